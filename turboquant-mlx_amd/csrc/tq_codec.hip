@@ -1,7 +1,7 @@
 // PolarQuant codec kernels for gfx950: fused encode, dequantise, query pre-rotation and the
 // per-row-butterfly QK scoring.  One wavefront owns one vector; the Walsh-Hadamard butterfly
 // and the norm reduction run on lane exchanges, never through LDS barriers.
-#include "tq_common.h"
+#include "tq_codec_stream.h"
 
 #include <math.h>
 #include <cmath>
@@ -11,15 +11,7 @@
 namespace {
 
 using namespace tqd;
-
-constexpr int kWavesPerBlock = 4;
-constexpr int kBlock = kWavesPerBlock * TQ_WAVE;
-
-struct Thresholds { float t[15]; };
-
-struct RowMap {
-  int64_t n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride;
-};
+using namespace tqc;
 
 // Optional row copies done by the wavefront that encodes a row (the append of a cache that keeps
 // float16 keys beside its packed values): key row `row` of k_src (dtype k_dtype) goes, converted to
@@ -136,290 +128,6 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(const T* __restrict__ x,
   }
 }
 
-// ---------------------------------------------------------------- encode, d = 128
-// The streaming encoder for the cache's own head dimension (every width; the notes below describe three bits,
-// the width-dependent parts are the level table and the word assembly at the end of a pass).  Four lanes own one vector, so a wavefront
-// encodes 16 vectors per pass: lane ls = lane % 4 of a vector holds the four 8-element chunks
-// c = ls + 4k (k = 0..3), element e = 32k + 8ls + j.  Each load instruction therefore reads 64
-// contiguous bytes per vector; butterfly stages 1, 2, 4, 32 and 64 and five of the seven levels of
-// the sum-of-squares tree stay inside a lane, and stages 8 and 16 are quad-permute lane exchanges
-// folded into the add.  Results are bit-identical to encode_kernel:
-//  * the sum of squares is added in the same stride-halving tree order;
-//  * x / n is computed as q = x*r, q += r * fma(-n, q, x) with r = 1/n correctly rounded, which
-//    yields the correctly rounded quotient (checked against IEEE division on 3e10 operand pairs
-//    with |x| <= n), at 3 operations per element instead of a full division;
-//  * the count of thresholds exceeded is g + (w > t[g]) where g is a guess that the host has verified to be
-//    the count or one less for every w: v = fma(w, alpha, beta + 2^20 + 32) lies in [2^20, 2^21), where
-//    floats are 1/8 apart, so bits 3..8 of v are 32 + floor(alpha*w + beta) (to within the rounding to
-//    1/8) and, masked, are the byte offset into a 64-entry LDS table of (t[g], g) pairs whose entries
-//    below / above the seven levels hold (+inf, 0) / (-inf, 6): no clamp, no float-to-int convert, no
-//    address shift.  A NaN norm forces all indices of the vector to 0 (as comparisons with NaN do).
-// Packed words leave through LDS so that a wavefront stores 208 contiguous words per pass.
-// Mixed-precision FMA on one half of a packed fp16 pair (HI = 0: low half, 1: high half), so that fp16
-// inputs need no separate widening instruction.  A product is taken as fma(a, b, -0): adding -0 changes
-// no value, not even the sign of a zero, so it rounds exactly like the float32 multiply of the widened
-// operands.
-template <int HI>
-__device__ __forceinline__ float mix_sq(uint32_t h2, float negzero) {           // widen(h) * widen(h)
-  float d;
-  if (HI) asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(h2), "v"(negzero));
-  else    asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[0,0,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(h2), "v"(negzero));
-  return d;
-}
-template <int HI>
-__device__ __forceinline__ float mix_mul(uint32_t h2, float b, float negzero) { // widen(h) * b
-  float d;
-  if (HI) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h2), "v"(b), "v"(negzero));
-  else    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h2), "v"(b), "v"(negzero));
-  return d;
-}
-template <int HI>
-__device__ __forceinline__ float mix_fma_addend(float a, float b, uint32_t h2) { // fma(a, b, widen(h))
-  float d;
-  if (HI) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(d) : "v"(a), "v"(b), "v"(h2));
-  else    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(d) : "v"(a), "v"(b), "v"(h2));
-  return d;
-}
-
-// The 8 * BITS bits that hold elements 8c .. 8c+7 (chunk c) of a packed d = 128 row: word and shifts.  Three-bit
-// rows hold ten fields per word, so a chunk may straddle two words (chunk 15 is all of word 12: taken as word
-// 11 >> 30, which is 0, | word 12); the other widths divide the word.
-template <int BITS>
-struct Chunk {
-  static constexpr int kPd = BITS == 3 ? 13 : 4 * BITS;       // words per row
-  static constexpr uint32_t kPairMask = (1u << (2 * BITS)) - 1u;
-  __device__ static __forceinline__ void pos(int c, int& w0, int& sh_lo, int& sh_hi) {
-    if (BITS == 3) {
-      w0 = (c == 15) ? 11 : (8 * c) / 10;
-      const int s0 = (c == 15) ? 10 : (8 * c) % 10;
-      sh_lo = 3 * s0;
-      sh_hi = 30 - 3 * s0;
-    } else {
-      constexpr int kPerWord = 4 / BITS;
-      w0 = c / kPerWord;
-      sh_lo = (c % kPerWord) * 8 * BITS;
-      sh_hi = 0;
-    }
-  }
-  __device__ static __forceinline__ uint32_t field(const uint32_t* at_w0, int sh_lo, int sh_hi) {
-    if (BITS == 3) return ((at_w0[0] >> sh_lo) | (at_w0[1] << sh_hi)) & 0xFFFFFFu;
-    if (BITS == 4) return at_w0[0];
-    return (at_w0[0] >> sh_lo) & ((1u << (8 * BITS)) - 1u);
-  }
-};
-
-constexpr int kEncVecs = 16;      // vectors per wavefront pass
-constexpr int kEncPasses = 4;     // passes per wavefront once there are rows enough to fill the chip
-
-// alpha and beta of the level guess; beta0 = beta without the 2^20 + 32 that places the guess in the mantissa
-struct EncodeGuess { float alpha, beta, beta0; };
-
-// BITS = 3: every threshold j sits in cell j of the guess (level_guess_search), and the table is written down
-// directly.  Other widths: any guess line under which no cell holds two thresholds (level_cells_search); cell
-// c = floor(alpha * w + beta0) then knows the count g of thresholds below its lower edge and the one threshold it
-// may hold (else +inf: nothing to compare with), both derived here from the thresholds themselves.
-template <typename T, int BITS = 3>
-__global__ __launch_bounds__(kBlock) void encode128x3_kernel(const T* __restrict__ x,
-                                                             const float* __restrict__ signs, Thresholds thr,
-                                                             EncodeGuess gs, uint32_t* __restrict__ packed,
-                                                             float* __restrict__ norms, RowMap rm, int passes) {
-  constexpr bool kHalfWidth = sizeof(T) == 2;
-  constexpr int NM = kHalfWidth ? 4 : 8;                       // sign masks per chunk
-  constexpr int NB = (1 << BITS) - 1;                          // thresholds
-  constexpr int kPd = Chunk<BITS>::kPd;
-  constexpr int kCells = BITS == 4 ? 128 : 64;                 // cells of the level guess (fifteen thresholds need finer ones)
-  __shared__ __align__(8) uint2 lvl_s[kCells];                 // (threshold bits, guess) by kCells / 2 + floor(alpha*w + beta0)
-  __shared__ __align__(16) float sg_s[128];
-  __shared__ uint32_t chunk_s[kWavesPerBlock][kEncVecs * 16 + 4];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ls = lane & 3, v = lane >> 2;
-  if (tid < kCells) {
-    const int gq = tid - kCells / 2;
-    if (BITS == 3) {
-      float t = gq < 0 ? INFINITY : -INFINITY;
-#pragma unroll
-      for (int i = 0; i < 7; ++i) t = (gq == i) ? thr.t[i] : t;
-      lvl_s[tid] = make_uint2(__float_as_uint(t), (uint32_t)(gq < 0 ? 0 : (gq > 6 ? 6 : gq)));
-    } else {
-      int g = 0;                                               // thresholds below the cell's lower edge
-#pragma unroll
-      for (int i = 0; i < NB; ++i) g += (__fmaf_rn(thr.t[i], gs.alpha, gs.beta0) < (float)gq) ? 1 : 0;
-      float t = INFINITY;                                      // threshold number g, if it lies inside the cell
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        t = (i == g && __fmaf_rn(thr.t[i], gs.alpha, gs.beta0) < (float)(gq + 1)) ? thr.t[i] : t;
-      lvl_s[tid] = make_uint2(__float_as_uint(t), (uint32_t)g);
-    }
-  }
-  if (tid < 128) sg_s[tid] = signs[tid];
-  __syncthreads();
-
-  // sign flips as xor masks on the raw input bits
-  uint32_t sm[4][NM];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float4 a = *reinterpret_cast<const float4*>(&sg_s[32 * k + 8 * ls]);
-    const float4 b = *reinterpret_cast<const float4*>(&sg_s[32 * k + 8 * ls + 4]);
-    const float sv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    if (kHalfWidth) {
-#pragma unroll
-      for (int jp = 0; jp < 4; ++jp)
-        sm[k][jp] = ((__float_as_uint(sv[2 * jp]) >> 16) & 0x8000u) | (__float_as_uint(sv[2 * jp + 1]) & 0x80000000u);
-    } else {
-#pragma unroll
-      for (int j = 0; j < NM; ++j) sm[k][j] = __float_as_uint(sv[j & 7]) & 0x80000000u;
-    }
-  }
-  // lanes 1 and 2 of a vector take their inputs negated (folded into the sign masks): butterfly_4lane_neg12
-  if (ls == 1 || ls == 2) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int j = 0; j < NM; ++j) sm[k][j] ^= kHalfWidth ? 0x80008000u : 0x80000000u;
-  }
-  const float m1 = (ls & 1) ? 1.0f : -1.0f, m2 = (ls & 2) ? 1.0f : -1.0f;
-  uint32_t* chunks = chunk_s[wave];
-
-  // first batch of 16 rows of this wavefront and its place in the (group, row) map
-  const uint32_t batch0 = ((uint32_t)blockIdx.x * kWavesPerBlock + wave) * (uint32_t)passes;
-  uint32_t row0 = batch0 * kEncVecs;
-  uint32_t grp = row0 / (uint32_t)rm.rows_per_group;
-  uint32_t rin = row0 - grp * (uint32_t)rm.rows_per_group;
-
-  // 16-bit inputs: the rows of the next pass are fetched while the current one is computed
-  uint4 nraw[4] = {};
-  if (kHalfWidth && row0 < (uint32_t)rm.n_rows) {
-    const T* xr = x + ((int64_t)row0 + v) * 128 + 8 * ls;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) nraw[k] = *reinterpret_cast<const uint4*>(xr + 32 * k);
-  }
-  for (int pass = 0; pass < passes; ++pass) {
-    if (row0 >= (uint32_t)rm.n_rows) break;                    // uniform over the wavefront
-    // ---- load, flip signs, widen (fp16: the packed pairs stay as they are and are widened inside the
-    // mixed-precision multiplies below)
-    constexpr bool kMix = __is_same(T, __half);
-    float xs[4][8];
-    uint32_t hw[4][4];
-    const T* xr = x + ((int64_t)row0 + v) * 128 + 8 * ls;
-    if (kHalfWidth) {
-      uint4 raw[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) raw[k] = nraw[k];
-      if (pass + 1 < passes && row0 + kEncVecs < (uint32_t)rm.n_rows) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nraw[k] = *reinterpret_cast<const uint4*>(xr + kEncVecs * 128 + 32 * k);
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t w[4] = {raw[k].x ^ sm[k][0], raw[k].y ^ sm[k][1], raw[k].z ^ sm[k][2], raw[k].w ^ sm[k][3]};
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-          hw[k][jp] = w[jp];
-          if (!kMix) {
-            xs[k][2 * jp] = __uint_as_float(w[jp] << 16);
-            xs[k][2 * jp + 1] = __uint_as_float(w[jp] & 0xFFFF0000u);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint4 a = *reinterpret_cast<const uint4*>(xr + 32 * k);
-        const uint4 b = *reinterpret_cast<const uint4*>(xr + 32 * k + 4);
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) xs[k][j] = __uint_as_float(w[j] ^ sm[k][j & (NM - 1)]);
-      }
-    }
-    const float negzero = -0.0f;
-    // ---- sum of squares: strides 64, 32 (k), 16, 8 (lanes), 4, 2, 1 (j)
-    float t8[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float sq[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (kMix) sq[k] = (j & 1) ? mix_sq<1>(hw[k][j >> 1], negzero) : mix_sq<0>(hw[k][j >> 1], negzero);
-        else sq[k] = xs[k][j] * xs[k][j];
-      }
-      t8[j] = (sq[0] + sq[2]) + (sq[1] + sq[3]);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t8[j] = t8[j] + quad_xor2(t8[j]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t8[j] = t8[j] + quad_xor1(t8[j]);
-    const float ss = ((t8[0] + t8[4]) + (t8[2] + t8[6])) + ((t8[1] + t8[5]) + (t8[3] + t8[7]));
-    const float nrm = sqrtf(ss);
-    const float safe = fmaxf(nrm, 1e-8f);
-    const float rinv = 1.0f / safe;
-    // a norm that overflowed to infinity: x / inf is 0 for every finite x, which q = x * 0 already is; the
-    // correction term must then not multiply infinity by that zero
-    const float nsafe = (safe == INFINITY) ? 0.0f : -safe;
-    // ---- unit vector
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (kMix) {
-          const uint32_t h2 = hw[k][j >> 1];
-          const float q0 = (j & 1) ? mix_mul<1>(h2, rinv, negzero) : mix_mul<0>(h2, rinv, negzero);
-          const float rem = (j & 1) ? mix_fma_addend<1>(nsafe, q0, h2) : mix_fma_addend<0>(nsafe, q0, h2);
-          xs[k][j] = __fmaf_rn(rem, rinv, q0);
-        } else {
-          const float q0 = xs[k][j] * rinv;
-          const float rem = __fmaf_rn(nsafe, q0, xs[k][j]);
-          xs[k][j] = __fmaf_rn(rem, rinv, q0);
-        }
-      }
-    butterfly_4lane_neg12(xs, m1, m2);
-    // ---- levels, 8 * BITS bits per chunk
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      uint32_t bits24 = 0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float w = xs[k][j];
-        const uint32_t off = __float_as_uint(__fmaf_rn(w, gs.alpha, gs.beta)) & (uint32_t)((kCells - 1) << 3);
-        const uint2 lv = *reinterpret_cast<const uint2*>(reinterpret_cast<const unsigned char*>(lvl_s) + off);
-        const uint32_t idx = lv.y + ((w > __uint_as_float(lv.x)) ? 1u : 0u);
-        bits24 |= idx << (BITS * j);
-      }
-      chunks[v * 16 + ls + 4 * k] = (nrm != nrm) ? 0u : bits24;
-    }
-    // ---- words.  Three bits: word wd of a row holds elements 10wd .. 10wd+9 = chunks (5wd)/4 and the next;
-    // four bits: a chunk is a word; two bits / one bit: two / four chunks make a word
-    uint32_t* prow = packed + ((int64_t)grp * rm.packed_group_stride + rin) * kPd;
-#pragma unroll
-    for (int it = 0; it < (kEncVecs * kPd + 63) / 64; ++it) {
-      const int id = it * 64 + lane;
-      if (id < kEncVecs * kPd) {
-        const int vv = id / kPd, wd = id - kPd * vv;
-        uint32_t word;
-        if (BITS == 3) {
-          const int a = (5 * wd) >> 2, sh = 3 * ((10 * wd) & 7);
-          const uint32_t lo = chunks[vv * 16 + a], hi = chunks[vv * 16 + a + 1];
-          word = ((lo >> sh) | (hi << (24 - sh))) & (wd == 12 ? 0xFFFFFFu : 0x3FFFFFFFu);
-        } else if (BITS == 4) {
-          word = chunks[vv * 16 + wd];
-        } else if (BITS == 2) {
-          word = chunks[vv * 16 + 2 * wd] | (chunks[vv * 16 + 2 * wd + 1] << 16);
-        } else {
-          word = chunks[vv * 16 + 4 * wd] | (chunks[vv * 16 + 4 * wd + 1] << 8) | (chunks[vv * 16 + 4 * wd + 2] << 16) |
-                 (chunks[vv * 16 + 4 * wd + 3] << 24);
-        }
-        prow[id] = word;
-      }
-    }
-    if (ls == 0) norms[(int64_t)grp * rm.norms_group_stride + rin + v] = nrm;
-    row0 += kEncVecs;
-    rin += kEncVecs;
-    if (rin >= (uint32_t)rm.rows_per_group) { rin = 0; ++grp; }
-  }
-}
-
 // ---------------------------------------------------------------- dequant
 template <int D, int BITS>
 __device__ __forceinline__ void load_centroid_values(const uint32_t* __restrict__ prow, const float* cb,
@@ -472,159 +180,6 @@ __global__ __launch_bounds__(kBlock) void dequant_kernel(const uint32_t* __restr
       int e = lane + 64 * i;
       if (e < D) store_from_float<TO>(orow + e, ((v[i] * s) * sg[i]) * nrm);
     }
-  }
-}
-
-// ---------------------------------------------------------------- dequant, d = 128
-// Same four-lanes-per-vector layout as encode128x3_kernel, every width.  The packed words of a pass (208 at
-// three bits) are read with coalesced loads into LDS; a lane cuts the 8 * BITS bits of each of its chunks out
-// of one or two words and looks centroid pairs up in a table of 4^BITS entries (c[a]*s, c[b]*s).  Arithmetic per
-// element, in this order, as in dequant_kernel: butterfly, * s, * sign, * norm, round to TO.
-template <typename TO, int BITS = 3>
-__global__ __launch_bounds__(kBlock) void dequant128x3_kernel(const uint32_t* __restrict__ packed,
-                                                              const float* __restrict__ norms, Codebook cbk,
-                                                              const float* __restrict__ signs, float s,
-                                                              TO* __restrict__ out, RowMap rm, int passes) {
-  using CK = Chunk<BITS>;
-  constexpr int kPd = CK::kPd;
-  constexpr int kPairs = 1 << (2 * BITS);                      // entries of the centroid-pair table
-  constexpr int kWordLoads = (kEncVecs * kPd + 63) / 64;       // wave-wide loads of a pass's packed words
-  __shared__ __align__(16) float sg_s[128];
-  // centroid pairs, and after them the same pairs negated: lanes 1 and 2 of a vector read those (butterfly_4lane_neg12)
-  __shared__ __align__(8) float2 pair_s[2 * kPairs];
-  __shared__ uint32_t words_s[kWavesPerBlock][kEncVecs * kPd + 3];
-  // Outputs leave through LDS: 16 rows of 256 (16-bit) or 512 (float32) bytes at a padded pitch (conflict-free
-  // 16-byte writes per lane and reads per row segment), so that every store instruction writes 1 KB of
-  // contiguous memory
-  constexpr int kPitch = sizeof(TO) == 2 ? 320 : 528;          // row of 256 / 512 bytes plus padding
-  __shared__ __align__(16) unsigned char orow_s[kWavesPerBlock][kEncVecs * kPitch];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ls = lane & 3, v = lane >> 2;
-  if (tid < kPairs) {                                          // kBlock = 256 threads cover the largest table
-    float clo = 0.0f, chi = 0.0f;
-#pragma unroll
-    for (int i = 0; i < (1 << BITS); ++i) {
-      clo = ((tid & ((1 << BITS) - 1)) == i) ? cbk.c[i] : clo;
-      chi = ((tid >> BITS) == i) ? cbk.c[i] : chi;
-    }
-    pair_s[tid] = make_float2(clo * s, chi * s);
-    pair_s[kPairs + tid] = make_float2(-(clo * s), -(chi * s));
-  }
-  if (tid >= 128) sg_s[tid - 128] = signs[tid - 128];
-  __syncthreads();
-
-  uint32_t sm[4][8];                                           // sign bit of each element of this lane
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float4 a = *reinterpret_cast<const float4*>(&sg_s[32 * k + 8 * ls]);
-    const float4 b = *reinterpret_cast<const float4*>(&sg_s[32 * k + 8 * ls + 4]);
-    const float sv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sm[k][j] = __float_as_uint(sv[j]) & 0x80000000u;
-  }
-  const float m1 = (ls & 1) ? 1.0f : -1.0f, m2 = (ls & 2) ? 1.0f : -1.0f;
-  const float2* my_pairs = pair_s + ((ls == 1 || ls == 2) ? kPairs : 0);
-  uint32_t* words = words_s[wave];
-  // words / shifts of the bits of chunk c = ls + 4k (elements 8c .. 8c+7)
-  int cw[4], csl[4], csh[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) CK::pos(ls + 4 * k, cw[k], csl[k], csh[k]);
-
-  const uint32_t batch0 = ((uint32_t)blockIdx.x * kWavesPerBlock + wave) * (uint32_t)passes;
-  uint32_t row0 = batch0 * kEncVecs;
-  uint32_t grp = row0 / (uint32_t)rm.rows_per_group;
-  uint32_t rin = row0 - grp * (uint32_t)rm.rows_per_group;
-
-  // the packed words and the norm of the next pass are fetched while the current one is computed
-  uint32_t pw[kWordLoads];
-  float pn = 0.0f;
-  auto fetch = [&](uint32_t g_, uint32_t r_) {
-    const uint32_t* prow = packed + ((int64_t)g_ * rm.packed_group_stride + r_) * kPd;
-    pn = norms[(int64_t)g_ * rm.norms_group_stride + r_ + v];
-#pragma unroll
-    for (int it = 0; it < kWordLoads; ++it) {
-      const int id = it * 64 + lane;
-      pw[it] = (id < kEncVecs * kPd) ? prow[id] : 0u;
-    }
-  };
-  if (row0 < (uint32_t)rm.n_rows) fetch(grp, rin);
-  for (int pass = 0; pass < passes; ++pass) {
-    if (row0 >= (uint32_t)rm.n_rows) break;                    // uniform over the wavefront
-    const float nrm = pn;
-#pragma unroll
-    for (int it = 0; it < kWordLoads; ++it) {
-      const int id = it * 64 + lane;
-      if (id < kEncVecs * kPd) words[id] = pw[it];
-    }
-    uint32_t nrin = rin + kEncVecs, ngrp = grp;
-    if (nrin >= (uint32_t)rm.rows_per_group) { nrin = 0; ++ngrp; }
-    if (pass + 1 < passes && row0 + kEncVecs < (uint32_t)rm.n_rows) fetch(ngrp, nrin);
-    float xs[4][8];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t f = CK::field(words + v * kPd + cw[k], csl[k], csh[k]);
-#pragma unroll
-      for (int jp = 0; jp < 4; ++jp) {
-        const float2 c2 = my_pairs[(f >> (2 * BITS * jp)) & CK::kPairMask];
-        xs[k][2 * jp] = c2.x;
-        xs[k][2 * jp + 1] = c2.y;
-      }
-    }
-    butterfly_4lane_neg12(xs, m1, m2);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float r[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float t = (xs[k][j] * s) * nrm;
-        asm volatile("" : "+v"(t));                            // keep the multiply out of the narrowing convert
-        r[j] = t;
-      }
-      if (sizeof(TO) == 4) {
-        uint4 a, b;
-        a.x = __float_as_uint(r[0]) ^ sm[k][0]; a.y = __float_as_uint(r[1]) ^ sm[k][1];
-        a.z = __float_as_uint(r[2]) ^ sm[k][2]; a.w = __float_as_uint(r[3]) ^ sm[k][3];
-        b.x = __float_as_uint(r[4]) ^ sm[k][4]; b.y = __float_as_uint(r[5]) ^ sm[k][5];
-        b.z = __float_as_uint(r[6]) ^ sm[k][6]; b.w = __float_as_uint(r[7]) ^ sm[k][7];
-        *reinterpret_cast<uint4*>(&orow_s[wave][v * kPitch + 128 * k + 32 * ls]) = a;
-        *reinterpret_cast<uint4*>(&orow_s[wave][v * kPitch + 128 * k + 32 * ls + 16]) = b;
-      } else {
-        uint32_t w[4];
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-          uint32_t lo, hi;
-          if (__is_same(TO, __half)) {
-            lo = __half_as_ushort(__float2half_rn(r[2 * jp]));
-            hi = __half_as_ushort(__float2half_rn(r[2 * jp + 1]));
-          } else {
-            lo = __bfloat16_as_ushort(__float2bfloat16(r[2 * jp]));
-            hi = __bfloat16_as_ushort(__float2bfloat16(r[2 * jp + 1]));
-          }
-          w[jp] = (lo | (hi << 16)) ^ ((sm[k][2 * jp] >> 16) | sm[k][2 * jp + 1]);
-        }
-        *reinterpret_cast<uint4*>(&orow_s[wave][v * kPitch + 64 * k + 16 * ls]) = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    }
-    {
-      unsigned char* oblock = reinterpret_cast<unsigned char*>(out + ((int64_t)grp * rm.out_group_stride + rin) * 128);
-      constexpr int kPiecesPerRow = 8 * (int)sizeof(TO);           // 16-byte pieces in a row: 16 or 32
-#pragma unroll
-      for (int i = 0; i < (int)(2 * sizeof(TO)); ++i) {            // 4 or 8 KB per pass
-        const int piece = i * 64 + lane;
-        // a streaming store (the "nt" hint): the rows are not read again by this kernel and a pass writes more than the
-        // caches hold -- 115 -> 99 us per 1 M float32 rows, 75 -> 66 us for fp16
-        typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(
-            *reinterpret_cast<const piece_t*>(&orow_s[wave][(piece / kPiecesPerRow) * kPitch + (piece % kPiecesPerRow) * 16]),
-            reinterpret_cast<piece_t*>(oblock + piece * 16));
-      }
-    }
-    row0 += kEncVecs;
-    rin = nrin;
-    grp = ngrp;
   }
 }
 
@@ -836,12 +391,43 @@ bool level_guess_search(const float* t, int nb, EncodeGuess& out) {
   return true;
 }
 
-// Passes per wavefront of the four-lanes-per-vector kernels: several, to spread the set-up cost,
-// once every CU has a few workgroups anyway.
-int fast_passes(int64_t n_rows) {
-  const int64_t rows_per_block_pass = (int64_t)kEncVecs * kWavesPerBlock;
-  return (n_rows >= rows_per_block_pass * kEncPasses * 256 * 4) ? kEncPasses : 1;
+// Rows from which the streaming kernels are ahead of one wavefront per vector (encode_kernel, dequant_kernel): below,
+// the chip is not full either way and the chain of a single vector spread over 64 lanes is the shorter one.  Measured on
+// both sides of each line (us, streaming / one wavefront per vector; encode, then dequant to fp16):
+//   d =  64:  4 097 rows 4.7 / 4.0 and 4.0 / 3.1,  16 385 rows 4.9 / 9.9 and 4.2 / 4.8,  262 147 rows 14 / 69 and 9.1 / 30
+//   d = 128:  4 097 rows 4.7 / 4.3 and 4.0 / 3.4,  16 385 rows 5.4 / 11.0 and 4.5 / 5.7,  80 056 rows 9.8 / 26 and 7.7 / 14
+//   d = 256:  2 049 rows 4.7 / 4.5 and 4.2 / 3.2,   8 193 rows 5.3 / 7.3 and 4.6 / 5.1,  262 147 rows 42 / 134 and 30 / 54
+int64_t stream_min_rows(int dim, bool encode) {
+  if (dim == 64) return encode ? 6144 : 12288;
+  if (dim == 128) return encode ? 5120 : 8192;
+  return encode ? 3072 : 6144;
 }
+
+RowMap row_map(int64_t n_rows, int64_t rows_per_group, int64_t packed_group_stride, int64_t norms_group_stride,
+               int64_t out_group_stride) {
+  RowMap rm{n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride, 0, 0};
+  // row / d = (row * m) >> (31 + s) with s = ceil(log2 d), m = ceil(2^(31 + s) / d), exact for row < 2^31: the error
+  // row * (m d - 2^(31 + s)) stays below 2^31 * 2^s; m < 2^32 because d > 2^(s - 1)
+  const uint64_t d = (uint64_t)rows_per_group;
+  if (d > 1 && d < ((uint64_t)1 << 31)) {
+    int s = 1;
+    while (((uint64_t)1 << s) < d) ++s;
+    const unsigned __int128 top = (unsigned __int128)1 << (31 + s);
+    rm.group_mul = (uint32_t)((top + d - 1) / d);
+    rm.group_shift = (uint32_t)(s - 1);
+  }
+  return rm;
+}
+
+// The streaming kernels index rows with 32 bits: rows of the call, and of the storage they lie in.
+bool rows_fit_32_bits(const RowMap& rm, int64_t n_groups) {
+  const int64_t most = (int64_t)1 << 31;
+  return rm.n_rows < most && n_groups * rm.packed_group_stride + rm.rows_per_group < most &&
+         n_groups * rm.out_group_stride + rm.rows_per_group < most;
+}
+
+// d = 128, groups of a multiple of 16 rows: the form without per-row destinations, at any size
+bool whole_batches(int dim, const RowMap& rm) { return dim == 128 && rm.rows_per_group % VecLanes<128>::kVecs == 0; }
 
 int grid_for_rows(int64_t rows) {
   int64_t blocks = (rows + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -984,22 +570,18 @@ extern "C" int tq_encode(const void* x, int x_dtype, const float* signs, const f
   for (int i = 0; i < 15; ++i) thr.t[i] = INFINITY;
   for (int i = 0; i < nb; ++i)
     thr.t[i] = (variant == TQ_ENCODE_MLX) ? double_rounding_threshold(boundaries[i], s) : boundaries[i];
-  RowMap rm{n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0};
+  const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
   hipStream_t stream = (hipStream_t)stream_;
   const int grid = grid_for_rows(n_rows);
   EncodeGuess gs{};
-  if (dim == 128 && rows_per_group % kEncVecs == 0 && n_rows < (int64_t)1 << 31 &&
-      tq::aligned(x, 16) && level_guess(thr.t, nb, gs)) {
-    const int passes = fast_passes(n_rows);
-    const int64_t rows_per_block = (int64_t)kEncVecs * passes * kWavesPerBlock;
-    const int fgrid = (int)((n_rows + rows_per_block - 1) / rows_per_block);
-#define LAUNCH_ENC128(T)                                                                                          \
-    TQ_DISPATCH_BITS(bits, (encode128x3_kernel<T, B_><<<fgrid, kBlock, 0, stream>>>((const T*)x, signs, thr, gs, packed, \
-                                                                                   norms, rm, passes)))
-    if (x_dtype == TQ_F32) { LAUNCH_ENC128(float); }
-    else if (x_dtype == TQ_F16) { LAUNCH_ENC128(__half); }
-    else { LAUNCH_ENC128(__hip_bfloat16); }
-#undef LAUNCH_ENC128
+  const bool whole = whole_batches(dim, rm);
+  if (dim >= 64 && (whole || n_rows >= stream_min_rows(dim, true)) && n_rows < (int64_t)1 << 31 &&
+      (whole || rows_fit_32_bits(rm, n_groups)) && tq::aligned(x, 16) && level_guess(thr.t, nb, gs)) {
+    const EncodeCall c{x, x_dtype, signs, thr, gs, packed, norms, rm, bits, stream};
+    if (whole) launch_encode_rows<128, false>(c);
+    else if (dim == 64) launch_encode_rows<64, true>(c);
+    else if (dim == 128) launch_encode_rows<128, true>(c);
+    else launch_encode_rows<256, true>(c);
     TQ_CHECK_LAUNCH("tq_encode launch");
     return TQ_OK;
   }
@@ -1041,7 +623,7 @@ int vonly_append(const void* k_new, int k_dtype, const void* v_new, int v_dtype,
   for (int i = 0; i < 15; ++i) thr.t[i] = INFINITY;
   for (int i = 0; i < nb; ++i)
     thr.t[i] = (variant == TQ_ENCODE_MLX) ? double_rounding_threshold(boundaries[i], s) : boundaries[i];
-  RowMap rm{n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0};
+  const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
   if (pos_dev && (!tq::aligned(pos_dev, 8) || pos_cap < 1))
     return tq::fail(TQ_ERR_ARG, "tq_vonly_append_at: position_dev must be 8-byte aligned and t_alloc >= 1");
   RowCopy rc{k_new, (__half*)k_f16, v_raw, k_group_stride, v_raw_group_stride, k_dtype, pos_dev, pos_cap};
@@ -1099,21 +681,18 @@ extern "C" int tq_dequant(const uint32_t* packed, const float* norms, const floa
   Codebook cb;
   for (int i = 0; i < 16; ++i) cb.c[i] = i < (1 << bits) ? centroids[i] : 0.0f;
   const float s = (float)(1.0 / sqrt((double)dim));
-  RowMap rm{n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride};
+  const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride);
   hipStream_t stream = (hipStream_t)stream_;
   const int grid = grid_for_rows(n_rows);
-  if (dim == 128 && rows_per_group % kEncVecs == 0 && n_rows < (int64_t)1 << 31 &&
-      tq::aligned(out, 16) && (out_group_stride * 128 * (int64_t)tq::dtype_size(out_dtype)) % 16 == 0) {
-    const int passes = fast_passes(n_rows);
-    const int64_t rows_per_block = (int64_t)kEncVecs * passes * kWavesPerBlock;
-    const int fgrid = (int)((n_rows + rows_per_block - 1) / rows_per_block);
-#define LAUNCH_DEQ128(TO)                                                                                       \
-    TQ_DISPATCH_BITS(bits, (dequant128x3_kernel<TO, B_><<<fgrid, kBlock, 0, stream>>>(packed, norms, cb, signs, s, \
-                                                                                     (TO*)out, rm, passes)))
-    if (out_dtype == TQ_F32) { LAUNCH_DEQ128(float); }
-    else if (out_dtype == TQ_F16) { LAUNCH_DEQ128(__half); }
-    else { LAUNCH_DEQ128(__hip_bfloat16); }
-#undef LAUNCH_DEQ128
+  const bool whole = whole_batches(dim, rm);
+  if (dim >= 64 && (whole || n_rows >= stream_min_rows(dim, false)) && n_rows < (int64_t)1 << 31 &&
+      (whole || rows_fit_32_bits(rm, n_groups)) && tq::aligned(out, 16) &&
+      (out_group_stride * dim * (int64_t)tq::dtype_size(out_dtype)) % 16 == 0) {
+    const DequantCall c{packed, norms, cb, signs, s, out, out_dtype, rm, bits, stream};
+    if (whole) launch_dequant_rows<128, false>(c);
+    else if (dim == 64) launch_dequant_rows<64, true>(c);
+    else if (dim == 128) launch_dequant_rows<128, true>(c);
+    else launch_dequant_rows<256, true>(c);
     TQ_CHECK_LAUNCH("tq_dequant launch");
     return TQ_OK;
   }

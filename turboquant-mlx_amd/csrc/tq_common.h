@@ -213,6 +213,10 @@ __device__ __forceinline__ float quad_xor2(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));   // lanes 2,3,0,1
 }
 
+__device__ __forceinline__ float oct_mirror(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));  // lanes 7,6,...,0 of eight
+}
+
 // Raw butterfly of a 128-vector spread over four lanes (element e = 32k + 8*ls + j in xs[k][j] of
 // lane ls), stages in the order of strides 1, 2, ..., 64.  flip1 / flip2 are 0x80000000 in the
 // lanes whose ls has bit 0 / bit 1 set (the upper element of a pair computes partner - own).
@@ -252,15 +256,30 @@ __device__ __forceinline__ void butterfly_4lane(float (&xs)[4][8], uint32_t flip
   }
 }
 
-// butterfly_4lane for inputs that the lanes with ls = 1 and ls = 2 hold NEGATED -- a sign the caller folds into the
-// sign flip or the table it applies to its inputs anyway.  Each of the two lane-exchange stages is then ONE fused
-// multiply-add, own + partner * (+-1), instead of a sign flip and an add: with the value a of the lower lane and b
-// of the upper lane of a pair, (own, partner, factor) = (a, -b, -1) gives a + b and (-b, a, +1) gives a - b; in the
-// pairs whose results the next stage wants negated, (-a, b, -1) gives -(a + b) and (b, -a, +1) gives -(a - b).  A
-// product with +-1 is exact, so every output is the same single rounding of the same sum as in butterfly_4lane:
-// identical bits (the sign of a zero aside, which no consumer looks at).  m1 = (ls & 1) ? 1 : -1,
-// m2 = (ls & 2) ? 1 : -1.  Outputs are not negated in any lane.
-__device__ __forceinline__ void butterfly_4lane_neg12(float (&xs)[4][8], float m1, float m2) {
+// Layout of the streaming codec for d = 64, 128 and 256: kLanes = d / 32 lanes own a vector, lane with logical number
+// ls holds xs[k][j] = element 8 kLanes k + 8 ls + j.  Of eight lanes (d = 256) the upper four are numbered in reverse
+// (physical 4, 5, 6, 7 = logical 7, 6, 5, 4): then xor 1, xor 2 and the mirror of eight lanes (a DPP pattern, where
+// xor 4 is none) each flip exactly one bit of the logical number.
+template <int D>
+struct VecLanes {
+  static constexpr int kLanes = D / 32;
+  static constexpr int kVecs = 64 / kLanes;                    // vectors per wavefront pass
+  __device__ static __forceinline__ int logical(int lane) {
+    const int p = lane & (kLanes - 1);
+    return (kLanes == 8 && (p & 4)) ? (p ^ 3) : p;
+  }
+};
+
+// Raw butterfly of vectors in that layout, stages in the order of strides 1, 2, ..., d / 2, for inputs that the lanes
+// with an odd number of bits set in ls hold NEGATED -- a sign the caller folds into the sign flip or the table it
+// applies to its inputs anyway.  Each lane-exchange stage is then ONE fused multiply-add, own + partner * (+-1),
+// instead of a sign flip and an add: with the value a of the lower lane and b of the upper lane of a pair,
+// (own, partner, factor) = (a, -b, -1) gives a + b and (-b, a, +1) gives a - b; in the pairs whose results a later
+// stage wants negated, (-a, b, -1) gives -(a + b) and (b, -a, +1) gives -(a - b).  A product with +-1 is exact, so
+// every output is the same single rounding of the same sum as in raw_butterfly: identical bits (the sign of a zero
+// aside, which no consumer looks at).  m[b] = (ls & (1 << b)) ? 1 : -1.  Outputs are not negated in any lane.
+template <int LANES>
+__device__ __forceinline__ void butterfly_lanes_neg(float (&xs)[4][8], const float (&m)[3]) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
 #pragma unroll
@@ -274,25 +293,31 @@ __device__ __forceinline__ void butterfly_4lane_neg12(float (&xs)[4][8], float m
         }
   }
   // v_fmac_f32 with the partner lane's value as its DPP operand, eight registers per statement (the compiler does
-  // not form this instruction from a quad permute and a fused multiply-add: it leaves the permute a move of its
+  // not form this instruction from a lane permute and a fused multiply-add: it leaves the permute a move of its
   // own).  A DPP read of a register that a vector instruction has just written needs two wait states, which the
   // compiler does not count across an asm statement: each statement starts with them.
 #define TQ_FMAC8(PERM, M, R)                                                                                        \
   asm("s_nop 1\n\t"                                                                                                \
-      "v_fmac_f32_dpp %0, %0, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %1, %1, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %2, %2, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %3, %3, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %4, %4, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %5, %5, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %6, %6, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                 \
-      "v_fmac_f32_dpp %7, %7, %8 quad_perm:" PERM " row_mask:0xf bank_mask:0xf"                                      \
+      "v_fmac_f32_dpp %0, %0, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %1, %1, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %2, %2, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %3, %3, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %4, %4, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %5, %5, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %6, %6, %8 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
+      "v_fmac_f32_dpp %7, %7, %8 " PERM " row_mask:0xf bank_mask:0xf"                                                \
       : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3]), "+v"(R[4]), "+v"(R[5]), "+v"(R[6]), "+v"(R[7])              \
       : "v"(M))
 #pragma unroll
-  for (int k = 0; k < 4; ++k) TQ_FMAC8("[1,0,3,2]", m1, xs[k]);
+  for (int k = 0; k < 4; ++k) TQ_FMAC8("quad_perm:[1,0,3,2]", m[0], xs[k]);
+  if constexpr (LANES >= 4) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) TQ_FMAC8("[2,3,0,1]", m2, xs[k]);
+    for (int k = 0; k < 4; ++k) TQ_FMAC8("quad_perm:[2,3,0,1]", m[1], xs[k]);
+  }
+  if constexpr (LANES >= 8) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) TQ_FMAC8("row_half_mirror", m[2], xs[k]);
+  }
 #undef TQ_FMAC8
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -321,6 +346,14 @@ __device__ __forceinline__ float sum_over_rows(float v) {
   v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Between LDS stores of some lanes and loads of others of the SAME wavefront.  The hardware executes a wavefront's LDS
+// operations in order and needs nothing; the compiler, to which the lanes are threads, may otherwise forward or move a
+// load over a store that it takes to be another thread's.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
 }
 
 __device__ __forceinline__ float wave_max(float v) {
