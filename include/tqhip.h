@@ -101,6 +101,18 @@ int tq_encode(const void* x, int x_dtype, const float* signs, const float* bound
               int dim, int bits, int variant, tq_stream_t stream);
 
 /*
+ * tq_encode for the key rows and the value rows of one insert in ONE launch: one data type, row count, width and set
+ * of boundaries, each side with its own signs and destination (strides in rows, common to both).  Same bits as two
+ * tq_encode calls.  Stands for the two encodes of TurboQuantKVCache.update_and_fetch (reference
+ * turboquant_mlx/cache.py:140-160).
+ */
+int tq_encode_kv(const void* k, const float* k_signs, uint32_t* k_packed, float* k_norms,
+                 const void* v, const float* v_signs, uint32_t* v_packed, float* v_norms,
+                 int x_dtype, const float* boundaries, int64_t n_groups, int64_t rows_per_group,
+                 int64_t packed_group_stride, int64_t norms_group_stride,
+                 int dim, int bits, int variant, tq_stream_t stream);
+
+/*
  * Append new tokens to a cache that keeps float16 keys beside PolarQuant values, in ONE launch:
  * every new value row is encoded exactly as tq_encode does (bit-identical words and norms), and
  * the wavefront that encodes row (g, i) also stores the key row, converted to float16 with
@@ -134,6 +146,40 @@ int tq_dequant(const uint32_t* packed, const float* norms, const float* centroid
                int64_t n_groups, int64_t rows_per_group,
                int64_t packed_group_stride, int64_t norms_group_stride, int64_t out_group_stride,
                int dim, int bits, tq_stream_t stream);
+
+/*
+ * tq_dequant for the keys and the values of the same rows in ONE launch (one width, codebook, output type; strides in
+ * rows, common to both).  Same values as two tq_dequant calls.  Stands for the dequantised fetch of
+ * TurboQuantKVCache.update_and_fetch (reference turboquant_mlx/cache.py:171-218).
+ */
+int tq_dequant_kv(const uint32_t* k_packed, const float* k_norms, const float* k_signs, void* k_out,
+                  const uint32_t* v_packed, const float* v_norms, const float* v_signs, void* v_out,
+                  const float* centroids, int out_dtype, int64_t n_groups, int64_t rows_per_group,
+                  int64_t packed_group_stride, int64_t norms_group_stride, int64_t out_group_stride,
+                  int dim, int bits, tq_stream_t stream);
+
+/*
+ * Sets up fresh storage in ONE launch: for every segment and every group g < n_groups, the first copy_bytes of the
+ * group come from src + g * src_group_stride and bytes zero_from .. zero_to - 1 become zero; the rest of the group is
+ * left alone (its rows are about to be written).  All sizes, strides and pointers are multiples of 4 bytes (16-byte
+ * accesses where all are multiples of 16).  Stands for the zero-filled allocation and the prefix copy of a growing
+ * cache (reference turboquant_mlx/cache.py:100-123).
+ */
+#define TQ_FILL_MAX_SEGMENTS 8
+typedef struct tq_fill_segment {
+  void* dst;
+  const void* src;                       /* NULL when copy_bytes is 0 */
+  int64_t dst_group_stride, src_group_stride, copy_bytes, zero_from, zero_to, n_groups;
+} tq_fill_segment;
+int tq_fill_rows(const tq_fill_segment* segments, int n_segments, tq_stream_t stream);
+
+/*
+ * The +-1 diagonals of up to four seeds: signs[i * dim + e] for seeds[i], the native generator of
+ * random_diagonal_sign (splitmix64; see the Python package) evaluated on the GPU without a host-to-device copy.
+ * Stands for random_diagonal_sign (reference turboquant_mlx/rotation.py:37-49), whose MLX stream it is NOT.
+ */
+#define TQ_SIGNS_MAX_SEEDS 4
+int tq_random_signs(const uint64_t* seeds /* HOST */, int n_seeds, int dim, float* signs, tq_stream_t stream);
 
 /*
  * q_rot[h] = butterfly(q[h] * signs), no 1/sqrt(dim).

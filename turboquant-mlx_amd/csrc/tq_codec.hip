@@ -36,10 +36,11 @@ struct RowCopy {
 // flip, raw butterfly, count of thresholds exceeded (strict >), pack.  `thr` holds the decision
 // thresholds in the domain of the raw butterfly output (see encode_thresholds below).
 template <int D, int BITS, typename T>
-__global__ __launch_bounds__(kBlock) void encode_kernel(const T* __restrict__ x,
-                                                        const float* __restrict__ signs,
-                                                        Thresholds thr, uint32_t* __restrict__ packed,
-                                                        float* __restrict__ norms, RowMap rm, RowCopy rc) {
+__global__ __launch_bounds__(kBlock) void encode_kernel(EncodeSides sides, Thresholds thr, RowMap rm, RowCopy rc) {
+  const T* __restrict__ x = (const T*)sides.s[blockIdx.y].x;
+  const float* __restrict__ signs = sides.s[blockIdx.y].signs;
+  uint32_t* __restrict__ packed = sides.s[blockIdx.y].packed;
+  float* __restrict__ norms = sides.s[blockIdx.y].norms;
   constexpr int EPL = Lay<D>::EPL;
   constexpr int VPW = Pk<BITS>::VPW;
   constexpr int PDIM = Pk<BITS>::pdim(D);
@@ -148,10 +149,11 @@ __device__ __forceinline__ void load_centroid_values(const uint32_t* __restrict_
 }
 
 template <int D, int BITS, typename TO>
-__global__ __launch_bounds__(kBlock) void dequant_kernel(const uint32_t* __restrict__ packed,
-                                                         const float* __restrict__ norms, Codebook cbk,
-                                                         const float* __restrict__ signs, float s,
-                                                         TO* __restrict__ out, RowMap rm) {
+__global__ __launch_bounds__(kBlock) void dequant_kernel(DequantSides sides, Codebook cbk, float s, RowMap rm) {
+  const uint32_t* __restrict__ packed = sides.s[blockIdx.y].packed;
+  const float* __restrict__ norms = sides.s[blockIdx.y].norms;
+  const float* __restrict__ signs = sides.s[blockIdx.y].signs;
+  TO* __restrict__ out = (TO*)sides.s[blockIdx.y].out;
   constexpr int EPL = Lay<D>::EPL;
   constexpr int PDIM = Pk<BITS>::pdim(D);
   __shared__ float cb[16];
@@ -327,36 +329,46 @@ bool level_cells_search(const float* t, int nb, EncodeGuess& out) {
   return true;
 }
 
-// Search results are kept for the last few threshold sets seen (a process that alternates widths or threshold
-// rules between calls -- caches of different bits, keys and values under different rules -- would otherwise repeat
-// a search of several milliseconds at every switch).  The lock covers the table only, not the search: two threads
-// that miss on the same set both search and store the same result.
-bool level_guess(const float* t, int nb, EncodeGuess& out) {
+// Thresholds and level guess of the encoder for the last few (boundaries, dim, variant) seen, by value: a process that
+// alternates widths or threshold rules between calls -- caches of different bits, keys and values under different
+// rules -- would otherwise repeat a search of several milliseconds at every switch, and every call the bisections of
+// double_rounding_threshold (2 us at three bits).  The lock covers the table only, not the search: two threads that
+// miss on the same set both search and store the same result.
+struct EncodePlan {
+  Thresholds thr;
+  EncodeGuess gs;
+  bool has_guess;
+};
+
+EncodePlan encode_plan(const float* boundaries, int dim, int bits, int variant) {
   constexpr int kSlots = 8;
-  struct Slot { float t[15]; int nb; bool ok; EncodeGuess g; };
+  struct Slot { float b[15]; int nb, dim, variant; EncodePlan p; };
   static std::mutex mu;
   static Slot slots[kSlots];
   static int n_used = 0, next = 0;
+  const int nb = (1 << bits) - 1;
   {
     std::lock_guard<std::mutex> lock(mu);
     for (int i = 0; i < n_used; ++i)
-      if (slots[i].nb == nb && memcmp(slots[i].t, t, nb * sizeof(float)) == 0) {
-        out = slots[i].g;
-        return slots[i].ok;
-      }
+      if (slots[i].nb == nb && slots[i].dim == dim && slots[i].variant == variant &&
+          memcmp(slots[i].b, boundaries, nb * sizeof(float)) == 0)
+        return slots[i].p;
   }
   Slot s{};
   s.nb = nb;
-  memcpy(s.t, t, nb * sizeof(float));
-  s.ok = (nb == 7) ? level_guess_search(t, nb, s.g) : level_cells_search(t, nb, s.g);
+  s.dim = dim;
+  s.variant = variant;
+  memcpy(s.b, boundaries, nb * sizeof(float));
+  for (int i = 0; i < 15; ++i) s.p.thr.t[i] = INFINITY;
+  tq::encode_thresholds(boundaries, dim, bits, variant, s.p.thr.t);
+  s.p.has_guess = (nb == 7) ? level_guess_search(s.p.thr.t, nb, s.p.gs) : level_cells_search(s.p.thr.t, nb, s.p.gs);
   {
     std::lock_guard<std::mutex> lock(mu);
     slots[next] = s;
     next = (next + 1) % kSlots;
     if (n_used < kSlots) ++n_used;
   }
-  out = s.g;
-  return s.ok;
+  return s.p;
 }
 
 bool level_guess_search(const float* t, int nb, EncodeGuess& out) {
@@ -508,9 +520,7 @@ int encode_pair(const void* k_new, int k_dtype, const float* k_signs, uint32_t* 
                 const void* v_new, int v_dtype, const float* v_signs, uint32_t* v_packed, float* v_norms,
                 const float* boundaries, int bits, int64_t n_rows, int64_t group_stride, int variant, tq_stream_t stream_,
                 const int64_t* pos_dev) {
-  Thresholds thr;
-  for (int i = 0; i < 15; ++i) thr.t[i] = INFINITY;
-  encode_thresholds(boundaries, 128, bits, variant, thr.t);
+  const Thresholds thr = encode_plan(boundaries, 128, bits, variant).thr;
   PairSide k{k_new, k_signs, k_packed, k_norms, k_dtype}, v{v_new, v_signs, v_packed, v_norms, v_dtype};
   const int grid = (int)((2 * n_rows + kWavesPerBlock - 1) / kWavesPerBlock);
   TQ_DISPATCH_BITS(bits, (encode_pair_kernel<B_><<<grid, kBlock, 0, (hipStream_t)stream_>>>(k, v, thr, n_rows, group_stride, pos_dev)));
@@ -549,51 +559,112 @@ extern "C" const char* tq_status_string(int status) {
   return status <= TQ_ERR_HIP ? "hip error" : "unknown";
 }
 
-extern "C" int tq_encode(const void* x, int x_dtype, const float* signs, const float* boundaries,
-                         uint32_t* packed, float* norms, int64_t n_groups, int64_t rows_per_group,
-                         int64_t packed_group_stride, int64_t norms_group_stride, int dim, int bits,
-                         int variant, tq_stream_t stream_) {
+namespace {
+// The rows of one tensor, or of the keys and the values (n_sides = 2): arguments checked here, `who` names the entry.
+int encode_sides(const char* who, const EncodeSides& sides, int n_sides, int x_dtype, const float* boundaries, int64_t n_groups,
+                 int64_t rows_per_group, int64_t packed_group_stride, int64_t norms_group_stride, int dim, int bits,
+                 int variant, hipStream_t stream) {
   if (int rc = tq::check_dim_bits(dim, bits)) return rc;
-  if (tq::check_dtype(x_dtype)) return tq::fail(TQ_ERR_DTYPE, "tq_encode: unknown x_dtype %d", x_dtype);
+  if (tq::check_dtype(x_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown x_dtype %d", who, x_dtype);
   if (variant != TQ_ENCODE_MLX && variant != TQ_ENCODE_METAL)
-    return tq::fail(TQ_ERR_ARG, "tq_encode: unknown variant %d", variant);
-  if (n_groups < 0 || rows_per_group < 0) return tq::fail(TQ_ERR_ARG, "tq_encode: negative row count");
+    return tq::fail(TQ_ERR_ARG, "%s: unknown variant %d", who, variant);
+  if (n_groups < 0 || rows_per_group < 0) return tq::fail(TQ_ERR_ARG, "%s: negative row count", who);
   const int64_t n_rows = n_groups * rows_per_group;
   if (n_rows == 0) return TQ_OK;
-  if (!x || !signs || !boundaries || !packed || !norms) return tq::fail(TQ_ERR_NULL, "tq_encode: null pointer");
-  if (!tq::aligned(x, tq::dtype_size(x_dtype)) || !tq::aligned(signs, 4) || !tq::aligned(packed, 4) ||
-      !tq::aligned(norms, 4))
-    return tq::fail(TQ_ERR_ALIGN, "tq_encode: misaligned pointer");
-  const int nb = (1 << bits) - 1;
-  Thresholds thr;
-  const float s = (float)(1.0 / sqrt((double)dim));
-  for (int i = 0; i < 15; ++i) thr.t[i] = INFINITY;
-  for (int i = 0; i < nb; ++i)
-    thr.t[i] = (variant == TQ_ENCODE_MLX) ? double_rounding_threshold(boundaries[i], s) : boundaries[i];
+  if (!boundaries) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  bool wide = true;                                            // 16-byte loads of the input rows
+  for (int i = 0; i < n_sides; ++i) {
+    const EncodeSide& s = sides.s[i];
+    if (!s.x || !s.signs || !s.packed || !s.norms) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+    if (!tq::aligned(s.x, tq::dtype_size(x_dtype)) || !tq::aligned(s.signs, 4) || !tq::aligned(s.packed, 4) ||
+        !tq::aligned(s.norms, 4))
+      return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+    wide = wide && tq::aligned(s.x, 16);
+  }
   const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
-  hipStream_t stream = (hipStream_t)stream_;
-  const int grid = grid_for_rows(n_rows);
-  EncodeGuess gs{};
+  const EncodePlan plan = encode_plan(boundaries, dim, bits, variant);
   const bool whole = whole_batches(dim, rm);
-  if (dim >= 64 && (whole || n_rows >= stream_min_rows(dim, true)) && n_rows < (int64_t)1 << 31 &&
-      (whole || rows_fit_32_bits(rm, n_groups)) && tq::aligned(x, 16) && level_guess(thr.t, nb, gs)) {
-    const EncodeCall c{x, x_dtype, signs, thr, gs, packed, norms, rm, bits, stream};
+  if (dim >= 64 && (whole || n_rows * n_sides >= stream_min_rows(dim, true)) && n_rows < (int64_t)1 << 31 &&
+      (whole || rows_fit_32_bits(rm, n_groups)) && wide && plan.has_guess) {
+    const EncodeCall c{sides, n_sides, x_dtype, plan.thr, plan.gs, rm, bits, stream};
     if (whole) launch_encode_rows<128, false>(c);
     else if (dim == 64) launch_encode_rows<64, true>(c);
     else if (dim == 128) launch_encode_rows<128, true>(c);
     else launch_encode_rows<256, true>(c);
-    TQ_CHECK_LAUNCH("tq_encode launch");
-    return TQ_OK;
-  }
-#define LAUNCH_ENC(T)                                                                               \
-  TQ_DISPATCH_DIM(dim, TQ_DISPATCH_BITS(bits, (encode_kernel<D_, B_, T><<<grid, kBlock, 0, stream>>>( \
-                                                  (const T*)x, signs, thr, packed, norms, rm, RowCopy{}))))
-  if (x_dtype == TQ_F32) { LAUNCH_ENC(float); }
-  else if (x_dtype == TQ_F16) { LAUNCH_ENC(__half); }
-  else { LAUNCH_ENC(__hip_bfloat16); }
+  } else {
+    const dim3 grid(grid_for_rows(n_rows), n_sides);
+#define LAUNCH_ENC(T)                                                                                                 \
+    TQ_DISPATCH_DIM(dim, TQ_DISPATCH_BITS(bits, (encode_kernel<D_, B_, T><<<grid, kBlock, 0, stream>>>(                \
+                                                    sides, plan.thr, rm, RowCopy{}))))
+    if (x_dtype == TQ_F32) { LAUNCH_ENC(float); }
+    else if (x_dtype == TQ_F16) { LAUNCH_ENC(__half); }
+    else { LAUNCH_ENC(__hip_bfloat16); }
 #undef LAUNCH_ENC
-  TQ_CHECK_LAUNCH("tq_encode launch");
+  }
+  TQ_CHECK_LAUNCH(who);
   return TQ_OK;
+}
+
+int dequant_sides(const char* who, const DequantSides& sides, int n_sides, const float* centroids, int out_dtype,
+                  int64_t n_groups, int64_t rows_per_group, int64_t packed_group_stride, int64_t norms_group_stride,
+                  int64_t out_group_stride, int dim, int bits, hipStream_t stream) {
+  if (int rc = tq::check_dim_bits(dim, bits)) return rc;
+  if (tq::check_dtype(out_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown out_dtype %d", who, out_dtype);
+  if (n_groups < 0 || rows_per_group < 0) return tq::fail(TQ_ERR_ARG, "%s: negative row count", who);
+  const int64_t n_rows = n_groups * rows_per_group;
+  if (n_rows == 0) return TQ_OK;
+  if (!centroids) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  bool wide = (out_group_stride * dim * (int64_t)tq::dtype_size(out_dtype)) % 16 == 0;   // 16-byte stores of the output rows
+  for (int i = 0; i < n_sides; ++i) {
+    const DequantSide& s = sides.s[i];
+    if (!s.packed || !s.norms || !s.signs || !s.out) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+    if (!tq::aligned(s.packed, 4) || !tq::aligned(s.norms, 4) || !tq::aligned(s.signs, 4) ||
+        !tq::aligned(s.out, tq::dtype_size(out_dtype)))
+      return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+    wide = wide && tq::aligned(s.out, 16);
+  }
+  Codebook cb;
+  for (int i = 0; i < 16; ++i) cb.c[i] = i < (1 << bits) ? centroids[i] : 0.0f;
+  const float s = (float)(1.0 / sqrt((double)dim));
+  const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride);
+  const bool whole = whole_batches(dim, rm);
+  if (dim >= 64 && (whole || n_rows * n_sides >= stream_min_rows(dim, false)) && n_rows < (int64_t)1 << 31 &&
+      (whole || rows_fit_32_bits(rm, n_groups)) && wide) {
+    const DequantCall c{sides, n_sides, cb, s, out_dtype, rm, bits, stream};
+    if (whole) launch_dequant_rows<128, false>(c);
+    else if (dim == 64) launch_dequant_rows<64, true>(c);
+    else if (dim == 128) launch_dequant_rows<128, true>(c);
+    else launch_dequant_rows<256, true>(c);
+  } else {
+    const dim3 grid(grid_for_rows(n_rows), n_sides);
+#define LAUNCH_DEQ(T)                                                                                                 \
+    TQ_DISPATCH_DIM(dim, TQ_DISPATCH_BITS(bits, (dequant_kernel<D_, B_, T><<<grid, kBlock, 0, stream>>>(sides, cb, s, rm))))
+    if (out_dtype == TQ_F32) { LAUNCH_DEQ(float); }
+    else if (out_dtype == TQ_F16) { LAUNCH_DEQ(__half); }
+    else { LAUNCH_DEQ(__hip_bfloat16); }
+#undef LAUNCH_DEQ
+  }
+  TQ_CHECK_LAUNCH(who);
+  return TQ_OK;
+}
+}  // namespace
+
+extern "C" int tq_encode(const void* x, int x_dtype, const float* signs, const float* boundaries,
+                         uint32_t* packed, float* norms, int64_t n_groups, int64_t rows_per_group,
+                         int64_t packed_group_stride, int64_t norms_group_stride, int dim, int bits,
+                         int variant, tq_stream_t stream_) {
+  return encode_sides("tq_encode", EncodeSides{{{x, signs, packed, norms}, {}}}, 1, x_dtype, boundaries, n_groups,
+                      rows_per_group, packed_group_stride, norms_group_stride, dim, bits, variant, (hipStream_t)stream_);
+}
+
+extern "C" int tq_encode_kv(const void* k, const float* k_signs, uint32_t* k_packed, float* k_norms, const void* v,
+                            const float* v_signs, uint32_t* v_packed, float* v_norms, int x_dtype,
+                            const float* boundaries, int64_t n_groups, int64_t rows_per_group,
+                            int64_t packed_group_stride, int64_t norms_group_stride, int dim, int bits, int variant,
+                            tq_stream_t stream_) {
+  return encode_sides("tq_encode_kv", EncodeSides{{{k, k_signs, k_packed, k_norms}, {v, v_signs, v_packed, v_norms}}}, 2,
+                      x_dtype, boundaries, n_groups, rows_per_group, packed_group_stride, norms_group_stride, dim, bits,
+                      variant, (hipStream_t)stream_);
 }
 
 namespace {
@@ -617,21 +688,17 @@ int vonly_append(const void* k_new, int k_dtype, const void* v_new, int v_dtype,
       !tq::aligned(v_signs, 4) || !tq::aligned(k_f16, 2) || !tq::aligned(v_packed, 4) || !tq::aligned(v_norms, 4) ||
       (v_raw && !tq::aligned(v_raw, tq::dtype_size(v_dtype))))
     return tq::fail(TQ_ERR_ALIGN, "tq_vonly_append: misaligned pointer");
-  const int nb = (1 << bits) - 1;
-  Thresholds thr;
-  const float s = (float)(1.0 / sqrt((double)dim));
-  for (int i = 0; i < 15; ++i) thr.t[i] = INFINITY;
-  for (int i = 0; i < nb; ++i)
-    thr.t[i] = (variant == TQ_ENCODE_MLX) ? double_rounding_threshold(boundaries[i], s) : boundaries[i];
+  const Thresholds thr = encode_plan(boundaries, dim, bits, variant).thr;
   const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
   if (pos_dev && (!tq::aligned(pos_dev, 8) || pos_cap < 1))
     return tq::fail(TQ_ERR_ARG, "tq_vonly_append_at: position_dev must be 8-byte aligned and t_alloc >= 1");
   RowCopy rc{k_new, (__half*)k_f16, v_raw, k_group_stride, v_raw_group_stride, k_dtype, pos_dev, pos_cap};
   hipStream_t stream = (hipStream_t)stream_;
   const int grid = grid_for_rows(n_rows);
+  const EncodeSides sides{{{v_new, v_signs, v_packed, v_norms}, {}}};
 #define LAUNCH_APP(T)                                                                               \
   TQ_DISPATCH_DIM(dim, TQ_DISPATCH_BITS(bits, (encode_kernel<D_, B_, T><<<grid, kBlock, 0, stream>>>( \
-                                                  (const T*)v_new, v_signs, thr, v_packed, v_norms, rm, rc))))
+                                                  sides, thr, rm, rc))))
   if (v_dtype == TQ_F32) { LAUNCH_APP(float); }
   else if (v_dtype == TQ_F16) { LAUNCH_APP(__half); }
   else { LAUNCH_APP(__hip_bfloat16); }
@@ -669,41 +736,109 @@ extern "C" int tq_dequant(const uint32_t* packed, const float* norms, const floa
                           const float* signs, void* out, int out_dtype, int64_t n_groups,
                           int64_t rows_per_group, int64_t packed_group_stride, int64_t norms_group_stride,
                           int64_t out_group_stride, int dim, int bits, tq_stream_t stream_) {
-  if (int rc = tq::check_dim_bits(dim, bits)) return rc;
-  if (tq::check_dtype(out_dtype)) return tq::fail(TQ_ERR_DTYPE, "tq_dequant: unknown out_dtype %d", out_dtype);
-  if (n_groups < 0 || rows_per_group < 0) return tq::fail(TQ_ERR_ARG, "tq_dequant: negative row count");
-  const int64_t n_rows = n_groups * rows_per_group;
-  if (n_rows == 0) return TQ_OK;
-  if (!packed || !norms || !centroids || !signs || !out) return tq::fail(TQ_ERR_NULL, "tq_dequant: null pointer");
-  if (!tq::aligned(packed, 4) || !tq::aligned(norms, 4) || !tq::aligned(signs, 4) ||
-      !tq::aligned(out, tq::dtype_size(out_dtype)))
-    return tq::fail(TQ_ERR_ALIGN, "tq_dequant: misaligned pointer");
-  Codebook cb;
-  for (int i = 0; i < 16; ++i) cb.c[i] = i < (1 << bits) ? centroids[i] : 0.0f;
-  const float s = (float)(1.0 / sqrt((double)dim));
-  const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride);
-  hipStream_t stream = (hipStream_t)stream_;
-  const int grid = grid_for_rows(n_rows);
-  const bool whole = whole_batches(dim, rm);
-  if (dim >= 64 && (whole || n_rows >= stream_min_rows(dim, false)) && n_rows < (int64_t)1 << 31 &&
-      (whole || rows_fit_32_bits(rm, n_groups)) && tq::aligned(out, 16) &&
-      (out_group_stride * dim * (int64_t)tq::dtype_size(out_dtype)) % 16 == 0) {
-    const DequantCall c{packed, norms, cb, signs, s, out, out_dtype, rm, bits, stream};
-    if (whole) launch_dequant_rows<128, false>(c);
-    else if (dim == 64) launch_dequant_rows<64, true>(c);
-    else if (dim == 128) launch_dequant_rows<128, true>(c);
-    else launch_dequant_rows<256, true>(c);
-    TQ_CHECK_LAUNCH("tq_dequant launch");
-    return TQ_OK;
+  return dequant_sides("tq_dequant", DequantSides{{{packed, norms, signs, out}, {}}}, 1, centroids, out_dtype, n_groups,
+                       rows_per_group, packed_group_stride, norms_group_stride, out_group_stride, dim, bits,
+                       (hipStream_t)stream_);
+}
+
+extern "C" int tq_dequant_kv(const uint32_t* k_packed, const float* k_norms, const float* k_signs, void* k_out,
+                             const uint32_t* v_packed, const float* v_norms, const float* v_signs, void* v_out,
+                             const float* centroids, int out_dtype, int64_t n_groups, int64_t rows_per_group,
+                             int64_t packed_group_stride, int64_t norms_group_stride, int64_t out_group_stride, int dim,
+                             int bits, tq_stream_t stream_) {
+  return dequant_sides("tq_dequant_kv", DequantSides{{{k_packed, k_norms, k_signs, k_out}, {v_packed, v_norms, v_signs, v_out}}},
+                       2, centroids, out_dtype, n_groups, rows_per_group, packed_group_stride, norms_group_stride,
+                       out_group_stride, dim, bits, (hipStream_t)stream_);
+}
+
+// ---------------------------------------------------------------- storage set-up
+
+namespace {
+// One launch for everything that a cache's fresh storage needs besides its new rows: per segment and group, words
+// 0 .. copy - 1 from the old storage, zeros in words zero_from .. zero_to - 1.
+struct FillArgs {
+  struct Segment {
+    uint32_t* dst;
+    const uint32_t* src;
+    int64_t dst_stride, src_stride, copy, zero_from, zero_to, n_groups;
+    int wide;                                                  // every bound a multiple of four words, 16-byte aligned
+  } s[TQ_FILL_MAX_SEGMENTS];
+};
+
+template <typename V>
+__device__ __forceinline__ void fill_group(const FillArgs::Segment& s, int64_t g) {
+  constexpr int64_t W = sizeof(V) / 4;
+  V* dst = reinterpret_cast<V*>(s.dst + g * s.dst_stride);
+  const V* src = reinterpret_cast<const V*>(s.src + g * s.src_stride);
+  const int64_t step = (int64_t)gridDim.x * kBlock, first = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  for (int64_t i = first; i < s.copy / W; i += step) dst[i] = src[i];
+  for (int64_t i = s.zero_from / W + first; i < s.zero_to / W; i += step) dst[i] = V{};
+}
+
+__global__ __launch_bounds__(kBlock) void fill_rows_kernel(FillArgs a) {
+  const FillArgs::Segment& s = a.s[blockIdx.y];
+  for (int64_t g = blockIdx.z; g < s.n_groups; g += gridDim.z) {
+    if (s.wide) fill_group<uint4>(s, g);
+    else fill_group<uint32_t>(s, g);
   }
-#define LAUNCH_DEQ(T)                                                                                 \
-  TQ_DISPATCH_DIM(dim, TQ_DISPATCH_BITS(bits, (dequant_kernel<D_, B_, T><<<grid, kBlock, 0, stream>>>( \
-                                                  packed, norms, cb, signs, s, (T*)out, rm))))
-  if (out_dtype == TQ_F32) { LAUNCH_DEQ(float); }
-  else if (out_dtype == TQ_F16) { LAUNCH_DEQ(__half); }
-  else { LAUNCH_DEQ(__hip_bfloat16); }
-#undef LAUNCH_DEQ
-  TQ_CHECK_LAUNCH("tq_dequant launch");
+}
+
+struct Seeds { uint64_t s[TQ_SIGNS_MAX_SEEDS]; };
+
+__device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
+  z += 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+
+__global__ __launch_bounds__(kBlock) void random_signs_kernel(Seeds seeds, int dim, float* __restrict__ out) {
+  const uint64_t base = splitmix64(seeds.s[blockIdx.x]);
+  for (int i = threadIdx.x; i < dim; i += kBlock)
+    out[(int64_t)blockIdx.x * dim + i] = (splitmix64(base + (uint64_t)i) >> 63) ? 1.0f : -1.0f;
+}
+}  // namespace
+
+extern "C" int tq_fill_rows(const tq_fill_segment* segments, int n_segments, tq_stream_t stream_) {
+  const char* who = "tq_fill_rows";
+  if (n_segments < 0 || n_segments > TQ_FILL_MAX_SEGMENTS) return tq::fail(TQ_ERR_ARG, "%s: %d segments", who, n_segments);
+  if (n_segments == 0) return TQ_OK;
+  if (!segments) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  FillArgs a{};
+  int64_t most = 0, groups = 1;
+  for (int i = 0; i < n_segments; ++i) {
+    const tq_fill_segment& g = segments[i];
+    if (g.n_groups < 0 || g.copy_bytes < 0 || g.zero_from < 0 || g.zero_to < g.zero_from)
+      return tq::fail(TQ_ERR_ARG, "%s: segment %d has a negative size", who, i);
+    if (!g.dst || (g.copy_bytes > 0 && !g.src)) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+    const int64_t bits = g.dst_group_stride | g.src_group_stride | g.copy_bytes | g.zero_from | g.zero_to |
+                         (int64_t)(uintptr_t)g.dst | (int64_t)(uintptr_t)g.src;
+    if (bits & 3) return tq::fail(TQ_ERR_ALIGN, "%s: segment %d is not made of 4-byte words", who, i);
+    a.s[i] = {(uint32_t*)g.dst, (const uint32_t*)g.src, g.dst_group_stride / 4, g.src_group_stride / 4, g.copy_bytes / 4,
+              g.zero_from / 4, g.zero_to / 4, g.n_groups, (bits & 15) == 0};
+    const int64_t words = (g.copy_bytes + g.zero_to - g.zero_from) / 4 / ((bits & 15) == 0 ? 4 : 1);
+    most = words > most ? words : most;
+    groups = g.n_groups > groups ? g.n_groups : groups;
+  }
+  if (most == 0) return TQ_OK;
+  const int64_t x = (most + kBlock - 1) / kBlock;
+  const dim3 grid((unsigned)(x < 256 ? x : 256), n_segments, (unsigned)(groups < 1024 ? groups : 1024));
+  fill_rows_kernel<<<grid, kBlock, 0, (hipStream_t)stream_>>>(a);
+  TQ_CHECK_LAUNCH("tq_fill_rows launch");
+  return TQ_OK;
+}
+
+extern "C" int tq_random_signs(const uint64_t* seeds, int n_seeds, int dim, float* signs, tq_stream_t stream_) {
+  const char* who = "tq_random_signs";
+  if (n_seeds < 0 || n_seeds > TQ_SIGNS_MAX_SEEDS) return tq::fail(TQ_ERR_ARG, "%s: %d seeds", who, n_seeds);
+  if (dim < 1) return tq::fail(TQ_ERR_DIM, "%s: dim %d", who, dim);
+  if (n_seeds == 0) return TQ_OK;
+  if (!seeds || !signs) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (!tq::aligned(signs, 4)) return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+  Seeds s{};
+  for (int i = 0; i < n_seeds; ++i) s.s[i] = seeds[i];
+  random_signs_kernel<<<n_seeds, kBlock, 0, (hipStream_t)stream_>>>(s, dim, signs);
+  TQ_CHECK_LAUNCH("tq_random_signs launch");
   return TQ_OK;
 }
 

@@ -21,6 +21,23 @@ struct RowMap {
   uint32_t group_mul, group_shift;
 };
 
+// What an encode or dequantise launch reads and writes; a launch takes one such side, or the keys' and the values' of
+// the same rows (blockIdx.y) with one RowMap, codebook and data type.
+struct EncodeSide {
+  const void* x;
+  const float* signs;
+  uint32_t* packed;
+  float* norms;
+};
+struct DequantSide {
+  const uint32_t* packed;
+  const float* norms;
+  const float* signs;
+  void* out;
+};
+struct EncodeSides { EncodeSide s[2]; };
+struct DequantSides { DequantSide s[2]; };
+
 __device__ __forceinline__ void group_of(const RowMap& rm, uint32_t row, uint32_t& g, uint32_t& r) {
   g = rm.group_mul ? (__umulhi(row, rm.group_mul) >> rm.group_shift) : row;
   r = row - g * (uint32_t)rm.rows_per_group;
@@ -114,10 +131,12 @@ constexpr int kEncPasses = 4;     // passes per wavefront once there are rows en
 // per pass and the destination rows of the pass are shared through LDS; rows past the end repeat the last one and
 // are not stored.  What it costs over the other form is a dozen instructions per 2048 elements.
 template <int D, typename T, int BITS, bool RAGGED>
-__global__ __launch_bounds__(kBlock) void encode_rows_kernel(const T* __restrict__ x,
-                                                             const float* __restrict__ signs, Thresholds thr,
-                                                             EncodeGuess gs, uint32_t* __restrict__ packed,
-                                                             float* __restrict__ norms, RowMap rm, int passes) {
+__global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, Thresholds thr, EncodeGuess gs, RowMap rm,
+                                                             int passes) {
+  const T* __restrict__ x = (const T*)sides.s[blockIdx.y].x;
+  const float* __restrict__ signs = sides.s[blockIdx.y].signs;
+  uint32_t* __restrict__ packed = sides.s[blockIdx.y].packed;
+  float* __restrict__ norms = sides.s[blockIdx.y].norms;
   using VL = VecLanes<D>;
   constexpr int kLanes = VL::kLanes, kVecs = VL::kVecs, kChunks = D / 8;
   constexpr bool kHalfWidth = sizeof(T) == 2;
@@ -355,10 +374,12 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(const T* __restrict
 // looks centroid pairs up in a table of 4^BITS entries (c[a]*s, c[b]*s).  Arithmetic per element, in this order, as in
 // dequant_kernel: butterfly, * s, * sign, * norm, round to TO.  RAGGED as in the encoder.
 template <int D, typename TO, int BITS, bool RAGGED>
-__global__ __launch_bounds__(kBlock) void dequant_rows_kernel(const uint32_t* __restrict__ packed,
-                                                              const float* __restrict__ norms, Codebook cbk,
-                                                              const float* __restrict__ signs, float s,
-                                                              TO* __restrict__ out, RowMap rm, int passes) {
+__global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides, Codebook cbk, float s, RowMap rm,
+                                                              int passes) {
+  const uint32_t* __restrict__ packed = sides.s[blockIdx.y].packed;
+  const float* __restrict__ norms = sides.s[blockIdx.y].norms;
+  const float* __restrict__ signs = sides.s[blockIdx.y].signs;
+  TO* __restrict__ out = (TO*)sides.s[blockIdx.y].out;
   using CK = Chunk<D, BITS>;
   using VL = VecLanes<D>;
   constexpr int kLanes = VL::kLanes, kVecs = VL::kVecs;
@@ -536,24 +557,20 @@ __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(const uint32_t* __
 // ---------------------------------------------------------------- launches
 
 struct EncodeCall {
-  const void* x;
+  EncodeSides sides;
+  int n_sides;
   int x_dtype;
-  const float* signs;
   Thresholds thr;
   EncodeGuess gs;
-  uint32_t* packed;
-  float* norms;
   RowMap rm;
   int bits;
   hipStream_t stream;
 };
 struct DequantCall {
-  const uint32_t* packed;
-  const float* norms;
+  DequantSides sides;
+  int n_sides;
   Codebook cb;
-  const float* signs;
   float s;
-  void* out;
   int out_dtype;
   RowMap rm;
   int bits;
@@ -574,10 +591,11 @@ inline int stream_grid(int64_t n_rows, int passes) {
 
 template <int D, bool RAGGED>
 void launch_encode_rows(const EncodeCall& c) {
-  const int passes = stream_passes<D>(c.rm.n_rows), grid = stream_grid<D>(c.rm.n_rows, passes);
+  const int passes = stream_passes<D>(c.rm.n_rows * c.n_sides);
+  const dim3 grid(stream_grid<D>(c.rm.n_rows, passes), c.n_sides);
 #define TQ_LAUNCH_ENC(T)                                                                                             \
   TQ_DISPATCH_BITS(c.bits, (encode_rows_kernel<D, T, B_, RAGGED><<<grid, kBlock, 0, c.stream>>>(                      \
-                               (const T*)c.x, c.signs, c.thr, c.gs, c.packed, c.norms, c.rm, passes)))
+                               c.sides, c.thr, c.gs, c.rm, passes)))
   if (c.x_dtype == TQ_F32) { TQ_LAUNCH_ENC(float); }
   else if (c.x_dtype == TQ_F16) { TQ_LAUNCH_ENC(__half); }
   else { TQ_LAUNCH_ENC(__hip_bfloat16); }
@@ -586,10 +604,11 @@ void launch_encode_rows(const EncodeCall& c) {
 
 template <int D, bool RAGGED>
 void launch_dequant_rows(const DequantCall& c) {
-  const int passes = stream_passes<D>(c.rm.n_rows), grid = stream_grid<D>(c.rm.n_rows, passes);
+  const int passes = stream_passes<D>(c.rm.n_rows * c.n_sides);
+  const dim3 grid(stream_grid<D>(c.rm.n_rows, passes), c.n_sides);
 #define TQ_LAUNCH_DEQ(TO)                                                                                            \
   TQ_DISPATCH_BITS(c.bits, (dequant_rows_kernel<D, TO, B_, RAGGED><<<grid, kBlock, 0, c.stream>>>(                    \
-                               c.packed, c.norms, c.cb, c.signs, c.s, (TO*)c.out, c.rm, passes)))
+                               c.sides, c.cb, c.s, c.rm, passes)))
   if (c.out_dtype == TQ_F32) { TQ_LAUNCH_DEQ(float); }
   else if (c.out_dtype == TQ_F16) { TQ_LAUNCH_DEQ(__half); }
   else { TQ_LAUNCH_DEQ(__hip_bfloat16); }

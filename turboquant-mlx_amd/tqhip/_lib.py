@@ -20,7 +20,7 @@ _p = C.c_void_p
 _i = C.c_int
 _l = C.c_int64
 _f = C.c_float
-_fp = C.POINTER(C.c_float)
+_fp = C.c_void_p                    # small host tables: a ctypes float array or the address of one
 _z = C.c_size_t
 
 
@@ -61,12 +61,24 @@ class PackedCacheDesc(C.Structure):
     ]
 
 
+class FillSegment(C.Structure):
+    """Mirror of struct tq_fill_segment."""
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("dst_group_stride", C.c_int64), ("src_group_stride", C.c_int64),
+                ("copy_bytes", C.c_int64), ("zero_from", C.c_int64), ("zero_to", C.c_int64), ("n_groups", C.c_int64)]
+
+
+FILL_MAX_SEGMENTS = 8              # TQ_FILL_MAX_SEGMENTS of include/tqhip.h
+
 # name -> (restype, argtypes); the authoritative list of exported symbols
 PROTOTYPES = {
     "tq_version": (_i, []),
     "tq_last_error": (C.c_char_p, []),
     "tq_status_string": (C.c_char_p, [_i]),
     "tq_encode": (_i, [_p, _i, _p, _fp, _p, _p, _l, _l, _l, _l, _i, _i, _i, _p]),
+    "tq_encode_kv": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i, _fp, _l, _l, _l, _l, _i, _i, _i, _p]),
+    "tq_dequant_kv": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _fp, _i, _l, _l, _l, _l, _l, _i, _i, _p]),
+    "tq_fill_rows": (_i, [C.POINTER(FillSegment), _i, _p]),
+    "tq_random_signs": (_i, [C.POINTER(C.c_uint64), _i, _i, _p, _p]),
     "tq_vonly_append": (_i, [_p, _i, _p, _i, _p, _fp, _p, _p, _p, _p, _l, _l, _l, _l, _l, _l, _i, _i, _i, _p]),
     "tq_dequant": (_i, [_p, _p, _fp, _p, _p, _i, _l, _l, _l, _l, _l, _i, _i, _p]),
     "tq_prerotate_query": (_i, [_p, _i, _p, _p, _l, _i, _p]),

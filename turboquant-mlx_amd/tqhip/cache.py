@@ -34,33 +34,41 @@ class _Quantizer:
     random_diagonal_sign derives from `seed` (whose generator is this package's own, not MLX's): the way to
     read a cache written by the reference, which stores only the seed (cache.py:286)."""
 
-    def __init__(self, dim, bits, seed, device, signs=None, sign_stream="native"):
+    def __init__(self, dim, bits, seed, device, signs=None, sign_stream="native", made=None, tables=None):
+        """made: the sign vector of `seed` where the caller has it already; tables: (centroids, boundaries) of `bits`."""
         self.dim = dim
         self.bits = bits
-        self.signs = (random_diagonal_sign(dim, seed=seed, device=device, stream=sign_stream) if signs is None
-                      else _checked_signs(signs, dim, device))
-        self.centroids = gaussian_codebook(bits)
-        self.boundaries = gaussian_boundaries(self.centroids)
+        if signs is not None:
+            self.signs = _checked_signs(signs, dim, device)
+        else:
+            self.signs = made if made is not None else random_diagonal_sign(dim, seed=seed, device=device, stream=sign_stream)
+        self.centroids, self.boundaries = tables if tables is not None else _tables(bits)
+
+
+def _tables(bits):
+    centroids = gaussian_codebook(bits)
+    return centroids, gaussian_boundaries(centroids)
 
 
 def _round_up(n, step):
     return ((n + step - 1) // step) * step
 
 
+def _is_grouped(t: torch.Tensor, inner: int) -> bool:
+    """Whether _group_stride can describe t."""
+    if inner == 1 and t.dim() == 3:
+        return t.stride(2) == 1 and t.stride(0) == t.shape[1] * t.stride(1)
+    return (t.stride(3) == 1 and t.stride(2) == inner and t.stride(1) % inner == 0
+            and t.stride(0) == t.shape[1] * t.stride(1))
+
+
 def _group_stride(t: torch.Tensor, inner: int) -> int:
     """Rows between consecutive (b, h) groups of a [B, H, T, inner] (or [B, H, T] with inner=1)
     tensor whose rows are dense and whose batch stride is H head strides -- true for the cache's
     own allocations and for time-slices of them."""
-    if inner == 1 and t.dim() == 3:
-        ok = t.stride(2) == 1 and t.stride(0) == t.shape[1] * t.stride(1)
-        gs = t.stride(1)
-    else:
-        ok = (t.stride(3) == 1 and t.stride(2) == inner and t.stride(1) % inner == 0
-              and t.stride(0) == t.shape[1] * t.stride(1))
-        gs = t.stride(1) // inner
-    if not ok:
+    if not _is_grouped(t, inner):
         raise ValueError("cache storage must be row-contiguous [B, H, T, *]; call .contiguous() first")
-    return gs
+    return t.stride(1) // inner
 
 
 class TurboQuantKVCache:
@@ -126,39 +134,67 @@ class TurboQuantKVCache:
                 return t.device
         return torch.device("cuda")
 
-    def _ensure_quantizer(self, k_dim, v_dim, device=None):
-        device = device if device is not None else self._device()
-        if not self.v_only and self._k_q is None:
-            self._k_q = _Quantizer(k_dim, self.quant_bits, self.seed, device, self._k_signs_given, self.sign_stream)
+    def _ensure_quantizer(self, k_dim, v_dim, device=None, in_order=True):
+        """in_order: what uses the sign vectors runs on the current stream (or waits for it), as the inserts do.  False
+        makes them with a blocking copy, for a restored cache that may be read from any stream at once."""
+        new_k, new_v = not self.v_only and self._k_q is None, self._v_q is None
+        if not (new_k or new_v):
+            return
+        device = torch.device(device) if device is not None else self._device()
+        ask = []                                             # (seed, dim) of the vectors to derive
+        if new_k and self._k_signs_given is None:
+            ask.append((self.seed, k_dim))
+        if new_v and self._v_signs_given is None:
+            ask.append((self.seed + 1, v_dim))
+        made = {}
+        if in_order and ask and self.sign_stream == "native" and device.type == "cuda" and len({d for _, d in ask}) == 1:
+            made = dict(zip((s for s, _ in ask), ops.random_signs([s for s, _ in ask], ask[0][1], device)))
+        tables = _tables(self.quant_bits)
+        if new_k:
+            self._k_q = _Quantizer(k_dim, self.quant_bits, self.seed, device, self._k_signs_given, self.sign_stream,
+                                   made.get(self.seed), tables)
             self._k_dim = k_dim
             self._k_pdim = ops.packed_dim(k_dim, self.quant_bits)
-        if self._v_q is None:
-            self._v_q = _Quantizer(v_dim, self.quant_bits, self.seed + 1, device, self._v_signs_given, self.sign_stream)
+        if new_v:
+            self._v_q = _Quantizer(v_dim, self.quant_bits, self.seed + 1, device, self._v_signs_given, self.sign_stream,
+                                   made.get(self.seed + 1), tables)
             self._v_dim = v_dim
             self._v_pdim = ops.packed_dim(v_dim, self.quant_bits)
 
-    def _grow(self, old_p, old_n, B, H, n, pdim, prev, device):
-        new_p = torch.zeros((B, H, n, pdim), dtype=torch.uint32, device=device)
-        new_n = torch.zeros((B, H, n), dtype=torch.float32, device=device)
-        if old_p is not None and prev > 0:
-            new_p[..., :prev, :] = old_p[..., :prev, :]
-            new_n[..., :prev] = old_n[..., :prev]
-        return new_p, new_n
+    def _grow(self, old, shape, inner, prev, incoming, dtype, device, fill):
+        """Fresh storage [B, H, n(, inner)] holding the first `prev` rows of `old`, zero from row prev + incoming on; the
+        rows between are about to be written.  The copy and the zeros join `fill`."""
+        new = torch.empty(shape, dtype=dtype, device=device)
+        n = shape[2]
+        if old is None or prev == 0:
+            fill.add(new, inner, incoming, n)
+        elif old.dtype == dtype and old.device == new.device and old.shape[:2] == new.shape[:2] and _is_grouped(old, inner):
+            fill.add(new, inner, prev + incoming, n, src=old, src_stride=_group_stride(old, inner), copy=prev)
+        else:
+            new.zero_()
+            new[:, :, :prev] = old[:, :, :prev]
+        return new
 
-    def _ensure_storage(self, B, H, num_new, device):
+    def _ensure_storage(self, B, H, num_new, device, incoming=0, fill=None):
+        """Room for num_new more positions (cache.py:100-123); the caller writes the first `incoming` of them itself."""
         prev = self.offset
         needed = prev + num_new
         if self.v_packed is None or needed > self.v_packed.shape[2]:
-            self._reallocate(B, H, _round_up(needed, self.step), device)
+            self._reallocate(B, H, _round_up(needed, self.step), device, incoming, fill)
 
-    def _reallocate(self, B, H, n, device):
+    def _reallocate(self, B, H, n, device, incoming=0, fill=None):
         """Fresh contiguous storage of n positions per (b, h) holding the first `offset` positions."""
         prev = self.offset
+        own = fill if fill is not None else ops.StorageFill()
         if not self.v_only:
-            self.k_packed, self.k_norms = self._grow(self.k_packed, self.k_norms, B, H, n,
-                                                     self._k_pdim, prev, device)
-        self.v_packed, self.v_norms = self._grow(self.v_packed, self.v_norms, B, H, n,
-                                                 self._v_pdim, prev, device)
+            self.k_packed, self.k_norms = (
+                self._grow(self.k_packed, (B, H, n, self._k_pdim), self._k_pdim, prev, incoming, torch.uint32, device, own),
+                self._grow(self.k_norms, (B, H, n), 1, prev, incoming, torch.float32, device, own))
+        self.v_packed, self.v_norms = (
+            self._grow(self.v_packed, (B, H, n, self._v_pdim), self._v_pdim, prev, incoming, torch.uint32, device, own),
+            self._grow(self.v_norms, (B, H, n), 1, prev, incoming, torch.float32, device, own))
+        if fill is None:
+            own.run()
 
     # ---------------------------------------------------------------- codec calls
     def _encode(self, x, q, packed, norms, B, H, S, dim, prev):
@@ -168,12 +204,43 @@ class TurboQuantKVCache:
                         norms_group_stride=_group_stride(norms, 1), dim=dim, bits=self.quant_bits,
                         variant=self.encode_variant, packed_row_offset=prev, norms_row_offset=prev)
 
-    def _dequant_range(self, packed, norms, q, dim, buf, B, H, start, count):
-        """Dequantise positions [start, start+count) of every (b, h) into buf[..., start:start+count, :]."""
-        ops.dequant_into(packed, norms, q.centroids, q.signs, buf, n_groups=B * H, rows_per_group=count,
-                         packed_group_stride=_group_stride(packed, packed.shape[3]),
-                         norms_group_stride=_group_stride(norms, 1), out_group_stride=buf.shape[2], dim=dim, bits=self.quant_bits,
-                         packed_row_offset=start, norms_row_offset=start, out_row_offset=start)
+    def _encode_pair(self, keys, values, B, H, S, k_dim, v_dim, prev):
+        """Key and value rows at positions prev .. prev + S - 1, in one launch where one describes both."""
+        gs = _group_stride(self.v_packed, self._v_pdim)
+        if (keys.dtype == values.dtype and k_dim == v_dim and _group_stride(self.k_packed, self._k_pdim) == gs
+                and _group_stride(self.k_norms, 1) == gs and _group_stride(self.v_norms, 1) == gs):
+            kq, vq = self._k_q, self._v_q
+            ops.encode_kv_into(keys, kq.signs, self.k_packed, self.k_norms, values, vq.signs, self.v_packed, self.v_norms,
+                               vq.boundaries, n_groups=B * H, rows_per_group=S, group_stride=gs, dim=v_dim,
+                               bits=self.quant_bits, variant=self.encode_variant, row_offset=prev)
+        else:
+            self._encode(values, self._v_q, self.v_packed, self.v_norms, B, H, S, v_dim, prev)
+            self._encode(keys, self._k_q, self.k_packed, self.k_norms, B, H, S, k_dim, prev)
+
+    def _sides(self):
+        """(packed, norms, quantizer, dim) of the stored tensors."""
+        v = (self.v_packed, self.v_norms, self._v_q, self._v_dim)
+        return [v] if self.v_only else [(self.k_packed, self.k_norms, self._k_q, self._k_dim), v]
+
+    def _dequant_rows(self, outs, B, H, start, count, out_start):
+        """Positions start .. start + count - 1 of every (b, h) of each stored tensor into rows out_start .. of its
+        contiguous [B, H, T, dim] tensor in `outs`: one launch where one describes both."""
+        sides = self._sides()
+        if len(sides) == 2:
+            (kp, kn, kq, kd), (vp, vn, vq, vd) = sides
+            ko, vo = outs
+            gs = _group_stride(vp, vp.shape[3])
+            if (ko.dtype == vo.dtype and ko.shape == vo.shape and _group_stride(kp, kp.shape[3]) == gs
+                    and _group_stride(kn, 1) == gs and _group_stride(vn, 1) == gs and kq.centroids is vq.centroids):
+                ops.dequant_kv_into(kp, kn, kq.signs, ko, vp, vn, vq.signs, vo, vq.centroids, n_groups=B * H,
+                                    rows_per_group=count, group_stride=gs, out_group_stride=vo.shape[2], dim=vd,
+                                    bits=self.quant_bits, row_offset=start, out_row_offset=out_start)
+                return
+        for (packed, norms, q, dim), out in zip(sides, outs):
+            ops.dequant_into(packed, norms, q.centroids, q.signs, out, n_groups=B * H, rows_per_group=count,
+                             packed_group_stride=_group_stride(packed, packed.shape[3]),
+                             norms_group_stride=_group_stride(norms, 1), out_group_stride=out.shape[2], dim=dim,
+                             bits=self.quant_bits, packed_row_offset=start, norms_row_offset=start, out_row_offset=out_start)
 
     def _full_dequant(self, packed, norms, q, dim, B, H, total, dtype):
         """cache.py:125-129: every stored position, as a fresh [B, H, total, dim] tensor."""
@@ -184,45 +251,38 @@ class TurboQuantKVCache:
                          out_group_stride=total, dim=dim, bits=self.quant_bits)
         return out
 
-    def _incremental(self, packed, norms, q, dim, buf, B, H, prev, total, dtype):
-        """Decode step of cache.py:171-180 / 192-207: dequantise only the new rows, in half
-        precision (dequant_fp16), cast to the cache dtype, into the persistent buffer."""
-        if total > self._deq_alloc_for(buf):
-            na = _round_up(total, self.step)
-            grown = torch.zeros((B, H, na, dim), dtype=dtype, device=buf.device)
-            grown[..., :self._deq_offset, :] = buf[..., :self._deq_offset, :]
-            buf = grown
-        if dtype == torch.float16:
-            self._dequant_range(packed, norms, q, dim, buf, B, H, prev, total - prev)
+    def _buffers(self, B, H, n, dtypes, device):
+        return [torch.empty((B, H, n, side[3]), dtype=dt, device=device) for side, dt in zip(self._sides(), dtypes)]
+
+    def _incremental(self, bufs, B, H, prev, total, dtypes):
+        """Decode step of cache.py:171-180 / 192-207: dequantise only the new rows, in half precision (dequant_fp16),
+        cast to the cache dtype, into the persistent buffers."""
+        if total > bufs[0].shape[2]:
+            fill = ops.StorageFill()
+            grown = self._buffers(B, H, _round_up(total, self.step), dtypes, bufs[0].device)
+            for new, old in zip(grown, bufs):
+                fill.add(new, new.shape[3], total, new.shape[2], src=old, src_stride=old.shape[2], copy=self._deq_offset)
+            fill.run()
+            bufs = grown
+        if all(dt == torch.float16 for dt in dtypes):
+            self._dequant_rows(bufs, B, H, prev, total - prev, prev)
         else:
-            tmp = torch.empty((B, H, total - prev, dim), dtype=torch.float16, device=buf.device)
-            ops.dequant_into(packed, norms, q.centroids, q.signs, tmp, n_groups=B * H,
-                             rows_per_group=total - prev,
-                             packed_group_stride=_group_stride(packed, packed.shape[3]),
-                             norms_group_stride=_group_stride(norms, 1), out_group_stride=total - prev, dim=dim,
-                             bits=self.quant_bits, packed_row_offset=prev, norms_row_offset=prev)
-            buf[..., prev:total, :] = tmp.to(dtype)
-        return buf
-
-    @staticmethod
-    def _deq_alloc_for(buf):
-        return buf.shape[2]
-
-    def _prefill_buffer(self, packed, norms, q, dim, B, H, total, dtype):
-        """cache.py:182-188 / 208-218: full dequant into a fresh step-rounded buffer."""
-        alloc = _round_up(total, self.step)
-        buf = torch.zeros((B, H, alloc, dim), dtype=dtype, device=packed.device)
-        self._dequant_range(packed, norms, q, dim, buf, B, H, 0, total)
-        return buf, alloc
+            tmp = self._buffers(B, H, total - prev, [torch.float16] * len(bufs), bufs[0].device)
+            self._dequant_rows(tmp, B, H, prev, total - prev, 0)
+            for buf, rows in zip(bufs, tmp):
+                buf[:, :, prev:total].copy_(rows)
+        return bufs
 
     # ---------------------------------------------------------------- cache.py:131-218
-    def _zero_like(self, t: torch.Tensor) -> torch.Tensor:
+    def _zero_like(self, t: torch.Tensor, fill) -> torch.Tensor:
         """A zero scalar of t's dtype on t's device, made once: the source of the stride-0 placeholders
-        (a fresh one per step would cost a fill launch each)."""
+        (a fresh one per step would cost a fill launch each).  A new one's bytes join `fill`."""
         key = (t.dtype, t.device)
         z = self.__dict__.setdefault("_zero_scalars", {}).get(key)
         if z is None:
-            z = self._zero_scalars[key] = t.new_zeros(())
+            base = t.new_empty(8)
+            fill.add(base, 1, 0, 8)
+            z = self._zero_scalars[key] = base[0]
         return z
 
     def reserve(self, B: int, H: int, n_positions: int, dim: int, device="cuda"):
@@ -295,47 +355,60 @@ class TurboQuantKVCache:
         device = values.device
         self._dtype = keys.dtype
         self._ensure_quantizer(k_dim, v_dim, device)
-        self._ensure_storage(B, H, S, device)
         prev = self.offset
-
-        self._encode(values, self._v_q, self.v_packed, self.v_norms, B, H, S, v_dim, prev)
-        if not self.v_only:
-            self._encode(keys, self._k_q, self.k_packed, self.k_norms, B, H, S, k_dim, prev)
-
-        self.offset += S
-        total = self.offset
+        total = prev + S
+        fill = ops.StorageFill()
+        self._ensure_storage(B, H, S, device, incoming=S, fill=fill)
+        dtypes = [values.dtype] if self.v_only else [keys.dtype, values.dtype]
+        fresh = None if self.fused else self._fetch_buffers(B, H, prev, total, dtypes, device, fill)
+        zeros = [self._zero_like(t, fill) for t in ((keys, values) if self.fused else (keys,) if self.v_only else ())]
+        fill.run()
+        if self.v_only:
+            self._encode(values, self._v_q, self.v_packed, self.v_norms, B, H, S, v_dim, prev)
+        else:
+            self._encode_pair(keys, values, B, H, S, k_dim, v_dim, prev)
+        self.offset = total
 
         if self.fused:
             # zero placeholders of the right shape that own no memory (stride-0 views)
-            return (self._zero_like(keys).expand(B, H, total, k_dim),
-                    self._zero_like(values).expand(B, H, total, v_dim))
-
-        incremental = S <= 4 and self._v_deq_buf is not None and self._deq_offset == prev
-
+            return zeros[0].expand(B, H, total, k_dim), zeros[1].expand(B, H, total, v_dim)
+        out = self._fetch(fresh, B, H, prev, total, dtypes)
         if self.v_only:
-            if incremental:
-                self._v_deq_buf = self._incremental(self.v_packed, self.v_norms, self._v_q, v_dim,
-                                                    self._v_deq_buf, B, H, prev, total, values.dtype)
-                self._deq_alloc = self._v_deq_buf.shape[2]
-            else:
-                self._v_deq_buf, self._deq_alloc = self._prefill_buffer(
-                    self.v_packed, self.v_norms, self._v_q, v_dim, B, H, total, values.dtype)
-            self._deq_offset = total
-            return self._zero_like(keys).expand(B, H, total, k_dim), self._v_deq_buf[..., :total, :]
+            return zeros[0].expand(B, H, total, k_dim), out[0]
+        return out[0], out[1]
 
-        if incremental:
-            self._k_deq_buf = self._incremental(self.k_packed, self.k_norms, self._k_q, k_dim,
-                                                self._k_deq_buf, B, H, prev, total, keys.dtype)
-            self._v_deq_buf = self._incremental(self.v_packed, self.v_norms, self._v_q, v_dim,
-                                                self._v_deq_buf, B, H, prev, total, values.dtype)
-            self._deq_alloc = self._v_deq_buf.shape[2]
+    def _fetch_buffers(self, B, H, prev, total, dtypes, device, fill):
+        """The dequantised buffers a fetch of the first `total` positions goes to: None where the new rows join the present
+        ones (cache.py:171-180, 192-207), else fresh step-rounded ones, whose tails join `fill` (cache.py:182-188, 208-218)."""
+        if total - prev <= 4 and self._v_deq_buf is not None and self._deq_offset == prev:
+            return None
+        bufs = self._buffers(B, H, _round_up(total, self.step), dtypes, device)
+        for buf in bufs:
+            fill.add(buf, buf.shape[3], total, buf.shape[2])
+        return bufs
+
+    def _fetch(self, fresh, B, H, prev, total, dtypes):
+        """Dequantise into the buffers of _fetch_buffers; views of their first `total` positions."""
+        if fresh is None:
+            bufs = self._incremental([self._v_deq_buf] if self.v_only else [self._k_deq_buf, self._v_deq_buf],
+                                     B, H, prev, total, dtypes)
         else:
-            self._k_deq_buf, _ = self._prefill_buffer(self.k_packed, self.k_norms, self._k_q, k_dim,
-                                                      B, H, total, keys.dtype)
-            self._v_deq_buf, self._deq_alloc = self._prefill_buffer(
-                self.v_packed, self.v_norms, self._v_q, v_dim, B, H, total, values.dtype)
+            bufs = fresh
+            self._dequant_rows(bufs, B, H, 0, total, 0)
+        self._v_deq_buf = bufs[-1]
+        if not self.v_only:
+            self._k_deq_buf = bufs[0]
+        self._deq_alloc = self._v_deq_buf.shape[2]
         self._deq_offset = total
-        return self._k_deq_buf[..., :total, :], self._v_deq_buf[..., :total, :]
+        return [buf[:, :, :total] for buf in bufs]
+
+    def fetch_values(self, prev, dtype):
+        """The dequantised values of a v_only cache whose positions from `prev` on an owner has encoded itself."""
+        B, H = self.v_packed.shape[:2]
+        fill = ops.StorageFill()
+        fresh = self._fetch_buffers(B, H, prev, self.offset, [dtype], self.v_packed.device, fill)
+        fill.run()
+        return self._fetch(fresh, B, H, prev, self.offset, [dtype])[0]
 
     # ---------------------------------------------------------------- cache.py:220-247
     def empty(self):
@@ -446,7 +519,7 @@ class TurboQuantKVCache:
         if obj.v_packed is not None:
             obj._v_pdim = obj.v_packed.shape[-1]
         if obj._k_dim is not None and obj._v_dim is not None:
-            obj._ensure_quantizer(obj._k_dim, obj._v_dim)
+            obj._ensure_quantizer(obj._k_dim, obj._v_dim, in_order=False)
         return obj
 
     # ---------------------------------------------------------------- from_kvcache

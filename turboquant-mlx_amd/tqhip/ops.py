@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import weakref
 
 import torch
 
@@ -62,20 +63,32 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _host_table(x):
-    """Small table (boundaries / centroids) as a ctypes float array.  Accepts tensors, lists."""
-    if isinstance(x, torch.Tensor):
-        key = (x.data_ptr(), x._version, x.numel())
-        hit = _host_table.cache.get(key)
-        if hit is None:
-            hit = _lib.host_floats(x.detach().float().cpu().tolist())
-            if len(_host_table.cache) > 256:
-                _host_table.cache.clear()
-            _host_table.cache[key] = hit
-        return hit
-    return _lib.host_floats(x)
+    """Small table (boundaries / centroids) as the library takes it: a ctypes float array, or the address of a float32
+    CPU tensor's data (read during the call only).  Accepts tensors, lists."""
+    if not isinstance(x, torch.Tensor):
+        return _lib.host_floats(x)
+    if x.is_cuda:
+        return _device_table(x)
+    if x.dtype == torch.float32 and x.is_contiguous():
+        return x.data_ptr()
+    return _lib.host_floats(x.tolist())
 
 
-_host_table.cache = {}
+_device_tables = {}
+
+
+def _device_table(x: torch.Tensor):
+    """Host copy of a table that a caller keeps on the GPU, made once per tensor (a copy synchronises, and cannot run
+    under HIP-graph capture).  Held with a weak reference to the tensor and its version: another tensor at the same
+    address, or the same one after an in-place change, is copied anew."""
+    hit = _device_tables.get(id(x))
+    if hit is not None and hit[0]() is x and hit[1] == x._version:
+        return hit[2]
+    table = _lib.host_floats(x.detach().float().cpu().tolist())
+    if len(_device_tables) > 256:
+        _device_tables.clear()
+    _device_tables[id(x)] = (weakref.ref(x), x._version, table)
+    return table
 
 
 def _as_f32_dev(x, like: torch.Tensor) -> torch.Tensor:
@@ -175,6 +188,80 @@ def encode_into(x: torch.Tensor, signs: torch.Tensor, boundaries, packed: torch.
         C.c_void_p(norms.data_ptr() + norms_row_offset * 4),
         n_groups, rows_per_group, packed_group_stride, norms_group_stride,
         dim, bits, var, _stream(x)))
+
+
+def encode_kv_into(k: torch.Tensor, k_signs, k_packed, k_norms, v: torch.Tensor, v_signs, v_packed, v_norms, boundaries, *,
+                   n_groups: int, rows_per_group: int, group_stride: int, dim: int, bits: int, variant: str = "mlx",
+                   row_offset: int = 0) -> None:
+    """encode_into for key rows and value rows of one dtype and shape in one launch (tq_encode_kv); group_stride (rows)
+    is that of all four destinations."""
+    _need_gpu(k, k_signs, k_packed, k_norms, v, v_signs, v_packed, v_norms)
+    k, v = k.contiguous(), v.contiguous()
+    words, floats = row_offset * packed_dim(dim, bits) * 4, row_offset * 4
+    _lib.check(_lib.load().tq_encode_kv(
+        k.data_ptr(), k_signs.data_ptr(), k_packed.data_ptr() + words, k_norms.data_ptr() + floats,
+        v.data_ptr(), v_signs.data_ptr(), v_packed.data_ptr() + words, v_norms.data_ptr() + floats,
+        _dt(k), _host_table(boundaries), n_groups, rows_per_group, group_stride, group_stride, dim, bits,
+        {"mlx": _lib.TQ_ENCODE_MLX, "metal": _lib.TQ_ENCODE_METAL}[variant], _stream(k)))
+
+
+def dequant_kv_into(k_packed, k_norms, k_signs, k_out: torch.Tensor, v_packed, v_norms, v_signs, v_out: torch.Tensor, centroids, *,
+                    n_groups: int, rows_per_group: int, group_stride: int, out_group_stride: int, dim: int, bits: int,
+                    row_offset: int = 0, out_row_offset: int = 0) -> None:
+    """dequant_into for keys and values of one shape and output dtype in one launch (tq_dequant_kv)."""
+    _need_gpu(k_packed, k_norms, k_signs, k_out, v_packed, v_norms, v_signs, v_out)
+    words, floats = row_offset * packed_dim(dim, bits) * 4, row_offset * 4
+    at = out_row_offset * dim * k_out.element_size()
+    _lib.check(_lib.load().tq_dequant_kv(
+        k_packed.data_ptr() + words, k_norms.data_ptr() + floats, k_signs.data_ptr(), k_out.data_ptr() + at,
+        v_packed.data_ptr() + words, v_norms.data_ptr() + floats, v_signs.data_ptr(), v_out.data_ptr() + at,
+        _host_table(centroids), _dt(k_out), n_groups, rows_per_group, group_stride, group_stride, out_group_stride, dim, bits,
+        _stream(k_out)))
+
+
+class StorageFill:
+    """Collects what fresh cache storage needs besides its new rows -- the prefix of the storage it replaces, zeros behind
+    the new rows -- and does it in one launch (tq_fill_rows).  Keeps the tensors alive until then."""
+
+    def __init__(self):
+        self._segments, self._keep = [], []
+
+    def add(self, dst: torch.Tensor, inner: int, zero_from: int, zero_to: int, src: torch.Tensor | None = None, src_stride: int = 0,
+            copy: int = 0) -> None:
+        """dst: contiguous [..., T, inner] (or [..., T] with inner 1), its leading axes are the groups: rows `copy` from src
+        (rows src_stride apart per group) first, zeros in rows zero_from .. zero_to - 1."""
+        if copy == 0 and zero_to <= zero_from:
+            return
+        if not dst.is_cuda:                                  # storage of a cache that has not met the GPU yet
+            axis = dst.dim() - (2 if inner > 1 else 1)
+            if copy:
+                dst.narrow(axis, 0, copy).copy_(src.narrow(axis, 0, copy))
+            dst.narrow(axis, zero_from, max(0, zero_to - zero_from)).zero_()
+            return
+        row = inner * dst.element_size()
+        rows = dst.shape[-2] if inner > 1 else dst.shape[-1]
+        groups = dst.numel() // max(1, rows * inner)
+        from_ = (0, 0) if src is None else (src.data_ptr(), src_stride * row)
+        self._segments.append((dst.data_ptr(), from_[0], rows * row, from_[1], copy * row,
+                               zero_from * row, max(zero_from, zero_to) * row, groups))
+        self._keep.append((dst, src))
+
+    def run(self) -> None:
+        segs, self._segments = self._segments, []
+        for at in range(0, len(segs), _lib.FILL_MAX_SEGMENTS):
+            part = segs[at:at + _lib.FILL_MAX_SEGMENTS]
+            arr = (_lib.FillSegment * len(part))(*part)
+            _lib.check(_lib.load().tq_fill_rows(arr, len(part), _stream(self._keep[0][0])))
+        self._keep = []
+
+
+def random_signs(seeds, dim: int, device) -> torch.Tensor:
+    """(len(seeds), dim) float32 rows of +-1, row i = sign_pattern(dim, seeds[i]) of the rotation module, made on the GPU on
+    the current stream (tq_random_signs)."""
+    out = torch.empty((len(seeds), dim), dtype=torch.float32, device=device)
+    arr = (C.c_uint64 * len(seeds))(*[s & 0xFFFFFFFFFFFFFFFF for s in seeds])
+    _lib.check(_lib.load().tq_random_signs(arr, len(seeds), dim, out.data_ptr(), _stream(out)))
+    return out
 
 
 def vonly_append_into(keys: torch.Tensor, values: torch.Tensor, signs: torch.Tensor, boundaries,

@@ -37,7 +37,7 @@ class VOnlyTurboQuantCache:
         B, H, S, v_dim = values.shape
         tq._dtype = keys.dtype
         tq._ensure_quantizer(keys.shape[-1], v_dim, values.device)
-        tq._ensure_storage(B, H, S, values.device)
+        tq._ensure_storage(B, H, S, values.device, incoming=S)
         tq._encode(values, tq._v_q, tq.v_packed, tq.v_norms, B, H, S, v_dim, tq.offset)
         tq.offset += S
 
@@ -61,8 +61,8 @@ class VOnlyTurboQuantCache:
         if have_v != n or not tq.v_packed.is_contiguous() or not tq.v_norms.is_contiguous():
             tq._reallocate(B, H, n, device)
 
-    # Decode-sized inserts of a fused cache go through one launch (key rows to float16, value rows
-    # raw and encoded) instead of two slice assignments, a cast and the encoder.
+    # Decode-sized inserts go through one launch (key rows to float16, value rows raw and encoded) instead of two
+    # slice assignments, a cast and the encoder.
     _FUSED_APPEND_MAX_TOKENS = 16
 
     def _append_fused(self, keys, values) -> bool:
@@ -174,7 +174,9 @@ class VOnlyTurboQuantCache:
         # The decode kernels read float16 keys: bf16 / float32 keys are stored as float16 (exact for bf16
         # values inside the float16 range, which keys are); the reference keeps whatever dtype it is
         # given (v_only_cache.py:41-47), so `state` then differs in the dtype of its first entry.
-        if self.fused and self._append_fused(keys, values):
+        prev = self._v_tq.offset
+        appended = self._append_fused(keys, values)
+        if appended:
             k_out = self._k_cache.keys[..., :self._k_cache.offset, :]
         else:
             k16 = keys if keys.dtype == torch.float16 else keys.to(torch.float16)
@@ -187,18 +189,16 @@ class VOnlyTurboQuantCache:
             if self._zero is None or self._zero_key != key:          # one element, made once
                 self._zero, self._zero_key = torch.zeros((1, 1, 1, 1), dtype=values.dtype, device=values.device), key
             return k_out, self._zero.expand(B, H, self._v_tq.offset, v_dim)
+        tq = self._v_tq
+        B, H, S, v_dim = values.shape
         if self._no_v_buffer:                                    # v_only_cache.py:54-75
-            tq = self._v_tq
-            B, H, S, v_dim = values.shape
-            tq._dtype = keys.dtype
-            tq._ensure_quantizer(keys.shape[-1], v_dim, values.device)
-            tq._ensure_storage(B, H, S, values.device)
-            prev = tq.offset
-            tq._encode(values, tq._v_q, tq.v_packed, tq.v_norms, B, H, S, v_dim, prev)
-            tq.offset += S
+            if not appended:
+                self._encode_only(keys, values)
             v_out = tq._full_dequant(tq.v_packed, tq.v_norms, tq._v_q, v_dim, B, H, tq.offset, values.dtype)
+        elif appended:
+            v_out = tq.fetch_values(prev, values.dtype)
         else:
-            _, v_out = self._v_tq.update_and_fetch(keys, values)
+            _, v_out = tq.update_and_fetch(keys, values)
         return k_out, v_out
 
     @property
@@ -235,7 +235,7 @@ class VOnlyTurboQuantCache:
             tq.meta_state = parts[3]
             tq._v_pdim = tq.v_packed.shape[-1]
             if tq._v_dim is not None:                     # usable at once (attention straight off the restored cache),
-                tq._ensure_quantizer(tq._v_dim, tq._v_dim, tq.v_packed.device)   # not only after the next insert
+                tq._ensure_quantizer(tq._v_dim, tq._v_dim, tq.v_packed.device, in_order=False)   # not only after the next insert
         return obj
 
     @classmethod
