@@ -182,6 +182,16 @@ int tq_fill_rows(const tq_fill_segment* segments, int n_segments, tq_stream_t st
 int tq_random_signs(const uint64_t* seeds /* HOST */, int n_seeds, int dim, float* signs, tq_stream_t stream);
 
 /*
+ * Index rows to packed words and back (reference turboquant_mlx/packing.py:26-56 and 59-87): rows of dim indices,
+ * integers of index_bytes = 1, 4 or 8 bytes, to rows of ceil(dim / vpw) words, and rows of words_per_row words to rows of
+ * dim <= words_per_row * vpw bytes.  Packing adds the shifted indices without masking them, modulo 2^32.
+ */
+int tq_pack_indices(const void* indices, int index_bytes, uint32_t* packed, int64_t n_rows, int dim, int bits,
+                    tq_stream_t stream);
+int tq_unpack_indices(const uint32_t* packed, uint8_t* indices, int64_t n_rows, int words_per_row, int dim, int bits,
+                      tq_stream_t stream);
+
+/*
  * q_rot[h] = butterfly(q[h] * signs), no 1/sqrt(dim).
  * Replaces prerotate_query (metal_kernels_v4.py:119-150, kernel 37-62).
  *   q [n_heads, dim] dtype q_dtype -> q_rot [n_heads, dim] float32

@@ -144,12 +144,25 @@ def _head_layout_2d(t: torch.Tensor) -> tuple[torch.Tensor, int]:
 
 # ------------------------------------------------------------------ packing (integer plumbing)
 
+def _native_pack(t: torch.Tensor) -> bool:
+    """Integer plumbing also runs on the CPU, on tensor subclasses and under functional transforms: as tensor operations."""
+    return t.is_cuda and t.numel() > 0 and type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+
+
 def pack_indices(indices: torch.Tensor, bits: int) -> torch.Tensor:
     """packing.py:26-56.  (..., dim) integer indices -> (..., packed_dim) uint32."""
     vpw = VALS_PER_WORD[bits]
     shape = indices.shape
     dim = shape[-1]
     pd = packed_dim(dim, bits)
+    if _native_pack(indices):
+        if indices.dtype not in (torch.uint8, torch.int32, torch.int64):
+            indices = indices.to(torch.int64)
+        flat = indices.contiguous()
+        out = torch.empty((*shape[:-1], pd), dtype=torch.uint32, device=flat.device)
+        _lib.check(_lib.load().tq_pack_indices(flat.data_ptr(), flat.element_size(), out.data_ptr(), flat.numel() // dim,
+                                               dim, bits, _stream(flat)))
+        return out
     flat = indices.reshape(-1, dim).to(torch.int64)
     if dim % vpw:
         flat = torch.nn.functional.pad(flat, (0, pd * vpw - dim))
@@ -163,6 +176,13 @@ def unpack_indices(packed: torch.Tensor, bits: int, dim: int) -> torch.Tensor:
     """packing.py:59-87.  (..., packed_dim) uint32 -> (..., dim) uint8."""
     vpw = VALS_PER_WORD[bits]
     shape = packed.shape
+    if dim > 0 and _native_pack(packed):
+        words = _u32(packed).contiguous()
+        dim = min(dim, shape[-1] * vpw)
+        out = torch.empty((*shape[:-1], dim), dtype=torch.uint8, device=words.device)
+        _lib.check(_lib.load().tq_unpack_indices(words.data_ptr(), out.data_ptr(), words.numel() // shape[-1], shape[-1],
+                                                 dim, bits, _stream(words)))
+        return out
     w = _u32(packed).contiguous().view(torch.int32).to(torch.int64) & 0xFFFFFFFF
     shifts = torch.arange(vpw, device=w.device, dtype=torch.int64) * bits
     vals = (w.unsqueeze(-1) >> shifts) & BIT_MASK[bits]
