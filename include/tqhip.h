@@ -306,9 +306,20 @@ int tq_flash_decode(const float* q_rot,
                     const tq_decode_shape* shape /* host */, tq_stream_t stream);
 
 /*
+ * An attention mask as the additive float32 rows that the decode kernels read: mask[s * seq_stride + h * head_stride +
+ * p * pos_stride] (strides in elements) of a tq_dtype or TQ_MASK_BOOL (bytes; nonzero = attend: 0, else -inf) to
+ * out[(s * n_heads + h) * row_len + p], p < seq_len <= row_len.  The mask preparation of turboquant_attention
+ * (fused_attention.py:81-92).
+ */
+#define TQ_MASK_BOOL 3
+int tq_mask_rows(const void* mask, int mask_dtype, int64_t seq_stride, int64_t head_stride, int64_t pos_stride, float* out,
+                 int n_seq, int n_heads, int64_t seq_len, int64_t row_len, tq_stream_t stream);
+
+/*
  * Which tile pass tq_flash_decode takes on the matrix-core path for a batch of this shape:
  * 0 = one workgroup per 512-position tile; n >= 2 = the streaming pass, one workgroup per
- * n * 256 consecutive positions (large unmasked batches).  Informational: lets a caller or a test
+ * n * 256 consecutive positions (large batches; masked != 0: a mask with a row per query head -- one that the
+ * heads share counts as none).  Informational: lets a caller or a test
  * know which kernel a shape exercises.  No counterpart in the reference (one kernel per call,
  * flash_attention.py:168-274).  The plan sees no pointers: it describes three-bit tensors (rows at any
  * 4-byte offset) and tensors of widths 1, 2 and 4 that are 16-byte aligned; tq_flash_decode sends a

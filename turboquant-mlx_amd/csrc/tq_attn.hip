@@ -1022,7 +1022,8 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
   int tile_pos = tqm::kTilePos;
   a.len_dev = len_dev; a.len_bias = len_bias;             // a length read on the device: an upper bound on the host, like a ragged batch
   // the streaming pass takes rows at any 4-byte offset at three bits only (the other widths: 16-byte aligned tensors)
-  const bool stream_ok = MODE == tqm::kFlash && !sh.mask &&
+  // and a mask only where the query heads share it (one value per position)
+  const bool stream_ok = MODE == tqm::kFlash && (!sh.mask || sh.mask_head_stride == 0) &&
                          (sh.bits == 3 || (tq::aligned(k_packed, 16) && tq::aligned(v_packed, 16)));
   const int n_steps = stream_ok ? flash_stream_steps(sh.n_seq, sh.n_kv_heads, sh.seq_len,
                                                      sh.seq_offsets != nullptr || len_dev != nullptr) : 0;
@@ -1424,6 +1425,49 @@ extern "C" int tq_sparse_v_matvec(const float* weights, const uint32_t* v_packed
   return launch_decode<kWeights>(weights, TQ_F32, nullptr, nullptr, nullptr, v_packed, v_norms, nullptr,
                                  centroids, signs, out, workspace, workspace_bytes, sh, thr,
                                  (hipStream_t)stream_, "tq_sparse_v_matvec");
+}
+
+namespace {
+// Rows of an attention mask in any of its forms as the additive float32 rows that the kernels read: bool (true = attend)
+// becomes 0 / -inf, the 16-bit types are widened.  A handful of microseconds of tensor operations and one full copy per
+// query head otherwise (8 sequences, 6003 positions, boolean padding mask: 24 launches, 154 us of host time).
+struct MaskRows {
+  const void* mask;
+  float* out;
+  int64_t seq_stride, head_stride, pos_stride, seq_len, row_len;
+  int32_t n_heads, dtype;
+};
+
+__global__ __launch_bounds__(256) void mask_rows_kernel(MaskRows a) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p >= a.seq_len) return;
+  const int head = blockIdx.y, seq = blockIdx.z;
+  const int64_t at = seq * a.seq_stride + head * a.head_stride + p * a.pos_stride;
+  float v;
+  if (a.dtype == TQ_MASK_BOOL) v = reinterpret_cast<const uint8_t*>(a.mask)[at] ? 0.0f : -INFINITY;
+  else if (a.dtype == TQ_F16) v = __half2float(reinterpret_cast<const __half*>(a.mask)[at]);
+  else if (a.dtype == TQ_BF16) v = __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(a.mask)[at] << 16);
+  else v = reinterpret_cast<const float*>(a.mask)[at];
+  a.out[((int64_t)seq * a.n_heads + head) * a.row_len + p] = v;
+}
+}  // namespace
+
+extern "C" int tq_mask_rows(const void* mask, int mask_dtype, int64_t seq_stride, int64_t head_stride, int64_t pos_stride,
+                            float* out, int n_seq, int n_heads, int64_t seq_len, int64_t row_len, tq_stream_t stream_) {
+  const char* who = "tq_mask_rows";
+  if (mask_dtype != TQ_MASK_BOOL && tq::check_dtype(mask_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown dtype %d", who, mask_dtype);
+  if (n_seq < 0 || n_heads < 0 || seq_len < 0 || row_len < seq_len || n_seq > 65535 || n_heads > 65535 || seq_len >= (int64_t)1 << 38)
+    return tq::fail(TQ_ERR_ARG, "%s: %d x %d rows of %lld positions at a stride of %lld", who, n_seq, n_heads, (long long)seq_len,
+                    (long long)row_len);
+  if (n_seq == 0 || n_heads == 0 || seq_len == 0) return TQ_OK;
+  if (!mask || !out) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if ((mask_dtype != TQ_MASK_BOOL && !tq::aligned(mask, tq::dtype_size(mask_dtype))) || !tq::aligned(out, 4))
+    return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+  const dim3 grid((unsigned)((seq_len + 255) / 256), n_heads, n_seq);
+  mask_rows_kernel<<<grid, 256, 0, (hipStream_t)stream_>>>(
+      MaskRows{mask, out, seq_stride, head_stride, pos_stride, seq_len, row_len, n_heads, mask_dtype});
+  TQ_CHECK_LAUNCH("tq_mask_rows launch");
+  return TQ_OK;
 }
 
 extern "C" int tq_flash_decode_plan(int n_seq, int n_kv_heads, int64_t max_seq_len, int ragged, int masked) {

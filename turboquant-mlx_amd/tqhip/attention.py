@@ -54,7 +54,9 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
     if fused and v_buffer is None and (thr == 0.0 or one_call_thr):
         m = None
         if mask is not None:
-            m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
+            m = ops.decode_mask_rows(mask, B, n_q, total, queries.device)
+            if m is None:
+                m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
         od = queries.dtype if queries.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
         if ops.vonly_sparse_supported(dim, bits, n_rep) and total > 0 and dim == cache._v_dim:
             # one call: the kernels rotate the query themselves
@@ -116,7 +118,9 @@ def vonly_decode_attention(queries: torch.Tensor, cache, attn_scale: float, mask
     if thr == 0.0 or (ops.vonly_threshold_supported(dim, bits, n_rep) and total > 0):
         m = None
         if mask is not None:
-            m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
+            m = ops.decode_mask_rows(mask, B, n_q, total, queries.device)
+            if m is None:
+                m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
         od = queries.dtype if queries.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
         out = ops.vonly_decode(queries[:, :, 0, :], kc.keys, tq.v_packed, tq.v_norms, vq.centroids, vq.signs,
                                dim, bits, attn_scale, n_rep=n_rep, seq_len=total, mask=m, out_dtype=od,

@@ -647,10 +647,43 @@ def _mask_layout(mask, n_seq: int, n_q: int, seq_len: int, device):
         m = m.unsqueeze(0)
     if m.shape[-1] != seq_len or m.shape[0] not in (1, n_seq) or m.shape[1] not in (1, n_q):
         raise ValueError(f"mask shape {tuple(mask.shape)} not broadcastable to ({n_seq}, {n_q}, {seq_len})")
-    m = m.contiguous()
-    ss = m.shape[1] * seq_len if m.shape[0] == n_seq and n_seq > 1 else 0
-    hs = seq_len if m.shape[1] == n_q and n_q > 1 else 0
+    if m.dim() > 3 or m.stride(-1) != 1 or min(m.stride()) < 0:
+        m = m.contiguous()
+    ss = m.stride(0) if m.shape[0] == n_seq and n_seq > 1 else 0
+    hs = m.stride(1) if m.shape[1] == n_q and n_q > 1 else 0
     return m, (ss, hs)
+
+
+_MASK_DTYPES = {torch.bool: _lib.TQ_MASK_BOOL, **_DTYPES}
+
+
+def decode_mask_rows(mask: torch.Tensor, n_seq: int, n_q: int, seq_len: int, device):
+    """A mask of a decode step in the forms of fused_attention.py:81-92 -- (B, H, 1, T), (B, 1, T), (H, T) or (T,) -- as
+    additive float32 rows (1 or n_seq, 1 or n_q, T): the mask's own memory where it is float32 already, else one launch
+    (tq_mask_rows).  None for forms that need more than that (the caller builds the rows with tensor operations)."""
+    if mask.device != device or mask.dtype not in _MASK_DTYPES or type(mask) is not torch.Tensor:
+        return None
+    d = mask.dim()
+    if d == 4:
+        m = mask[:, :, 0, :]
+    elif d == 3:
+        m = mask[:, 0:1, :]
+    elif d in (1, 2):
+        m = mask[None] if d == 2 else mask[None, None]
+    else:
+        return None
+    b, h, t = m.shape
+    if t != seq_len or t == 0 or h not in (1, n_q) or b == 0 or 1 < b < n_seq:
+        return None
+    m = m[:n_seq]
+    b = m.shape[0]
+    if m.dtype == torch.float32 and m.stride(2) == 1:
+        return m
+    row_len = (t + 3) // 4 * 4                        # 16-byte rows: the kernels read four positions at a time
+    out = torch.empty((b, h, row_len), dtype=torch.float32, device=m.device)
+    sb, sh, st = m.stride()
+    _lib.check(_lib.load().tq_mask_rows(m.data_ptr(), _MASK_DTYPES[m.dtype], sb, sh, st, out.data_ptr(), b, h, t, row_len, _stream(m)))
+    return out[:, :, :t]
 
 
 def flash_decode(q_rot: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids,
