@@ -586,6 +586,25 @@ int tq_prefill_attn(const void* q, int q_dtype,
 size_t tq_prefill_workspace_bytes(int n_q_heads, int64_t n_rows, int64_t kv_len, int dim);
 
 /*
+ * tq_prefill_attn for a batch of sequences of one length in one call: q and out [n_seq, n_kv*n_rep, n_rows, dim], the rows of
+ * sequence s and kv head h of a packed tensor / norms at s * *_seq_stride + h * *_head_stride (rows).  Workspace:
+ * tq_prefill_batch_workspace_bytes, 256-byte aligned.
+ */
+int tq_prefill_attn_batch(const void* q, int q_dtype,
+                          const uint32_t* k_packed, const float* k_norms,
+                          const uint32_t* v_packed, const float* v_norms,
+                          const float* k_centroids /* host */, const float* v_centroids /* host */,
+                          const float* k_signs, const float* v_signs,
+                          void* out, int out_dtype, void* workspace, size_t workspace_bytes,
+                          int n_seq, int n_kv_heads, int n_rep, int64_t n_rows, int64_t kv_len, int64_t q_pos0,
+                          int64_t k_seq_stride, int64_t kn_seq_stride, int64_t v_seq_stride, int64_t vn_seq_stride,
+                          int64_t k_head_stride, int64_t kn_head_stride, int64_t v_head_stride, int64_t vn_head_stride,
+                          int dim, int bits, float attn_scale, int flags, tq_stream_t stream);
+
+size_t tq_prefill_batch_workspace_bytes(int n_seq, int n_kv_heads, int n_rep, int64_t n_rows, int64_t kv_len,
+                                        int64_t q_pos0, int dim, int flags);
+
+/*
  * Measurement aid, no counterpart in the reference (its benches time whole kernels with mx.eval,
  * scripts/bench_sparse_v.py:49-57): ONE launch that streams `bytes` bytes from `src` (16-byte aligned,
  * a multiple of 16) through n_workgroups workgroups (256 threads with eight loads in flight each; 512 threads with

@@ -108,6 +108,9 @@ PROTOTYPES = {
     "tq_prefill_attn": (_i, [_p, _i, _p, _p, _p, _p, _fp, _fp, _p, _p, _p, _i, _p, _z, _i, _i, _l, _l, _l,
                             _l, _l, _l, _l, _i, _i, _f, _i, _p]),
     "tq_prefill_workspace_bytes": (_z, [_i, _l, _l, _i]),
+    "tq_prefill_attn_batch": (_i, [_p, _i, _p, _p, _p, _p, _fp, _fp, _p, _p, _p, _i, _p, _z, _i, _i, _i, _l, _l, _l,
+                                  _l, _l, _l, _l, _l, _l, _l, _l, _i, _i, _f, _i, _p]),
+    "tq_prefill_batch_workspace_bytes": (_z, [_i, _i, _i, _l, _l, _l, _i, _i]),
     "tq_probe_read": (_i, [_p, _z, _p, _i, _z, _p]),
 }
 

@@ -154,9 +154,6 @@ def turboquant_prefill_attention(queries: torch.Tensor, cache, attn_scale: float
     n_kv = cache.k_packed.shape[1]
     n_rep = n_q // n_kv
     kq, vq = cache._k_q, cache._v_q
-    outs = [ops.prefill_attention(queries[b], cache.k_packed[b], cache.k_norms[b], cache.v_packed[b],
-                                  cache.v_norms[b], kq.centroids, vq.centroids, kq.signs, vq.signs, dim,
-                                  cache.quant_bits, attn_scale, n_rep=n_rep, kv_len=total, q_pos0=total - S,
-                                  causal=causal)
-            for b in range(B)]
-    return torch.stack(outs, dim=0)
+    return ops.prefill_attention_batch(queries, cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms, kq.centroids,
+                                       vq.centroids, kq.signs, vq.signs, dim, cache.quant_bits, attn_scale, n_rep=n_rep,
+                                       kv_len=total, q_pos0=total - S, causal=causal)

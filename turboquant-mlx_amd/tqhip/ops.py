@@ -1173,3 +1173,40 @@ def prefill_attention(q: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_c
         k_packed.stride(0) // pd, k_norms.stride(0), v_packed.stride(0) // pd, v_norms.stride(0),
         dim, bits, float(attn_scale), (1 if causal else 0) | (2 if fp16_query else 0), stream))
     return out
+
+
+def prefill_attention_batch(q: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, k_signs,
+                            v_signs, dim: int, bits: int, attn_scale: float, *, n_rep: int, kv_len: int, q_pos0: int,
+                            causal: bool = True) -> torch.Tensor:
+    """prefill_attention for every sequence of a cache in one launch (tq_prefill_attn_batch): q (B, n_q, n_rows, dim),
+    k_packed / v_packed (B, n_kv, T_alloc, pdim), k_norms / v_norms (B, n_kv, T_alloc) -> (B, n_q, n_rows, dim) in q's dtype
+    (float32 for one that is no kernel dtype)."""
+    _need_gpu(q, k_packed, k_norms, v_packed, v_norms)
+    B, n_q, n_rows, _ = q.shape
+    n_kv = k_norms.shape[1]
+    _check_gqa(n_q, n_kv, n_rep)
+    pd = packed_dim(dim, bits)
+    if q.dtype not in _DTYPES:
+        q = q.float()
+    q = q.contiguous()
+    k_packed, ks = _kv_layout(_u32(k_packed), pd, False)
+    v_packed, vs = _kv_layout(_u32(v_packed), pd, False)
+    k_norms, kns = _norm_layout(k_norms.to(torch.float32))
+    v_norms, vns = _norm_layout(v_norms.to(torch.float32))
+    _check_rows(kv_len, False, B, k_packed=k_packed, k_norms=k_norms, v_packed=v_packed, v_norms=v_norms)
+    out = torch.empty((B, n_q, n_rows, dim), dtype=q.dtype, device=q.device)
+    if n_rows == 0:
+        return out
+    k_signs = _as_f32_dev(k_signs, q)
+    v_signs = _as_f32_dev(v_signs, q)
+    flags = 1 if causal else 0
+    lib = _lib.load()
+    need = lib.tq_prefill_batch_workspace_bytes(B, n_kv, n_rep, n_rows, kv_len, q_pos0, dim, flags)
+    stream = _stream(q)
+    ws = _workspace(q.device, stream.value or 0, need)
+    _lib.check(lib.tq_prefill_attn_batch(
+        q.data_ptr(), _dt(q), k_packed.data_ptr(), k_norms.data_ptr(), v_packed.data_ptr(), v_norms.data_ptr(),
+        _host_table(k_centroids), _host_table(v_centroids), k_signs.data_ptr(), v_signs.data_ptr(), out.data_ptr(), _dt(out),
+        ws.data_ptr(), ws.numel(), B, n_kv, n_rep, n_rows, kv_len, q_pos0, ks[0], kns[0], vs[0], vns[0], ks[1], kns[1], vs[1],
+        vns[1], dim, bits, float(attn_scale), flags, stream))
+    return out
