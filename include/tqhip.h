@@ -544,6 +544,20 @@ int tq_flash_decode_from_q(const void* q, int q_dtype, const float* k_signs,
                            const tq_decode_shape* shape /* host */, tq_stream_t stream);
 
 /*
+ * The chain of turboquant_attention (fused_attention.py:56-121: prerotate_query -> prerot_fused_qk_scores -> * attn_scale + mask
+ * -> softmax -> sparse_v_matvec(threshold)) at float32 fidelity for a batch of one length in one call of three launches: the
+ * split operands of tq_prerot_qk_scores and tq_sparse_v_matvec (TQ_MMA_SPLIT), the softmax between them in float32.  Arguments
+ * as tq_flash_decode_from_q; workspace tq_vonly_sparse_workspace_bytes.  A row whose positions are all masked out is NaN, as in
+ * tq_softmax_rows.  dim 128, n_rep <= 16, a non-empty cache without seq_offsets (TQ_ERR_UNSUPPORTED otherwise).
+ */
+int tq_composed_decode(const void* q, int q_dtype, const float* k_signs,
+                       const uint32_t* k_packed, const float* k_norms,
+                       const uint32_t* v_packed, const float* v_norms,
+                       const float* k_centroids, const float* v_centroids, const float* v_signs,
+                       float threshold, void* out, void* workspace, size_t workspace_bytes,
+                       const tq_decode_shape* shape /* host */, tq_stream_t stream);
+
+/*
  * Bytes of workspace the op needs for this shape (host computation, no GPU call).  The workspace
  * holds per-tile partial results between the two passes of a call; its contents need not be
  * preserved or cleared between calls.  Calls that share a workspace must be ordered (same stream);

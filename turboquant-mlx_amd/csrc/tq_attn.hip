@@ -1085,6 +1085,30 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
   return TQ_OK;
 }
 
+// Merge pass of value sums whose weights are final.
+int launch_weights_merge(const float* ws_S, const float* ws_ml, int n_parts, int tile_pos, const float* v_signs, void* out,
+                         const tq_decode_shape& sh, hipStream_t stream, const char* who) {
+  dim3 mgrid(sh.n_kv_heads * sh.n_rep, sh.n_seq);
+  const float inv_dim = 1.0f / (float)sh.dim;
+  // partials per lane group and round: one round of loads where 64, 128 or 256 partials cover the sequence
+#define LAUNCH_MERGE_SU(TO, U_)                                                                             \
+  tqm::decode_merge_rows_kernel<TO, false, U_><<<mgrid, tqm::kMergeThreads, 0, stream>>>(                     \
+      ws_S, ws_ml, sh.seq_offsets, sh.seq_len, n_parts, sh.n_kv_heads, sh.n_rep, v_signs, inv_dim, (TO*)out, tile_pos)
+#define LAUNCH_MERGE_S(TO)                                                                                  \
+  do {                                                                                                      \
+    if (n_parts <= 64) LAUNCH_MERGE_SU(TO, 8);                                                              \
+    else if (n_parts <= 128) LAUNCH_MERGE_SU(TO, 16);                                                       \
+    else LAUNCH_MERGE_SU(TO, 32);                                                                           \
+  } while (0)
+  if (sh.out_dtype == TQ_F16) { LAUNCH_MERGE_S(__half); }
+  else if (sh.out_dtype == TQ_BF16) { LAUNCH_MERGE_S(__hip_bfloat16); }
+  else { LAUNCH_MERGE_S(float); }
+#undef LAUNCH_MERGE_S
+#undef LAUNCH_MERGE_SU
+  TQ_CHECK_LAUNCH(who);
+  return TQ_OK;
+}
+
 // Second and third pass of the thresholded decode steps: weights 2^(s - M) / L from the scores and per-tile
 // statistics, weights below the threshold dropped, value sums per tile; then the merge pass.
 int launch_soft_weights(const float* scores, const float* stats, int stats_tile_pos, float* ws_S, float* ws_ml, int64_t t_pad, int n_tiles,
@@ -1128,25 +1152,7 @@ int launch_soft_weights(const float* scores, const float* stats, int stats_tile_
   }
   TQ_CHECK_LAUNCH(who);
 
-  dim3 mgrid(n_q, sh.n_seq);
-  const float inv_dim = 1.0f / (float)sh.dim;
-  // partials per lane group and round: one round of loads where 64, 128 or 256 partials cover the sequence
-#define LAUNCH_MERGE_SU(TO, U_)                                                                             \
-  tqm::decode_merge_rows_kernel<TO, false, U_><<<mgrid, tqm::kMergeThreads, 0, stream>>>(                     \
-      ws_S, ws_ml, sh.seq_offsets, sh.seq_len, n_parts, sh.n_kv_heads, sh.n_rep, v_signs, inv_dim, (TO*)out, tile_pos)
-#define LAUNCH_MERGE_S(TO)                                                                                  \
-  do {                                                                                                      \
-    if (n_parts <= 64) LAUNCH_MERGE_SU(TO, 8);                                                              \
-    else if (n_parts <= 128) LAUNCH_MERGE_SU(TO, 16);                                                       \
-    else LAUNCH_MERGE_SU(TO, 32);                                                                           \
-  } while (0)
-  if (sh.out_dtype == TQ_F16) { LAUNCH_MERGE_S(__half); }
-  else if (sh.out_dtype == TQ_BF16) { LAUNCH_MERGE_S(__hip_bfloat16); }
-  else { LAUNCH_MERGE_S(float); }
-#undef LAUNCH_MERGE_S
-#undef LAUNCH_MERGE_SU
-  TQ_CHECK_LAUNCH(who);
-  return TQ_OK;
+  return launch_weights_merge(ws_S, ws_ml, n_parts, tile_pos, v_signs, out, sh, stream, who);
 }
 
 // Thresholded V-only decode on the matrix cores: scores pass (fp16 keys -> scores in log2 units + per-tile
@@ -1710,6 +1716,60 @@ extern "C" int tq_flash_decode_from_q(const void* q, int q_dtype, const float* k
   sh.allow_mma = 1;
   return launch_packed_mfma<tqm::kFlash>(nullptr, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs,
                                          out, workspace, workspace_bytes, sh, 0.0f, stream, who, q, q_dtype, k_signs);
+}
+
+extern "C" int tq_composed_decode(const void* q, int q_dtype, const float* k_signs, const uint32_t* k_packed,
+                                  const float* k_norms, const uint32_t* v_packed, const float* v_norms,
+                                  const float* k_centroids, const float* v_centroids, const float* v_signs,
+                                  float threshold, void* out, void* workspace, size_t workspace_bytes,
+                                  const tq_decode_shape* shape, tq_stream_t stream_) {
+  const char* who = "tq_composed_decode";
+  if (int rc = check_shape(shape, who, 128)) return rc;
+  const tq_decode_shape& sh = *shape;
+  if (tq::check_dtype(q_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown q_dtype %d", who, q_dtype);
+  if (!q || !k_signs || !k_centroids || !v_centroids || !v_signs || !out || !k_packed || !k_norms || !v_packed || !v_norms)
+    return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (!(threshold >= 0.0f)) return tq::fail(TQ_ERR_ARG, "%s: threshold must be >= 0", who);
+  if (!(sh.dim == 128 && sh.n_rep <= tqm::kHeadsMax && sh.seq_len > 0 && !sh.seq_offsets &&
+        tq::aligned(q, (int)tq::dtype_size(q_dtype))))
+    return tq::fail(TQ_ERR_UNSUPPORTED, "%s: dim 128, n_rep <= 16 and a non-empty cache of one length only "
+                                        "(compose tq_prerot_qk_scores, tq_softmax_rows and tq_sparse_v_matvec otherwise)", who);
+  const int n_q = sh.n_kv_heads * sh.n_rep;
+  const size_t need = vonly_sparse_ws_bytes(sh.n_seq, n_q, sh.seq_len);
+  if (!workspace || workspace_bytes < need)
+    return tq::fail(TQ_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
+  if (!tq::aligned(workspace, 16)) return tq::fail(TQ_ERR_ALIGN, "%s: workspace must be 16-byte aligned", who);
+  const int64_t t_pad = (sh.seq_len + 3) & ~(int64_t)3;
+  const int n_tiles = (int)((sh.seq_len + tqm::kTilePos - 1) / tqm::kTilePos);
+  float* scores = (float*)workspace;
+  float* stats = scores + (size_t)sh.n_seq * n_q * t_pad;
+  float* ws_S = stats + (((size_t)sh.n_seq * n_q * n_tiles * 2 + 3) & ~(size_t)3);
+  float* ws_ml = ws_S + (size_t)sh.n_seq * n_q * n_tiles * tqm::kD;
+  hipStream_t stream = (hipStream_t)stream_;
+  const dim3 grid(n_tiles, sh.n_kv_heads, sh.n_seq);
+
+  tqm::SplitArgs a{};
+  a.q_raw = q; a.q_dtype = q_dtype; a.k_signs = k_signs;
+  a.mask = sh.mask; a.mask_seq_stride = sh.mask_seq_stride; a.mask_head_stride = sh.mask_head_stride;
+  a.stats = stats; a.scores = scores; a.w_stride = t_pad;
+  a.packed = k_packed; a.norms = k_norms;
+  a.seq_stride = sh.k_seq_stride; a.head_stride = sh.k_head_stride;
+  a.norms_seq_stride = sh.kn_seq_stride; a.norms_head_stride = sh.kn_head_stride;
+  a.seq_len = sh.seq_len; a.n_kv = sh.n_kv_heads; a.n_rep = sh.n_rep; a.n_tiles = n_tiles;
+  a.scale = 1.0f / (float)sh.dim; a.scale2 = sh.attn_scale * tqm::kLog2e;
+  Codebook cb;
+  fill_codebook(cb, k_centroids, sh.bits);
+  launch_split_tiles_bits(sh.bits, tqm::kSoftScores, grid, a, cb, stream);
+  TQ_CHECK_LAUNCH(who);
+
+  a.weights = scores; a.packed = v_packed; a.norms = v_norms;
+  a.seq_stride = sh.v_seq_stride; a.head_stride = sh.v_head_stride;
+  a.norms_seq_stride = sh.vn_seq_stride; a.norms_head_stride = sh.vn_head_stride;
+  a.ws_S = ws_S; a.ws_ml = ws_ml; a.threshold = threshold;
+  fill_codebook(cb, v_centroids, sh.bits);
+  launch_split_tiles_bits(sh.bits, tqm::kSoftWeights, grid, a, cb, stream);
+  TQ_CHECK_LAUNCH(who);
+  return launch_weights_merge(ws_S, ws_ml, n_tiles, tqm::kTilePos, v_signs, out, sh, stream, who);
 }
 
 extern "C" int tq_vonly_decode_step_at(const tq_vonly_cache_desc* c, const void* k_new, int k_dtype, const void* v_new,

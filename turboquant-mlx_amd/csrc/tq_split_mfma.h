@@ -17,6 +17,12 @@
 //   weights    p = w * norm in float32 (the reference's order, (w * norm) * c), positions below the threshold
 //              dropped, then scaled per wave by a power of two that puts the wave's largest p near 2^13 -- so that
 //              weights many decades below the largest still have normal hi and lo parts -- and split.
+//
+// The composed decode step (pre-rotation, scores, softmax, thresholded value sum: tq_composed_decode) takes the same two passes
+// as kSoftScores and kSoftWeights, for a batch: the query is rotated inside, the scores leave scaled and masked in log2 units
+// with the statistics (maximum, sum of 2^(s - maximum)) of each tile, and the value pass makes the weights 2^(s - M) / L of the
+// whole row itself.  As five operations (rotation, scores, a row softmax that reads every score eleven times, values, merge)
+// plus a conversion and a copy, 28 / 4 heads over 65 536 positions took 60 us, of which the softmax 18; in three launches 31.
 #pragma once
 
 #include "tq_packed_mfma.h"
@@ -50,11 +56,18 @@ __device__ __forceinline__ void fill_split_table(uint2* lut, const Codebook& cb,
 
 struct SplitArgs {
   const float* q_rot;         // scores: [n_q, 128] f32, pre-rotated
-  const float* weights;       // values: [n_q, w_stride] f32
+  const void* q_raw;          // kSoftScores: [n_seq, n_q, 128] of q_dtype, rotated inside
+  const float* k_signs;
+  const float* mask;          // kSoftScores: additive rows or NULL
+  float* stats;               // soft modes: [n_seq * n_kv, n_tiles, n_rep, 2]
+  int64_t seq_stride, norms_seq_stride, mask_seq_stride, mask_head_stride;
+  int32_t q_dtype;
+  float scale2;               // kSoftScores: attention scale times log2 e
+  const float* weights;       // values: [n_seq * n_q, w_stride] f32 weights; kSoftWeights: scores in log2 units
   int64_t w_stride;
   const uint32_t* packed;     // keys (scores) or values
   const float* norms;
-  float* scores;              // scores: [n_q, seq_len] f32
+  float* scores;              // scores: [n_q, seq_len] f32; kSoftScores: [n_seq * n_q, w_stride]
   float* ws_S;                // values: partial sums [n_kv, n_tiles, n_rep, 128]
   float* ws_ml;               //         their (0, sum of weights) pairs
   int64_t seq_len;
@@ -64,26 +77,29 @@ struct SplitArgs {
   float threshold;            // values
 };
 
-// MODE = kScores or kWeights.  grid = (n_tiles, n_kv), 512 threads.
+// MODE = kScores, kWeights: grid = (n_tiles, n_kv); kSoftScores, kSoftWeights: (n_tiles, n_kv, n_seq).  512 threads.
 template <int MODE, int BITS>
 __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void split_tile_kernel(SplitArgs a, Codebook cb) {
   using VF = VField<BITS>;
   constexpr int kPd = VF::kPd;
-  constexpr bool SCORES = MODE == kScores;
+  constexpr bool SCORES = MODE == kScores || MODE == kSoftScores;
+  constexpr bool SOFT_S = MODE == kSoftScores, SOFT_W = MODE == kSoftWeights;
   __shared__ __align__(16) unsigned char big_s[32768];      // per-wave 4 KB areas, later the merge deposits
   __shared__ __align__(16) uint2 lut_s[VF::kLut < 64 ? 64 : VF::kLut];
   __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];
   __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kD / 2];
   __shared__ __align__(16) float n_s[kWaves][kWavePos];
   __shared__ __align__(16) MergeLds<kWaves> mg_s;
+  __shared__ float m_s[kWaves][kHeadsMax], l_s[kWaves][kHeadsMax];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int n16 = lane & 15, g = lane >> 4;
-  const int tile = blockIdx.x, kvh = blockIdx.y;
+  const int tile = blockIdx.x, kvh = blockIdx.y, seq = (SOFT_S || SOFT_W) ? blockIdx.z : 0;
   const int n_rep = a.n_rep;
-  const int64_t q_row0 = (int64_t)kvh * n_rep;
+  const int64_t grp = (int64_t)seq * a.n_kv + kvh;
+  const int64_t q_row0 = grp * n_rep;
   const int64_t len = a.seq_len;
   const int64_t tile_p0 = (int64_t)tile * kTilePos;
   if (tile_p0 >= len) return;
@@ -95,16 +111,17 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
 
   // ---- loads ----------------------------------------------------------------------------------------------------
   float2 my_q[2];
-  if (SCORES) {
+  if (MODE == kScores) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int w = tid + i * kMfmaThreads;
       my_q[i] = (w < n_rep * (kD / 2)) ? reinterpret_cast<const float2*>(a.q_rot + q_row0 * kD)[w] : make_float2(0.f, 0.f);
     }
   }
-  const float my_n = a.norms[(int64_t)kvh * a.norms_head_stride + tile_p0 + crow];
+  const int64_t seq_rows = (SOFT_S || SOFT_W) ? (int64_t)seq * a.seq_stride : 0;
+  const float my_n = a.norms[((SOFT_S || SOFT_W) ? (int64_t)seq * a.norms_seq_stride : 0) + (int64_t)kvh * a.norms_head_stride + tile_p0 + crow];
   PackedBlockT<kPd> blk;
-  load_block<MODE == kWeights>(blk, a.packed + ((int64_t)kvh * a.head_stride + tile_p0 + wrow0) * kPd, lane, wrow0, rows_here);
+  load_block<!SCORES>(blk, a.packed + (seq_rows + (int64_t)kvh * a.head_stride + tile_p0 + wrow0) * kPd, lane, wrow0, rows_here);
   // given weights: lane (head n16, group g) takes positions 16t + 4g + j
   float wgt[4][4];
   if (!SCORES) {
@@ -114,7 +131,7 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
       const int row0 = wrow0 + 16 * t + 4 * g;
       const float* src = a.weights + (q_row0 + n16) * a.w_stride + tile_p0 + row0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wgt[t][j] = 0.0f;
+      for (int j = 0; j < 4; ++j) wgt[t][j] = SOFT_W ? -INFINITY : 0.0f;
       if (n16 < n_rep) {
         if (vec_ok && row0 + 4 <= rows_here) {
           const f4 v = *reinterpret_cast<const f4*>(src);
@@ -127,8 +144,42 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
       }
     }
   }
+  // kSoftWeights: the statistics of the row's tiles, thread = head tid % 16, tiles tid / 16 + 32 u
+  float M_part = -INFINITY, L_part = 0.0f;
+  if (SOFT_W) {
+    const float* st = a.stats + grp * a.n_tiles * (int64_t)(n_rep * 2);
+    const int h = tid & 15;
+    if (h < n_rep) {
+      for (int t0 = tid >> 4; t0 < a.n_tiles; t0 += 128) {
+        float2 ml[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          ml[u] = (t0 + 32 * u < a.n_tiles) ? *reinterpret_cast<const float2*>(st + (int64_t)(t0 + 32 * u) * (n_rep * 2) + 2 * h)
+                                            : make_float2(-INFINITY, 0.0f);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float Mn = fmaxf(M_part, ml[u].x);
+          L_part = (Mn == -INFINITY) ? L_part + ml[u].y                  // zeros, or the NaN of a tile without a number
+                                     : L_part * __builtin_amdgcn_exp2f(M_part - Mn) + ml[u].y * __builtin_amdgcn_exp2f(ml[u].x - Mn);
+          M_part = Mn;
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 16; d <= 32; d <<= 1) {
+      const float Mo = shfl_xor_f(M_part, d), Lo = shfl_xor_f(L_part, d);
+      const float Mn = fmaxf(M_part, Mo);
+      L_part = (Mn == -INFINITY) ? L_part + Lo : L_part * __builtin_amdgcn_exp2f(M_part - Mn) + Lo * __builtin_amdgcn_exp2f(Mo - Mn);
+      M_part = Mn;
+    }
+    if (lane < kHeadsMax) {
+      m_s[wave][lane] = M_part;
+      l_s[wave][lane] = L_part;
+    }
+  }
   if (tid < 64) fill_split_table<BITS>(lut_s, cb, tid);
-  if (SCORES) {
+  if (SOFT_S) rotate_query_rows<kWaves>(a.q_raw, a.q_dtype, a.k_signs, q_row0, n_rep, wave, lane, q_s, ql_s);
+  if (MODE == kScores) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const __half2 h = __floats2half2_rn(my_q[i].x, my_q[i].y);
@@ -155,6 +206,8 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) VF::pos(4 * kb + g, kw0[kb], ksl[kb], ksh[kb]);
     float s[4][4];
+    const bool mask_vec = SOFT_S && a.mask && ((reinterpret_cast<uintptr_t>(a.mask) & 15) == 0) && ((a.mask_seq_stride & 3) == 0) &&
+                          ((a.mask_head_stride & 3) == 0);                                         // uniform
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -176,6 +229,36 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
       }
       const float4 kn4 = *reinterpret_cast<const float4*>(&n_s[wave][16 * t + 4 * g]);
       s[t][0] = acc[0] * kn4.x; s[t][1] = acc[1] * kn4.y; s[t][2] = acc[2] * kn4.z; s[t][3] = acc[3] * kn4.w;
+      if (SOFT_S) {
+        const int row0 = wrow0 + 16 * t + 4 * g;
+        float mk[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (a.mask && n16 < n_rep)
+          load_mask4(a.mask + (int64_t)seq * a.mask_seq_stride + ((int64_t)kvh * n_rep + n16) * a.mask_head_stride + tile_p0 + row0,
+                     row0, rows_here, mask_vec, mk);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = s[t][j] * a.scale2;
+          s[t][j] = (row0 + j < rows_here) ? (a.mask ? __builtin_fmaf(mk[j], kLog2e, v) : v) : -INFINITY;
+        }
+      }
+    }
+    if (SOFT_S) {                                          // statistics of head n16 over the wave's positions
+      float m = -INFINITY, l = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
+      m = max_over_rows(m);
+      const float msafe = (m == -INFINITY) ? 0.0f : m;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) l += __builtin_amdgcn_exp2f(s[t][j] - msafe);
+      l = sum_over_rows(l);
+      if (g == 0) {
+        m_s[wave][n16] = m;
+        l_s[wave][n16] = l;
+      }
     }
     // The wave's 64 x n_rep scores leave through its LDS area (the key image has been consumed): a store
     // instruction then writes whole 256-byte runs of a head's row.  Area = [16 heads][16 units of 4 positions],
@@ -183,14 +266,15 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
     f4* sc = reinterpret_cast<f4*>(stage);
 #pragma unroll
     for (int t = 0; t < 4; ++t) sc[n16 * 16 + ((4 * t + g) ^ n16)] = f4{s[t][0], s[t][1], s[t][2], s[t][3]};
-    const bool vec_ok = ((len & 3) == 0) && ((reinterpret_cast<uintptr_t>(a.scores) & 15) == 0);   // uniform
+    const int64_t row_len = SOFT_S ? a.w_stride : len;
+    const bool vec_ok = ((row_len & 3) == 0) && ((reinterpret_cast<uintptr_t>(a.scores) & 15) == 0);   // uniform
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int h = 4 * i + g, unit = n16;
       if (h < n_rep) {
         const f4 v = sc[h * 16 + (unit ^ h)];
         const int row0 = wrow0 + 4 * unit;
-        float* dst = a.scores + (q_row0 + h) * len + tile_p0 + row0;
+        float* dst = a.scores + (q_row0 + h) * row_len + tile_p0 + row0;
         if (vec_ok && row0 + 4 <= rows_here) {
           __builtin_nontemporal_store(v, reinterpret_cast<f4*>(dst));     // streaming store: 10.9 -> 10.3 us at 65 536 positions
         } else {
@@ -200,10 +284,43 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
         }
       }
     }
+    if (SOFT_S) {
+      __syncthreads();
+      if (tid < n_rep) {
+        float M = m_s[0][tid], L = 0.0f;
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) M = fmaxf(M, m_s[w][tid]);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          const float mw = m_s[w][tid];
+          L += (mw == -INFINITY) ? l_s[w][tid] * 0.0f : l_s[w][tid] * __builtin_amdgcn_exp2f(mw - M);   // a NaN stays one
+        }
+        float* st = a.stats + (grp * a.n_tiles + tile) * (int64_t)(n_rep * 2);
+        st[2 * tid] = M;
+        st[2 * tid + 1] = L;
+      }
+    }
   } else {
     // ---- values: p = w * norm (weights below the threshold dropped), scaled per wave, split into hi and lo
     float p[4][4];
     float pmax = 0.0f, l = 0.0f;
+    if (SOFT_W) {                                          // the weight 2^(s - M) / L; a row without a visible position: 0 * inf = NaN,
+      float M = -INFINITY, L = 0.0f;                       // as a softmax over nothing is
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) M = fmaxf(M, m_s[w][n16]);
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const float mw = m_s[w][n16];
+        L += (mw == -INFINITY) ? l_s[w][n16] * 0.0f : l_s[w][n16] * __builtin_amdgcn_exp2f(mw - M);
+      }
+      if (M == -INFINITY) M = 0.0f;
+      const float inv_l = 1.0f / L;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          wgt[t][j] = (n16 < n_rep && wrow0 + 16 * t + 4 * g + j < rows_here) ? __builtin_amdgcn_exp2f(wgt[t][j] - M) * inv_l : 0.0f;
+    }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float4 n4 = *reinterpret_cast<const float4*>(&n_s[wave][16 * t + 4 * g]);
@@ -264,8 +381,8 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
         accS[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, Ah), __builtin_bit_cast(h8, Bh), accS[et], 0, 0, 0);
       }
     }
-    float* pS = a.ws_S + ((int64_t)kvh * a.n_tiles + tile) * (int64_t)(n_rep * kD);
-    float* pml = a.ws_ml + ((int64_t)kvh * a.n_tiles + tile) * (int64_t)(n_rep * 2);
+    float* pS = a.ws_S + (grp * a.n_tiles + tile) * (int64_t)(n_rep * kD);
+    float* pml = a.ws_ml + (grp * a.n_tiles + tile) * (int64_t)(n_rep * 2);
     merge_waves<kWaves>(mg_s, big_s, 4096, accS, 0.0f, l, inv_tscale, kSplitTableUnscale, n_rep, pS, pml);
   }
 }
@@ -273,6 +390,8 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
 template <int BITS>
 void launch_split_tiles(int mode, dim3 grid, const SplitArgs& a, const Codebook& cb, hipStream_t stream) {
   if (mode == kScores) split_tile_kernel<kScores, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, cb);
+  else if (mode == kSoftScores) split_tile_kernel<kSoftScores, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, cb);
+  else if (mode == kSoftWeights) split_tile_kernel<kSoftWeights, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, cb);
   else split_tile_kernel<kWeights, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, cb);
 }
 #ifndef TQ_WIDTH_HERE

@@ -71,6 +71,17 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
         out = out[:, :, None, :]
         return out if out.dtype == queries.dtype else out.to(queries.dtype)
 
+    if v_buffer is None and B > 0 and total > 0 and dim == cache._v_dim and ops.vonly_sparse_supported(dim, bits, n_rep):
+        # the same chain in three launches for the whole batch
+        m = None
+        if mask is not None:
+            m = ops.decode_mask_rows(mask, B, n_q, total, queries.device)
+            if m is None:
+                m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
+        out = ops.composed_decode(queries[:, :, 0, :], kq.signs, cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms,
+                                  kq.centroids, vq.centroids, vq.signs, dim, bits, attn_scale, n_rep=n_rep, seq_len=total,
+                                  mask=m, threshold=thr)[:, :, None, :]
+        return out if out.dtype == queries.dtype else out.to(queries.dtype)
     outputs = []
     for b in range(B):
         kp = cache.k_packed[b, :, :total, :]

@@ -816,6 +816,47 @@ def flash_decode_from_q(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v
     return out
 
 
+_COMPOSED_WORKSPACE = 256 << 20    # bytes of scores that one call of composed_decode may keep
+
+
+def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs, dim: int,
+                    bits: int, attn_scale: float, *, n_rep: int, seq_len: int, mask=None, threshold: float = 0.0) -> torch.Tensor:
+    """prerotate_query, prerot_fused_qk_scores, softmax_rows and sparse_v_matvec for every sequence of a cache in three
+    launches (tq_composed_decode), float32 fidelity.  q (n_seq, n_q, dim); K / V in cache layout (n_seq, n_kv, T_alloc, *);
+    returns (n_seq, n_q, dim) in q's dtype (float32 for one that is no kernel dtype).  Shapes of vonly_sparse_supported.
+    Batches whose scores would not fit the workspace bound go in several calls."""
+    _need_gpu(q, k_packed, k_norms, v_packed, v_norms, mask)
+    n_seq, n_q, _ = q.shape
+    _check_gqa(n_q, k_norms.shape[-2], n_rep)
+    pd = packed_dim(dim, bits)
+    if q.dtype not in _DTYPES:
+        q = q.float()
+    q = q.contiguous()
+    k_packed, ks = _kv_layout(_u32(k_packed), pd, False)
+    v_packed, vs = _kv_layout(_u32(v_packed), pd, False)
+    k_norms, kns = _norm_layout(k_norms.to(torch.float32))
+    v_norms, vns = _norm_layout(v_norms.to(torch.float32))
+    _check_rows(seq_len, False, n_seq, k_packed=k_packed, k_norms=k_norms, v_packed=v_packed, v_norms=v_norms)
+    k_signs, v_signs = _as_f32_dev(k_signs, q), _as_f32_dev(v_signs, q)
+    mask, ms = _mask_layout(mask, n_seq, n_q, seq_len, q.device)
+    out = torch.empty((n_seq, n_q, dim), dtype=q.dtype, device=q.device)
+    lib = _lib.load()
+    stream = _stream(q)
+    per_call = max(1, min(n_seq, _COMPOSED_WORKSPACE // max(1, lib.tq_vonly_sparse_workspace_bytes(1, n_q, seq_len))))
+    ws = _workspace(q.device, stream.value or 0, lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len))
+    for first in range(0, n_seq, per_call):
+        n = min(per_call, n_seq - first)
+        sh = _decode_shape(n_seq=n, n_kv=n_q // n_rep, n_rep=n_rep, dim=dim, bits=bits, block_size=16, seq_len=seq_len,
+                           seq_offsets=None, k_strides=ks, kn_strides=kns, v_strides=vs, vn_strides=vns,
+                           mask=mask if mask is None or ms[0] == 0 else mask[first:], mask_strides=ms, attn_scale=attn_scale,
+                           out_dtype=q.dtype)
+        _lib.check(lib.tq_composed_decode(
+            q[first:].data_ptr(), _dt(q), k_signs.data_ptr(), k_packed[first:].data_ptr(), k_norms[first:].data_ptr(),
+            v_packed[first:].data_ptr(), v_norms[first:].data_ptr(), _host_table(k_centroids), _host_table(v_centroids),
+            v_signs.data_ptr(), threshold, out[first:].data_ptr(), ws.data_ptr(), ws.numel(), C.byref(sh), stream))
+    return out
+
+
 def flash_attention_turboquant(q_rot, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids,
                                v_signs, dim: int, bits: int, attn_scale: float, block_size: int = 16,
                                n_rep: int = 1, precision: str = "fp16") -> torch.Tensor:
