@@ -544,6 +544,18 @@ int tq_flash_decode_from_q(const void* q, int q_dtype, const float* k_signs,
                            const tq_decode_shape* shape /* host */, tq_stream_t stream);
 
 /*
+ * tq_prerotate_query and tq_flash_decode for dim 64 in one call (the kernel rotates the query: same bits), float32 fidelity on
+ * the matrix cores: the fused decode step of turboquant_attention at that head dimension (fused_attention.py:56-121).
+ * Arguments and workspace as tq_flash_decode, q [n_seq, n_kv*n_rep, 64] of q_dtype.
+ */
+int tq_flash_decode_from_q64(const void* q, int q_dtype, const float* k_signs,
+                             const uint32_t* k_packed, const float* k_norms,
+                             const uint32_t* v_packed, const float* v_norms,
+                             const float* k_centroids, const float* v_centroids, const float* v_signs,
+                             void* out, void* workspace, size_t workspace_bytes,
+                             const tq_decode_shape* shape /* host */, tq_stream_t stream);
+
+/*
  * The chain of turboquant_attention (fused_attention.py:56-121: prerotate_query -> prerot_fused_qk_scores -> * attn_scale + mask
  * -> softmax -> sparse_v_matvec(threshold)) at float32 fidelity for a batch of one length in one call of three launches: the
  * split operands of tq_prerot_qk_scores and tq_sparse_v_matvec (TQ_MMA_SPLIT), the softmax between them in float32.  Arguments

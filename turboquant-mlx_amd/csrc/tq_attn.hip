@@ -31,6 +31,7 @@ struct DecodeArgs {
   // query side
   const void* q;                // kPackedK: q_rot f32; kDenseK: q (dtype QT); kWeights: weights f32 [n_q, T]
   // key side
+  const float* k_signs;         // kPackedK in split_decode_kernel: set when q is the query itself, rotated there
   const uint32_t* k_packed;
   const float* k_norms;
   const __half* k_dense;
@@ -562,6 +563,8 @@ __global__ __launch_bounds__(kThreads) void decode_tile_kernel(DecodeArgs a, Cod
   }
 }
 
+#include "tq_split_dims.h"
+
 // ---------------------------------------------------------------- merge pass
 // grid = (n_q, n_seq), 256 threads.  Lane group ph = tid / (D/4) folds tiles ph, ph + P, ... (4
 // elements per lane, P = 1024 / D groups) -- with a running maximum for the softmax modes, a plain
@@ -674,7 +677,7 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
                   const void* k_dense, const uint32_t* v_packed, const float* v_norms,
                   const float* k_centroids, const float* v_centroids, const float* v_signs, void* out,
                   void* workspace, size_t workspace_bytes, const tq_decode_shape& sh, float threshold,
-                  hipStream_t stream, const char* who, int phases = 3) {
+                  hipStream_t stream, const char* who, int phases = 3, const float* k_signs = nullptr) {
   const int n_q = sh.n_kv_heads * sh.n_rep;
   const size_t need = ws_bytes(sh.n_seq, n_q, sh.seq_len, sh.dim);
   if (!workspace || workspace_bytes < need)
@@ -683,7 +686,7 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
   const int n_tiles = n_tiles_for(sh.seq_len);
   const int n_tiles_max = n_tiles > 0 ? n_tiles : 1;
   DecodeArgs a{};
-  a.q = q;
+  a.q = q; a.k_signs = k_signs;
   a.k_packed = k_packed; a.k_norms = k_norms; a.k_dense = (const __half*)k_dense;
   a.v_packed = v_packed; a.v_norms = v_norms;
   a.seq_offsets = sh.seq_offsets; a.mask = sh.mask;
@@ -705,6 +708,18 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
   fill_codebook(kcb, k_centroids, sh.bits);
   fill_codebook(vcb, v_centroids, sh.bits);
   if (n_tiles > 0 && (phases & 1)) {
+    // d = 64 and 256 with matrix instructions allowed: the split tile kernel (same tiles and partials); packed keys exist up
+    // to d = 128.  d = 32, and float32 arithmetic asked for: the vector kernel.
+    if (KMODE != kWeights && sh.allow_mma && (sh.dim == 64 || (KMODE == kDenseK && sh.dim == 256))) {
+      a.n_rgroups = (sh.n_rep + kSplitHeads - 1) / kSplitHeads;
+      dim3 sgrid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
+      if (sh.dim == 64) {
+        TQ_DISPATCH_BITS(sh.bits, (split_decode_kernel<64, B_, KMODE == kDenseK><<<sgrid, kThreads, 0, stream>>>(a, q_dtype, kcb, vcb)));
+      } else {
+        TQ_DISPATCH_BITS(sh.bits, (split_decode_kernel<256, B_, true><<<sgrid, kThreads, 0, stream>>>(a, q_dtype, kcb, vcb)));
+      }
+      TQ_CHECK_LAUNCH(who);
+    } else {
     dim3 grid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
 #define LAUNCH_TILE(QT)                                                                              \
   TQ_DISPATCH_DIM(sh.dim, TQ_DISPATCH_BITS(sh.bits, (decode_tile_kernel<D_, B_, KMODE, QT>            \
@@ -714,6 +729,7 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
     else { LAUNCH_TILE(float); }
 #undef LAUNCH_TILE
     TQ_CHECK_LAUNCH(who);
+    }
   }
   if (!(phases & 2)) return TQ_OK;
   dim3 mgrid(n_q, sh.n_seq);
@@ -1716,6 +1732,25 @@ extern "C" int tq_flash_decode_from_q(const void* q, int q_dtype, const float* k
   sh.allow_mma = 1;
   return launch_packed_mfma<tqm::kFlash>(nullptr, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs,
                                          out, workspace, workspace_bytes, sh, 0.0f, stream, who, q, q_dtype, k_signs);
+}
+
+extern "C" int tq_flash_decode_from_q64(const void* q, int q_dtype, const float* k_signs, const uint32_t* k_packed,
+                                        const float* k_norms, const uint32_t* v_packed, const float* v_norms,
+                                        const float* k_centroids, const float* v_centroids, const float* v_signs, void* out,
+                                        void* workspace, size_t workspace_bytes, const tq_decode_shape* shape,
+                                        tq_stream_t stream_) {
+  const char* who = "tq_flash_decode_from_q64";
+  if (int rc = check_shape(shape, who, 128)) return rc;
+  if (tq::check_dtype(q_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown q_dtype %d", who, q_dtype);
+  if (!q || !k_signs || !k_centroids || !v_centroids || !v_signs || !out) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (shape->seq_len > 0 && (!k_packed || !k_norms || !v_packed || !v_norms))
+    return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (shape->dim != 64 || !tq::aligned(q, (int)tq::dtype_size(q_dtype)))
+    return tq::fail(TQ_ERR_UNSUPPORTED, "%s: dim 64 only (call tq_prerotate_query and tq_flash_decode otherwise)", who);
+  tq_decode_shape sh = *shape;
+  sh.allow_mma = 1;
+  return launch_decode<kPackedK>(q, q_dtype, k_packed, k_norms, nullptr, v_packed, v_norms, k_centroids, v_centroids, v_signs,
+                                 out, workspace, workspace_bytes, sh, 0.0f, (hipStream_t)stream_, who, 3, k_signs);
 }
 
 extern "C" int tq_composed_decode(const void* q, int q_dtype, const float* k_signs, const uint32_t* k_packed,

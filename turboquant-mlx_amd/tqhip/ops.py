@@ -769,13 +769,25 @@ def flash_decode_from_q(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v
     itself: the pre-rotation of prerotate_query happens inside the attention kernels (tq_flash_decode_from_q).
     q (n_seq, n_q, dim) fp16 / bf16 / float32; other arguments as flash_decode.  Matrix-core shapes only
     (vonly_sparse_supported); callers fall back to prerotate_query + flash_decode otherwise."""
+    if not vonly_sparse_supported(dim, bits, n_rep):
+        _need_gpu(q, k_packed, k_norms, v_packed, v_norms, seq_offsets)
+        _check_gqa(q.shape[1], k_norms.shape[-2], n_rep)
+        raise ValueError("flash_decode_from_q needs dim 128 and n_rep <= 16; use prerotate_query + flash_decode")
+    return flash_from_query(q, k_signs, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs, dim, bits,
+                            attn_scale, n_rep=n_rep, seq_len=seq_len, seq_offsets=seq_offsets, max_seq_len=max_seq_len, mask=mask,
+                            out_dtype=out_dtype, sparse_v_threshold=sparse_v_threshold, validate_offsets=validate_offsets)
+
+
+def flash_from_query(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs, dim: int,
+                     bits: int, attn_scale: float, *, n_rep: int = 1, seq_len: int | None = None, seq_offsets=None,
+                     max_seq_len: int | None = None, mask=None, out_dtype=torch.float32, sparse_v_threshold: float = 0.0,
+                     validate_offsets: bool = False) -> torch.Tensor:
+    """flash_decode_from_q, and without a threshold also d = 64 (tq_flash_decode_from_q64, any n_rep)."""
     _need_gpu(q, k_packed, k_norms, v_packed, v_norms, seq_offsets)
     n_seq, n_q, _ = q.shape
     ragged = seq_offsets is not None
     n_kv = k_norms.shape[-2]
     _check_gqa(n_q, n_kv, n_rep)
-    if not vonly_sparse_supported(dim, bits, n_rep):
-        raise ValueError("flash_decode_from_q needs dim 128 and n_rep <= 16; use prerotate_query + flash_decode")
     pd = packed_dim(dim, bits)
     if q.dtype not in _DTYPES:
         q = q.float()
@@ -809,6 +821,11 @@ def flash_decode_from_q(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v
     need = (lib.tq_vonly_sparse_workspace_bytes(n_seq, n_q, T) if thr > 0.0
             else lib.tq_workspace_bytes(_lib.TQ_OP_FLASH_DECODE, n_seq, n_q, T, dim))
     ws = _workspace(q.device, stream.value or 0, need)
+    if dim == 64:
+        _lib.check(lib.tq_flash_decode_from_q64(
+            _ptr(q), _dt(q), _ptr(k_signs), _ptr(k_packed), _ptr(k_norms), _ptr(v_packed), _ptr(v_norms),
+            _host_table(k_centroids), _host_table(v_centroids), _ptr(v_signs), _ptr(out), _ptr(ws), ws.numel(), C.byref(sh), stream))
+        return out
     _lib.check(lib.tq_flash_decode_from_q(
         _ptr(q), _dt(q), _ptr(k_signs), _ptr(k_packed), _ptr(k_norms), _ptr(v_packed), _ptr(v_norms),
         _host_table(k_centroids), _host_table(v_centroids), _ptr(v_signs), thr, _ptr(out),
