@@ -711,7 +711,8 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
     // d = 64 and 256 with matrix instructions allowed: the split tile kernel (same tiles and partials); packed keys exist up
     // to d = 128.  d = 32, and float32 arithmetic asked for: the vector kernel.
     if (KMODE != kWeights && sh.allow_mma && (sh.dim == 64 || (KMODE == kDenseK && sh.dim == 256))) {
-      a.n_rgroups = (sh.n_rep + kSplitHeads - 1) / kSplitHeads;
+      const int heads = sh.dim == 256 ? kSplitHeads<256> : kSplitHeads<64>;
+      a.n_rgroups = (sh.n_rep + heads - 1) / heads;
       dim3 sgrid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
       if (sh.dim == 64) {
         TQ_DISPATCH_BITS(sh.bits, (split_decode_kernel<64, B_, KMODE == kDenseK><<<sgrid, kThreads, 0, stream>>>(a, q_dtype, kcb, vcb)));

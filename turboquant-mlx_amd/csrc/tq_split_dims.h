@@ -9,7 +9,9 @@
 // so that magnitudes outside the range of fp16 change nothing (see tq_split_mfma.h).
 #pragma once
 
-constexpr int kSplitHeads = 16;      // query heads of a kv head that one workgroup serves
+// query heads of a kv head that one workgroup serves: at d = 256 eight, whose sums leave room for three workgroups in a CU's LDS
+// (4 sequences x 32 / 8 heads x 16 000 positions, fp16 keys: a call takes 150 us with one workgroup of sixteen heads a CU, 84 us with three of eight)
+template <int D> constexpr int kSplitHeads = D == 256 ? 8 : 16;
 
 // power of two that brings `largest` to [2^13, 2^14), and its inverse; both normal
 __device__ __forceinline__ void split_scale(float largest, float& up, float& down) {
@@ -27,26 +29,27 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   using tqm::u4;
   using VF = tqm::VField<BITS>;
   constexpr int PD = Pk<BITS>::pdim(D), PSTR = PD | 1, VPW = Pk<BITS>::VPW;
+  constexpr int kH = kSplitHeads<D>;
   constexpr int KB = D / 32;                                   // contraction steps of a score
   constexpr int EL = D >= 128 ? 8 : D / 16;                    // consecutive elements of a value row per lane and pass
   constexpr int NP = D / (16 * EL);
   constexpr int EPL = D / 64;
   constexpr int kRows = 64 * PSTR + 4;                         // a field's second word may lie past the last row
   constexpr int kQ = D / 2 + 4;                                // words per query row, rows in different banks
-  constexpr int kWaveWords = (DENSE ? 1 : 2) * kRows > kSplitHeads * D ? (DENSE ? 1 : 2) * kRows : kSplitHeads * D;
+  constexpr int kWaveWords = (DENSE ? 1 : 2) * kRows > kH * D ? (DENSE ? 1 : 2) * kRows : kH * D;
   constexpr int kLutN = VF::kLut < 64 ? 64 : VF::kLut;
   constexpr float kLog2eF = 1.44269504088896340736f;
   __shared__ __align__(16) uint32_t area_s[kWaves][(kWaveWords + 3) & ~3];   // per wave: packed rows, then its sums [16][D]
-  __shared__ __align__(16) uint32_t qh_s[kSplitHeads][kQ], ql_s[kSplitHeads][kQ];
-  __shared__ float qdown_s[kSplitHeads];
+  __shared__ __align__(16) uint32_t qh_s[kH][kQ], ql_s[kH][kQ];
+  __shared__ float qdown_s[kH];
   __shared__ __align__(16) uint2 lutk_s[DENSE ? 1 : kLutN], lutv_s[kLutN];
   __shared__ __align__(16) float kn_s[kWaves][64], vn_s[kWaves][64];
-  __shared__ float m_s[kWaves][kSplitHeads], l_s[kWaves][kSplitHeads];
+  __shared__ float m_s[kWaves][16], l_s[kWaves][16];
 
   const int tile = blockIdx.x;
   const int kvh = blockIdx.y / a.n_rgroups;
-  const int r0 = (blockIdx.y % a.n_rgroups) * kSplitHeads;
-  const int n_local = min(kSplitHeads, a.n_rep - r0);
+  const int r0 = (blockIdx.y % a.n_rgroups) * kH;
+  const int n_local = min(kH, a.n_rep - r0);
   const int seq = blockIdx.z;
   const int n_q = a.n_kv * a.n_rep;
   const int64_t q_row0 = (int64_t)seq * n_q + (int64_t)kvh * a.n_rep + r0;
@@ -80,9 +83,9 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
     my_vn = a.v_norms[(int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first + w0 + lane];
   }
   const bool rotate = !DENSE && a.k_signs;                      // the query itself: q * signs and the butterfly of tq_prerotate_query
-  float v[kSplitHeads / kWaves][EPL];
+  float v[kH / kWaves][EPL];
 #pragma unroll
-  for (int it = 0; it < kSplitHeads / kWaves; ++it) {
+  for (int it = 0; it < kH / kWaves; ++it) {
     const int r = wave + it * kWaves;
 #pragma unroll
     for (int i = 0; i < EPL; ++i) {
@@ -105,7 +108,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   if (!DENSE) kn_s[wave][lane] = my_kn;
   vn_s[wave][lane] = my_vn;
 #pragma unroll
-  for (int it = 0; it < kSplitHeads / kWaves; ++it) {
+  for (int it = 0; it < kH / kWaves; ++it) {
     const int r = wave + it * kWaves;
     if (rotate && r < n_local) raw_butterfly<D>(v[it], lane);   // uniform over the wave
     float largest = 0.0f;
@@ -124,6 +127,16 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
       lo[lane + 64 * i] = __float2half_rn(x - __half2float(h));
     }
   }
+  // fp16 keys: row n16 of a group of 16 positions, one group ahead of its products (rows past the end: the last that exists)
+  u4 kd[2][DENSE ? KB : 1];
+  auto load_keys = [&](int t, u4 (&k)[DENSE ? KB : 1]) {
+    if constexpr (DENSE) {
+      const int64_t row = krow0 + (rows > 0 ? w0 + min(16 * t + n16, rows - 1) : p0);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) k[kb] = *reinterpret_cast<const u4*>(a.k_dense + row * D + 8 * g + 32 * kb);
+    }
+  };
+  load_keys(0, kd[0]);
   if (!DENSE && wave == 0) tqm::fill_split_table<BITS>(lutk_s, kcb, lane);
   if (wave == 1) tqm::fill_split_table<BITS>(lutv_s, vcb, lane);
   __syncthreads();
@@ -132,20 +145,17 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   u4 qh[KB], ql[KB];
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
-    qh[kb] = *reinterpret_cast<const u4*>(&qh_s[n16][16 * kb + 4 * g]);
-    ql[kb] = *reinterpret_cast<const u4*>(&ql_s[n16][16 * kb + 4 * g]);
+    qh[kb] = *reinterpret_cast<const u4*>(&qh_s[n16 & (kH - 1)][16 * kb + 4 * g]);
+    ql[kb] = *reinterpret_cast<const u4*>(&ql_s[n16 & (kH - 1)][16 * kb + 4 * g]);
   }
-  const float qdown = qdown_s[n16];
+  const float qdown = qdown_s[n16 & (kH - 1)];      // columns past the last head repeat others and are dropped
   float s[4][4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     if constexpr (DENSE) {
-      const int64_t row = krow0 + w0 + min(16 * t + n16, rows > 0 ? rows - 1 : 0) - (rows > 0 ? 0 : w0 - p0);   // an existing row
-      const __half* src = a.k_dense + row * D + 8 * g;
-      u4 k[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) k[kb] = *reinterpret_cast<const u4*>(src + 32 * kb);
+      u4 (&k)[KB] = kd[t & 1];
+      if (t < 3) load_keys(t + 1, kd[(t + 1) & 1]);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, k[kb]), __builtin_bit_cast(h8, ql[kb]), acc, 0, 0, 0);
@@ -269,7 +279,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e4 = 0; e4 < EL; e4 += 4)
-        *reinterpret_cast<f4*>(dep + (4 * g + j) * D + EL * (n16 + 16 * np) + e4) =
+        if (kH == 16 || 4 * g + j < kH) *reinterpret_cast<f4*>(dep + (4 * g + j) * D + EL * (n16 + 16 * np) + e4) =
             f4{acc[np][e4][j] * unscale, acc[np][e4 + 1][j] * unscale, acc[np][e4 + 2][j] * unscale, acc[np][e4 + 3][j] * unscale};
   if (g == 0) {
     m_s[wave][n16] = m;
