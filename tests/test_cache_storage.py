@@ -1,0 +1,65 @@
+"""Growth of cache storage without a GPU: what the storage fill is asked to copy and to zero, on CPU tensors."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import tqhip  # noqa: E402
+from tqhip import ops  # noqa: E402
+
+B, H = 2, 3
+
+
+def _grown(cache, dim, n):
+    """A cache of n positions on the CPU whose stored words and norms are numbered."""
+    cache._ensure_quantizer(dim, dim, torch.device("cpu"))
+    cache._ensure_storage(B, H, n, torch.device("cpu"))
+    for t in _stored(cache):
+        t[:, :, :n] = torch.arange(1, t[:, :, :n].numel() + 1, dtype=torch.int32).reshape(t[:, :, :n].shape).to(t.dtype)
+    cache.offset = n
+    return cache
+
+
+def _stored(cache):
+    ts = [cache.v_packed, cache.v_norms] + ([] if cache.v_only else [cache.k_packed, cache.k_norms])
+    return [t.view(torch.int32) if t.dtype == torch.uint32 else t for t in ts]
+
+
+@pytest.mark.parametrize("v_only", [False, True])
+@pytest.mark.parametrize("dim,bits", [(d, b) for d in (32, 64, 128, 256) for b in (1, 2, 3, 4)])
+def test_growth_keeps_the_stored_prefix(dim, bits, v_only):
+    """(32, 1) packs a vector into one word: storage [B, H, T, 1], whose last axis is not the positions."""
+    cache = _grown(tqhip.TurboQuantKVCache(bits=bits, v_only=v_only), dim, 250)
+    before = [t[:, :, :250].clone() for t in _stored(cache)]
+    assert all(not t[:, :, 250:].any() for t in _stored(cache))
+    cache._ensure_storage(B, H, 10, torch.device("cpu"))
+    for t, want in zip(_stored(cache), before):
+        assert t.shape[2] == 512 and torch.equal(t[:, :, :250], want) and not t[:, :, 250:].any()
+
+
+@pytest.mark.parametrize("dim,bits", [(d, b) for d in (32, 64, 128, 256) for b in (1, 2, 3, 4)])
+def test_fill_segments_stay_inside_the_tensors(monkeypatch, dim, bits):
+    """The byte ranges that a GPU launch would get for the same growth."""
+    segments = []
+
+    def add(self, dst, inner, zero_from, zero_to, src=None, src_stride=0, copy=0, axis=None):
+        groups, rows = dst.shape[:axis].numel(), dst.shape[axis]
+        assert dst.is_contiguous() and groups * rows * inner == dst.numel() and groups == B * H
+        s = ops.StorageFill.segment(dst, src, groups, rows, inner, zero_from, zero_to, src_stride, copy)
+        _, _, dst_stride, src_stride, copy_bytes, z0, z1, n = s
+        assert (n - 1) * dst_stride + max(copy_bytes, z1) <= dst.nbytes and copy_bytes <= z0 <= z1 <= dst_stride
+        if copy_bytes:
+            assert src.dtype == dst.dtype and (n - 1) * src_stride + copy_bytes <= src.nbytes
+        segments.append(s)
+
+    cache = _grown(tqhip.TurboQuantKVCache(bits=bits), dim, 250)
+    monkeypatch.setattr(ops.StorageFill, "add", add)
+    cache._ensure_storage(B, H, 10, torch.device("cpu"), incoming=10)
+    assert len(segments) == 4
+
+
+def test_fill_refuses_rows_outside_the_tensor():
+    fill = ops.StorageFill()
+    with pytest.raises(ValueError):
+        fill.add(torch.zeros(1, 2, 8, 1), 1, 4, 8)                 # the trailing axis taken for the rows
+    with pytest.raises(ValueError):
+        fill.segment(torch.zeros(2, 8, 4), torch.zeros(2, 4, 4), 2, 8, 4, 4, 8, 5, 4)

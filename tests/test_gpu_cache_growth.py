@@ -1,0 +1,46 @@
+"""Caches whose storage grows while they are filled, against a cache filled by one insert."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tq():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a GPU: torch.cuda.is_available() is False")
+    import tqhip
+    return tqhip
+
+
+def _rows(dim, n, seed=0, B=2, H=4):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.randn((B, H, n, dim), generator=g, device="cuda").half() for _ in range(2)]
+
+
+def _same(a, b):
+    for x, y in zip(a, b):
+        x, y = (t.view(torch.int32) if t.dtype == torch.uint32 else t for t in (x, y))
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dim,bits", [(32, 1), (32, 2), (64, 1), (128, 3)])      # (32, 1): one word a row
+@pytest.mark.parametrize("kind", ["default", "fused", "vonly", "vonly_nobuf"])
+def test_storage_grows_with_its_contents(tq, dim, bits, kind):
+    k, v = _rows(dim, 530)
+
+    def make():
+        if kind.startswith("vonly"):
+            return tq.VOnlyTurboQuantCache(bits=bits, no_v_buffer=kind == "vonly_nobuf")
+        return tq.TurboQuantKVCache(bits=bits, fused=kind == "fused")
+    whole, parts = make(), make()
+    want = whole.update_and_fetch(k, v)
+    got = None
+    for lo, hi in ((0, 100), (100, 255), (255, 258), (258, 500), (500, 530)):
+        got = parts.update_and_fetch(k[:, :, lo:hi], v[:, :, lo:hi])
+    _same(parts.state, whole.state)
+    _same(got, want)
+    store = parts._v_tq if kind.startswith("vonly") else parts
+    for t in (store.v_packed, store.v_norms):
+        assert not (t.view(torch.int32) if t.dtype == torch.uint32 else t)[:, :, 530:].any()

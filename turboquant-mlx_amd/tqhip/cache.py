@@ -167,9 +167,10 @@ class TurboQuantKVCache:
         new = torch.empty(shape, dtype=dtype, device=device)
         n = shape[2]
         if old is None or prev == 0:
-            fill.add(new, inner, incoming, n)
+            fill.add(new, inner, incoming, n, axis=2)
         elif old.dtype == dtype and old.device == new.device and old.shape[:2] == new.shape[:2] and _is_grouped(old, inner):
-            fill.add(new, inner, prev + incoming, n, src=old, src_stride=_group_stride(old, inner), copy=prev)
+            fill.add(new, inner, prev + incoming, n, src=old, src_stride=_group_stride(old, inner), copy=prev,
+                     axis=2)
         else:
             new.zero_()
             new[:, :, :prev] = old[:, :, :prev]
@@ -261,7 +262,7 @@ class TurboQuantKVCache:
             fill = ops.StorageFill()
             grown = self._buffers(B, H, _round_up(total, self.step), dtypes, bufs[0].device)
             for new, old in zip(grown, bufs):
-                fill.add(new, new.shape[3], total, new.shape[2], src=old, src_stride=old.shape[2], copy=self._deq_offset)
+                fill.add(new, new.shape[3], total, new.shape[2], src=old, src_stride=old.shape[2], copy=self._deq_offset, axis=2)
             fill.run()
             bufs = grown
         if all(dt == torch.float16 for dt in dtypes):
@@ -384,7 +385,7 @@ class TurboQuantKVCache:
             return None
         bufs = self._buffers(B, H, _round_up(total, self.step), dtypes, device)
         for buf in bufs:
-            fill.add(buf, buf.shape[3], total, buf.shape[2])
+            fill.add(buf, buf.shape[3], total, buf.shape[2], axis=2)
         return bufs
 
     def _fetch(self, fresh, B, H, prev, total, dtypes):

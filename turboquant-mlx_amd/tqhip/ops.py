@@ -247,24 +247,35 @@ class StorageFill:
         self._segments, self._keep = [], []
 
     def add(self, dst: torch.Tensor, inner: int, zero_from: int, zero_to: int, src: torch.Tensor | None = None, src_stride: int = 0,
-            copy: int = 0) -> None:
-        """dst: contiguous [..., T, inner] (or [..., T] with inner 1), its leading axes are the groups: rows `copy` from src
-        (rows src_stride apart per group) first, zeros in rows zero_from .. zero_to - 1."""
+            copy: int = 0, axis: int | None = None) -> None:
+        """dst: contiguous, its rows along `axis` (default: the last but one, or the last with inner 1), `inner` elements each;
+        the axes before are the groups: rows `copy` from src (rows src_stride apart per group) first, zeros in rows
+        zero_from .. zero_to - 1.  Storage of one word a row has a trailing axis of 1 that only the caller can tell from rows."""
         if copy == 0 and zero_to <= zero_from:
             return
-        if not dst.is_cuda:                                  # storage of a cache that has not met the GPU yet
+        if axis is None:
             axis = dst.dim() - (2 if inner > 1 else 1)
+        rows = dst.shape[axis]
+        if dst.shape[axis + 1:].numel() != inner or max(copy, zero_to) > rows:
+            raise ValueError(f"rows of {inner} elements up to {max(copy, zero_to)} along axis {axis} of {tuple(dst.shape)}")
+        if not dst.is_cuda:                                  # storage of a cache that has not met the GPU yet
             if copy:
                 dst.narrow(axis, 0, copy).copy_(src.narrow(axis, 0, copy))
             dst.narrow(axis, zero_from, max(0, zero_to - zero_from)).zero_()
             return
-        row = inner * dst.element_size()
-        rows = dst.shape[-2] if inner > 1 else dst.shape[-1]
-        groups = dst.numel() // max(1, rows * inner)
-        from_ = (0, 0) if src is None else (src.data_ptr(), src_stride * row)
-        self._segments.append((dst.data_ptr(), from_[0], rows * row, from_[1], copy * row,
-                               zero_from * row, max(zero_from, zero_to) * row, groups))
+        self._segments.append(self.segment(dst, src, dst.shape[:axis].numel(), rows, inner, zero_from, zero_to, src_stride, copy))
         self._keep.append((dst, src))
+
+    @staticmethod
+    def segment(dst, src, groups: int, rows: int, inner: int, zero_from: int, zero_to: int, src_stride: int, copy: int) -> tuple:
+        """The fields of struct tq_fill_segment, checked against the bytes that the tensors hold."""
+        row = inner * dst.element_size()
+        if src is not None and copy > 0:
+            held = src.untyped_storage().nbytes() - src.storage_offset() * src.element_size()
+            if ((groups - 1) * src_stride + copy) * row > held:
+                raise ValueError(f"{groups} groups of {copy} rows, {src_stride} apart, exceed the {held} bytes of the source")
+        return (dst.data_ptr(), 0 if src is None else src.data_ptr(), rows * row, 0 if src is None else src_stride * row, copy * row,
+                zero_from * row, max(zero_from, zero_to) * row, groups)
 
     def run(self) -> None:
         segs, self._segments = self._segments, []
