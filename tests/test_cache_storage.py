@@ -63,3 +63,31 @@ def test_fill_refuses_rows_outside_the_tensor():
         fill.add(torch.zeros(1, 2, 8, 1), 1, 4, 8)                 # the trailing axis taken for the rows
     with pytest.raises(ValueError):
         fill.segment(torch.zeros(2, 8, 4), torch.zeros(2, 4, 4), 2, 8, 4, 4, 8, 5, 4)
+
+
+@pytest.mark.parametrize("v_only", [False, True])
+@pytest.mark.parametrize("was,now", [(a, b) for a in (torch.float16, torch.bfloat16, torch.float32)
+                                     for b in (torch.float16, torch.bfloat16, torch.float32)])
+def test_buffer_growth_casts_rows_of_another_dtype(monkeypatch, was, now, v_only):
+    """Dequantised buffers that grow under rows of another dtype: the prefix is cast, never copied byte by byte."""
+    cache = _grown(tqhip.TurboQuantKVCache(bits=3, v_only=v_only), 128, 256)
+    sides = 1 if v_only else 2
+    old = [torch.randn(B, H, 256, 128).to(was) for _ in range(sides)]
+    cache._deq_offset = 256
+    raw = []
+    add = ops.StorageFill.add
+
+    def checked(self, dst, inner, zero_from, zero_to, src=None, src_stride=0, copy=0, axis=None):
+        if copy:
+            raw.append(src.dtype)
+            assert src.dtype == dst.dtype
+            ops.StorageFill.segment(dst, src, B * H, dst.shape[axis], inner, zero_from, zero_to, src_stride, copy)
+        return add(self, dst, inner, zero_from, zero_to, src=src, src_stride=src_stride, copy=copy, axis=axis)
+
+    monkeypatch.setattr(ops.StorageFill, "add", checked)
+    monkeypatch.setattr(tqhip.TurboQuantKVCache, "_dequant_rows", lambda self, outs, *a: [o.zero_() for o in outs if o.shape[2] == 1])
+    grown = cache._incremental(list(old), B, H, 256, 257, [now] * sides)
+    assert len(raw) == (sides if was == now else 0)
+    for new, o in zip(grown, old):
+        assert new.dtype == now and new.shape[2] == 512
+        assert torch.equal(new[:, :, :256], o.to(now)) and not new[:, :, 257:].any()

@@ -44,3 +44,23 @@ def test_storage_grows_with_its_contents(tq, dim, bits, kind):
     store = parts._v_tq if kind.startswith("vonly") else parts
     for t in (store.v_packed, store.v_norms):
         assert not (t.view(torch.int32) if t.dtype == torch.uint32 else t)[:, :, 530:].any()
+
+
+@pytest.mark.parametrize("kind", ["default", "vonly"])
+@pytest.mark.parametrize("was,now", [(torch.float16, torch.float16), (torch.float16, torch.bfloat16), (torch.bfloat16, torch.float16),
+                                     (torch.float16, torch.float32), (torch.float32, torch.float16), (torch.bfloat16, torch.float32)])
+def test_buffer_grows_under_tokens_of_another_dtype(tq, was, now, kind):
+    """A prompt in one dtype, tokens in another, over a boundary of 256 positions, where the dequantised buffers grow: every
+    position is what a full dequantisation in its own dtype gives, cast to the buffer's."""
+    B, H, n, dim = 2, 4, 254, 128
+    k, v = _rows(dim, n + 4)
+    cls = tq.VOnlyTurboQuantCache if kind == "vonly" else tq.TurboQuantKVCache
+    cache = cls(bits=3)
+    cache.update_and_fetch(k[:, :, :n].to(was), v[:, :, :n].to(was))
+    prompt = cache._v_tq._v_deq_buf[:, :, :n].clone() if kind == "vonly" else cache._v_deq_buf[:, :, :n].clone()
+    for i in range(n, n + 4):
+        _, got = cache.update_and_fetch(k[:, :, i:i + 1].to(now), v[:, :, i:i + 1].to(now))
+    store = cache._v_tq if kind == "vonly" else cache
+    full = store._full_dequant(store.v_packed, store.v_norms, store._v_q, dim, B, H, n + 4, torch.float16)
+    assert got.dtype == now and torch.equal(got[:, :, :n], prompt.to(now))
+    assert torch.equal(got[:, :, n + 2:], full[:, :, n + 2:].to(now))       # the tokens after the growth

@@ -262,7 +262,11 @@ class TurboQuantKVCache:
             fill = ops.StorageFill()
             grown = self._buffers(B, H, _round_up(total, self.step), dtypes, bufs[0].device)
             for new, old in zip(grown, bufs):
-                fill.add(new, new.shape[3], total, new.shape[2], src=old, src_stride=old.shape[2], copy=self._deq_offset, axis=2)
+                if new.dtype == old.dtype and new.shape[:2] == old.shape[:2] and new.shape[3] == old.shape[3]:
+                    fill.add(new, new.shape[3], total, new.shape[2], src=old, src_stride=old.shape[2], copy=self._deq_offset, axis=2)
+                else:                                        # rows of another dtype than before: cast, as a slice assignment does
+                    new[:, :, :self._deq_offset] = old[:, :, :self._deq_offset]
+                    fill.add(new, new.shape[3], total, new.shape[2], axis=2)
             fill.run()
             bufs = grown
         if all(dt == torch.float16 for dt in dtypes):

@@ -271,6 +271,8 @@ class StorageFill:
         """The fields of struct tq_fill_segment, checked against the bytes that the tensors hold."""
         row = inner * dst.element_size()
         if src is not None and copy > 0:
+            if src.dtype != dst.dtype:
+                raise ValueError(f"rows of {src.dtype} cannot be copied into {dst.dtype} as they are")
             held = src.untyped_storage().nbytes() - src.storage_offset() * src.element_size()
             if ((groups - 1) * src_stride + copy) * row > held:
                 raise ValueError(f"{groups} groups of {copy} rows, {src_stride} apart, exceed the {held} bytes of the source")
