@@ -91,3 +91,62 @@ def test_buffer_growth_casts_rows_of_another_dtype(monkeypatch, was, now, v_only
     for new, o in zip(grown, old):
         assert new.dtype == now and new.shape[2] == 512
         assert torch.equal(new[:, :, :256], o.to(now)) and not new[:, :, 257:].any()
+
+
+class _LateFill(ops.StorageFill):
+    """A storage fill that does its work in run(), as on the GPU."""
+
+    def __init__(self):
+        super().__init__()
+        self.asked = []
+
+    def add(self, *args, **kw):
+        self.asked.append((args, kw))
+
+    def run(self):
+        for args, kw in self.asked:
+            super().add(*args, **kw)
+        self.asked = []
+
+
+def _words(cache, n):
+    return [t[:, :, :n].clone() for t in _stored(cache)]
+
+
+@pytest.mark.parametrize("mode", [dict(), dict(fused=True), dict(v_only=True)])
+@pytest.mark.parametrize("at", range(8))
+def test_a_failed_allocation_leaves_the_cache_as_it_was(monkeypatch, mode, at):
+    """Allocation number `at` of an insert that grows the storage fails; the caller makes room and tries again."""
+    monkeypatch.setattr(ops, "StorageFill", _LateFill)
+    for name in ("encode_into", "encode_kv_into", "dequant_into", "dequant_kv_into"):
+        monkeypatch.setattr(ops, name, lambda *a, **kw: None)
+    cache = _grown(tqhip.TurboQuantKVCache(bits=3, **mode), 128, 250)
+    want = _words(cache, 250)
+    kept = _stored(cache)
+    x = torch.randn(B, H, 10, 128).half()
+    left = [at]
+
+    def failing(real):
+        def alloc(*args, **kw):
+            left[0] -= 1
+            if left[0] < 0:
+                raise torch.OutOfMemoryError("no room")
+            return real(*args, **kw)
+        return alloc
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", failing(torch.empty))
+        m.setattr(torch.Tensor, "new_empty", failing(torch.Tensor.new_empty))
+        try:
+            cache.update_and_fetch(x, x)
+            failed = False
+        except torch.OutOfMemoryError:
+            failed = True
+    assert failed == (left[0] < 0)
+    if failed:
+        assert cache.offset == 250 and all(a.data_ptr() == b.data_ptr() for a, b in zip(_stored(cache), kept))
+        out = cache.update_and_fetch(x, x)
+        if cache.fused:
+            assert not any(t.any() for t in out)
+    assert cache.offset == 260
+    for got, w in zip(_words(cache, 250), want):
+        assert torch.equal(got, w)

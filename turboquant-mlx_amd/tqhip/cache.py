@@ -176,26 +176,31 @@ class TurboQuantKVCache:
             new[:, :, :prev] = old[:, :, :prev]
         return new
 
-    def _ensure_storage(self, B, H, num_new, device, incoming=0, fill=None):
+    def _ensure_storage(self, B, H, num_new, device, incoming=0):
         """Room for num_new more positions (cache.py:100-123); the caller writes the first `incoming` of them itself."""
-        prev = self.offset
-        needed = prev + num_new
-        if self.v_packed is None or needed > self.v_packed.shape[2]:
-            self._reallocate(B, H, _round_up(needed, self.step), device, incoming, fill)
+        if self._lacks_room(num_new):
+            self._reallocate(B, H, _round_up(self.offset + num_new, self.step), device, incoming)
 
-    def _reallocate(self, B, H, n, device, incoming=0, fill=None):
+    def _lacks_room(self, num_new):
+        return self.v_packed is None or self.offset + num_new > self.v_packed.shape[2]
+
+    def _reallocate(self, B, H, n, device, incoming=0):
         """Fresh contiguous storage of n positions per (b, h) holding the first `offset` positions."""
+        fill = ops.StorageFill()
+        new = self._grown_storage(B, H, n, device, incoming, fill)
+        fill.run()
+        self.__dict__.update(new)
+
+    def _grown_storage(self, B, H, n, device, incoming, fill):
+        """The tensors of _reallocate by name, whole once `fill` has run.  The cache keeps what it has until then: an
+        allocation that fails on the way leaves it as it was."""
         prev = self.offset
-        own = fill if fill is not None else ops.StorageFill()
-        if not self.v_only:
-            self.k_packed, self.k_norms = (
-                self._grow(self.k_packed, (B, H, n, self._k_pdim), self._k_pdim, prev, incoming, torch.uint32, device, own),
-                self._grow(self.k_norms, (B, H, n), 1, prev, incoming, torch.float32, device, own))
-        self.v_packed, self.v_norms = (
-            self._grow(self.v_packed, (B, H, n, self._v_pdim), self._v_pdim, prev, incoming, torch.uint32, device, own),
-            self._grow(self.v_norms, (B, H, n), 1, prev, incoming, torch.float32, device, own))
-        if fill is None:
-            own.run()
+        new = {}
+        for side, pdim in ((("v", self._v_pdim),) if self.v_only else (("k", self._k_pdim), ("v", self._v_pdim))):
+            packed, norms = side + "_packed", side + "_norms"
+            new[packed] = self._grow(getattr(self, packed), (B, H, n, pdim), pdim, prev, incoming, torch.uint32, device, fill)
+            new[norms] = self._grow(getattr(self, norms), (B, H, n), 1, prev, incoming, torch.float32, device, fill)
+        return new
 
     # ---------------------------------------------------------------- codec calls
     def _encode(self, x, q, packed, norms, B, H, S, dim, prev):
@@ -279,15 +284,16 @@ class TurboQuantKVCache:
         return bufs
 
     # ---------------------------------------------------------------- cache.py:131-218
-    def _zero_like(self, t: torch.Tensor, fill) -> torch.Tensor:
+    def _zero_like(self, t: torch.Tensor, fill, made: dict) -> torch.Tensor:
         """A zero scalar of t's dtype on t's device, made once: the source of the stride-0 placeholders
-        (a fresh one per step would cost a fill launch each).  A new one's bytes join `fill`."""
+        (a fresh one per step would cost a fill launch each).  A new one's bytes join `fill`, itself `made`, which
+        the caller keeps once the fill has run."""
         key = (t.dtype, t.device)
-        z = self.__dict__.setdefault("_zero_scalars", {}).get(key)
+        z = self.__dict__.setdefault("_zero_scalars", {}).get(key, made.get(key))
         if z is None:
             base = t.new_empty(8)
             fill.add(base, 1, 0, 8)
-            z = self._zero_scalars[key] = base[0]
+            z = made[key] = base[0]
         return z
 
     def reserve(self, B: int, H: int, n_positions: int, dim: int, device="cuda"):
@@ -363,11 +369,15 @@ class TurboQuantKVCache:
         prev = self.offset
         total = prev + S
         fill = ops.StorageFill()
-        self._ensure_storage(B, H, S, device, incoming=S, fill=fill)
+        new = self._grown_storage(B, H, _round_up(total, self.step), device, S, fill) if self._lacks_room(S) else {}
         dtypes = [values.dtype] if self.v_only else [keys.dtype, values.dtype]
         fresh = None if self.fused else self._fetch_buffers(B, H, prev, total, dtypes, device, fill)
-        zeros = [self._zero_like(t, fill) for t in ((keys, values) if self.fused else (keys,) if self.v_only else ())]
-        fill.run()
+        made = {}
+        zeros = [self._zero_like(t, fill, made) for t in ((keys, values) if self.fused else (keys,) if self.v_only else ())]
+        fill.run()                                           # every allocation has succeeded: now the cache may change
+        self.__dict__.update(new)
+        if made:
+            self._zero_scalars.update(made)
         if self.v_only:
             self._encode(values, self._v_q, self.v_packed, self.v_norms, B, H, S, v_dim, prev)
         else:
