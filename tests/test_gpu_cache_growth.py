@@ -64,3 +64,12 @@ def test_buffer_grows_under_tokens_of_another_dtype(tq, was, now, kind):
     full = store._full_dequant(store.v_packed, store.v_norms, store._v_q, dim, B, H, n + 4, torch.float16)
     assert got.dtype == now and torch.equal(got[:, :, :n], prompt.to(now))
     assert torch.equal(got[:, :, n + 2:], full[:, :, n + 2:].to(now))       # the tokens after the growth
+
+
+@pytest.mark.parametrize("kind", ["default", "fused", "vonly"])
+def test_inserts_without_a_sequence(tq, kind):
+    x = torch.randn(0, 4, 20, 128, device="cuda").half()
+    cache = tq.VOnlyTurboQuantCache(bits=3) if kind == "vonly" else tq.TurboQuantKVCache(bits=3, fused=kind == "fused")
+    for n in (20, 40):
+        k, v = cache.update_and_fetch(x, x)
+        assert k.shape == v.shape == (0, 4, n, 128) and cache.offset == n

@@ -251,7 +251,7 @@ class StorageFill:
         """dst: contiguous, its rows along `axis` (default: the last but one, or the last with inner 1), `inner` elements each;
         the axes before are the groups: rows `copy` from src (rows src_stride apart per group) first, zeros in rows
         zero_from .. zero_to - 1.  Storage of one word a row has a trailing axis of 1 that only the caller can tell from rows."""
-        if copy == 0 and zero_to <= zero_from:
+        if (copy == 0 and zero_to <= zero_from) or dst.numel() == 0:
             return
         if axis is None:
             axis = dst.dim() - (2 if inner > 1 else 1)
