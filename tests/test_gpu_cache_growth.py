@@ -73,3 +73,28 @@ def test_inserts_without_a_sequence(tq, kind):
     for n in (20, 40):
         k, v = cache.update_and_fetch(x, x)
         assert k.shape == v.shape == (0, 4, n, 128) and cache.offset == n
+
+
+@pytest.mark.parametrize("nobuf", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int32])
+def test_vonly_insert_of_keys_that_are_no_kernel_dtype(tq, dtype, nobuf):
+    """Cast to float16, as any other key, whatever the number of new rows."""
+    k, v = _rows(128, 40)
+    k = (k * 8).round()
+    want, got = (tq.VOnlyTurboQuantCache(bits=3, no_v_buffer=nobuf) for _ in range(2))
+    for lo, hi in ((0, 30), (30, 39), (39, 40)):
+        a = want.update_and_fetch(k[:, :, lo:hi], v[:, :, lo:hi])
+        b = got.update_and_fetch(k[:, :, lo:hi].to(dtype), v[:, :, lo:hi])
+        _same(a, b)
+    _same(want.state, got.state)
+
+
+def test_vonly_insert_of_no_rows(tq):
+    x = torch.randn(2, 4, 0, 128, device="cuda").half()
+    cache = tq.VOnlyTurboQuantCache(bits=3)
+    for _ in range(2):
+        k, v = cache.update_and_fetch(x, x)
+        assert k.shape == v.shape == (2, 4, 0, 128) and cache.offset == 0
+    k, v = _rows(128, 5)
+    cache.update_and_fetch(k, v)
+    assert cache.update_and_fetch(x, x)[1].shape == (2, 4, 5, 128)
