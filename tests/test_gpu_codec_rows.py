@@ -95,3 +95,28 @@ def test_codec_rows_nan(tq, dim):
     wp, wn = o.fused_quantize(x[ok], s, b, dim, 3)
     assert np.array_equal(gp[ok], wp) and np.array_equal(gn[ok], wn)
     assert (gp[bad] == 0).all() and np.isnan(gn[bad]).all()
+
+
+# decision boundaries far out, where only rows along a Hadamard vector (one butterfly output of sqrt(dim)) reach them: the level
+# table of the streaming encoder has 64 cells (128 at four bits), and at d = 256 outputs beyond it are clamped into the last
+@pytest.mark.parametrize("dim,bounds", [
+    (256, [14.0]), (256, [-14.0]), (256, [11.4]), (256, [15.9]), (256, [-13.0, 0.0, 13.0]), (256, [10.0, 12.5, 15.0]),
+    (256, [-15.0, -14.0, -13.0, 0.0, 13.0, 14.0, 15.0]), (256, [float(i) * 2.1 for i in range(-7, 8)]),
+    (256, [-15.5] + [0.3 * i for i in range(-6, 7)] + [15.5]), (128, [11.0]), (128, [-11.2, 0.0, 11.2]), (128, [30.0]), (64, [7.9]),
+])
+def test_boundaries_near_the_largest_output(tq, dim, bounds):
+    bits = {1: 1, 3: 2, 7: 3, 15: 4}[len(bounds)]
+    rng = np.random.default_rng(dim)
+    n = 6151
+    x = _rows(rng, n, dim)
+    s = o.random_diagonal_sign(dim, 42)
+    for r in range(100, 1600):                          # along +- a Hadamard vector of the signed rows, with and without noise
+        k = int(rng.integers(0, dim))
+        h = np.array([(-1.0) ** bin(j & k).count("1") for j in range(dim)])
+        x[r] = (rng.choice([-1.0, 1.0]) * h + rng.choice([0.0, 0.1, 0.5]) * rng.standard_normal(dim)) * s
+    b = np.asarray(bounds, dtype=np.float32)
+    gp, gn = tq.fused_quantize(torch.from_numpy(x).cuda(), torch.from_numpy(s).cuda(), b, dim, bits)
+    wp, wn = o.fused_quantize(x, s, b, dim, bits)
+    idx = o.unpack_indices(wp, bits, dim)
+    assert idx.max() > 0 or max(bounds) > dim ** 0.5
+    assert np.array_equal(gp.cpu().numpy(), wp) and np.array_equal(gn.cpu().numpy(), wn)

@@ -287,7 +287,9 @@ float double_rounding_threshold(float b, float s) {
 // further margin of 0.01), beta a multiple of 1/8.  The kernel evaluates v = fma(w, alpha, beta + 2^20 + 32)
 // in float: one rounding, to a multiple of 1/8, i.e. at most 1/16 away from alpha*w + beta, so
 // floor(v) - 2^20 - 32 is the count of thresholds below w or one less for every w.  |w| <= sqrt(128)
-// (raw butterfly of a unit vector), so the guess must stay within +-32 of zero for the 64-entry table (three bits).
+// (raw butterfly of a unit vector; up to d = 128), so the guess must stay within +-32 of zero for the 64-entry table
+// (three bits).  At d = 256 |w| reaches 16 and the kernel clamps to the table's first and last cell: every threshold
+// must then lie in a cell of the table (here they lie in cells 0 .. nb - 1).
 // False when no such line exists (then the generic kernel counts the thresholds one by one).
 bool level_guess_search(const float* t, int nb, EncodeGuess& out);
 
@@ -296,7 +298,8 @@ bool level_guess_search(const float* t, int nb, EncodeGuess& out);
 // The kernel's cell of w is floor(alpha * w + beta0) or, for w within 1/16 below a cell edge, the next one; with no
 // threshold that close below an edge the count "thresholds below the cell + (w > the threshold inside it)" is the
 // count of thresholds below w either way.  The candidate with the widest margin is taken.
-bool level_cells_search(const float* t, int nb, EncodeGuess& out) {
+// clamped (d = 256): thresholds outside the table's cells refuse the line.  Otherwise no w reaches such a threshold.
+bool level_cells_search(const float* t, int nb, bool clamped, EncodeGuess& out) {
   for (int i = 0; i < nb; ++i)
     if (!std::isfinite(t[i]) || (i > 0 && !(t[i] > t[i - 1]))) return false;
   const int half = nb == 15 ? 64 : 32;                              // the kernel's table has 2 * half cells
@@ -314,7 +317,7 @@ bool level_cells_search(const float* t, int nb, EncodeGuess& out) {
       for (int j = 0; j < nb && ok; ++j) {
         const double u = a * (double)t[j] + b;
         const double c = std::floor(u), f = u - c;
-        if (f < margin || f > 1.0 - margin || c <= prev_cell) ok = false;
+        if (f < margin || f > 1.0 - margin || c <= prev_cell || (clamped && (c < -half || c > half - 1))) ok = false;
         prev_cell = c;
         slack = std::fmin(slack, std::fmin(f - margin, 1.0 - margin - f));
       }
@@ -361,7 +364,7 @@ EncodePlan encode_plan(const float* boundaries, int dim, int bits, int variant) 
   memcpy(s.b, boundaries, nb * sizeof(float));
   for (int i = 0; i < 15; ++i) s.p.thr.t[i] = INFINITY;
   tq::encode_thresholds(boundaries, dim, bits, variant, s.p.thr.t);
-  s.p.has_guess = (nb == 7) ? level_guess_search(s.p.thr.t, nb, s.p.gs) : level_cells_search(s.p.thr.t, nb, s.p.gs);
+  s.p.has_guess = (nb == 7) ? level_guess_search(s.p.thr.t, nb, s.p.gs) : level_cells_search(s.p.thr.t, nb, dim > 128, s.p.gs);
   {
     std::lock_guard<std::mutex> lock(mu);
     slots[next] = s;
