@@ -120,3 +120,28 @@ def test_boundaries_near_the_largest_output(tq, dim, bounds):
     idx = o.unpack_indices(wp, bits, dim)
     assert idx.max() > 0 or max(bounds) > dim ** 0.5
     assert np.array_equal(gp.cpu().numpy(), wp) and np.array_equal(gn.cpu().numpy(), wn)
+
+
+@pytest.mark.parametrize("call", ["append", "encode"])
+def test_small_calls_do_not_wait_for_the_level_search(tq, call):
+    """The search for the streaming encoder's level line (13 ms at four bits) is no part of a call that does not take it: a
+    token's append, a few rows.  Each call has boundaries that no call has had before."""
+    import time
+    dim, bits, n = 64, 4, 8
+    s = torch.from_numpy(o.random_diagonal_sign(dim, 42)).cuda()
+    base = np.asarray(o.gaussian_boundaries(o.gaussian_codebook(bits)), dtype=np.float32)
+    x = torch.randn(1, 1, n, dim, device="cuda").half()
+    k, v = (torch.zeros(1, 1, n, dim, dtype=torch.float16, device="cuda") for _ in range(2))
+    vp = torch.zeros(1, 1, n, tq.packed_dim(dim, bits), dtype=torch.int32, device="cuda").view(torch.uint32)
+    vn = torch.zeros(1, 1, n, device="cuda")
+    took = []
+    for i in range(12):
+        b = base * np.float32(1.0 + 0.01 * i + (0.003 if call == "encode" else 0.0))
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        if call == "append":
+            tq.ops.vonly_append_into(x, x, s, b, k, v, vp, vn, position=0, bits=bits)
+        else:
+            tq.fused_quantize(x[0, 0], s, b, dim, bits)
+        took.append(time.perf_counter() - t0)
+    assert sorted(took)[len(took) // 2] < 2e-3, took

@@ -334,42 +334,61 @@ bool level_cells_search(const float* t, int nb, bool clamped, EncodeGuess& out) 
 
 // Thresholds and level guess of the encoder for the last few (boundaries, dim, variant) seen, by value: a process that
 // alternates widths or threshold rules between calls -- caches of different bits, keys and values under different
-// rules -- would otherwise repeat a search of several milliseconds at every switch, and every call the bisections of
-// double_rounding_threshold (2 us at three bits).  The lock covers the table only, not the search: two threads that
-// miss on the same set both search and store the same result.
+// rules -- would otherwise repeat the search for a guess at every switch, and every call the bisections of
+// double_rounding_threshold (2 us at three bits).  The search (0.3 ms at three bits, 13 ms at four) is made for callers
+// that use the guess only: a token's step never waits for it.  The lock covers the table only, not the search: two
+// threads that miss on the same set both search and store the same result.
 struct EncodePlan {
   Thresholds thr;
   EncodeGuess gs;
   bool has_guess;
 };
 
-EncodePlan encode_plan(const float* boundaries, int dim, int bits, int variant) {
-  constexpr int kSlots = 8;
-  struct Slot { float b[15]; int nb, dim, variant; EncodePlan p; };
+EncodePlan encode_plan(const float* boundaries, int dim, int bits, int variant, bool want_guess) {
+  constexpr int kSlots = 32;                                         // every width, head dimension and rule there is, and a few given tables
+  struct Slot { float b[15]; int nb, dim, variant; bool searched; EncodePlan p; };
   static std::mutex mu;
   static Slot slots[kSlots];
   static int n_used = 0, next = 0;
   const int nb = (1 << bits) - 1;
-  {
-    std::lock_guard<std::mutex> lock(mu);
+  auto find = [&]() -> Slot* {                                        // under the lock
     for (int i = 0; i < n_used; ++i)
       if (slots[i].nb == nb && slots[i].dim == dim && slots[i].variant == variant &&
           memcmp(slots[i].b, boundaries, nb * sizeof(float)) == 0)
-        return slots[i].p;
-  }
+        return &slots[i];
+    return nullptr;
+  };
   Slot s{};
-  s.nb = nb;
-  s.dim = dim;
-  s.variant = variant;
-  memcpy(s.b, boundaries, nb * sizeof(float));
-  for (int i = 0; i < 15; ++i) s.p.thr.t[i] = INFINITY;
-  tq::encode_thresholds(boundaries, dim, bits, variant, s.p.thr.t);
-  s.p.has_guess = (nb == 7) ? level_guess_search(s.p.thr.t, nb, s.p.gs) : level_cells_search(s.p.thr.t, nb, dim > 128, s.p.gs);
+  bool known = false;
   {
     std::lock_guard<std::mutex> lock(mu);
-    slots[next] = s;
-    next = (next + 1) % kSlots;
-    if (n_used < kSlots) ++n_used;
+    if (const Slot* hit = find()) {
+      if (hit->searched || !want_guess) return hit->p;
+      s = *hit;
+      known = true;
+    }
+  }
+  if (!known) {
+    s.nb = nb;
+    s.dim = dim;
+    s.variant = variant;
+    memcpy(s.b, boundaries, nb * sizeof(float));
+    for (int i = 0; i < 15; ++i) s.p.thr.t[i] = INFINITY;
+    tq::encode_thresholds(boundaries, dim, bits, variant, s.p.thr.t);
+  }
+  if (want_guess) {
+    s.p.has_guess = (nb == 7) ? level_guess_search(s.p.thr.t, nb, s.p.gs) : level_cells_search(s.p.thr.t, nb, dim > 128, s.p.gs);
+    s.searched = true;
+  }
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (Slot* hit = find()) {
+      if (!hit->searched) *hit = s;
+    } else {
+      slots[next] = s;
+      next = (next + 1) % kSlots;
+      if (n_used < kSlots) ++n_used;
+    }
   }
   return s.p;
 }
@@ -523,7 +542,7 @@ int encode_pair(const void* k_new, int k_dtype, const float* k_signs, uint32_t* 
                 const void* v_new, int v_dtype, const float* v_signs, uint32_t* v_packed, float* v_norms,
                 const float* boundaries, int bits, int64_t n_rows, int64_t group_stride, int variant, tq_stream_t stream_,
                 const int64_t* pos_dev) {
-  const Thresholds thr = encode_plan(boundaries, 128, bits, variant).thr;
+  const Thresholds thr = encode_plan(boundaries, 128, bits, variant, false).thr;
   PairSide k{k_new, k_signs, k_packed, k_norms, k_dtype}, v{v_new, v_signs, v_packed, v_norms, v_dtype};
   const int grid = (int)((2 * n_rows + kWavesPerBlock - 1) / kWavesPerBlock);
   TQ_DISPATCH_BITS(bits, (encode_pair_kernel<B_><<<grid, kBlock, 0, (hipStream_t)stream_>>>(k, v, thr, n_rows, group_stride, pos_dev)));
@@ -585,10 +604,11 @@ int encode_sides(const char* who, const EncodeSides& sides, int n_sides, int x_d
     wide = wide && tq::aligned(s.x, 16);
   }
   const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
-  const EncodePlan plan = encode_plan(boundaries, dim, bits, variant);
   const bool whole = whole_batches(dim, rm);
-  if (dim >= 64 && (whole || n_rows * n_sides >= stream_min_rows(dim, true)) && n_rows < (int64_t)1 << 31 &&
-      (whole || rows_fit_32_bits(rm, n_groups)) && wide && plan.has_guess) {
+  const bool stream_form = dim >= 64 && (whole || n_rows * n_sides >= stream_min_rows(dim, true)) && n_rows < (int64_t)1 << 31 &&
+                           (whole || rows_fit_32_bits(rm, n_groups)) && wide;
+  const EncodePlan plan = encode_plan(boundaries, dim, bits, variant, stream_form);
+  if (stream_form && plan.has_guess) {
     const EncodeCall c{sides, n_sides, x_dtype, plan.thr, plan.gs, rm, bits, stream};
     if (whole) launch_encode_rows<128, false>(c);
     else if (dim == 64) launch_encode_rows<64, true>(c);
@@ -691,7 +711,7 @@ int vonly_append(const void* k_new, int k_dtype, const void* v_new, int v_dtype,
       !tq::aligned(v_signs, 4) || !tq::aligned(k_f16, 2) || !tq::aligned(v_packed, 4) || !tq::aligned(v_norms, 4) ||
       (v_raw && !tq::aligned(v_raw, tq::dtype_size(v_dtype))))
     return tq::fail(TQ_ERR_ALIGN, "tq_vonly_append: misaligned pointer");
-  const Thresholds thr = encode_plan(boundaries, dim, bits, variant).thr;
+  const Thresholds thr = encode_plan(boundaries, dim, bits, variant, false).thr;
   const RowMap rm = row_map(n_rows, rows_per_group, packed_group_stride, norms_group_stride, 0);
   if (pos_dev && (!tq::aligned(pos_dev, 8) || pos_cap < 1))
     return tq::fail(TQ_ERR_ARG, "tq_vonly_append_at: position_dev must be 8-byte aligned and t_alloc >= 1");
