@@ -284,9 +284,11 @@ typedef struct tq_decode_shape {
   int64_t mask_head_stride;  /* floats between query heads (0 = shared) */
   float attn_scale;
   int32_t out_dtype;         /* TQ_F32, TQ_F16 or TQ_BF16 */
-  int32_t allow_mma;         /* 1: use the fp16 matrix-core kernels where the shape allows (d = 128,
-                                n_rep <= 16, every width 1-4; operands rounded to fp16, float32
-                                accumulation);
+  int32_t allow_mma;         /* 1: use the matrix-core kernels where the shape allows, float32 accumulation, every
+                                width 1-4: d = 128, n_rep <= 16 with operands rounded to fp16; d = 64, and
+                                d = 256 over fp16 keys, any n_rep, with operands split into an fp16 value and the
+                                fp16 remainder of its rounding (22 bits; fp16 keys are exact).  d = 32 and what
+                                else there is: the float32 vector kernels;
                                 0: float32 vector-ALU kernels only */
 } tq_decode_shape;
 
@@ -334,8 +336,9 @@ int tq_flash_decode_plan(int n_seq, int n_kv_heads, int64_t max_seq_len, int rag
  * fused_attention.py:50-121 in one launch for the cache of v_only_cache.py:24-127.
  *   q [n_seq, n_kv*n_rep, dim] dtype q_dtype;  k_f16 rows of dim halfs;  out as tq_flash_decode.
  * With allow_mma, d = 128 and n_rep <= 16 the tile pass runs on the matrix cores for values of every
- * width (bits 1-4, as adaptive.py:26 / v_only_cache.py:41 take them); other shapes take the float32 kernels.
- * Alignment: k_f16 16 bytes (TQ_ERR_ALIGN otherwise).  The matrix-core pass reads q in 16-byte pieces: a q
+ * width (bits 1-4, as adaptive.py:26 / v_only_cache.py:41 take them); d = 64 and 256 run there with split operands
+ * (tq_decode_shape.allow_mma); other shapes take the float32 kernels.
+ * Alignment: k_f16 16 bytes (TQ_ERR_ALIGN otherwise).  The matrix-core pass of d = 128 reads q in 16-byte pieces: a q
  * that is not 16-byte aligned (a view at an odd element offset) is served by the float32 kernels instead,
  * same result to their rounding, several times slower.
  */

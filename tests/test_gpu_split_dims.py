@@ -26,9 +26,9 @@ def _case(tq, B, n_kv, n_rep, T, D, bits, seed=1):
     return mk(B, n_kv * n_rep, D), pack(), mk(B, n_kv, T).abs() * 8 + 0.1, pack(), mk(B, n_kv, T).abs() * 8 + 0.1, mk(B, n_kv, T, D).half()
 
 
-# float32 arithmetic on both sides, sums in another order and operands of 22 bits: a few 2^-22 of the magnitudes summed,
-# which scores of up to 30 in the exponent multiply
-_REL = 3e-5
+# float32 arithmetic on both sides, sums in another order and operands of 22 bits.  A score that is off by a few 2^-24 of its
+# magnitude, up to 30 here, moves its weight by that much: 30 x 4 x 6e-8, half of it to either side.
+_REL = 4e-6
 
 
 @pytest.mark.parametrize("bits", [1, 2, 3, 4])
@@ -93,3 +93,78 @@ def test_split_dims_against_float64(tq):
            / np.linalg.norm(want) for pr in ("fp16", "fp32")]
     print("relative error, split / float32 kernels:", err)
     assert err[0] <= max(4 * err[1], 1e-6), err
+
+
+def _had(D):
+    i = np.arange(D)
+    return np.array([[(-1.0) ** bin(a & b).count("1") for b in i] for a in i])
+
+
+def _float64(tq, q, kp, kn, kd, vp, vn, c, signs, D, bits, sc, n_rep, mask):
+    """The step in 64 bits: kp / kn packed keys in the rotated domain, or kd fp16 keys."""
+    cc = torch.from_numpy(np.asarray(c, dtype=np.float64))
+    B, n_kv, T = vn.shape
+    vals = cc[tq.unpack_indices(vp, bits, D).cpu().long()] * vn.cpu().double()[..., None]
+    keys = kd.cpu().double() if kp is None else cc[tq.unpack_indices(kp, bits, D).cpu().long()] * (kn.cpu().double() / D)[..., None]
+    rep = lambda t: t.repeat_interleave(n_rep, dim=1)   # noqa: E731
+    s = (rep(keys) * q.cpu().double()[:, :, None, :]).sum(-1) * sc + (0 if mask is None else mask.cpu().double())
+    s = torch.nan_to_num(s, neginf=-np.inf)
+    w = torch.softmax(s, dim=-1)
+    rot = (rep(vals) * torch.where(w > 0, w, 0.0)[..., None]).sum(2)
+    return (rot @ torch.from_numpy(_had(D)) * signs.cpu().double() / D).numpy()
+
+
+@pytest.mark.parametrize("D,packed", [(64, True), (64, False), (256, False)])
+@pytest.mark.parametrize("octaves", [0, 3, 13])
+def test_split_dims_heads_of_different_magnitude(tq, D, packed, octaves):
+    """Heads of one wave that attend rows whose value norms lie far apart: head h sees the positions h, h + 8, ... only, whose
+    norms are 2^(-octaves h).  Per head, no further from 64-bit arithmetic than the float32 kernel, a few units of float32
+    (2^-24 = 6e-8) allowed for sums in another order."""
+    B, n_kv, n_rep, T, bits = 2, 2, 8, 700, 3
+    c = o.gaussian_codebook(bits)
+    q, kp, kn, vp, vn, kd = _case(tq, B, n_kv, n_rep, T, D, bits)
+    signs = torch.from_numpy(o.random_diagonal_sign(D, 43)).cuda()
+    pos = torch.arange(T, device="cuda") % n_rep
+    vn = (vn * torch.exp2(-octaves * pos.float())).contiguous()
+    head = torch.arange(n_kv * n_rep, device="cuda") % n_rep
+    mask = torch.where(pos[None, :] == head[:, None], 0.0, float("-inf")).float()[None].expand(B, -1, -1).contiguous()
+    sc = 1.0 / (8.0 * D ** 0.5) if packed else D ** -0.5
+
+    def run(precision):
+        if packed:
+            return tq.flash_decode(q, kp, kn, vp, vn, c, c, signs, D, bits, sc, n_rep=n_rep, mask=mask, precision=precision)
+        return tq.vonly_decode(q, kd, vp, vn, c, signs, D, bits, sc, n_rep=n_rep, mask=mask, precision=precision)
+    want = _float64(tq, q, kp if packed else None, kn, kd, vp, vn, c, signs, D, bits, sc, n_rep, mask)
+    err = [np.linalg.norm(run(p).cpu().double().numpy() - want, axis=-1) / np.linalg.norm(want, axis=-1) for p in ("fp16", "fp32")]
+    print(D, packed, octaves, "largest relative error of a head, split / float32:", err[0].max(), err[1].max())
+    assert err[0].max() <= 1.5 * err[1].max() + 1.2e-7, (err[0].max(), err[1].max())
+
+
+@pytest.mark.parametrize("D", [64, 256])
+def test_split_dims_infinite_keys(tq, D):
+    """Keys that overflowed float16: a head whose score of such a position is -inf leaves it out, as the float32 kernel does."""
+    B, n_kv, n_rep, T, bits = 1, 2, 4, 300, 3
+    c = o.gaussian_codebook(bits)
+    q, _, _, vp, vn, kd = _case(tq, B, n_kv, n_rep, T, D, bits)
+    signs = torch.from_numpy(o.random_diagonal_sign(D, 43)).cuda()
+    q[..., 7] = q[..., 7].abs() + 0.25
+    q[0, 3] = torch.randint(-8, 9, (D,), device="cuda").float()              # no remainder: exact in fp16
+    q[0, 3, 7] = 2.0
+    for at, value in ((5, float("-inf")), (70, float("-inf")), (299, float("-inf")), (130, 65504.0)):
+        kd[:, :, at, 7] = value
+    args = (q, kd, vp, vn, c, signs, D, bits, D ** -0.5)
+    got, want = tq.vonly_decode(*args, n_rep=n_rep), tq.vonly_decode(*args, n_rep=n_rep, precision="fp32")
+    assert bool(torch.isfinite(want).all()) and bool(torch.isfinite(got).all())
+    assert (got - want).abs().max() <= _REL * want.abs().max()
+
+
+@pytest.mark.parametrize("scale", [1e35, 1e-35])
+def test_split_dims_extreme_norms(tq, scale):
+    """Value norms near the ends of float32."""
+    D, bits, n_rep = 64, 3, 4
+    c = o.gaussian_codebook(bits)
+    q, kp, kn, vp, vn, _ = _case(tq, 1, 2, n_rep, 200, D, bits)
+    signs = torch.from_numpy(o.random_diagonal_sign(D, 43)).cuda()
+    args = (q, kp, kn, vp, vn * scale, c, c, signs, D, bits, 0.02)
+    got, want = tq.flash_decode(*args, n_rep=n_rep), tq.flash_decode(*args, n_rep=n_rep, precision="fp32")
+    assert bool(torch.isfinite(want).all()) and (got.double() - want.double()).abs().max() <= _REL * want.double().abs().max()

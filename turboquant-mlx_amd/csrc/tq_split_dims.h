@@ -5,18 +5,20 @@
 // The vector kernel decodes every element for eight heads with multiply-adds: its time is vector arithmetic (2 sequences x
 // 32 / 8 heads x 8 190 positions of d = 64 at four bits: 20.4 us for 9 MB; this kernel, query rotation included, 10.6).  Here a wave's 64 positions and 16 heads are
 // products of 16x16x32 matrix instructions.  Operands keep 22 bits: queries, weights and centroids enter as an fp16 value and
-// the fp16 remainder of its rounding, keys in fp16 are exact; queries are scaled per head and weights per wave by powers of two,
-// so that magnitudes outside the range of fp16 change nothing (see tq_split_mfma.h).
+// the fp16 remainder of its rounding, keys in fp16 are exact; queries and, in each wave, weights times value norms are scaled per
+// head by powers of two, so that magnitudes outside the range of fp16 change nothing, nor does a head whose value norms lie many
+// octaves below another's (see tq_split_mfma.h).  Infinite keys and queries give the infinite scores of the vector kernel: a
+// remainder never meets them.
 #pragma once
 
 // query heads of a kv head that one workgroup serves: at d = 256 eight, whose sums leave room for three workgroups in a CU's LDS
 // (4 sequences x 32 / 8 heads x 16 000 positions, fp16 keys: a call takes 150 us with one workgroup of sixteen heads a CU, 84 us with three of eight)
 template <int D> constexpr int kSplitHeads = D == 256 ? 8 : 16;
 
-// power of two that brings `largest` to [2^13, 2^14), and its inverse; both normal
+// power of two that brings `largest` to [2^13, 2^14), and its inverse: normal for every float (a largest below 2^-113 stays as
+// many octaves below)
 __device__ __forceinline__ void split_scale(float largest, float& up, float& down) {
-  int ex = (int)((__float_as_uint(largest) >> 23) & 0xFF);
-  ex = ex < 40 ? (ex < 1 ? 140 : 40) : (ex > 230 ? 230 : ex);
+  const int ex = min(max((int)((__float_as_uint(largest) >> 23) & 0xFF), 14), 254);
   up = __uint_as_float((uint32_t)(254 - ex + 13) << 23);
   down = __uint_as_float((uint32_t)(ex - 13) << 23);
 }
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
       const float x = v[it][i] * up;
       const __half h = __float2half_rn(x);
       hi[lane + 64 * i] = h;
-      lo[lane + 64 * i] = __float2half_rn(x - __half2float(h));
+      lo[lane + 64 * i] = __float2half_rn(fabsf(x) == INFINITY ? 0.0f : x - __half2float(h));
     }
   }
   // fp16 keys: row n16 of a group of 16 positions, one group ahead of its products (rows past the end: the last that exists)
@@ -152,13 +154,13 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   float s[4][4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    f4 acc = {0.f, 0.f, 0.f, 0.f}, rem = {0.f, 0.f, 0.f, 0.f};   // products of the values, products with a remainder
     if constexpr (DENSE) {
       u4 (&k)[KB] = kd[t & 1];
       if (t < 3) load_keys(t + 1, kd[(t + 1) & 1]);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, k[kb]), __builtin_bit_cast(h8, ql[kb]), acc, 0, 0, 0);
+        rem = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, k[kb]), __builtin_bit_cast(h8, ql[kb]), rem, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, k[kb]), __builtin_bit_cast(h8, qh[kb]), acc, 0, 0, 0);
       }
     } else {
@@ -174,16 +176,16 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
           kh[k] = e.x;
           kl[k] = e.y;
         }
-        // smallest terms first
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kl), __builtin_bit_cast(h8, qh[kb]), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kh), __builtin_bit_cast(h8, ql[kb]), acc, 0, 0, 0);
+        rem = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kl), __builtin_bit_cast(h8, qh[kb]), rem, 0, 0, 0);
+        rem = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kh), __builtin_bit_cast(h8, ql[kb]), rem, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kh), __builtin_bit_cast(h8, qh[kb]), acc, 0, 0, 0);
       }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int row = 16 * t + 4 * g + j;
-      float x = acc[j] * qdown;
+      // an infinite key times a remainder of 0 is no number: the product of the values is the score then
+      float x = (fabsf(acc[j]) == INFINITY ? acc[j] : acc[j] + rem[j]) * qdown;
       if (!DENSE) x = (x * tqm::kSplitTableUnscale * kn_s[wave][row]) * a.inv_dim;
       x *= a.attn_scale;
       if (row < rows) {
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
     }
   l = sum_over_rows(l);
   float up, down;
-  split_scale(wave_max(largest), up, down);
+  split_scale(max_over_rows(largest), up, down);                // of head n16
   u4 ph[2], pl[2];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
@@ -272,7 +274,9 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   // ---- the wave's sums into its own area (its packed rows have been consumed), then the four waves together
   wave_lds_fence();
   float* dep = reinterpret_cast<float*>(area_s[wave]);
-  const float unscale = down * tqm::kSplitTableUnscale;
+  float unscale[4];                                             // of heads 4 g + j, whose sums this lane holds
+#pragma unroll
+  for (int j = 0; j < 4; ++j) unscale[j] = __shfl(down, 4 * g + j) * tqm::kSplitTableUnscale;
 #pragma unroll
   for (int np = 0; np < NP; ++np)
 #pragma unroll
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
 #pragma unroll
       for (int e4 = 0; e4 < EL; e4 += 4)
         if (kH == 16 || 4 * g + j < kH) *reinterpret_cast<f4*>(dep + (4 * g + j) * D + EL * (n16 + 16 * np) + e4) =
-            f4{acc[np][e4][j] * unscale, acc[np][e4 + 1][j] * unscale, acc[np][e4 + 2][j] * unscale, acc[np][e4 + 3][j] * unscale};
+            f4{acc[np][e4][j], acc[np][e4 + 1][j], acc[np][e4 + 2][j], acc[np][e4 + 3][j]} * unscale[j];
   if (g == 0) {
     m_s[wave][n16] = m;
     l_s[wave][n16] = l;
