@@ -168,3 +168,20 @@ def test_split_dims_extreme_norms(tq, scale):
     args = (q, kp, kn, vp, vn * scale, c, c, signs, D, bits, 0.02)
     got, want = tq.flash_decode(*args, n_rep=n_rep), tq.flash_decode(*args, n_rep=n_rep, precision="fp32")
     assert bool(torch.isfinite(want).all()) and (got.double() - want.double()).abs().max() <= _REL * want.double().abs().max()
+
+
+@pytest.mark.parametrize("D,packed", [(64, True), (64, False), (256, False)])
+@pytest.mark.parametrize("scale", [1e4, 100.0, 1e-6])
+def test_split_dims_codebooks_of_another_scale(tq, D, packed, scale):
+    """A given codebook need not be that of a unit Gaussian."""
+    bits, n_rep = 3, 4
+    c = (np.asarray(o.gaussian_codebook(bits)) * scale).astype(np.float32)
+    q, kp, kn, vp, vn, kd = _case(tq, 1, 2, n_rep, 700, D, bits)
+    signs = torch.from_numpy(o.random_diagonal_sign(D, 43)).cuda()
+
+    def run(**kw):
+        if packed:
+            return tq.flash_decode(q, kp, kn, vp, vn, c, c, signs, D, bits, 0.02 / scale, n_rep=n_rep, **kw)
+        return tq.vonly_decode(q, kd, vp, vn, c, signs, D, bits, D ** -0.5, n_rep=n_rep, **kw)
+    got, want = run(), run(precision="fp32")
+    assert (got - want).abs().max() <= _REL * want.abs().max()

@@ -48,6 +48,7 @@ struct DecodeArgs {
   int64_t mask_seq_stride, mask_head_stride;
   int32_t n_kv, n_rep, n_rgroups, n_tiles_max;
   float attn_scale, inv_dim, threshold;
+  float k_table, v_table;       // split_decode_kernel: what an entry of its centroid tables counts
 };
 
 __device__ __forceinline__ void seq_range(const int32_t* seq_offsets, int64_t seq_len, int seq,
@@ -666,6 +667,19 @@ void fill_codebook(Codebook& cb, const float* c, int bits) {
   for (int i = 0; i < 16; ++i) cb.c[i] = (c && i < (1 << bits)) ? c[i] : 0.0f;
 }
 
+// The split kernels' tables hold fp16 pairs of kSplitTableScale times a centroid: full precision for codebooks whose largest
+// centroid lies between 2^-4 and 2^5, as those of unit Gaussians do.  Others are brought to [1, 2) by a power of two first.
+// Returns what a table entry counts.
+float fit_split_codebook(Codebook& cb) {
+  float largest = 0.0f;
+  for (int i = 0; i < 16; ++i) largest = fmaxf(largest, fabsf(cb.c[i]));
+  int ex = 0;
+  if (!(largest >= 0.0625f && largest <= 32.0f) && largest > 0.0f && largest < INFINITY) frexpf(largest, &ex), --ex;
+  if (ex)
+    for (int i = 0; i < 16; ++i) cb.c[i] = ldexpf(cb.c[i], -ex);
+  return ldexpf(tqm::kSplitTableUnscale, ex);
+}
+
 int check_heads(int n_kv, int n_rep, const char* who) {
   if (n_kv < 1) return tq::fail(TQ_ERR_ARG, "%s: n_kv_heads must be >= 1, got %d", who, n_kv);
   if (n_rep < 1) return tq::fail(TQ_ERR_NREP, "%s: n_rep must be >= 1, got %d", who, n_rep);
@@ -712,6 +726,8 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
     // to d = 128.  d = 32, and float32 arithmetic asked for: the vector kernel.
     if (KMODE != kWeights && sh.allow_mma && (sh.dim == 64 || (KMODE == kDenseK && sh.dim == 256))) {
       const int heads = sh.dim == 256 ? kSplitHeads<256> : kSplitHeads<64>;
+      a.k_table = fit_split_codebook(kcb);
+      a.v_table = fit_split_codebook(vcb);
       a.n_rgroups = (sh.n_rep + heads - 1) / heads;
       dim3 sgrid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
       if (sh.dim == 64) {

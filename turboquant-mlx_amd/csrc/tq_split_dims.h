@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
       const int row = 16 * t + 4 * g + j;
       // an infinite key times a remainder of 0 is no number: the product of the values is the score then
       float x = (fabsf(acc[j]) == INFINITY ? acc[j] : acc[j] + rem[j]) * qdown;
-      if (!DENSE) x = (x * tqm::kSplitTableUnscale * kn_s[wave][row]) * a.inv_dim;
+      if (!DENSE) x = (x * a.k_table * kn_s[wave][row]) * a.inv_dim;
       x *= a.attn_scale;
       if (row < rows) {
         if (a.mask && n16 < n_local)
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
   float* dep = reinterpret_cast<float*>(area_s[wave]);
   float unscale[4];                                             // of heads 4 g + j, whose sums this lane holds
 #pragma unroll
-  for (int j = 0; j < 4; ++j) unscale[j] = __shfl(down, 4 * g + j) * tqm::kSplitTableUnscale;
+  for (int j = 0; j < 4; ++j) unscale[j] = __shfl(down, 4 * g + j) * a.v_table;
 #pragma unroll
   for (int np = 0; np < NP; ++np)
 #pragma unroll
