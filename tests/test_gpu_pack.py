@@ -50,3 +50,18 @@ def test_pack_out_of_range_and_empty(tq):
         assert tq.pack_indices(idx[:0].cuda(), bits).shape == tq.pack_indices(idx[:0], bits).shape
         assert tq.unpack_indices(words[:0].cuda(), bits, 96).shape == (0, 96)
         assert tq.unpack_indices(words.cuda(), bits, 0).shape == (41, 0)
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+def test_packing_can_be_traced(tq, bits):
+    """A graph recorded from real tensors gives the words of the tensors that it is run on, not of those it was made with."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    dim = 40
+    a, b = (torch.randint(0, 1 << bits, (6, dim), device="cuda", dtype=torch.uint8) for _ in range(2))
+
+    def both(x):
+        p = tq.pack_indices(x, bits).view(torch.int32)
+        return p, tq.unpack_indices(p, bits, dim)
+    want = both(b)
+    got = make_fx(both)(a)(b)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], b)

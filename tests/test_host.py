@@ -377,3 +377,19 @@ def test_flash_decode_plan_follows_its_rule_on_host():
                         if got:
                             assert 2 <= got <= (4 if ragged else 8)
                             assert got * 256 * (-(-max_len // (got * 256)) - 1) < max_len
+
+
+def test_tracing_of_the_integer_plumbing_is_noticed():
+    """Where tensor operations are recorded, packing must stay tensor operations (the GPU route is a library call)."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    seen = []
+
+    def f(x):
+        seen.append(ops._observed())
+        return ops.pack_indices(x, 3).view(torch.int32)
+    x = torch.randint(0, 8, (3, 20), dtype=torch.uint8)
+    y = torch.randint(0, 8, (3, 20), dtype=torch.uint8)
+    want = f(y)
+    assert torch.equal(make_fx(f)(x)(y), want)
+    torch.jit.trace(lambda t: (seen.append(ops._observed()), t + 1)[1], x, check_trace=False)
+    assert seen == [False, True, True] and not ops._observed()

@@ -144,9 +144,17 @@ def _head_layout_2d(t: torch.Tensor) -> tuple[torch.Tensor, int]:
 
 # ------------------------------------------------------------------ packing (integer plumbing)
 
+def _observed() -> bool:
+    """Whether something records or rewrites the tensor operations of the caller: a dispatch mode (make_fx, flop counters), the
+    JIT's tracer, a compiler.  A library call would be missing from what they see."""
+    return torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+
+
 def _native_pack(t: torch.Tensor) -> bool:
-    """Integer plumbing also runs on the CPU, on tensor subclasses and under functional transforms: as tensor operations."""
-    return t.is_cuda and t.numel() > 0 and type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+    """Integer plumbing also runs on the CPU, on tensor subclasses, under functional transforms and under tracing: as tensor
+    operations."""
+    return (t.is_cuda and t.numel() > 0 and type(t) is torch.Tensor and not _observed()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
 def pack_indices(indices: torch.Tensor, bits: int) -> torch.Tensor:
