@@ -91,3 +91,15 @@ def test_composed_in_several_calls(tq, monkeypatch):
     whole = tq.turboquant_attention(q, cache, 0.09, mask)
     monkeypatch.setattr(tq.ops, "_COMPOSED_WORKSPACE", 100_000)
     assert torch.equal(whole, tq.turboquant_attention(q, cache, 0.09, mask))
+
+
+def test_composed_scores_are_temporaries(tq, monkeypatch):
+    """The scores of a call (7 MB here) are free again after it, whatever its length."""
+    cache, mk = _cache(tq, 1, 4, 65536, 3)
+    q = mk(1, 28, 1, D)
+    monkeypatch.setattr(tq.ops, "_workspaces", {})
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = tq.turboquant_attention(q, cache, 0.09)
+    kept = torch.cuda.memory_allocated() - before - out.numel() * out.element_size()
+    assert kept < 1 << 20, kept

@@ -854,7 +854,7 @@ def flash_from_query(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_no
     return out
 
 
-_COMPOSED_WORKSPACE = 256 << 20    # bytes of scores that one call of composed_decode may keep
+_COMPOSED_WORKSPACE = 256 << 20    # bytes of scores that one launch of composed_decode may take
 
 
 def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs, dim: int,
@@ -862,7 +862,8 @@ def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_nor
     """prerotate_query, prerot_fused_qk_scores, softmax_rows and sparse_v_matvec for every sequence of a cache in three
     launches (tq_composed_decode), float32 fidelity.  q (n_seq, n_q, dim); K / V in cache layout (n_seq, n_kv, T_alloc, *);
     returns (n_seq, n_q, dim) in q's dtype (float32 for one that is no kernel dtype).  Shapes of vonly_sparse_supported.
-    Batches whose scores would not fit the workspace bound go in several calls."""
+    Batches whose scores would not fit the workspace bound go in several calls.  The scores are a temporary of the call: the
+    workspace kept per stream is for partial sums, a few megabytes, and lives as long as the process."""
     _need_gpu(q, k_packed, k_norms, v_packed, v_norms, mask)
     n_seq, n_q, _ = q.shape
     _check_gqa(n_q, k_norms.shape[-2], n_rep)
@@ -881,7 +882,7 @@ def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_nor
     lib = _lib.load()
     stream = _stream(q)
     per_call = max(1, min(n_seq, _COMPOSED_WORKSPACE // max(1, lib.tq_vonly_sparse_workspace_bytes(1, n_q, seq_len))))
-    ws = _workspace(q.device, stream.value or 0, lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len))
+    ws = torch.empty(lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len), dtype=torch.uint8, device=q.device)
     for first in range(0, n_seq, per_call):
         n = min(per_call, n_seq - first)
         sh = _decode_shape(n_seq=n, n_kv=n_q // n_rep, n_rep=n_rep, dim=dim, bits=bits, block_size=16, seq_len=seq_len,
