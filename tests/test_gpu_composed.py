@@ -103,3 +103,15 @@ def test_composed_scores_are_temporaries(tq, monkeypatch):
     out = tq.turboquant_attention(q, cache, 0.09)
     kept = torch.cuda.memory_allocated() - before - out.numel() * out.element_size()
     assert kept < 1 << 20, kept
+
+
+@pytest.mark.parametrize("T", [5, 700])
+def test_queries_of_the_first_sequences(tq, T):
+    """Fewer queries than the cache holds sequences: those of the first ones, for a decode step and for a chunk."""
+    cache, mk = _cache(tq, 3, 2, T, 3)
+    q, rows = mk(3, 6, 1, D), mk(3, 6, 4, D)
+    whole, chunk = tq.turboquant_attention(q, cache, 0.09), tq.turboquant_prefill_attention(rows, cache, 0.09)
+    for n in (1, 2):
+        assert torch.equal(tq.turboquant_attention(q[:n], cache, 0.09), whole[:n])
+        got = tq.turboquant_prefill_attention(rows[:n], cache, 0.09)
+        assert (got - chunk[:n]).abs().max() <= 4e-3 * chunk.abs().max()        # fp16 results, another split of the positions

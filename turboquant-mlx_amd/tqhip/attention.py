@@ -31,6 +31,12 @@ def _mask_rows(mask, b: int, n_q: int, total: int):
     return m
 
 
+def _stored(cache, B):
+    """Packed keys and values and their norms of the first B sequences of the cache (which may hold more)."""
+    ts = (cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms)
+    return ts if ts[0].shape[0] <= B else tuple(t[:B] for t in ts)
+
+
 def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=None, v_buffer=None,
                          sparse_v_threshold: float | None = None, fused: bool = False) -> torch.Tensor:
     """fused_attention.py:20-125.  queries (B, n_heads, 1, dim) against a TurboQuantKVCache holding
@@ -78,9 +84,8 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
             m = ops.decode_mask_rows(mask, B, n_q, total, queries.device)
             if m is None:
                 m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
-        out = ops.composed_decode(queries[:, :, 0, :], kq.signs, cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms,
-                                  kq.centroids, vq.centroids, vq.signs, dim, bits, attn_scale, n_rep=n_rep, seq_len=total,
-                                  mask=m, threshold=thr)[:, :, None, :]
+        out = ops.composed_decode(queries[:, :, 0, :], kq.signs, *_stored(cache, B), kq.centroids, vq.centroids, vq.signs, dim,
+                                  bits, attn_scale, n_rep=n_rep, seq_len=total, mask=m, threshold=thr)[:, :, None, :]
         return out if out.dtype == queries.dtype else out.to(queries.dtype)
     outputs = []
     for b in range(B):
@@ -165,6 +170,5 @@ def turboquant_prefill_attention(queries: torch.Tensor, cache, attn_scale: float
     n_kv = cache.k_packed.shape[1]
     n_rep = n_q // n_kv
     kq, vq = cache._k_q, cache._v_q
-    return ops.prefill_attention_batch(queries, cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms, kq.centroids,
-                                       vq.centroids, kq.signs, vq.signs, dim, cache.quant_bits, attn_scale, n_rep=n_rep,
-                                       kv_len=total, q_pos0=total - S, causal=causal)
+    return ops.prefill_attention_batch(queries, *_stored(cache, B), kq.centroids, vq.centroids, kq.signs, vq.signs, dim,
+                                       cache.quant_bits, attn_scale, n_rep=n_rep, kv_len=total, q_pos0=total - S, causal=causal)
