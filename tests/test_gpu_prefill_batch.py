@@ -58,3 +58,45 @@ def test_prefill_batch(tq, B, n_kv, n_rep, T, S, bits, dtype, causal):
         one = tq.prefill_attention(q[b].cuda(), *(x[b] for x in dev), c, c, signs[1:129], signs[130:], D, bits, 0.05, n_rep=n_rep,
                                    kv_len=T, q_pos0=T - S, causal=causal)
         assert torch.allclose(one.float(), got[b].float(), rtol=2e-3 if dtype != torch.bfloat16 else 8e-3, atol=2e-3 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("n_kv,n_rep,n_rows,T,causal", [(8, 4, 1, 5262, True), (8, 4, 1, 5262, False), (4, 7, 3, 9001, True), (2, 6, 100, 2500, True),
+                                                        (1, 1, 1, 700, True), (8, 1, 33, 20000, True), (1, 8, 40, 16500, False)])
+def test_the_split_does_not_depend_on_the_bytes_at_hand(tq, n_kv, n_rep, n_rows, T, causal):
+    """Equal calls give equal bits, whatever workspace earlier calls left behind: through the package and through both C entries
+    with the workspace asked for and with a larger one."""
+    from tqhip import _lib
+    lib = _lib.load()
+    D, bits, n_q = 128, 3, n_kv * n_rep
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q = torch.randn(n_q, n_rows, D, generator=g, device="cuda")
+    kp, vp = (tq.pack_indices(torch.randint(0, 8, (n_kv, T, D), generator=g, device="cuda", dtype=torch.uint8), bits) for _ in range(2))
+    kn, vn = (torch.rand(n_kv, T, generator=g, device="cuda") * 8 + 1 for _ in range(2))
+    ks, vs = (torch.from_numpy(o.random_diagonal_sign(D, s)).cuda() for s in (42, 43))
+    c = torch.tensor(np.asarray(o.gaussian_codebook(bits), dtype=np.float32))
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def entry(batch, extra):
+        flags, pos0 = int(causal), T - n_rows
+        need = (lib.tq_prefill_batch_workspace_bytes(1, n_kv, n_rep, n_rows, T, pos0, D, flags) if batch
+                else lib.tq_prefill_workspace_bytes(n_q, n_rows, T, D))
+        ws = torch.empty(need + extra, dtype=torch.uint8, device="cuda")
+        out = torch.empty(n_q, n_rows, D, device="cuda")
+        p = [t.data_ptr() for t in (q, kp, kn, vp, vn, c, c, ks, vs, out, ws)]
+        head = (p[0], 0, *p[1:10], 0, p[10], ws.numel())
+        tail = (T, T, T, T, D, bits, 0.02, flags, stream)
+        rc = (lib.tq_prefill_attn_batch(*head, 1, n_kv, n_rep, n_rows, T, pos0, 0, 0, 0, 0, *tail) if batch
+              else lib.tq_prefill_attn(*head, n_kv, n_rep, n_rows, T, pos0, *tail))
+        assert rc == 0, lib.tq_last_error()
+        torch.cuda.synchronize()
+        return out
+    for batch in (False, True):
+        assert torch.equal(entry(batch, 0), entry(batch, 64 << 20))
+
+    def package():
+        return tq.prefill_attention(q, kp, kn, vp, vn, c, c, ks, vs, D, bits, 0.02, n_rep=n_rep, causal=causal)
+    tq.ops._workspaces.clear()
+    before = package()
+    tq.ops._workspace(q.device, stream, 64 << 20)
+    assert torch.equal(before, package()) and torch.equal(before, entry(True, 0))
+    tq.ops._workspaces.clear()

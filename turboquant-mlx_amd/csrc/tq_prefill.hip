@@ -155,7 +155,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 void prefill_tile_kernel(PrefillArgs a, Codebook kcb, Codebook vcb) {
   using PF = PackedField<BITS>;
   constexpr int kPdim = PF::kPd;                    // words per packed row
-  constexpr int kStageWords = kBlkPos * kPdim;      // packed words per block and tensor (832 at three bits)
   constexpr int kLut = PF::kLut < 64 ? 64 : PF::kLut;
   __shared__ __align__(16) _Float16 Ks2[2][kBlkPos * kKStride];
   __shared__ __align__(16) _Float16 Vt2[2][kD * kVStride];
@@ -672,7 +671,8 @@ int64_t row_workgroups(int n_rep, int64_t n_rows) {
 //  - workgroups of about the same length (a chunk at the end of a long cache): rounds of 256 times the blocks of a split;
 //  - of different lengths (a prompt under the causal rule, longest first): the even share of all blocks, at least the
 //    longest workgroup.
-// At least 8 blocks of positions per split, at most 32 splits, and never more than `fit`.
+// At least 8 blocks of positions per split, at most 32 splits, and never more than `fit`.  A plan is a function of the shape
+// alone, never of the bytes at hand: results of equal calls are equal whatever ran before.
 SplitPlan plan_splits(int n_seq, int n_kv, int n_rep, int64_t n_rows, int64_t kv_len, int64_t q_pos0, bool causal, int64_t fit) {
   const int64_t blocks = (kv_len + kBlkPos - 1) / kBlkPos;
   const int64_t wgs = row_workgroups(n_rep, n_rows), cols = wgs * n_kv * n_seq;
@@ -726,8 +726,8 @@ struct PrefillCall {
   hipStream_t stream;
 };
 
-// `need`: the workspace that the entry point asks its callers for
-int prefill(const char* who, const PrefillCall& c, size_t need) {
+// `need`: the workspace that the entry point asks its callers for; `most`: the splits that it has room for
+int prefill(const char* who, const PrefillCall& c, size_t need, int64_t most) {
   if (c.flags & ~(TQ_PREFILL_CAUSAL | TQ_PREFILL_FP16_QUERY))
     return tq::fail(TQ_ERR_ARG, "%s: unknown flag bits 0x%x", who, c.flags);
   const bool causal = c.flags & TQ_PREFILL_CAUSAL;
@@ -757,8 +757,7 @@ int prefill(const char* who, const PrefillCall& c, size_t need) {
   const int n_q = c.n_kv_heads * c.n_rep;
   const size_t rows = (size_t)c.n_seq * n_q * (size_t)c.n_rows;
   const int64_t kv_eff = visible(c.kv_len, c.q_pos0, c.n_rows, causal);
-  const int64_t fit = c.workspace_bytes < 512 ? 0 : (int64_t)((c.workspace_bytes - 512) / (rows * (kD + 2) * sizeof(float)));
-  const SplitPlan plan = plan_splits(c.n_seq, c.n_kv_heads, c.n_rep, c.n_rows, kv_eff, c.q_pos0, causal, fit);
+  const SplitPlan plan = plan_splits(c.n_seq, c.n_kv_heads, c.n_rep, c.n_rows, kv_eff, c.q_pos0, causal, most);
   const int64_t row_wgs = row_workgroups(c.n_rep, c.n_rows);
   const int64_t grid = row_wgs * plan.n_splits * c.n_seq * c.n_kv_heads;
   if (grid >= (int64_t)1 << 31) return tq::fail(TQ_ERR_ARG, "%s: %lld query rows are too many", who, (long long)c.n_rows);
@@ -808,12 +807,16 @@ int prefill(const char* who, const PrefillCall& c, size_t need) {
 
 }  // namespace
 
-// The size for any position of the chunk: the plan of rows that all see the whole cache, which splits the most.
+// Splits of rows that all see the whole cache, a head of each kind a workgroup: what tq_prefill_attn has room for, which learns
+// of the position of the chunk and of the heads that share keys only at the call (its plan may want more: the batch entry, whose
+// size query knows them, gives it those).
+static SplitPlan plan_any_position(int n_q_heads, int64_t n_rows, int64_t kv_len) {
+  return plan_splits(1, n_q_heads, 1, n_rows, kv_len, 0, false, 32);
+}
+
 extern "C" size_t tq_prefill_workspace_bytes(int n_q_heads, int64_t n_rows, int64_t kv_len, int dim) {
   if (n_q_heads < 1 || n_rows < 1 || kv_len < 1 || dim != kD) return 0;
-  const SplitPlan p = plan_splits(1, n_q_heads, 1, n_rows, kv_len, 0, false, 32);
-  const size_t need = workspace_of(p.n_splits, (size_t)n_q_heads * (size_t)n_rows) + 512;
-  return need;
+  return workspace_of(plan_any_position(n_q_heads, n_rows, kv_len).n_splits, (size_t)n_q_heads * (size_t)n_rows) + 512;
 }
 
 extern "C" size_t tq_prefill_batch_workspace_bytes(int n_seq, int n_kv_heads, int n_rep, int64_t n_rows, int64_t kv_len,
@@ -831,13 +834,15 @@ extern "C" int tq_prefill_attn(const void* q, int q_dtype, const uint32_t* k_pac
                                int64_t n_rows, int64_t kv_len, int64_t q_pos0, int64_t k_head_stride,
                                int64_t kn_head_stride, int64_t v_head_stride, int64_t vn_head_stride, int dim,
                                int bits, float attn_scale, int flags, tq_stream_t stream) {
-  const size_t need = n_kv_heads > 0 && n_rep > 0 ? tq_prefill_workspace_bytes(n_kv_heads * n_rep, n_rows, kv_len, dim) : 0;
+  const bool sizes = n_kv_heads > 0 && n_rep > 0 && n_rows > 0 && kv_len > 0;
+  const size_t need = sizes ? tq_prefill_workspace_bytes(n_kv_heads * n_rep, n_rows, kv_len, dim) : 0;
+  const int64_t most = sizes ? plan_any_position(n_kv_heads * n_rep, n_rows, kv_len).n_splits : 1;
   return prefill("tq_prefill_attn",
                  PrefillCall{q, q_dtype, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, k_signs, v_signs, out,
                              out_dtype, workspace, workspace_bytes, 1, n_kv_heads, n_rep, n_rows, kv_len, q_pos0, 0, 0, 0, 0,
                              k_head_stride, kn_head_stride, v_head_stride, vn_head_stride, dim, bits, attn_scale, flags,
                              (hipStream_t)stream},
-                 need);
+                 need, most);
 }
 
 extern "C" int tq_prefill_attn_batch(const void* q, int q_dtype, const uint32_t* k_packed, const float* k_norms,
@@ -855,5 +860,5 @@ extern "C" int tq_prefill_attn_batch(const void* q, int q_dtype, const uint32_t*
                              out_dtype, workspace, workspace_bytes, n_seq, n_kv_heads, n_rep, n_rows, kv_len, q_pos0,
                              k_seq_stride, kn_seq_stride, v_seq_stride, vn_seq_stride, k_head_stride, kn_head_stride,
                              v_head_stride, vn_head_stride, dim, bits, attn_scale, flags, (hipStream_t)stream},
-                 need);
+                 need, 32);
 }

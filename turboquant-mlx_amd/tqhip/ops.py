@@ -1205,7 +1205,7 @@ def prefill_attention(q: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_c
                       k_signs, v_signs, dim: int, bits: int, attn_scale: float, *, n_rep: int = 1,
                       kv_len: int | None = None, q_pos0: int | None = None, causal: bool = True,
                       out_dtype=None, fp16_query: bool = False) -> torch.Tensor:
-    """Chunked-prefill attention over packed K and V on the matrix cores (tq_prefill_attn).
+    """Chunked-prefill attention over packed K and V on the matrix cores (tq_prefill_attn_batch).
 
     The reference dequantises the whole cache and calls stock SDPA for this step (cache.py:125-129,
     209-210); here the packed rows are decoded tile by tile in LDS and never written back.
@@ -1243,15 +1243,16 @@ def prefill_attention(q: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_c
     k_signs = _as_f32_dev(k_signs, q)
     v_signs = _as_f32_dev(v_signs, q)
     lib = _lib.load()
-    need = lib.tq_prefill_workspace_bytes(n_q, n_rows, T, dim)
+    flags = (1 if causal else 0) | (2 if fp16_query else 0)
+    need = lib.tq_prefill_batch_workspace_bytes(1, n_kv, n_rep, n_rows, T, pos0, dim, flags)
     stream = _stream(q)
     ws = _workspace(q.device, stream.value or 0, max(need, 256))
-    _lib.check(lib.tq_prefill_attn(
+    _lib.check(lib.tq_prefill_attn_batch(
         _ptr(q), _dt(q), _ptr(k_packed), _ptr(k_norms), _ptr(v_packed), _ptr(v_norms),
         _host_table(k_centroids), _host_table(v_centroids), _ptr(k_signs), _ptr(v_signs),
-        _ptr(out), _dt(out), _ptr(ws), ws.numel(), n_kv, n_rep, n_rows, T, pos0,
+        _ptr(out), _dt(out), _ptr(ws), ws.numel(), 1, n_kv, n_rep, n_rows, T, pos0, 0, 0, 0, 0,
         k_packed.stride(0) // pd, k_norms.stride(0), v_packed.stride(0) // pd, v_norms.stride(0),
-        dim, bits, float(attn_scale), (1 if causal else 0) | (2 if fp16_query else 0), stream))
+        dim, bits, float(attn_scale), flags, stream))
     return out
 
 
