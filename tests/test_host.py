@@ -393,3 +393,11 @@ def test_tracing_of_the_integer_plumbing_is_noticed():
     assert torch.equal(make_fx(f)(x)(y), want)
     torch.jit.trace(lambda t: (seen.append(ops._observed()), t + 1)[1], x, check_trace=False)
     assert seen == [False, True, True] and not ops._observed()
+
+
+@pytest.mark.parametrize("dim,n_rep,threshold", [(64, 4, 1e-5), (32, 4, 0.0), (256, 4, 0.0), (128, 17, 0.0), (128, 32, 1e-5)])
+def test_decode_from_the_query_refuses_what_no_entry_serves(dim, n_rep, threshold):
+    """Never the step without its threshold, nor another head dimension: refused before the tensors are looked at."""
+    t = torch.zeros(1)
+    with pytest.raises(ValueError, match="dim 64 without a threshold"):
+        ops.flash_from_query(t, t, t, t, t, t, t, t, t, dim, 3, 0.1, n_rep=n_rep, sparse_v_threshold=threshold)

@@ -804,6 +804,10 @@ def flash_from_query(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_no
                      max_seq_len: int | None = None, mask=None, out_dtype=torch.float32, sparse_v_threshold: float = 0.0,
                      validate_offsets: bool = False) -> torch.Tensor:
     """flash_decode_from_q, and without a threshold also d = 64 (tq_flash_decode_from_q64, any n_rep)."""
+    thresholded = sparse_v_threshold is not None and sparse_v_threshold > 0.0
+    if not (vonly_sparse_supported(dim, bits, n_rep) or (dim == 64 and not thresholded)):
+        raise ValueError("one call from the query needs dim 128 and n_rep <= 16, or dim 64 without a threshold; "
+                         "use prerotate_query + flash_decode")
     _need_gpu(q, k_packed, k_norms, v_packed, v_norms, seq_offsets)
     n_seq, n_q, _ = q.shape
     ragged = seq_offsets is not None
