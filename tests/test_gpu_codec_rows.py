@@ -145,3 +145,21 @@ def test_small_calls_do_not_wait_for_the_level_search(tq, call):
             tq.fused_quantize(x[0, 0], s, b, dim, bits)
         took.append(time.perf_counter() - t0)
     assert sorted(took)[len(took) // 2] < 2e-3, took
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("bounds", [[-30.0], [-60.0, -40.0, 0.5], [0.3]])
+def test_infinities_under_boundaries_that_no_output_reaches(tq, dim, bounds):
+    """A row with an infinity has an infinite norm and outputs that are no numbers: every index 0."""
+    rng = np.random.default_rng(dim)
+    x = _rows(rng, 6151, dim)
+    x[20:40, 3] = np.inf
+    x[40:60, dim - 1] = -np.inf
+    s = o.random_diagonal_sign(dim, 42)
+    b = np.asarray(bounds, dtype=np.float32)
+    bits = {1: 1, 3: 2}[len(bounds)]
+    with np.errstate(invalid="ignore"):
+        wp, wn = o.fused_quantize(x, s, b, dim, bits)
+    assert not wp[20:60].any()
+    gp, gn = tq.fused_quantize(torch.from_numpy(x).cuda(), torch.from_numpy(s).cuda(), b, dim, bits)
+    assert np.array_equal(gp.cpu().numpy(), wp) and np.array_equal(gn.cpu().numpy(), wn)

@@ -298,7 +298,8 @@ bool level_guess_search(const float* t, int nb, EncodeGuess& out);
 // The kernel's cell of w is floor(alpha * w + beta0) or, for w within 1/16 below a cell edge, the next one; with no
 // threshold that close below an edge the count "thresholds below the cell + (w > the threshold inside it)" is the
 // count of thresholds below w either way.  The candidate with the widest margin is taken.
-// clamped (d = 256): thresholds outside the table's cells refuse the line.  Otherwise no w reaches such a threshold.
+// A threshold below the table's first cell refuses the line: no number reaches it, but an output that is no number (a row with
+// an infinity) reads the first cell, whose count must be 0.  clamped (d = 256): one above the last cell does as well.
 bool level_cells_search(const float* t, int nb, bool clamped, EncodeGuess& out) {
   for (int i = 0; i < nb; ++i)
     if (!std::isfinite(t[i]) || (i > 0 && !(t[i] > t[i - 1]))) return false;
@@ -317,7 +318,7 @@ bool level_cells_search(const float* t, int nb, bool clamped, EncodeGuess& out) 
       for (int j = 0; j < nb && ok; ++j) {
         const double u = a * (double)t[j] + b;
         const double c = std::floor(u), f = u - c;
-        if (f < margin || f > 1.0 - margin || c <= prev_cell || (clamped && (c < -half || c > half - 1))) ok = false;
+        if (f < margin || f > 1.0 - margin || c <= prev_cell || c < -half || (clamped && c > half - 1)) ok = false;
         prev_cell = c;
         slack = std::fmin(slack, std::fmin(f - margin, 1.0 - margin - f));
       }
