@@ -194,12 +194,12 @@ class TurboQuantKVCache:
     def _grown_storage(self, B, H, n, device, incoming, fill):
         """The tensors of _reallocate by name, whole once `fill` has run.  The cache keeps what it has until then: an
         allocation that fails on the way leaves it as it was."""
-        prev = self.offset
-        new = {}
-        for side, pdim in ((("v", self._v_pdim),) if self.v_only else (("k", self._k_pdim), ("v", self._v_pdim))):
-            packed, norms = side + "_packed", side + "_norms"
-            new[packed] = self._grow(getattr(self, packed), (B, H, n, pdim), pdim, prev, incoming, torch.uint32, device, fill)
-            new[norms] = self._grow(getattr(self, norms), (B, H, n), 1, prev, incoming, torch.float32, device, fill)
+        prev, new = self.offset, {}
+        if not self.v_only:
+            new["k_packed"] = self._grow(self.k_packed, (B, H, n, self._k_pdim), self._k_pdim, prev, incoming, torch.uint32, device, fill)
+            new["k_norms"] = self._grow(self.k_norms, (B, H, n), 1, prev, incoming, torch.float32, device, fill)
+        new["v_packed"] = self._grow(self.v_packed, (B, H, n, self._v_pdim), self._v_pdim, prev, incoming, torch.uint32, device, fill)
+        new["v_norms"] = self._grow(self.v_norms, (B, H, n), 1, prev, incoming, torch.float32, device, fill)
         return new
 
     # ---------------------------------------------------------------- codec calls

@@ -259,33 +259,35 @@ class StorageFill:
         """dst: contiguous, its rows along `axis` (default: the last but one, or the last with inner 1), `inner` elements each;
         the axes before are the groups: rows `copy` from src (rows src_stride apart per group) first, zeros in rows
         zero_from .. zero_to - 1.  Storage of one word a row has a trailing axis of 1 that only the caller can tell from rows."""
-        if (copy == 0 and zero_to <= zero_from) or dst.numel() == 0:
+        held = dst.numel()
+        if held == 0 or (copy == 0 and zero_to <= zero_from):
             return
         if axis is None:
             axis = dst.dim() - (2 if inner > 1 else 1)
-        rows = dst.shape[axis]
-        if dst.shape[axis + 1:].numel() != inner or max(copy, zero_to) > rows:
+        rows = dst.size(axis)
+        if dst.stride(axis) != inner or copy > rows or zero_to > rows:
             raise ValueError(f"rows of {inner} elements up to {max(copy, zero_to)} along axis {axis} of {tuple(dst.shape)}")
         if not dst.is_cuda:                                  # storage of a cache that has not met the GPU yet
             if copy:
                 dst.narrow(axis, 0, copy).copy_(src.narrow(axis, 0, copy))
             dst.narrow(axis, zero_from, max(0, zero_to - zero_from)).zero_()
             return
-        self._segments.append(self.segment(dst, src, dst.shape[:axis].numel(), rows, inner, zero_from, zero_to, src_stride, copy))
+        self._segments.append(self.segment(dst, src, held // (rows * inner), rows, inner, zero_from, zero_to, src_stride, copy))
         self._keep.append((dst, src))
 
     @staticmethod
     def segment(dst, src, groups: int, rows: int, inner: int, zero_from: int, zero_to: int, src_stride: int, copy: int) -> tuple:
-        """The fields of struct tq_fill_segment, checked against the bytes that the tensors hold."""
+        """The fields of struct tq_fill_segment, the source checked against the bytes that it holds."""
         row = inner * dst.element_size()
-        if src is not None and copy > 0:
-            if src.dtype != dst.dtype:
-                raise ValueError(f"rows of {src.dtype} cannot be copied into {dst.dtype} as they are")
-            held = src.untyped_storage().nbytes() - src.storage_offset() * src.element_size()
-            if ((groups - 1) * src_stride + copy) * row > held:
-                raise ValueError(f"{groups} groups of {copy} rows, {src_stride} apart, exceed the {held} bytes of the source")
-        return (dst.data_ptr(), 0 if src is None else src.data_ptr(), rows * row, 0 if src is None else src_stride * row, copy * row,
-                zero_from * row, max(zero_from, zero_to) * row, groups)
+        if copy == 0:
+            return dst.data_ptr(), 0, rows * row, 0, 0, zero_from * row, zero_to * row, groups
+        if src.dtype != dst.dtype:
+            raise ValueError(f"rows of {src.dtype} cannot be copied into {dst.dtype} as they are")
+        held = src.untyped_storage().nbytes() - src.storage_offset() * src.element_size()
+        if ((groups - 1) * src_stride + copy) * row > held:
+            raise ValueError(f"{groups} groups of {copy} rows, {src_stride} apart, exceed the {held} bytes of the source")
+        return (dst.data_ptr(), src.data_ptr(), rows * row, src_stride * row, copy * row, zero_from * row, max(zero_from, zero_to) * row,
+                groups)
 
     def run(self) -> None:
         segs, self._segments = self._segments, []
