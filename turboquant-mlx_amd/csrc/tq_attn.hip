@@ -735,18 +735,17 @@ int launch_decode(const void* q, int q_dtype, const uint32_t* k_packed, const fl
       } else {
         TQ_DISPATCH_BITS(sh.bits, (split_decode_kernel<256, B_, true><<<sgrid, kThreads, 0, stream>>>(a, q_dtype, kcb, vcb)));
       }
-      TQ_CHECK_LAUNCH(who);
     } else {
-    dim3 grid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
+      dim3 grid(n_tiles, sh.n_kv_heads * a.n_rgroups, sh.n_seq);
 #define LAUNCH_TILE(QT)                                                                              \
-  TQ_DISPATCH_DIM(sh.dim, TQ_DISPATCH_BITS(sh.bits, (decode_tile_kernel<D_, B_, KMODE, QT>            \
-                                                        <<<grid, kThreads, 0, stream>>>(a, kcb, vcb))))
-    if (KMODE == kDenseK && q_dtype == TQ_F16) { LAUNCH_TILE(__half); }
-    else if (KMODE == kDenseK && q_dtype == TQ_BF16) { LAUNCH_TILE(__hip_bfloat16); }
-    else { LAUNCH_TILE(float); }
+      TQ_DISPATCH_DIM(sh.dim, TQ_DISPATCH_BITS(sh.bits, (decode_tile_kernel<D_, B_, KMODE, QT>        \
+                                                            <<<grid, kThreads, 0, stream>>>(a, kcb, vcb))))
+      if (KMODE == kDenseK && q_dtype == TQ_F16) { LAUNCH_TILE(__half); }
+      else if (KMODE == kDenseK && q_dtype == TQ_BF16) { LAUNCH_TILE(__hip_bfloat16); }
+      else { LAUNCH_TILE(float); }
 #undef LAUNCH_TILE
-    TQ_CHECK_LAUNCH(who);
     }
+    TQ_CHECK_LAUNCH(who);
   }
   if (!(phases & 2)) return TQ_OK;
   dim3 mgrid(n_q, sh.n_seq);
