@@ -3,7 +3,7 @@
 // positions and merge pass it shares with the vector kernel that it stands in for.
 //
 // The vector kernel decodes every element for eight heads with multiply-adds: its time is vector arithmetic (2 sequences x
-// 32 / 8 heads x 8 190 positions of d = 64 at four bits: 20.4 us for 9 MB; this kernel, query rotation included, 10.6).  Here a wave's 64 positions and 16 heads are
+// 32 / 8 heads x 8 190 positions of d = 64 at four bits: 20.4 us for 9 MB; this kernel, query rotation included, 10.2).  Here a wave's 64 positions and 16 heads are
 // products of 16x16x32 matrix instructions.  Operands keep 22 bits: queries, weights and centroids enter as an fp16 value and
 // the fp16 remainder of its rounding, keys in fp16 are exact; queries and, in each wave, weights times value norms are scaled per
 // head by powers of two, so that magnitudes outside the range of fp16 change nothing, nor does a head whose value norms lie many

@@ -348,8 +348,8 @@ def bench_packed_widths(iters, dev):
 
 
 def bench_codec_widths(iters, dev):
-    """Encode / dequantise 1 048 576 vectors at every width: the streaming kernels (row count a multiple of 16)
-    against the generic one-wavefront-per-vector kernels (one row fewer)."""
+    """Encode / dequantise 1 048 576 vectors at every width: the streaming kernels with whole passes in a group
+    against their form for any row count (one row fewer)."""
     signs = tqhip.random_diagonal_sign(128, 43, device=dev)
     n = 131072 * 8
     xs = [torch.randn((n, 128), device=dev, dtype=torch.float16) for _ in range(2)]
@@ -357,7 +357,7 @@ def bench_codec_widths(iters, dev):
         cb = gaussian_codebook(bits)
         bd = gaussian_boundaries(cb)
         pd = tqhip.packed_dim(128, bits)
-        for rows, kind in ((n, "streaming kernel"), (n - 1, "generic kernel")):
+        for rows, kind in ((n, "whole passes"), (n - 1, "any row count")):
             fns = [(lambda x=x: tqhip.fused_quantize(x[:rows], signs, bd, 128, bits)) for x in xs]
             report(f"encode d=128 {bits}-bit, {rows} vectors, {kind}", timeit(fns, max(10, iters // 4)), rows * (256 + 4 * pd + 4))
             p, nr = tqhip.fused_quantize(xs[0][:rows], signs, bd, 128, bits)
