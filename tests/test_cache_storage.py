@@ -150,3 +150,16 @@ def test_a_failed_allocation_leaves_the_cache_as_it_was(monkeypatch, mode, at):
     assert cache.offset == 260
     for got, w in zip(_words(cache, 250), want):
         assert torch.equal(got, w)
+
+
+def test_rows_that_one_side_never_held_are_zero(monkeypatch):
+    """A cache restored from the state of a v_only one has values and no keys: its first insert makes key storage whose rows
+    before the insert are zeros, not what memory held."""
+    cache = _grown(tqhip.TurboQuantKVCache(bits=3, v_only=True), 128, 250)
+    cache.v_only = False
+    cache._ensure_quantizer(128, 128, torch.device("cpu"))
+    real = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: real(*a, **kw).view(torch.uint8).fill_(7).view(kw["dtype"]))
+    cache._ensure_storage(B, H, 10, torch.device("cpu"), incoming=10)
+    for t in (cache.k_packed.view(torch.int32), cache.k_norms):
+        assert t.shape[2] == 512 and not t[:, :, :250].any() and not t[:, :, 260:].any()

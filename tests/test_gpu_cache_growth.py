@@ -98,3 +98,16 @@ def test_vonly_insert_of_no_rows(tq):
     k, v = _rows(128, 5)
     cache.update_and_fetch(k, v)
     assert cache.update_and_fetch(x, x)[1].shape == (2, 4, 5, 128)
+
+
+def test_insert_into_a_restored_v_only_cache(tq):
+    """Restored without its mode, it keeps keys from then on; the rows before are zeros."""
+    k, v = _rows(128, 5)
+    junk = torch.full((1 << 22,), 3, dtype=torch.int32, device="cuda")       # what the allocator hands out next
+    del junk
+    cache = tq.TurboQuantKVCache(bits=3, v_only=True)
+    cache.update_and_fetch(k[:, :, :3], v[:, :, :3])
+    back = tq.TurboQuantKVCache.from_state(cache.state, cache.meta_state)
+    back.update_and_fetch(k[:, :, 3:], v[:, :, 3:])
+    kp, kn, _, _ = back.state
+    assert not kp.view(torch.int32)[:, :, :3].any() and not kn[:, :, :3].any() and bool(kn[:, :, 3:].all())

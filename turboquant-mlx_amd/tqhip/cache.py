@@ -166,8 +166,10 @@ class TurboQuantKVCache:
         rows between are about to be written.  The copy and the zeros join `fill`."""
         new = torch.empty(shape, dtype=dtype, device=device)
         n = shape[2]
-        if old is None or prev == 0:
+        if prev == 0:
             fill.add(new, inner, incoming, n, axis=2)
+        elif old is None:                                    # rows that this side never held, as of a restored v_only cache: zeros
+            fill.add(new, inner, 0, n, axis=2)
         elif old.dtype == dtype and old.device == new.device and old.shape[:2] == new.shape[:2] and _is_grouped(old, inner):
             fill.add(new, inner, prev + incoming, n, src=old, src_stride=_group_stride(old, inner), copy=prev,
                      axis=2)
