@@ -111,3 +111,10 @@ def test_insert_into_a_restored_v_only_cache(tq):
     back.update_and_fetch(k[:, :, 3:], v[:, :, 3:])
     kp, kn, _, _ = back.state
     assert not kp.view(torch.int32)[:, :, :3].any() and not kn[:, :, :3].any() and bool(kn[:, :, 3:].all())
+
+
+def test_fused_vonly_insert_refuses_other_key_dtypes(tq):
+    """As ever: a fused cache's small inserts go through the one-launch append, which takes kernel dtypes."""
+    k, v = _rows(128, 4)
+    with pytest.raises(ValueError, match="unsupported dtype"):
+        tq.VOnlyTurboQuantCache(bits=3, fused=True).update_and_fetch(k.double(), v)

@@ -69,8 +69,8 @@ class VOnlyTurboQuantCache:
         from . import ops
         kc, tq = self._k_cache, self._v_tq
         B, H, S, v_dim = values.shape
-        if (not 0 < S <= self._FUSED_APPEND_MAX_TOKENS or keys.shape != values.shape or not (keys.is_cuda and values.is_cuda)
-                or keys.dtype not in ops._DTYPES or values.dtype not in ops._DTYPES
+        if (not 0 < S <= self._FUSED_APPEND_MAX_TOKENS or keys.shape != values.shape or not values.is_cuda
+                or not (self.fused or (keys.is_cuda and keys.dtype in ops._DTYPES and values.dtype in ops._DTYPES))
                 or (kc.values is not None and kc.values.dtype != values.dtype)
                 or (kc.keys is not None and kc.keys.dtype != torch.float16)
                 or kc.offset != tq.offset):
