@@ -100,3 +100,25 @@ def test_the_split_does_not_depend_on_the_bytes_at_hand(tq, n_kv, n_rep, n_rows,
     tq.ops._workspace(q.device, stream, 64 << 20)
     assert torch.equal(before, package()) and torch.equal(before, entry(True, 0))
     tq.ops._workspaces.clear()
+
+
+@pytest.mark.parametrize("T", [70, 6000])                                 # one split, several
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_rows_whose_query_is_no_number(tq, T, bad):
+    """A row none of whose scores is a number comes out as zeros, whatever the number of splits; other rows do not notice."""
+    kp, kn, vp, vn, q = _case(1, 2, 3, T, 40, 3, torch.float32)
+    c = o.gaussian_codebook(3)
+    ks, vs = (torch.from_numpy(o.random_diagonal_sign(D, s)).cuda() for s in (42, 43))
+    dev = [torch.from_numpy(x).cuda() for x in (kp.view(np.int32), kn, vp.view(np.int32), vn)]
+
+    def run(x):
+        return tq.ops.prefill_attention_batch(x.cuda(), *dev, c, c, ks, vs, D, 3, 0.05, n_rep=3, kv_len=T, q_pos0=T - 40)
+    want = run(q)
+    hurt = q.clone()
+    hurt[0, 1, 7, 5] = bad
+    hurt[0, 4, 39, 127] = bad
+    got = run(hurt)
+    for h, r in ((1, 7), (4, 39)):
+        assert not got[0, h, r].any()
+        got[0, h, r] = want[0, h, r]
+    assert torch.equal(got, want)

@@ -563,6 +563,12 @@ void prefill_tile_kernel(PrefillArgs a, Codebook kcb, Codebook vcb) {
             f4{oacc[et][4 * qd], oacc[et][4 * qd + 1], oacc[et][4 * qd + 2], oacc[et][4 * qd + 3]};
     return;
   }
+  if (m_run == -INFINITY) {                                              // none of the row's scores was a number: zeros, as in the
+#pragma unroll                                                           // merge of several splits
+    for (int et = 0; et < 4; ++et)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[et][i] = 0.0f;
+  }
   // ---- out[r] = B(O[r]) * signs_V * unscale / l : strides 1, 2 (registers), 4 (halves), 8, 16 and 32, 64 (registers)
   const uint32_t flip = hl ? 0x80000000u : 0u;
 #pragma unroll
