@@ -85,7 +85,7 @@ def test_buffer_growth_casts_rows_of_another_dtype(monkeypatch, was, now, v_only
         return add(self, dst, inner, zero_from, zero_to, src=src, src_stride=src_stride, copy=copy, axis=axis)
 
     monkeypatch.setattr(ops.StorageFill, "add", checked)
-    monkeypatch.setattr(tqhip.TurboQuantKVCache, "_dequant_rows", lambda self, outs, *a: [o.zero_() for o in outs if o.shape[2] == 1])
+    monkeypatch.setattr(tqhip.TurboQuantKVCache, "_dequant_rows", lambda self, outs, *a: [o.zero_() for o in outs if o is not None and o.shape[2] == 1])
     grown = cache._incremental(list(old), B, H, 256, 257, [now] * sides)
     assert len(raw) == (sides if was == now else 0)
     for new, o in zip(grown, old):

@@ -118,3 +118,23 @@ def test_fused_vonly_insert_refuses_other_key_dtypes(tq):
     k, v = _rows(128, 4)
     with pytest.raises(ValueError, match="unsupported dtype"):
         tq.VOnlyTurboQuantCache(bits=3, fused=True).update_and_fetch(k.double(), v)
+
+
+_CASTS = [(a, b, c) for a in (torch.float16, torch.float32) for b in (torch.float16, torch.bfloat16, torch.float32)
+          for c in (torch.float16, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("was,now_k,now_v", _CASTS)
+def test_tokens_of_another_dtype_than_the_buffer(tq, was, now_k, now_v):
+    """A token's dequantised rows: in half precision, cast to the token's dtype, then to the buffer's; float16 tokens go into the
+    buffer as its dtype takes them."""
+    B, H, n, dim = 2, 4, 40, 128
+    k, v = _rows(dim, n + 1)
+    cache = tq.TurboQuantKVCache(bits=3)
+    cache.update_and_fetch(k[:, :, :n].to(was), v[:, :, :n].to(was))
+    got = cache.update_and_fetch(k[:, :, n:].to(now_k), v[:, :, n:].to(now_v))
+    sides = ((cache.k_packed, cache.k_norms, cache._k_q, now_k), (cache.v_packed, cache.v_norms, cache._v_q, now_v))
+    for out, (p, nr, q, now) in zip(got, sides):
+        half = now == torch.float16
+        full = cache._full_dequant(p, nr, q, dim, B, H, n + 1, was if half else torch.float16)[:, :, n:]
+        assert out.dtype == was and torch.equal(out[:, :, n:], full if half else full.to(now).to(was))

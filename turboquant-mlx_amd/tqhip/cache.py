@@ -232,9 +232,9 @@ class TurboQuantKVCache:
 
     def _dequant_rows(self, outs, B, H, start, count, out_start):
         """Positions start .. start + count - 1 of every (b, h) of each stored tensor into rows out_start .. of its
-        contiguous [B, H, T, dim] tensor in `outs`: one launch where one describes both."""
+        contiguous [B, H, T, dim] tensor in `outs` (None: not wanted): one launch where one describes both."""
         sides = self._sides()
-        if len(sides) == 2:
+        if len(sides) == 2 and outs[0] is not None and outs[1] is not None:
             (kp, kn, kq, kd), (vp, vn, vq, vd) = sides
             ko, vo = outs
             gs = _group_stride(vp, vp.shape[3])
@@ -245,6 +245,8 @@ class TurboQuantKVCache:
                                     bits=self.quant_bits, row_offset=start, out_row_offset=out_start)
                 return
         for (packed, norms, q, dim), out in zip(sides, outs):
+            if out is None:
+                continue
             ops.dequant_into(packed, norms, q.centroids, q.signs, out, n_groups=B * H, rows_per_group=count,
                              packed_group_stride=_group_stride(packed, packed.shape[3]),
                              norms_group_stride=_group_stride(norms, 1), out_group_stride=out.shape[2], dim=dim,
@@ -276,13 +278,15 @@ class TurboQuantKVCache:
                     fill.add(new, new.shape[3], total, new.shape[2], axis=2)
             fill.run()
             bufs = grown
-        if all(dt == torch.float16 for dt in dtypes):
-            self._dequant_rows(bufs, B, H, prev, total - prev, prev)
-        else:
+        half = [dt == torch.float16 for dt in dtypes]
+        if any(half):
+            self._dequant_rows([buf if h else None for buf, h in zip(bufs, half)], B, H, prev, total - prev, prev)
+        if not all(half):                                    # rows of another dtype: cast to theirs, then to the buffer's
             tmp = self._buffers(B, H, total - prev, [torch.float16] * len(bufs), bufs[0].device)
-            self._dequant_rows(tmp, B, H, prev, total - prev, 0)
-            for buf, rows in zip(bufs, tmp):
-                buf[:, :, prev:total].copy_(rows)
+            self._dequant_rows([None if h else rows for rows, h in zip(tmp, half)], B, H, prev, total - prev, 0)
+            for buf, rows, dt in zip(bufs, tmp, dtypes):
+                if dt != torch.float16:
+                    buf[:, :, prev:total].copy_(rows if buf.dtype == dt else rows.to(dt))
         return bufs
 
     # ---------------------------------------------------------------- cache.py:131-218
