@@ -185,3 +185,23 @@ def test_split_dims_codebooks_of_another_scale(tq, D, packed, scale):
         return tq.vonly_decode(q, kd, vp, vn, c, signs, D, bits, D ** -0.5, n_rep=n_rep, **kw)
     got, want = run(), run(precision="fp32")
     assert (got - want).abs().max() <= _REL * want.abs().max()
+
+
+@pytest.mark.parametrize("D,packed", [(64, True), (64, False), (256, False)])
+def test_split_dims_infinite_value_norms(tq, D, packed):
+    """One position, whose value norm is infinite: the infinities and the no-numbers of the float32 kernel."""
+    bits, n_rep = 3, 4
+    c = o.gaussian_codebook(bits)
+    q, kp, kn, vp, vn, kd = _case(tq, 2, 2, n_rep, 1, D, bits)
+    vn[1] = float("inf")
+    signs = torch.from_numpy(o.random_diagonal_sign(D, 43)).cuda()
+    vp[1, 0] = tq.pack_indices(torch.full((1, D), 6, device="cuda", dtype=torch.uint8), bits)     # one sign: one output is infinite
+
+    def run(**kw):
+        if packed:
+            return tq.flash_decode(q, kp, kn, vp, vn, c, c, signs, D, bits, 0.02, n_rep=n_rep, **kw)
+        return tq.vonly_decode(q, kd, vp, vn, c, signs, D, bits, D ** -0.5, n_rep=n_rep, **kw)
+    got, want = run(), run(precision="fp32")
+    assert int(torch.isinf(want).sum()) == n_rep and bool(torch.isfinite(want[0]).all())
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])

@@ -7,8 +7,8 @@
 // products of 16x16x32 matrix instructions.  Operands keep 22 bits: queries, weights and centroids enter as an fp16 value and
 // the fp16 remainder of its rounding, keys in fp16 are exact; queries and, in each wave, weights times value norms are scaled per
 // head by powers of two, so that magnitudes outside the range of fp16 change nothing, nor does a head whose value norms lie many
-// octaves below another's (see tq_split_mfma.h).  Infinite keys and queries give the infinite scores of the vector kernel: a
-// remainder never meets them.
+// octaves below another's (see tq_split_mfma.h).  Infinite keys and queries give the infinite scores of the vector kernel, infinite
+// value norms its infinite sums: a remainder never meets them.
 #pragma once
 
 // query heads of a kv head that one workgroup serves: at d = 256 eight, whose sums leave room for three workgroups in a CU's LDS
@@ -217,7 +217,18 @@ __global__ __launch_bounds__(kThreads) void split_decode_kernel(DecodeArgs a, in
     }
   l = sum_over_rows(l);
   float up, down;
-  split_scale(max_over_rows(largest), up, down);                // of head n16
+  largest = max_over_rows(largest);                             // of head n16
+  split_scale(largest, up, down);
+  if (__any(largest == INFINITY)) {                             // infinite value norms: the sign of the sum, times infinity
+    if (largest == INFINITY) {
+      up = 1.0f;
+      down = INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[t][j] = fabsf(s[t][j]) == INFINITY ? copysignf(16384.0f, s[t][j]) : s[t][j] * 0.0f;
+    }
+  }
   u4 ph[2], pl[2];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
