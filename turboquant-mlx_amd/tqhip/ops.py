@@ -147,7 +147,7 @@ def _head_layout_2d(t: torch.Tensor) -> tuple[torch.Tensor, int]:
 def _observed() -> bool:
     """Whether something records or rewrites the tensor operations of the caller: a dispatch mode (make_fx, flop counters), the
     JIT's tracer, a compiler.  A library call would be missing from what they see."""
-    return torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+    return torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None
 
 
 def _native_pack(t: torch.Tensor) -> bool:
@@ -861,6 +861,7 @@ def flash_from_query(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_no
 
 
 _COMPOSED_WORKSPACE = 256 << 20    # bytes of scores that one launch of composed_decode may take
+_COMPOSED_KEPT = 16 << 20          # and those that it may leave in the workspace of its stream
 
 
 def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids, v_signs, dim: int,
@@ -868,8 +869,9 @@ def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_nor
     """prerotate_query, prerot_fused_qk_scores, softmax_rows and sparse_v_matvec for every sequence of a cache in three
     launches (tq_composed_decode), float32 fidelity.  q (n_seq, n_q, dim); K / V in cache layout (n_seq, n_kv, T_alloc, *);
     returns (n_seq, n_q, dim) in q's dtype (float32 for one that is no kernel dtype).  Shapes of vonly_sparse_supported.
-    Batches whose scores would not fit the workspace bound go in several calls.  The scores are a temporary of the call: the
-    workspace kept per stream is for partial sums, a few megabytes, and lives as long as the process."""
+    Batches whose scores would not fit the workspace bound go in several calls.  Scores of more than a few megabytes are a temporary of
+    the call: the workspace kept per stream lives as long as the process (a smaller call goes through it, 1 - 2 us of 33 sooner:
+    28 / 4 heads over 65 536 positions take 9.3 MB)."""
     _need_gpu(q, k_packed, k_norms, v_packed, v_norms, mask)
     n_seq, n_q, _ = q.shape
     _check_gqa(n_q, k_norms.shape[-2], n_rep)
@@ -888,7 +890,8 @@ def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_nor
     lib = _lib.load()
     stream = _stream(q)
     per_call = max(1, min(n_seq, _COMPOSED_WORKSPACE // max(1, lib.tq_vonly_sparse_workspace_bytes(1, n_q, seq_len))))
-    ws = torch.empty(lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len), dtype=torch.uint8, device=q.device)
+    need = lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len)
+    ws = _workspace(q.device, stream.value or 0, need) if need <= _COMPOSED_KEPT else torch.empty(need, dtype=torch.uint8, device=q.device)
     for first in range(0, n_seq, per_call):
         n = min(per_call, n_seq - first)
         sh = _decode_shape(n_seq=n, n_kv=n_q // n_rep, n_rep=n_rep, dim=dim, bits=bits, block_size=16, seq_len=seq_len,
