@@ -192,6 +192,19 @@ int tq_unpack_indices(const uint32_t* packed, uint8_t* indices, int64_t n_rows, 
                       tq_stream_t stream);
 
 /*
+ * tq_encode and tq_dequant with the levels as one byte each, rows of dim bytes without gaps, in one launch: the bytes that
+ * tq_unpack_indices gives for the words of tq_encode, and the float32 rows that tq_dequant gives for the words of tq_pack_indices
+ * (bytes past the width included).  dim 64, 128 or 256, x and out 16-byte aligned, indices 16-byte (quantize) or 8-byte
+ * aligned; TQ_ERR_UNSUPPORTED for other calls and for boundaries that the streaming encoder has no level line for: nothing is
+ * launched then, and the two-step way serves.  Stands for PolarQuantizer.quantize / dequantize (reference
+ * turboquant_mlx/quantizer.py:85-132).
+ */
+int tq_quantize(const void* x, int x_dtype, const float* signs, const float* boundaries /* HOST */, uint8_t* indices, float* norms,
+                int64_t n_rows, int dim, int bits, int variant, tq_stream_t stream);
+int tq_dequantize(const uint8_t* indices, const float* norms, const float* centroids /* HOST */, const float* signs, float* out,
+                  int64_t n_rows, int dim, int bits, tq_stream_t stream);
+
+/*
  * q_rot[h] = butterfly(q[h] * signs), no 1/sqrt(dim).
  * Replaces prerotate_query (metal_kernels_v4.py:119-150, kernel 37-62).
  *   q [n_heads, dim] dtype q_dtype -> q_rot [n_heads, dim] float32

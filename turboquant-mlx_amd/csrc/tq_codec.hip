@@ -691,6 +691,57 @@ extern "C" int tq_encode_kv(const void* k, const float* k_signs, uint32_t* k_pac
                       variant, (hipStream_t)stream_);
 }
 
+// Any number of rows: the launch of its own that the bytes would need costs more than one wavefront per vector saves on few rows
+// (see stream_min_rows).
+extern "C" int tq_quantize(const void* x, int x_dtype, const float* signs, const float* boundaries, uint8_t* indices, float* norms,
+                           int64_t n_rows, int dim, int bits, int variant, tq_stream_t stream_) {
+  const char* who = "tq_quantize";
+  if (int rc = tq::check_dim_bits(dim, bits)) return rc;
+  if (tq::check_dtype(x_dtype)) return tq::fail(TQ_ERR_DTYPE, "%s: unknown x_dtype %d", who, x_dtype);
+  if (variant != TQ_ENCODE_MLX && variant != TQ_ENCODE_METAL) return tq::fail(TQ_ERR_ARG, "%s: unknown variant %d", who, variant);
+  if (n_rows < 0) return tq::fail(TQ_ERR_ARG, "%s: negative row count", who);
+  if (n_rows == 0) return TQ_OK;
+  if (!x || !signs || !boundaries || !indices || !norms) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (!tq::aligned(x, tq::dtype_size(x_dtype)) || !tq::aligned(signs, 4) || !tq::aligned(norms, 4))
+    return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+  if (dim < 64 || n_rows >= (int64_t)1 << 31 || !tq::aligned(x, 16) || !tq::aligned(indices, 16))
+    return tq::fail(TQ_ERR_UNSUPPORTED, "%s: rows of %d, %lld of them, or a pointer off 16 bytes", who, dim, (long long)n_rows);
+  const EncodePlan plan = encode_plan(boundaries, dim, bits, variant, true);
+  if (!plan.has_guess) return tq::fail(TQ_ERR_UNSUPPORTED, "%s: no level line for these boundaries", who);
+  const EncodeCall c{EncodeSides{{{x, signs, (uint32_t*)indices, norms}, {}}}, 1, x_dtype, plan.thr, plan.gs,
+                     row_map(n_rows, n_rows, 0, 0, 0), bits, (hipStream_t)stream_};
+  if (dim == 64) launch_encode_indices<64>(c);
+  else if (dim == 128) launch_encode_indices<128>(c);
+  else launch_encode_indices<256>(c);
+  TQ_CHECK_LAUNCH(who);
+  return TQ_OK;
+}
+
+extern "C" int tq_dequantize(const uint8_t* indices, const float* norms, const float* centroids, const float* signs, float* out,
+                             int64_t n_rows, int dim, int bits, tq_stream_t stream_) {
+  const char* who = "tq_dequantize";
+  if (int rc = tq::check_dim_bits(dim, bits)) return rc;
+  if (n_rows < 0) return tq::fail(TQ_ERR_ARG, "%s: negative row count", who);
+  if (n_rows == 0) return TQ_OK;
+  if (!indices || !norms || !centroids || !signs || !out) return tq::fail(TQ_ERR_NULL, "%s: null pointer", who);
+  if (!tq::aligned(norms, 4) || !tq::aligned(signs, 4) || !tq::aligned(out, 4)) return tq::fail(TQ_ERR_ALIGN, "%s: misaligned pointer", who);
+  if (dim < 64 || n_rows >= (int64_t)1 << 31 || !tq::aligned(indices, 8) || !tq::aligned(out, 16))
+    return tq::fail(TQ_ERR_UNSUPPORTED, "%s: rows of %d, %lld of them, or a misaligned pointer", who, dim, (long long)n_rows);
+  Codebook cb;
+  for (int i = 0; i < 16; ++i) cb.c[i] = i < (1 << bits) ? centroids[i] : 0.0f;
+  const RowMap rm = row_map(n_rows, n_rows, 0, 0, 0);
+  const DequantCall c{DequantSides{{{(const uint32_t*)indices, norms, signs, out}, {}}}, 1, cb, (float)(1.0 / sqrt((double)dim)), TQ_F32,
+                      rm, bits, (hipStream_t)stream_};
+  // bytes past the width: the two upper bits of a word reach the next chunk where dequant_sides streams its words, else they do not
+  const bool streams = whole_batches(dim, rm) || n_rows >= stream_min_rows(dim, false);
+  const uint32_t word_bits = bits == 3 && !streams ? 0x3FFFFFFFu : ~0u;
+  if (dim == 64) launch_dequant_indices<64>(c, word_bits);
+  else if (dim == 128) launch_dequant_indices<128>(c, word_bits);
+  else launch_dequant_indices<256>(c, word_bits);
+  TQ_CHECK_LAUNCH(who);
+  return TQ_OK;
+}
+
 namespace {
 int vonly_append(const void* k_new, int k_dtype, const void* v_new, int v_dtype,
                                const float* v_signs, const float* boundaries, void* k_f16, void* v_raw,

@@ -129,8 +129,12 @@ constexpr int kEncPasses = 4;     // passes per wavefront once there are rows en
 // destination rows are consecutive.  RAGGED = true takes any row count (a prompt's length is no multiple of
 // anything): a pass takes the next kVecs rows whatever their groups, every lane derives its own vector's group once
 // per pass and the destination rows of the pass are shared through LDS; rows past the end repeat the last one and
-// are not stored.  What it costs over the other form is a dozen instructions per 2048 elements.
-template <int D, typename T, int BITS, bool RAGGED>
+// and are not stored.  What it costs over the other form is a dozen instructions per 2048 elements.
+//
+// INDICES: the levels leave as one byte each instead of packed words, `packed` standing for n_rows x D bytes without groups
+// (RAGGED).  Bound by memory like the packing form (256 bytes in, 132 out per fp16 row of 128): 100 003 rows in one launch 13.4 us
+// against 12.7 us of encoding and 5.4 us of unpacking the words again.
+template <int D, typename T, int BITS, bool RAGGED, bool INDICES = false>
 __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, Thresholds thr, EncodeGuess gs, RowMap rm,
                                                              int passes) {
   const T* __restrict__ x = (const T*)sides.s[blockIdx.y].x;
@@ -146,8 +150,9 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
   constexpr int kCells = BITS == 4 ? 128 : 64;                 // cells of the level guess (fifteen thresholds need finer ones)
   __shared__ __align__(8) uint2 lvl_s[kCells];                 // (threshold bits, guess) by kCells / 2 + floor(alpha*w + beta0)
   __shared__ __align__(16) float sg_s[D];
-  __shared__ uint32_t chunk_s[kWavesPerBlock][kVecs * kChunks + 4];
-  __shared__ uint32_t dst_s[kWavesPerBlock][RAGGED ? kVecs : 1];   // destination row of each vector of the pass
+  constexpr int kIdxPitch = D + 16;                            // bytes per row of indices in LDS: conflict-free 8-byte writes
+  __shared__ __align__(16) uint32_t chunk_s[kWavesPerBlock][INDICES ? kVecs * kIdxPitch / 4 : kVecs * kChunks + 4];
+  __shared__ uint32_t dst_s[kWavesPerBlock][RAGGED && !INDICES ? kVecs : 1];   // destination row of each vector of the pass
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -264,7 +269,10 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
     // ---- where this lane's vector goes
     uint32_t my_g = grp, my_r = rin + v;
     const bool mine = !RAGGED || row0 + v < n_rows;
-    if (RAGGED) {
+    if (INDICES) {
+      my_g = 0;
+      my_r = row0 + v;
+    } else if (RAGGED) {
       group_of(rm, min(row0 + v, n_rows - 1), my_g, my_r);
       dst_s[wave][v] = my_g * (uint32_t)rm.packed_group_stride + my_r;
     }
@@ -318,7 +326,7 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
     // ---- levels, 8 * BITS bits per chunk
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      uint32_t bits24 = 0;
+      uint32_t bits24 = 0, top4 = 0;                           // INDICES: bytes of elements 0 .. 3 and 4 .. 7
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float w = xs[k][j];
@@ -328,11 +336,29 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
         const uint32_t off = __float_as_uint(cell) & (uint32_t)((kCells - 1) << 3);
         const uint2 lv = *reinterpret_cast<const uint2*>(reinterpret_cast<const unsigned char*>(lvl_s) + off);
         const uint32_t idx = lv.y + ((w > __uint_as_float(lv.x)) ? 1u : 0u);
-        bits24 |= idx << (BITS * j);
+        if constexpr (INDICES) (j < 4 ? bits24 : top4) |= idx << (8 * (j & 3));
+        else bits24 |= idx << (BITS * j);
       }
-      chunks[v * kChunks + ls + kLanes * k] = (nrm != nrm) ? 0u : bits24;
+      if constexpr (INDICES)
+        *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(chunks) + v * kIdxPitch + 8 * (ls + kLanes * k)) =
+            (nrm != nrm) ? make_uint2(0u, 0u) : make_uint2(bits24, top4);
+      else
+        chunks[v * kChunks + ls + kLanes * k] = (nrm != nrm) ? 0u : bits24;
     }
     wave_lds_fence();
+    if constexpr (INDICES) {                                   // 1 KB of consecutive bytes per store instruction
+      unsigned char* rows = reinterpret_cast<unsigned char*>(packed) + (int64_t)row0 * D;
+#pragma unroll
+      for (int it = 0; it < 2; ++it) {
+        const int piece = it * 64 + lane, vv = piece / (D / 16);
+        const uint4 val = *reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(chunks) + vv * kIdxPitch + 16 * (piece % (D / 16)));
+        if (row0 + vv < n_rows) *reinterpret_cast<uint4*>(rows + 16 * piece) = val;
+      }
+      wave_lds_fence();
+      if (ls == 0 && mine) norms[my_r] = nrm;
+      row0 += kVecs;
+      continue;
+    }
     // ---- words.  Three bits: word wd of a row holds elements 10wd .. 10wd+9 = chunks (5wd)/4 and the next;
     // four bits: a chunk is a word; two bits / one bit: two / four chunks make a word
     uint32_t* prow = packed + ((int64_t)grp * rm.packed_group_stride + rin) * kPd;
@@ -373,9 +399,16 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
 // read with coalesced loads into LDS; a lane cuts the 8 * BITS bits of each of its chunks out of one or two words and
 // looks centroid pairs up in a table of 4^BITS entries (c[a]*s, c[b]*s).  Arithmetic per element, in this order, as in
 // dequant_kernel: butterfly, * s, * sign, * norm, round to TO.  RAGGED as in the encoder.
-template <int D, typename TO, int BITS, bool RAGGED>
+//
+// INDICES: the levels come as one byte each, `packed` standing for n_rows x D bytes without groups (RAGGED).  A lane reads its
+// chunks as they lie (8 bytes each, 16 kLanes bytes of a row per instruction) and looks pairs up from them.  Bytes past the width
+// mean what packing them first would give: words of the summed, shifted bytes, cut to `word_bits` (three bits: whether the two
+// bits above a word's ten fields reach the next chunk depends on the kernel that reads the words); a wavefront that meets one
+// builds the words of its pass.  100 003 rows of 128 to float32 13.6 us against 8.1 us of packing and 11.6 us of this kernel
+// on the words.
+template <int D, typename TO, int BITS, bool RAGGED, bool INDICES = false>
 __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides, Codebook cbk, float s, RowMap rm,
-                                                              int passes) {
+                                                              int passes, uint32_t word_bits = ~0u) {
   const uint32_t* __restrict__ packed = sides.s[blockIdx.y].packed;
   const float* __restrict__ norms = sides.s[blockIdx.y].norms;
   const float* __restrict__ signs = sides.s[blockIdx.y].signs;
@@ -391,7 +424,8 @@ __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides
   // (butterfly_lanes_neg)
   __shared__ __align__(8) float2 pair_s[2 * kPairs];
   __shared__ uint32_t words_s[kWavesPerBlock][kVecs * kPd + 3];
-  __shared__ uint32_t src_s[kWavesPerBlock][RAGGED ? kVecs : 1], dst_s[kWavesPerBlock][RAGGED ? kVecs : 1];
+  constexpr bool kMapped = RAGGED && !INDICES;
+  __shared__ uint32_t src_s[kWavesPerBlock][kMapped ? kVecs : 1], dst_s[kWavesPerBlock][kMapped ? kVecs : 1];
   // Outputs leave through LDS: rows at a padded pitch (conflict-free 16-byte writes per lane and reads per row
   // segment), so that every store instruction writes 1 KB of contiguous memory
   constexpr int kPiecesPerRow = D * (int)sizeof(TO) / 16;
@@ -445,8 +479,16 @@ __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides
   uint32_t pw[kWordLoads];
   float pn = 0.0f;
   uint32_t my_out = 0;                                         // RAGGED: output row of this lane's vector in the fetched pass
+  uint2 pi[4];                                                 // INDICES: bytes of this lane's chunks
+  const uint8_t* ibytes = reinterpret_cast<const uint8_t*>(packed);
   auto fetch = [&](uint32_t first, uint32_t g_, uint32_t r_) {
-    if (RAGGED) {
+    if constexpr (INDICES) {
+      const uint32_t row = min(first + v, n_rows - 1);
+      pn = norms[row];
+      const uint8_t* src = ibytes + (int64_t)row * D + 8 * ls;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) pi[k] = *reinterpret_cast<const uint2*>(src + 8 * kLanes * k);
+    } else if (RAGGED) {
       uint32_t mg, mr;
       group_of(rm, min(first + v, n_rows - 1), mg, mr);
       src_s[wave][v] = mg * (uint32_t)rm.packed_group_stride + mr;
@@ -473,25 +515,61 @@ __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides
   for (int pass = 0; pass < passes; ++pass) {
     if (row0 >= n_rows) break;                                 // uniform over the wavefront
     const float nrm = pn;
-    if (RAGGED) dst_s[wave][v] = my_out;
+    uint2 ib[4];
+    if constexpr (INDICES) {
 #pragma unroll
-    for (int it = 0; it < kWordLoads; ++it) {
-      const int id = it * 64 + lane;
-      if (id < kVecs * kPd) words[id] = pw[it];
+      for (int k = 0; k < 4; ++k) ib[k] = pi[k];
+    } else {
+      if (RAGGED) dst_s[wave][v] = my_out;
+#pragma unroll
+      for (int it = 0; it < kWordLoads; ++it) {
+        const int id = it * 64 + lane;
+        if (id < kVecs * kPd) words[id] = pw[it];
+      }
     }
     uint32_t nrin = rin + kVecs, ngrp = grp;
     if (!RAGGED && nrin >= (uint32_t)rm.rows_per_group) { nrin = 0; ++ngrp; }
-    wave_lds_fence();
+    if (!INDICES) wave_lds_fence();
     if (pass + 1 < passes && row0 + kVecs < n_rows) fetch(row0 + kVecs, ngrp, nrin);
     float xs[4][8];
+    bool from_words = !INDICES;
+    if constexpr (INDICES) {
+      uint32_t past = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t f = CK::field(words + v * kPd + cw[k], csl[k], csh[k]);
+      for (int k = 0; k < 4; ++k) past |= ib[k].x | ib[k].y;
+      from_words = __any((past & (0x01010101u * (0x100u - (1u << BITS)))) != 0);
+      if (from_words) {
+        constexpr int VPW = Pk<BITS>::VPW;
+        for (int id = lane; id < kVecs * kPd; id += 64) {
+          const int vv = id / kPd, e0 = (id - vv * kPd) * VPW;
+          const uint8_t* src = ibytes + (int64_t)min(row0 + vv, n_rows - 1) * D + e0;
+          uint32_t word = 0;
+          for (int i = 0; i < min(VPW, D - e0); ++i) word += (uint32_t)src[i] << (BITS * i);
+          words[id] = word & word_bits;
+        }
+        wave_lds_fence();
+      } else {
 #pragma unroll
-      for (int jp = 0; jp < 4; ++jp) {
-        const float2 c2 = my_pairs[(f >> (2 * BITS * jp)) & CK::kPairMask];
-        xs[k][2 * jp] = c2.x;
-        xs[k][2 * jp + 1] = c2.y;
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int jp = 0; jp < 4; ++jp) {
+            const uint32_t b4 = jp < 2 ? ib[k].x : ib[k].y;
+            const float2 c2 = my_pairs[((b4 | (b4 >> (8 - BITS))) >> (16 * (jp & 1))) & CK::kPairMask];
+            xs[k][2 * jp] = c2.x;
+            xs[k][2 * jp + 1] = c2.y;
+          }
+      }
+    }
+    if (from_words) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t f = CK::field(words + v * kPd + cw[k], csl[k], csh[k]);
+#pragma unroll
+        for (int jp = 0; jp < 4; ++jp) {
+          const float2 c2 = my_pairs[(f >> (2 * BITS * jp)) & CK::kPairMask];
+          xs[k][2 * jp] = c2.x;
+          xs[k][2 * jp + 1] = c2.y;
+        }
       }
     }
     butterfly_lanes_neg<kLanes>(xs, m);
@@ -534,14 +612,15 @@ __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides
       // streaming stores (the "nt" hint): the rows are not read again by this kernel and a pass writes more than the
       // caches hold -- 115 -> 99 us per 1 M float32 rows, 75 -> 66 us for fp16 (d = 128)
       typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
-      unsigned char* oblock = reinterpret_cast<unsigned char*>(out + (RAGGED ? 0 : ((int64_t)grp * rm.out_group_stride + rin) * D));
+      unsigned char* oblock = reinterpret_cast<unsigned char*>(
+          out + (INDICES ? (int64_t)row0 * D : RAGGED ? 0 : ((int64_t)grp * rm.out_group_stride + rin) * D));
 #pragma unroll
       for (int i = 0; i < (int)(2 * sizeof(TO)); ++i) {            // 4 or 8 KB per pass
         const int piece = i * 64 + lane;
         const int vv = piece / kPiecesPerRow, pc = piece % kPiecesPerRow;
         const piece_t val = *reinterpret_cast<const piece_t*>(&orow_s[wave][vv * kPitch + pc * 16]);
-        if (!RAGGED) {
-          __builtin_nontemporal_store(val, reinterpret_cast<piece_t*>(oblock + piece * 16));
+        if (!kMapped) {
+          if (!RAGGED || row0 + vv < n_rows) __builtin_nontemporal_store(val, reinterpret_cast<piece_t*>(oblock + piece * 16));
         } else if (row0 + vv < n_rows) {
           __builtin_nontemporal_store(val, reinterpret_cast<piece_t*>(oblock + ((int64_t)dst_s[wave][vv] * kPiecesPerRow + pc) * 16));
         }
@@ -615,6 +694,27 @@ void launch_dequant_rows(const DequantCall& c) {
 #undef TQ_LAUNCH_DEQ
 }
 
+// levels as bytes: any number of rows, no groups
+template <int D>
+void launch_encode_indices(const EncodeCall& c) {
+  const int passes = stream_passes<D>(c.rm.n_rows);
+  const int grid = stream_grid<D>(c.rm.n_rows, passes);
+#define TQ_LAUNCH_ENC(T)                                                                                             \
+  TQ_DISPATCH_BITS(c.bits, (encode_rows_kernel<D, T, B_, true, true><<<grid, kBlock, 0, c.stream>>>(                  \
+                               c.sides, c.thr, c.gs, c.rm, passes)))
+  if (c.x_dtype == TQ_F32) { TQ_LAUNCH_ENC(float); }
+  else if (c.x_dtype == TQ_F16) { TQ_LAUNCH_ENC(__half); }
+  else { TQ_LAUNCH_ENC(__hip_bfloat16); }
+#undef TQ_LAUNCH_ENC
+}
+template <int D>
+void launch_dequant_indices(const DequantCall& c, uint32_t word_bits) {
+  const int passes = stream_passes<D>(c.rm.n_rows);
+  const int grid = stream_grid<D>(c.rm.n_rows, passes);
+  TQ_DISPATCH_BITS(c.bits, (dequant_rows_kernel<D, float, B_, true, true><<<grid, kBlock, 0, c.stream>>>(
+                               c.sides, c.cb, c.s, c.rm, passes, word_bits)));
+}
+
 // instantiated in translation units of their own, in parallel with the rest of the build
 extern template void launch_encode_rows<64, true>(const EncodeCall&);
 extern template void launch_encode_rows<256, true>(const EncodeCall&);
@@ -622,5 +722,11 @@ extern template void launch_encode_rows<128, true>(const EncodeCall&);
 extern template void launch_dequant_rows<64, true>(const DequantCall&);
 extern template void launch_dequant_rows<256, true>(const DequantCall&);
 extern template void launch_dequant_rows<128, true>(const DequantCall&);
+extern template void launch_encode_indices<64>(const EncodeCall&);
+extern template void launch_encode_indices<128>(const EncodeCall&);
+extern template void launch_encode_indices<256>(const EncodeCall&);
+extern template void launch_dequant_indices<64>(const DequantCall&, uint32_t);
+extern template void launch_dequant_indices<128>(const DequantCall&, uint32_t);
+extern template void launch_dequant_indices<256>(const DequantCall&, uint32_t);
 
 }  // namespace tqc

@@ -2,7 +2,7 @@
 //
 // Both are bound by memory: 141 bytes per row of 128 indices and one packed row of 52 bytes at three bits.  As a chain of
 // tensor operations in 64-bit integers (shift, mask, pad, sum) they moved 1 to 2 KB per index row: 100 003 rows of 128
-// at three bits took 130 us (unpack) and 140 us (pack), of a PolarQuantizer round trip of 332 us, which takes 42 us with these kernels.  Here a lane takes
+// at three bits took 130 us (unpack) and 140 us (pack), of a PolarQuantizer round trip of 332 us, which took 42 us with these kernels (24 us since it goes without words).  Here a lane takes
 // what one wide access holds: 16 indices of the output (one 16-byte store), or one packed word of the output (two to
 // eight 4-byte loads).
 #include "tq_common.h"

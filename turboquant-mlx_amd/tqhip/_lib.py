@@ -13,6 +13,7 @@ LIB_PATH = os.environ.get("TQHIP_LIB", os.path.join(_HERE, "lib", "libtqhip.so")
 
 TQ_F32, TQ_F16, TQ_BF16, TQ_MASK_BOOL = 0, 1, 2, 3
 TQ_ENCODE_MLX, TQ_ENCODE_METAL = 0, 1
+TQ_ERR_UNSUPPORTED = -10
 TQ_MMA_OFF, TQ_MMA_FP16, TQ_MMA_SPLIT = 0, 1, 2
 TQ_OP_SPARSE_V, TQ_OP_FLASH_DECODE, TQ_OP_VONLY_DECODE = 0, 1, 2
 
@@ -81,6 +82,8 @@ PROTOTYPES = {
     "tq_random_signs": (_i, [C.POINTER(C.c_uint64), _i, _i, _p, _p]),
     "tq_pack_indices": (_i, [_p, _i, _p, _l, _i, _i, _p]),
     "tq_unpack_indices": (_i, [_p, _p, _l, _i, _i, _i, _p]),
+    "tq_quantize": (_i, [_p, _i, _p, _fp, _p, _p, _l, _i, _i, _i, _p]),
+    "tq_dequantize": (_i, [_p, _p, _fp, _p, _p, _l, _i, _i, _p]),
     "tq_mask_rows": (_i, [_p, _i, _l, _l, _l, _p, _i, _i, _l, _l, _p]),
     "tq_vonly_append": (_i, [_p, _i, _p, _i, _p, _fp, _p, _p, _p, _p, _l, _l, _l, _l, _l, _l, _i, _i, _i, _p]),
     "tq_dequant": (_i, [_p, _p, _fp, _p, _p, _i, _l, _l, _l, _l, _l, _i, _i, _p]),

@@ -379,6 +379,42 @@ def fused_quantize(vectors: torch.Tensor, signs: torch.Tensor, boundaries, dim: 
     return packed, norms
 
 
+def quantize_indices(x: torch.Tensor, signs: torch.Tensor, boundaries, dim: int, bits: int, variant: str = "mlx"):
+    """fused_quantize and unpack_indices of (n, dim) rows: (n, dim) uint8 levels and (n,) float32 norms, in one launch
+    (tq_quantize) where it takes the call."""
+    if dim in (64, 128, 256) and x.dtype in _DTYPES and _native_pack(x):
+        rows = x.contiguous()
+        signs = _as_f32_dev(signs, rows)
+        n = rows.shape[0]
+        idx = torch.empty((n, dim), dtype=torch.uint8, device=rows.device)
+        norms = torch.empty((n,), dtype=torch.float32, device=rows.device)
+        rc = _lib.load().tq_quantize(rows.data_ptr(), _DTYPES[rows.dtype], signs.data_ptr(), _host_table(boundaries), idx.data_ptr(),
+                                     norms.data_ptr(), n, dim, bits,
+                                     {"mlx": _lib.TQ_ENCODE_MLX, "metal": _lib.TQ_ENCODE_METAL}[variant], _stream(rows))
+        if rc != _lib.TQ_ERR_UNSUPPORTED:
+            _lib.check(rc)
+            return idx, norms
+    packed, norms = fused_quantize(x, signs, boundaries, dim, bits, variant=variant)
+    return unpack_indices(packed, bits, dim), norms
+
+
+def dequantize_indices(indices: torch.Tensor, norms: torch.Tensor, centroids, signs: torch.Tensor, dim: int, bits: int) -> torch.Tensor:
+    """pack_indices and packed_dequantize of (n, dim) levels: (n, dim) float32, in one launch (tq_dequantize) for bytes."""
+    n = indices.shape[0]
+    if (dim in (64, 128, 256) and indices.dtype == torch.uint8 and _native_pack(indices) and norms.is_cuda
+            and norms.shape[0] == n and type(norms) is torch.Tensor):
+        rows = indices.contiguous()
+        norms = norms.to(torch.float32).contiguous()
+        signs = _as_f32_dev(signs, rows)
+        out = torch.empty((n, dim), dtype=torch.float32, device=rows.device)
+        rc = _lib.load().tq_dequantize(rows.data_ptr(), norms.data_ptr(), _host_table(centroids), signs.data_ptr(), out.data_ptr(), n,
+                                       dim, bits, _stream(rows))
+        if rc != _lib.TQ_ERR_UNSUPPORTED:
+            _lib.check(rc)
+            return out
+    return packed_dequantize(pack_indices(indices, bits), norms, centroids, signs, dim, bits)
+
+
 def dequant_into(packed: torch.Tensor, norms: torch.Tensor, centroids, signs: torch.Tensor,
                  out: torch.Tensor, *, n_groups: int, rows_per_group: int, packed_group_stride: int,
                  norms_group_stride: int, out_group_stride: int, dim: int, bits: int,

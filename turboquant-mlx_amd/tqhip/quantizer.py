@@ -48,13 +48,10 @@ class PolarQuantizer:
 
     def quantize(self, x: torch.Tensor):
         lead = x.shape[:-1]
-        packed, norms = ops.fused_quantize(x.reshape(-1, self.dim), self.signs, self.boundaries,
-                                           self.dim, self.bits, variant="mlx")
-        idx = ops.unpack_indices(packed, self.bits, self.dim)
+        idx, norms = ops.quantize_indices(x.reshape(-1, self.dim), self.signs, self.boundaries, self.dim, self.bits, variant="mlx")
         return idx.reshape(*lead, self.dim), norms.reshape(lead)
 
     def dequantize(self, indices: torch.Tensor, norms: torch.Tensor) -> torch.Tensor:
         lead = indices.shape[:-1]
-        packed = ops.pack_indices(indices.reshape(-1, self.dim), self.bits)
-        out = ops.packed_dequantize(packed, norms.reshape(-1), self.centroids, self.signs, self.dim, self.bits)
+        out = ops.dequantize_indices(indices.reshape(-1, self.dim), norms.reshape(-1), self.centroids, self.signs, self.dim, self.bits)
         return out.reshape(*lead, self.dim)
