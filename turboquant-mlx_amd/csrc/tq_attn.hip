@@ -978,7 +978,8 @@ void launch_packed_stream_bits(int bits, dim3 grid, const tqm::PackedArgs& a, co
 // per CU) about 4.2 us, and with more workgroups than that the launch runs in rounds whose set-up overlaps.
 // So: the smallest step count that brings the launch down to 256 workgroups, or the smallest that brings it
 // down to 512, whichever costs less; at most 8 steps, and at most 4 for ragged batches (true lengths
-// unknown on the host, max_seq_len is an upper bound), which keeps the tail of the launch short.  Measured,
+// unknown on the host, max_seq_len is an upper bound), which keeps the tail of the launch short (ragged batches without a mask
+// only learn from this that they stream: their steps are spread evenly, see launch_packed_mfma).  Measured,
 // one sequence of 32 / 8 heads: 24 576 positions 16.7 us with 3 steps (256 workgroups) against 17.9 with 2
 // (384) and 22.4 as single tiles; 18 432 positions 17.0 with 3 steps, 18.2 with 2, 22.0 as single tiles; 36 864
 // positions 21.7 with 3 (384 workgroups), 26.5 with 2 (576), 22.3 with 5 (232).
@@ -1059,7 +1060,16 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
                          (sh.bits == 3 || (tq::aligned(k_packed, 16) && tq::aligned(v_packed, 16)));
   const int n_steps = stream_ok ? flash_stream_steps(sh.n_seq, sh.n_kv_heads, sh.seq_len,
                                                      sh.seq_offsets != nullptr || len_dev != nullptr) : 0;
-  if (n_steps >= 2) {
+  // A ragged batch without a mask: equal ranges of the steps of all sequences (tq_packed_mfma.h, SPREAD), two workgroups per CU --
+  // as many as fit beside each other -- and as many partials as the workspace holds beside their list.
+  const int64_t spread = sh.seq_offsets && !sh.mask ? std::min<int64_t>(std::max(1, 512 / sh.n_kv_heads), (int64_t)sh.n_seq * (n_tiles - 2)) : 0;
+  if (n_steps >= 2 && spread >= 1) {
+    a.n_seq = sh.n_seq;
+    a.n_tiles_max = (int)spread + sh.n_seq;
+    a.ws_ml = a.ws_S + (size_t)a.n_tiles_max * n_q * tqm::kD;
+    a.parts = (int2*)(a.ws_ml + (size_t)a.n_tiles_max * n_q * 2);
+    launch_packed_stream_bits(sh.bits, dim3((unsigned)spread, sh.n_kv_heads), a, kcb, vcb, 0, stream);
+  } else if (n_steps >= 2) {
     tile_pos = tqm::kSStepPos * n_steps;
     a.n_tiles_max = (int)((sh.seq_len + tile_pos - 1) / tile_pos);
     dim3 grid(a.n_tiles_max, sh.n_kv_heads, sh.n_seq);
@@ -1108,7 +1118,7 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
 #define LAUNCH_MERGE_P(TO)                                                                                    \
   tqm::decode_merge_rows_kernel<TO, MODE == tqm::kFlash><<<mgrid, tqm::kMergeThreads, 0, stream>>>(            \
       a.ws_S, a.ws_ml, sh.seq_offsets, sh.seq_len, n_parts, sh.n_kv_heads, sh.n_rep, v_signs, inv_dim, (TO*)out, tile_pos, \
-      len_dev, len_bias)
+      len_dev, len_bias, a.parts)
   if (sh.out_dtype == TQ_F16) { LAUNCH_MERGE_P(__half); }
   else if (sh.out_dtype == TQ_BF16) { LAUNCH_MERGE_P(__hip_bfloat16); }
   else { LAUNCH_MERGE_P(float); }

@@ -368,6 +368,22 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+__device__ __forceinline__ int wave_total(int v) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, TQ_WAVE);
+  return v;
+}
+
+// inclusive sums over the lanes up to this one
+__device__ __forceinline__ int wave_scan(int v, int lane) {
+#pragma unroll
+  for (int d = 1; d < TQ_WAVE; d <<= 1) {
+    const int u = __shfl_up(v, d, TQ_WAVE);
+    v += lane >= d ? u : 0;
+  }
+  return v;
+}
+
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
   __half2 h = __floats2half2_rn(a, b);
   return *reinterpret_cast<uint32_t*>(&h);

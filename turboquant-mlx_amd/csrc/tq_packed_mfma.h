@@ -55,6 +55,8 @@ struct PackedArgs {
   float score_scale;          // (1/d) * attn_scale for kFlash, 1/d for kScores; times 1/key-table scale
   float v_unscale;            // 1 / the scale the value table was multiplied by on the host
   float threshold;            // kWeights
+  int32_t n_seq;              // spread streaming pass: sequences
+  int2* parts;                //   out, per sequence: its first partial of a kv head and their number (n_tiles_max = partials per kv head)
 };
 
 // copy one wave's 64 packed rows of PD words each (3328 bytes at three bits) from global memory into its LDS area:
@@ -624,6 +626,13 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
 // -inf scores.  Rows of the other widths are 16, 32 or 64 bytes: every row of a 16-byte aligned
 // tensor is aligned (the host sends other tensors to the tile pass), and a block is 64, 128 or 256 pieces.
 //
+// SPREAD (ragged batches): the grid is (gridDim.x, n_kv), about two workgroups per CU, and the steps of all sequences, one after
+// the other, are cut into gridDim.x equal ranges (at least two steps each), which the workgroups derive from the offsets.  A range
+// may end one sequence and begin the next: each piece leaves a partial of its own, number (workgroup + sequence) of its kv head --
+// along the list one or the other grows by one at every cut -- and the merge pass reads from a.parts which are a sequence's.
+// Against one workgroup per four steps of a sequence, whose set-up of about 5 us then stands beside 4 x 4.2 us of steps and
+// whose number is no multiple of what the chip holds: @SPREAD@
+//
 // Mask: one value per position, like the norms, two steps ahead of its use, so that a step that the mask excludes for a
 // wave (left padding) neither fetches its packed rows nor computes: 8 sequences x 32 / 8 heads of 6003 positions, a quarter of
 // them padding, 30.8 us in the tile pass, 20.9 us here.  A mask with a row per query head stays with the tile pass.
@@ -632,9 +641,17 @@ constexpr int kSThreads = kSWaves * 64;
 constexpr int kSStepPos = kSWaves * kWavePos;     // 256 positions per workgroup step
 constexpr int kSImageBytes = 4096;                // 209 pieces of 16 bytes, rounded up; 256 pieces at four bits
 
-template <int BITS, bool VQ = true, bool MASKED = false>
+// The arguments in the kernel's argument segment, and which of the two a form reads.
+typedef const __attribute__((address_space(4))) PackedArgs ConstArgs;
+template <bool AGAIN>
+__device__ __forceinline__ auto& args_of(const PackedArgs& args, ConstArgs* again) {
+  if constexpr (AGAIN) return *again;
+  else return args;
+}
+
+template <int BITS, bool VQ = true, bool MASKED = false, bool SPREAD = false>
 __global__ __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps) {
+void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_steps) {
   using VF = VField<BITS>;
   // A workgroup decodes up to 8 x 256 positions, which repays building the quad table (one for keys and values when
   // their codebooks are equal, VQ; else the values use their pair table).
@@ -653,14 +670,22 @@ void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps)
   __shared__ __align__(16) float alpha_s[kSWaves][kHeadsMax];
   __shared__ __align__(16) MergeLds<kSWaves> mg_s;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int wg = blockIdx.x, kvh = blockIdx.y;
+
+  // n_steps steps of sequence seq from position wg_p0 on, into partial `part`
+  auto run = [&](const int seq, const int64_t wg_p0, const int n_steps, const int64_t part) __attribute__((always_inline)) {
+  int tid = threadIdx.x;
+  ConstArgs* again = (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  // Several ranges in a row: what a range derives from the lane and from the arguments is derived again for the next one. Kept in
+  // registers from one to the next it costs 60 spilled ones.
+  if (SPREAD) asm volatile("" : "+v"(tid), "+s"(again));
+  auto& a = args_of<SPREAD>(args, again);
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, g = lane >> 4;
-  const int wg = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
   const int n_rep = a.n_rep;
   const int n_q = a.n_kv * n_rep;
   const int64_t q_row0 = (int64_t)seq * n_q + (int64_t)kvh * n_rep;
-
   int64_t first = 0, len = a.seq_len;
   if (a.seq_offsets) {
     first = a.seq_offsets[seq];
@@ -669,7 +694,6 @@ void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps)
     const int64_t want = *a.len_dev + a.len_bias;
     len = want < 0 ? 0 : (want < len ? want : len);
   }
-  const int64_t wg_p0 = (int64_t)wg * kSStepPos * n_steps;
   if (wg_p0 >= len) return;
 
   // ---- addresses: row 0 of the sequence for this kv head, misalignment of the wave's blocks
@@ -743,8 +767,10 @@ void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps)
   float knA, vnA, knB = 0.0f, vnB = 0.0f;
   issue(0, false, kqA, vqA, knA, vnA);
 
-  if (tid < 64) VF::fill(lutk_s, kcb, tid);
-  else if (tid < 128) VF::fill(lutv_s, vcb, tid - 64);
+  if (!SPREAD) {
+    if (tid < 64) VF::fill(lutk_s, kcb, tid);
+    else if (tid < 128) VF::fill(lutv_s, vcb, tid - 64);
+  }
   if (a.q_raw) {
     rotate_query_rows<kSWaves>(a.q_raw, a.q_dtype, a.k_signs, q_row0, n_rep, wave, lane, q_s, ql_s);
   } else {
@@ -757,7 +783,7 @@ void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps)
     }
   }
   __syncthreads();
-  if (KQUAD) {
+  if (KQUAD && !SPREAD) {
     VF::fill_quad(quad_s, lutk_s, tid, kSThreads);
     __syncthreads();
   }
@@ -919,11 +945,59 @@ void packed_stream_kernel(PackedArgs a, Codebook kcb, Codebook vcb, int n_steps)
   l += shfl_xor_f(l, 16);
   l += shfl_xor_f(l, 32);
   l *= inv_tscale;
-  const int64_t grp = (int64_t)seq * a.n_kv + kvh;
-  float* pS = a.ws_S + (grp * a.n_tiles_max + wg) * (int64_t)(n_rep * kD);
-  float* pml = a.ws_ml + (grp * a.n_tiles_max + wg) * (int64_t)(n_rep * 2);
+  float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
+  float* pml = a.ws_ml + part * (int64_t)(n_rep * 2);
   static_assert(2 * kSImageBytes >= 8 * kD * 4 && (2 * kSImageBytes) % 16 == 0, "a wave's image area holds its eight deposit rows");
-  merge_waves<kSWaves>(mg_s, big_s, 2 * kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml);
+  merge_waves<kSWaves>(mg_s, big_s, 2 * kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml, tid);
+  };
+
+  const PackedArgs& a = args;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if constexpr (!SPREAD) {
+    const int seq = blockIdx.z;
+    run(seq, (int64_t)wg * kSStepPos * max_steps, max_steps, ((int64_t)seq * a.n_kv + kvh) * a.n_tiles_max + wg);
+  } else {
+    // steps of all sequences in a row: this workgroup's are at .. end - 1, `base` those of the sequences before `seq`
+    if (tid < 64) VF::fill(lutk_s, kcb, tid);
+    else if (tid < 128) VF::fill(lutv_s, vcb, tid - 64);
+    __syncthreads();
+    if (KQUAD) VF::fill_quad(quad_s, lutk_s, tid, kSThreads);            // the first range's barrier makes it visible
+    auto steps_of = [&](int s) {
+      const int64_t len = s < a.n_seq ? (int64_t)a.seq_offsets[s + 1] - a.seq_offsets[s] : 0;
+      return len > 0 ? (int)((len + kSStepPos - 1) / kSStepPos) : 0;
+    };
+    int total = 0;
+    for (int s0 = 0; s0 < a.n_seq; s0 += 64) total += wave_total(steps_of(s0 + lane));
+    const int per = max(2, (total + (int)gridDim.x - 1) / (int)gridDim.x);
+    int at = wg * per, seq = 0, base = 0;
+    const int end = min(total, at + per);
+    const bool listing = wg == 0 && kvh == 0 && wave == 0;               // the merge pass's list of partials
+    bool found = false;
+    for (int s0 = 0, before = 0; s0 < a.n_seq; s0 += 64) {
+      const int mine = steps_of(s0 + lane), upto = before + wave_scan(mine, lane);
+      if (listing && s0 + lane < a.n_seq)
+        a.parts[s0 + lane] = make_int2((upto - mine) / per + s0 + lane, mine > 0 ? (upto - 1) / per - (upto - mine) / per + 1 : 0);
+      const uint64_t past = __ballot(upto > at);
+      if (!found && past) {
+        found = true;
+        const int l = __builtin_ctzll(past);
+        seq = s0 + l;
+        base = __builtin_amdgcn_readlane(upto - mine, l);
+      }
+      before = __builtin_amdgcn_readlane(upto, 63);
+    }
+    seq = __builtin_amdgcn_readfirstlane(seq);
+    while (at < end) {
+      const int have = steps_of(seq), n = min(end, base + have) - at;
+      if (n > 0) {
+        run(seq, (int64_t)(at - base) * kSStepPos, n, (int64_t)kvh * a.n_tiles_max + wg + seq);
+        __syncthreads();                                                 // the merge has read what the next range overwrites
+      }
+      at += n;
+      base += have;
+      ++seq;
+    }
+  }
 }
 
 // Scores pass of the thresholded flash step in the streaming form (packed K, no mask): the key half of
@@ -1376,7 +1450,7 @@ void packed_stream_weights_kernel(PackedArgs a, Codebook vcb, int n_steps) {
 // points, 1, 2 and 4 in translation units of their own (the widths compile in parallel).
 //   launch_packed_tiles: the tile pass in `mode`; shape (flash mode): kTilesOnePerCu when the grid gives a CU one
 //     workgroup at most, kTilesFourWaves for workgroups of four waves (tiles of 256 positions)
-//   launch_packed_stream: the streaming flash pass (no mask, or one that the query heads share); rows of widths other than 3 must be 16-byte aligned
+//   launch_packed_stream: the streaming flash pass (no mask, or one that the query heads share; a.parts set: the spread form, no mask); rows of widths other than 3 must be 16-byte aligned
 template <int BITS>
 void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb,
                          hipStream_t stream) {
@@ -1396,6 +1470,16 @@ void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, co
 template <int BITS>
 void launch_packed_stream(dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb, int n_steps,
                           hipStream_t stream) {
+  if (a.parts) {
+    if constexpr (VField<BITS>::kQuad) {
+      if (std::memcmp(kcb.c, vcb.c, sizeof(kcb.c)) != 0) {
+        packed_stream_kernel<BITS, false, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);
+        return;
+      }
+    }
+    packed_stream_kernel<BITS, true, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);
+    return;
+  }
   if constexpr (VField<BITS>::kQuad) {
     if (std::memcmp(kcb.c, vcb.c, sizeof(kcb.c)) != 0) {
       if (a.mask) packed_stream_kernel<BITS, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);
