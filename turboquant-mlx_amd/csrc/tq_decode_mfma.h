@@ -57,6 +57,10 @@ constexpr int kWavePos = 64;
 constexpr int kTilePos = kWaves * kWavePos;      // 512 positions per workgroup
 constexpr int kMfmaThreads = kWaves * 64;
 constexpr int kHeadsMax = 16;
+// Query rows in LDS, as words of two halves: four words more than a row has, so that the sixteen rows that one read takes
+// the same piece of lie in different banks (at 64 words every row begins in bank 0).
+constexpr int kQPitch = kD / 2 + 4;
+__device__ __forceinline__ constexpr int q_word(int w) { return w + (w / (kD / 2)) * (kQPitch - kD / 2); }
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr int kMergeThreads = 256;
 
@@ -521,8 +525,8 @@ __global__ __launch_bounds__(WAVES * 64) void vonly_scores_kernel(MfmaArgs a) {
   constexpr int kPos = WAVES * kWavePos;             // positions per workgroup
   constexpr int kThr = WAVES * 64;
   __shared__ __align__(16) unsigned char big_s[WAVES * 4096]; // per-wave 4 KB: K tiles, then the score block
-  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];
-  __shared__ __align__(16) uint32_t ql_s[QF32 ? kHeadsMax : 1][kD / 2];
+  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kQPitch];
+  __shared__ __align__(16) uint32_t ql_s[QF32 ? kHeadsMax : 1][kQPitch];
   __shared__ float m_s[WAVES][kHeadsMax], l_s[WAVES][kHeadsMax];
 
   const int tid = threadIdx.x;
@@ -579,8 +583,8 @@ __global__ __launch_bounds__(WAVES * 64) void vonly_scores_kernel(MfmaArgs a) {
     // bf16 queries become fp16 here, after every load of the pass has been requested: converting where the word
     // is loaded would wait for it before anything else is in flight
     if (!QF32 && a.q_bf16) my_q[i] = pack_h2(__uint_as_float(my_q[i] << 16), __uint_as_float(my_q[i] & 0xFFFF0000u));
-    (&q_s[0][0])[tid + i * kThr] = my_q[i];
-    if (QF32) (&ql_s[0][0])[tid + i * kThr] = my_ql[i];
+    (&q_s[0][0])[q_word(tid + i * kThr)] = my_q[i];
+    if (QF32) (&ql_s[0][0])[q_word(tid + i * kThr)] = my_ql[i];
   }
   __syncthreads();
 
@@ -719,8 +723,8 @@ __device__ __forceinline__ void vonly_stream_body(const MfmaArgs& a, const Codeb
   constexpr int kPieces = 8 * kPd + (MISALIGNED ? 1 : 0);   // 16-byte pieces of a step's 32 packed rows: 104 at three bits (+ 1 misaligned)
   __shared__ __align__(16) unsigned char big_s[NW * 4096];
   __shared__ uint32_t lut_s[VF::kLut < 64 ? 64 : VF::kLut];
-  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];
-  __shared__ __align__(16) uint32_t ql_s[QF32 ? kHeadsMax : 1][kD / 2];
+  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kQPitch];
+  __shared__ __align__(16) uint32_t ql_s[QF32 ? kHeadsMax : 1][kQPitch];
   __shared__ __align__(16) float nrm_s[NW][kStepPos];
   __shared__ __align__(16) float alpha_s[NW][kHeadsMax];
   __shared__ __align__(16) MergeLds<NW> mg_s;
@@ -825,8 +829,8 @@ __device__ __forceinline__ void vonly_stream_body(const MfmaArgs& a, const Codeb
     // bf16 queries become fp16 here, after every load of the pass has been requested: converting where the word
     // is loaded would wait for it before anything else is in flight
     if (!QF32 && a.q_bf16) my_q[i] = pack_h2(__uint_as_float(my_q[i] << 16), __uint_as_float(my_q[i] & 0xFFFF0000u));
-    (&q_s[0][0])[tid + i * kThr] = my_q[i];
-    if (QF32) (&ql_s[0][0])[tid + i * kThr] = my_ql[i];
+    (&q_s[0][0])[q_word(tid + i * kThr)] = my_q[i];
+    if (QF32) (&ql_s[0][0])[q_word(tid + i * kThr)] = my_ql[i];
   }
   __syncthreads();
 

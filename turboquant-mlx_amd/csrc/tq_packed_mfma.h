@@ -115,8 +115,8 @@ __device__ __forceinline__ void stage_block(const PackedBlockT<PD>& b, uint32_t*
 // rounding into q_s / ql_s.  Runs while the key/value loads are in flight.
 template <int N_WAVES>
 __device__ __forceinline__ void rotate_query_rows(const void* q_raw, int q_dtype, const float* k_signs, int64_t q_row0,
-                                                  int n_rep, int wave, int lane, uint32_t (*q_s)[kD / 2],
-                                                  uint32_t (*ql_s)[kD / 2]) {
+                                                  int n_rep, int wave, int lane, uint32_t (*q_s)[kQPitch],
+                                                  uint32_t (*ql_s)[kQPitch]) {
   const float s0 = k_signs[lane], s1 = k_signs[lane + 64];
 #pragma unroll
   for (int it = 0; it < kHeadsMax / N_WAVES; ++it) {
@@ -240,8 +240,8 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   __shared__ __align__(16) unsigned char big_s[NW * 4096];    // per-wave 4 KB areas, later S_all[NW][8][128]
   __shared__ uint32_t lutk_s[VF::kLut < 64 ? 64 : VF::kLut], lutv_s[VF::kLut < 64 ? 64 : VF::kLut];
   const uint2* quad_s = nullptr;
-  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];      // rotated queries as half2: rounded value ...
-  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kD / 2];     // ... and what the rounding lost
+  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kQPitch];      // rotated queries as half2: rounded value ...
+  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kQPitch];     // ... and what the rounding lost
   __shared__ __align__(16) float kn_s[NW][kWavePos], vn_s[NW][kWavePos];
   __shared__ float m_s[NW][kHeadsMax], l_s[NW][kHeadsMax];
   __shared__ __align__(16) MergeLds<NW> mg_s;
@@ -349,8 +349,8 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
       for (int i = 0; i < kQIt; ++i) {
         const __half2 h = __floats2half2_rn(my_q[i].x, my_q[i].y);
         const float2 back = __half22float2(h);
-        (&q_s[0][0])[tid + i * kThr] = *reinterpret_cast<const uint32_t*>(&h);
-        (&ql_s[0][0])[tid + i * kThr] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
+        (&q_s[0][0])[q_word(tid + i * kThr)] = *reinterpret_cast<const uint32_t*>(&h);
+        (&ql_s[0][0])[q_word(tid + i * kThr)] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
       }
     }
     // the score scale rides on the key norm: log2 units for the softmax, plain units for kScores
@@ -617,7 +617,10 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
 // computed.  The fixed work of a tile (query staging, tables, merge, partial store) is paid once
 // per n_steps * 256 positions and the merge pass sees that many fewer partials.
 //
-// Loads: at three bits a wave's 64 rows of 52 bytes start at an arbitrary multiple of 4 bytes (ragged
+// Loads: keys go from global memory into the registers of the lane that decodes them (KeyQuarter): a row's words are read by four
+// lanes, each 12 bytes and the shared last word at three bits.  Through an image like the values: 82 us where this takes 75 (sixteen ragged sequences); with the streaming hint, under which the two
+// reads of a line fetch it twice, 81.
+// Values need the same elements of several rows in one lane and pass through an image in LDS: at three bits a wave's 64 rows of 52 bytes start at an arbitrary multiple of 4 bytes (ragged
 // batches start a sequence at any row).  They are fetched as ALIGNED 16-byte pieces from the 16-byte
 // boundary at or below the first row (at most 209 pieces) into the wave's LDS image, and rows are
 // read from the image at the misalignment offset.  An aligned 16-byte piece never crosses a page,
@@ -631,7 +634,7 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
 // may end one sequence and begin the next: each piece leaves a partial of its own, number (workgroup + sequence) of its kv head --
 // along the list one or the other grows by one at every cut -- and the merge pass reads from a.parts which are a sequence's.
 // Against one workgroup per four steps of a sequence, whose set-up of about 5 us then stands beside 4 x 4.2 us of steps and
-// whose number is no multiple of what the chip holds: @SPREAD@
+// whose number is no multiple of what the chip holds: sixteen sequences of 4K to 32K positions, 32 / 8 heads, 125.7 -> 90.1 us (the pass 113.6 -> 80.6).
 //
 // Mask: one value per position, like the norms, two steps ahead of its use, so that a step that the mask excludes for a
 // wave (left padding) neither fetches its packed rows nor computes: 8 sequences x 32 / 8 heads of 6003 positions, a quarter of
@@ -640,6 +643,51 @@ constexpr int kSWaves = 4;
 constexpr int kSThreads = kSWaves * 64;
 constexpr int kSStepPos = kSWaves * kWavePos;     // 256 positions per workgroup step
 constexpr int kSImageBytes = 4096;                // 209 pieces of 16 bytes, rounded up; 256 pieces at four bits
+
+// What a lane needs of a packed key row as the A operand of four score products: the words of 32 elements, read from global memory
+// as they lie and cut up in registers.  Which elements meet in a product is free as long as the query's are chosen alike, so a
+// lane's are those of whole words: elements 32 g .. 32 g + 31, and at three bits, where a row is thirteen words of ten (the last
+// of eight), the three words 3 g .. 3 g + 2 and two elements of the last.
+template <int BITS>
+struct KeyQuarter {
+  static constexpr int kPd = VField<BITS>::kPd;
+  uint32_t w[BITS == 3 ? 4 : BITS];
+  __device__ __forceinline__ void load(const char* base, uint32_t row_bytes, int g) {
+    if constexpr (BITS == 3) {
+      typedef uint32_t u3 __attribute__((ext_vector_type(3), aligned(4)));
+      const u3 x = (*reinterpret_cast<const u3*>(base + (row_bytes + 12 * g)));
+      w[0] = x[0]; w[1] = x[1]; w[2] = x[2];
+      w[3] = *reinterpret_cast<const uint32_t*>(base + (row_bytes + 48));
+    } else if constexpr (BITS == 4) {
+      const u4 x = load_stream(base + (row_bytes + 16 * g));
+      w[0] = x[0]; w[1] = x[1]; w[2] = x[2]; w[3] = x[3];
+    } else if constexpr (BITS == 2) {
+      typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+      const u2 x = __builtin_nontemporal_load(reinterpret_cast<const u2*>(base + (row_bytes + 8 * g)));
+      w[0] = x[0]; w[1] = x[1];
+    } else {
+      w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + (row_bytes + 4 * g)));
+    }
+  }
+  // the fields of the eight elements of product kb from bit 0 on; bits above them are garbage
+  __device__ __forceinline__ uint32_t field(int kb, int g) const {
+    if constexpr (BITS == 3) {
+      if (kb < 3) return w[kb];                                          // elements 0 .. 7 of a word; 8 and 9 of all make the fourth
+      return (w[0] >> 24) | ((w[1] >> 18) & 0xFC0u) | ((w[2] >> 12) & 0x3F000u) | ((w[3] >> (6 * g)) << 18);
+    } else if constexpr (BITS == 4) {
+      return w[kb];
+    } else if constexpr (BITS == 2) {
+      return w[kb >> 1] >> (16 * (kb & 1));
+    } else {
+      return w[0] >> (8 * kb);
+    }
+  }
+  // the pair of query elements (in units of two) that meets fields 2 jp and 2 jp + 1 of product kb
+  __device__ static __forceinline__ int pair(int kb, int jp, int g) {
+    if constexpr (BITS == 3) return kb < 3 ? 15 * g + 5 * kb + jp : jp < 3 ? 15 * g + 5 * jp + 4 : 60 + g;
+    else return 16 * g + 4 * kb + jp;
+  }
+};
 
 // The arguments in the kernel's argument segment, and which of the two a form reads.
 typedef const __attribute__((address_space(4))) PackedArgs ConstArgs;
@@ -653,6 +701,7 @@ template <int BITS, bool VQ = true, bool MASKED = false, bool SPREAD = false>
 __global__ __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_steps) {
   using VF = VField<BITS>;
+  using KQ = KeyQuarter<BITS>;
   // A workgroup decodes up to 8 x 256 positions, which repays building the quad table (one for keys and values when
   // their codebooks are equal, VQ; else the values use their pair table).
   constexpr bool KQUAD = VF::kQuad, VQUAD = VF::kQuad && VQ;
@@ -660,11 +709,11 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   constexpr int kPieces = BITS == 3 ? 209 : 16 * kPd;           // 16-byte pieces of a wave's 64 rows (three bits: + misalignment)
   constexpr int kWhole = kPieces / 64, kRest = kPieces % 64;    // whole-wave stores into the image, lanes of the last one
   constexpr int kLoads = kWhole + (kRest ? 1 : 0);
-  __shared__ __align__(16) unsigned char big_s[kSWaves * 2 * kSImageBytes];   // per wave: K image, V image; later S_all[4][8][128]
+  __shared__ __align__(16) unsigned char big_s[kSWaves * kSImageBytes];   // per wave: image of its value rows; later S_all[4][8][128]
   __shared__ uint32_t lutk_s[VF::kLut < 64 ? 64 : VF::kLut], lutv_s[VF::kLut < 64 ? 64 : VF::kLut];
   __shared__ __align__(16) uint2 quad_s[KQUAD ? VF::kQuadEntries : 1];
-  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];
-  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kD / 2];
+  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kQPitch];
+  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kQPitch];
   __shared__ __align__(16) float kn_s[kSWaves][kWavePos], vn_s[kSWaves][kWavePos];
   __shared__ __align__(16) float mk_s[MASKED ? kSWaves : 1][kWavePos];
   __shared__ __align__(16) float alpha_s[kSWaves][kHeadsMax];
@@ -702,7 +751,6 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   const char* vrow0 = reinterpret_cast<const char*>(
       a.v_packed + ((int64_t)seq * a.v_seq_stride + (int64_t)kvh * a.v_head_stride + first) * kPd);
   // every block of this workgroup starts a multiple of 64 rows = 208 pieces after row wg_p0: one misalignment
-  const int kmis = BITS == 3 ? (int)((reinterpret_cast<uintptr_t>(krow0) + (uint64_t)wg_p0 * (kPd * 4)) & 15) : 0;
   const int vmis = BITS == 3 ? (int)((reinterpret_cast<uintptr_t>(vrow0) + (uint64_t)wg_p0 * (kPd * 4)) & 15) : 0;
   const float* knrow0 = a.k_norms + (int64_t)seq * a.kn_seq_stride + (int64_t)kvh * a.kn_head_stride + first;
   const float* vnrow0 = a.v_norms + (int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first;
@@ -720,23 +768,24 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   // finite, and its score is set to -inf.
   // Addresses are a base that is the same for the whole workgroup (its first piece / first norm) plus a 32-bit
   // offset per lane: one register per load instead of a 64-bit pointer.
-  const char* k_base = krow0 + wg_p0 * (kPd * 4) - kmis;
+  const char* k_base = krow0 + wg_p0 * (kPd * 4);
   const char* v_base = vrow0 + wg_p0 * (kPd * 4) - vmis;
   const float* kn_base = knrow0 + wg_p0;
   const float* vn_base = vnrow0 + wg_p0;
   // dead: the mask excludes every row of the step (uniform over the wave): its packed rows are all fetched from the first piece
-  auto issue = [&](int s, bool dead, u4 (&kq)[kLoads], u4 (&vq)[kLoads], float& kn, float& vn) {
+  auto issue = [&](int s, bool dead, KQ (&kq)[4], u4 (&vq)[kLoads], float& kn, float& vn) {
     const uint32_t row0 = (uint32_t)(s * kSStepPos + wave * kWavePos);   // first row of the wave's block, from wg_p0
     const int n_rows = rows_left_of(s);
     const int rows = dead ? 0 : n_rows;
     // offset of the last piece that holds a valid byte (pieces past it are fetched from there), first byte of the block
-    const uint32_t klast = rows ? ((uint32_t)(kmis + rows * (kPd * 4) - 1) & ~15u) : 0u;
+    const uint32_t kend = rows ? (uint32_t)rows - 1 : 0u;                 // keys past the last row: from there
     const uint32_t vlast = rows ? ((uint32_t)(vmis + rows * (kPd * 4) - 1) & ~15u) : 0u;
     const uint32_t blk = rows ? row0 * (kPd * 4) : 0u;
 #pragma unroll
+    for (int t = 0; t < 4; ++t) kq[t].load(k_base, blk + min((uint32_t)(16 * t + n16), kend) * (kPd * 4), g);
+#pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const uint32_t off = (uint32_t)(i * 64 + lane) * 16;
-      kq[i] = load_stream(k_base + (blk + min(off, klast)));
       vq[i] = load_stream(v_base + (blk + min(off, vlast)));
     }
     const uint32_t nrow = (lane < n_rows) ? row0 + lane : 0u;
@@ -763,7 +812,8 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
       my_q[i] = (w < n_rep * (kD / 2)) ? reinterpret_cast<const float2*>(a.q_rot + q_row0 * kD)[w] : make_float2(0.f, 0.f);
     }
   }
-  u4 kqA[kLoads], vqA[kLoads], kqB[kLoads], vqB[kLoads];
+  KQ kqA[4], kqB[4];                                              // the lane's quarters of rows 16 t + n16
+  u4 vqA[kLoads], vqB[kLoads];
   float knA, vnA, knB = 0.0f, vnB = 0.0f;
   issue(0, false, kqA, vqA, knA, vnA);
 
@@ -778,8 +828,8 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     for (int i = 0; i < 4; ++i) {
       const __half2 h = __floats2half2_rn(my_q[i].x, my_q[i].y);
       const float2 back = __half22float2(h);
-      (&q_s[0][0])[tid + i * kSThreads] = *reinterpret_cast<const uint32_t*>(&h);
-      (&ql_s[0][0])[tid + i * kSThreads] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
+      (&q_s[0][0])[q_word(tid + i * kSThreads)] = *reinterpret_cast<const uint32_t*>(&h);
+      (&ql_s[0][0])[q_word(tid + i * kSThreads)] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
     }
   }
   __syncthreads();
@@ -791,15 +841,14 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   u4 qreg[4], qlow[4];
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
-    qreg[kb] = *reinterpret_cast<const u4*>(&q_s[n16][(4 * kb + g) * 4]);
-    qlow[kb] = *reinterpret_cast<const u4*>(&ql_s[n16][(4 * kb + g) * 4]);
-  }
-  unsigned char* image = big_s + wave * (2 * kSImageBytes);
-  const uint32_t* kimg = reinterpret_cast<const uint32_t*>(image + kmis);
-  const uint32_t* vimg = reinterpret_cast<const uint32_t*>(image + kSImageBytes + vmis);
-  int kw0[4], ksl[4], ksh[4];
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) VF::pos(4 * kb + g, kw0[kb], ksl[kb], ksh[kb]);
+    for (int jp = 0; jp < 4; ++jp) {
+      qreg[kb][jp] = q_s[n16][KQ::pair(kb, jp, g)];
+      qlow[kb][jp] = ql_s[n16][KQ::pair(kb, jp, g)];
+    }
+  }
+  unsigned char* image = big_s + wave * kSImageBytes;
+  const uint32_t* vimg = reinterpret_cast<const uint32_t*>(image + vmis);
   int vw0, vsl, vsh;
   VF::pos(n16, vw0, vsl, vsh);
   const float kscale = a.score_scale * kLog2e;           // scores in log2 units
@@ -810,7 +859,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   float m_run = -INFINITY, R_run = -INFINITY, l_run = 0.0f, inv_tscale = 1.0f;
 
   // one step on the buffers (kq, vq, kn, vn); `next()` issues the loads of the following step
-  auto step = [&](int sidx, u4 (&kq)[kLoads], u4 (&vq)[kLoads], float kn, float vn_, float mk, auto&& next) {
+  auto step = [&](int sidx, KQ (&kq)[4], u4 (&vq)[kLoads], float kn, float vn_, float mk, auto&& next) {
     const int rows = rows_left_of(sidx);                 // uniform over the wave, at least 1 (the caller checks)
     // ---- the request for the next step's rows goes out first (the other buffer is free): what separates the arrival
     // of one step's rows from the request for the next is on the critical path of a loop that a memory round trip bounds
@@ -821,11 +870,10 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     if (MASKED && __all(mk == -INFINITY && __builtin_fabsf(kn) < INFINITY && __builtin_fabsf(vn_) < INFINITY)) return;
     // ---- images and norms into the wave's LDS area
     {
-      u4* k4 = reinterpret_cast<u4*>(image);
-      u4* v4 = reinterpret_cast<u4*>(image + kSImageBytes);
+      u4* v4 = reinterpret_cast<u4*>(image);
 #pragma unroll
-      for (int i = 0; i < kWhole; ++i) { k4[i * 64 + lane] = kq[i]; v4[i * 64 + lane] = vq[i]; }
-      if (kRest) { if (lane < kRest) { k4[kWhole * 64 + lane] = kq[kLoads - 1]; v4[kWhole * 64 + lane] = vq[kLoads - 1]; } }
+      for (int i = 0; i < kWhole; ++i) v4[i * 64 + lane] = vq[i];
+      if (kRest) { if (lane < kRest) v4[kWhole * 64 + lane] = vq[kLoads - 1]; }
       kn_s[wave][lane] = kn * kscale;
       vn_s[wave][lane] = vn_;
       if (MASKED) mk_s[wave][lane] = mk;
@@ -835,11 +883,9 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
-      const uint32_t* krow = kimg + (16 * t + n16) * kPd;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
-        const uint32_t f = VF::field_raw(krow + kw0[kb], ksl[kb], ksh[kb]);
-        const u4 ka = key_operand<BITS, KQUAD>(f, quad_s, lutk_s);
+        const u4 ka = key_operand<BITS, KQUAD>(kq[t].field(kb, g), quad_s, lutk_s);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, qreg[kb]),
                                                      acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, qlow[kb]),
@@ -947,8 +993,8 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   l *= inv_tscale;
   float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
   float* pml = a.ws_ml + part * (int64_t)(n_rep * 2);
-  static_assert(2 * kSImageBytes >= 8 * kD * 4 && (2 * kSImageBytes) % 16 == 0, "a wave's image area holds its eight deposit rows");
-  merge_waves<kSWaves>(mg_s, big_s, 2 * kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml, tid);
+  static_assert(kSImageBytes >= 8 * kD * 4 && kSImageBytes % 16 == 0, "a wave's image area holds its eight deposit rows");
+  merge_waves<kSWaves>(mg_s, big_s, kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml, tid);
   };
 
   const PackedArgs& a = args;
@@ -1019,8 +1065,8 @@ void packed_stream_scores_kernel(PackedArgs a, Codebook kcb, int n_steps) {
   __shared__ uint32_t lutk_s[VF::kLut < 64 ? 64 : VF::kLut];
   __shared__ __align__(16) uint2 quad_s[KQUAD ? VF::kQuadEntries : 1];
   // the rotated query (fp16 value and remainder, 8 KB) is staged in the image area: it is in registers before any image is written
-  uint32_t (*q_s)[kD / 2] = reinterpret_cast<uint32_t (*)[kD / 2]>(big_s);
-  uint32_t (*ql_s)[kD / 2] = reinterpret_cast<uint32_t (*)[kD / 2]>(big_s + kHeadsMax * (kD / 2) * 4);
+  uint32_t (*q_s)[kQPitch] = reinterpret_cast<uint32_t (*)[kQPitch]>(big_s);
+  uint32_t (*ql_s)[kQPitch] = reinterpret_cast<uint32_t (*)[kQPitch]>(big_s + kHeadsMax * kQPitch * 4);
   __shared__ __align__(16) float kn_s[kSWaves][kWavePos];
   __shared__ float m_s[kSWaves][kHeadsMax], l_s[kSWaves][kHeadsMax];
 
@@ -1085,8 +1131,8 @@ void packed_stream_scores_kernel(PackedArgs a, Codebook kcb, int n_steps) {
     for (int i = 0; i < 4; ++i) {
       const __half2 h = __floats2half2_rn(my_q[i].x, my_q[i].y);
       const float2 back = __half22float2(h);
-      (&q_s[0][0])[tid + i * kSThreads] = *reinterpret_cast<const uint32_t*>(&h);
-      (&ql_s[0][0])[tid + i * kSThreads] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
+      (&q_s[0][0])[q_word(tid + i * kSThreads)] = *reinterpret_cast<const uint32_t*>(&h);
+      (&ql_s[0][0])[q_word(tid + i * kSThreads)] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
     }
   }
   __syncthreads();

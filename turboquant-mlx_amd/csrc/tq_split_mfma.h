@@ -87,8 +87,8 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
   constexpr bool SOFT_S = MODE == kSoftScores, SOFT_W = MODE == kSoftWeights;
   __shared__ __align__(16) unsigned char big_s[32768];      // per-wave 4 KB areas, later the merge deposits
   __shared__ __align__(16) uint2 lut_s[VF::kLut < 64 ? 64 : VF::kLut];
-  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kD / 2];
-  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kD / 2];
+  __shared__ __align__(16) uint32_t q_s[kHeadsMax][kQPitch];
+  __shared__ __align__(16) uint32_t ql_s[kHeadsMax][kQPitch];
   __shared__ __align__(16) float n_s[kWaves][kWavePos];
   __shared__ __align__(16) MergeLds<kWaves> mg_s;
   __shared__ float m_s[kWaves][kHeadsMax], l_s[kWaves][kHeadsMax];
@@ -184,8 +184,8 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
     for (int i = 0; i < 2; ++i) {
       const __half2 h = __floats2half2_rn(my_q[i].x, my_q[i].y);
       const float2 back = __half22float2(h);
-      (&q_s[0][0])[tid + i * kMfmaThreads] = *reinterpret_cast<const uint32_t*>(&h);
-      (&ql_s[0][0])[tid + i * kMfmaThreads] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
+      (&q_s[0][0])[q_word(tid + i * kMfmaThreads)] = *reinterpret_cast<const uint32_t*>(&h);
+      (&ql_s[0][0])[q_word(tid + i * kMfmaThreads)] = pack_h2(my_q[i].x - back.x, my_q[i].y - back.y);
     }
   }
   n_s[wave][lane] = SCORES ? my_n * (a.scale * kSplitTableUnscale) : my_n;
