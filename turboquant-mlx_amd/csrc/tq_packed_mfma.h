@@ -689,6 +689,66 @@ struct KeyQuarter {
   }
 };
 
+// Scores of four 16-position tiles in the lanes of 16 / F query heads.  A score product leaves head n16 in lanes n16 + 16 g, position
+// 4 g + j of the tile in register j, and with few heads most lanes hold nothing: the arithmetic on the scores would run F times
+// for one use.  So the tiles F u .. F u + F - 1 share a register group, tile F u + f in lanes n16 = 16 f / F + head (one lane shift
+// within the rows of 16 per register in, half of one per register of weights out).  What lanes past the heads hold afterwards is
+// other tiles' numbers: rows of the value products that nothing reads.
+// Four heads: 75 -> 69 us for sixteen ragged sequences (64 instead of 180 vector operations on the scores of a step); with uniform block bounds and
+// offsets that never change in the requests of whole blocks 67 - 68.
+template <int F>
+struct HeadLanes {
+  static constexpr int kGroups = 4 / F, kStep = 16 / F;
+  typedef f4 Group;
+  // first position of group u in a lane
+  __device__ static __forceinline__ int row(int u, int n16, int g) { return 16 * (F * u + n16 / kStep) + 4 * g; }
+  template <int BY>
+  __device__ static __forceinline__ float into(float old, float x) {      // lanes BY .. BY + kStep - 1 of a row of 16: x of the lanes 0 .. kStep - 1
+    constexpr int kBanks = (kStep == 4 ? 0x1 : kStep == 8 ? 0x3 : 0xF) << (BY / 4);
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), 0x110 + BY, 0xF, kBanks, false));
+  }
+  __device__ static __forceinline__ void put(Group (&s)[kGroups], int t, const f4& acc) {
+    const int u = t / F, f = t % F;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (f == 0) s[u][j] = acc[j];
+      else if constexpr (F == 2) s[u][j] = into<8>(s[u][j], acc[j]);
+      else if constexpr (F == 4) s[u][j] = f == 1 ? into<4>(s[u][j], acc[j]) : f == 2 ? into<8>(s[u][j], acc[j]) : into<12>(s[u][j], acc[j]);
+    }
+  }
+  template <int BY>
+  __device__ static __forceinline__ uint32_t from(uint32_t x) {           // lanes 0 .. kStep - 1: x of the lanes BY further
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x100 + BY, 0xF, 0xF, true);
+  }
+  __device__ static __forceinline__ uint32_t take(uint32_t x, int f) {
+    if (f == 0) return x;
+    if constexpr (F == 2) return from<8>(x);
+    else if constexpr (F == 4) return f == 1 ? from<4>(x) : f == 2 ? from<8>(x) : from<12>(x);
+    return x;
+  }
+  template <int BY>
+  __device__ static __forceinline__ float ror(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x120 + BY, 0xF, 0xF, true));
+  }
+  __device__ static __forceinline__ float max_over_tiles(float x) {
+    if constexpr (F >= 2) x = fmaxf(x, ror<8>(x));
+    if constexpr (F >= 4) x = fmaxf(x, ror<4>(x));
+    return x;
+  }
+  __device__ static __forceinline__ float sum_over_tiles(float x) {
+    if constexpr (F >= 2) x += ror<8>(x);
+    if constexpr (F >= 4) x += ror<4>(x);
+    return x;
+  }
+};
+// Tiles that share registers at n_rep query heads per kv head.
+inline int tiles_per_group(int n_rep) { return n_rep <= 4 ? 4 : n_rep <= 8 ? 2 : 1; }
+
+// a value that every lane holds alike, as one
+__device__ __forceinline__ int64_t uniform64(int64_t x) {
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
+}
+
 // The arguments in the kernel's argument segment, and which of the two a form reads.
 typedef const __attribute__((address_space(4))) PackedArgs ConstArgs;
 template <bool AGAIN>
@@ -697,11 +757,12 @@ __device__ __forceinline__ auto& args_of(const PackedArgs& args, ConstArgs* agai
   else return args;
 }
 
-template <int BITS, bool VQ = true, bool MASKED = false, bool SPREAD = false>
+template <int BITS, bool VQ = true, bool MASKED = false, bool SPREAD = false, int F = 1>
 __global__ __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_steps) {
   using VF = VField<BITS>;
   using KQ = KeyQuarter<BITS>;
+  using Lanes = HeadLanes<F>;
   // A workgroup decodes up to 8 x 256 positions, which repays building the quad table (one for keys and values when
   // their codebooks are equal, VQ; else the values use their pair table).
   constexpr bool KQUAD = VF::kQuad, VQUAD = VF::kQuad && VQ;
@@ -743,6 +804,8 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     const int64_t want = *a.len_dev + a.len_bias;
     len = want < 0 ? 0 : (want < len ? want : len);
   }
+  first = uniform64(first);
+  len = uniform64(len);
   if (wg_p0 >= len) return;
 
   // ---- addresses: row 0 of the sequence for this kv head, misalignment of the wave's blocks
@@ -755,28 +818,39 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   const float* knrow0 = a.k_norms + (int64_t)seq * a.kn_seq_stride + (int64_t)kvh * a.kn_head_stride + first;
   const float* vnrow0 = a.v_norms + (int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first;
 
-  auto rows_left_of = [&](int s) {
-    const int64_t p0w = wg_p0 + (int64_t)s * kSStepPos + wave * kWavePos;
-    const int64_t left = s < n_steps ? len - p0w : 0;      // steps past the workgroup's last have no rows
-    return (int)(left < 0 ? 0 : (left > kWavePos ? kWavePos : left));
-  };
+  // rows of the wave's blocks from its first one on, steps past the workgroup's last without any (uniform like all that follows from it)
+  const int wave_rows = (int)min(len - wg_p0, (int64_t)n_steps * kSStepPos) - wave * kWavePos;
+  auto rows_left_of = [&](int s) { return min(max(wave_rows - s * kSStepPos, 0), kWavePos); };
   // Requests the rows of step s.  Every call issues the same loads whatever s is: a piece past the end of the sequence
   // is fetched from the last piece of the block that holds a valid byte, a norm past the end (and everything of a step
   // past the workgroup's last) from the first piece / row of the workgroup's range, which exists, so that no branch
   // surrounds a load -- the compiler can then count the requests in flight and wait for one buffer's rows while the
   // other buffer's are still on their way.  What comes back for a row that does not exist is real data of another row:
   // finite, and its score is set to -inf.
-  // Addresses are a base that is the same for the whole workgroup (its first piece / first norm) plus a 32-bit
-  // offset per lane: one register per load instead of a 64-bit pointer.
+  // Addresses are a base that is the same for the wavefront plus a 32-bit offset per lane, which for a whole block (all but a
+  // sequence's last) never changes: its loads take no vector instruction at all.
   const char* k_base = krow0 + wg_p0 * (kPd * 4);
   const char* v_base = vrow0 + wg_p0 * (kPd * 4) - vmis;
   const float* kn_base = knrow0 + wg_p0;
   const float* vn_base = vnrow0 + wg_p0;
+  // of the lane's last piece: from piece 64 kWhole on, those past the block's last from there
+  const uint32_t last_piece = min((uint32_t)lane * 16, ((uint32_t)(vmis + kWavePos * (kPd * 4) - 1) & ~15u) - kWhole * 1024);
   // dead: the mask excludes every row of the step (uniform over the wave): its packed rows are all fetched from the first piece
   auto issue = [&](int s, bool dead, KQ (&kq)[4], u4 (&vq)[kLoads], float& kn, float& vn) {
     const uint32_t row0 = (uint32_t)(s * kSStepPos + wave * kWavePos);   // first row of the wave's block, from wg_p0
     const int n_rows = rows_left_of(s);
     const int rows = dead ? 0 : n_rows;
+    if (rows == kWavePos) {
+      const char* kblk = k_base + (int64_t)row0 * (kPd * 4);
+      const char* vblk = v_base + (int64_t)row0 * (kPd * 4);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) kq[t].load(kblk + 16 * t * (kPd * 4), n16 * (kPd * 4), g);
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) vq[i] = load_stream(vblk + i * 1024 + (i < kWhole ? lane * 16 : last_piece));
+      kn = load_stream(kn_base + row0 + lane);
+      vn = load_stream(vn_base + row0 + lane);
+      return;
+    }
     // offset of the last piece that holds a valid byte (pieces past it are fetched from there), first byte of the block
     const uint32_t kend = rows ? (uint32_t)rows - 1 : 0u;                 // keys past the last row: from there
     const uint32_t vlast = rows ? ((uint32_t)(vmis + rows * (kPd * 4) - 1) & ~15u) : 0u;
@@ -879,7 +953,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
       if (MASKED) mk_s[wave][lane] = mk;
     }
     // ---- scores of the 64 rows (log2 units)
-    float s[4][4];
+    typename Lanes::Group s[Lanes::kGroups];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -891,33 +965,33 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, qlow[kb]),
                                                      acc, 0, 0, 0);
       }
-      const float4 kn4 = *reinterpret_cast<const float4*>(&kn_s[wave][16 * t + 4 * g]);
-      const float knv[4] = {kn4.x, kn4.y, kn4.z, kn4.w};
+      Lanes::put(s, t, acc);
+    }
+    const int row0 = Lanes::row(0, n16, g);               // the lane's first position; its others are 16 F u + j further
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[t][j] = acc[j] * knv[j];
+    for (int u = 0; u < Lanes::kGroups; ++u) {
+      s[u] *= *reinterpret_cast<const f4*>(&kn_s[wave][16 * F * u + row0]);
       if (MASKED) {
-        const float4 mk4 = *reinterpret_cast<const float4*>(&mk_s[wave][16 * t + 4 * g]);
-        const float mkv[4] = {mk4.x, mk4.y, mk4.z, mk4.w};
+        const f4 mk4 = *reinterpret_cast<const f4*>(&mk_s[wave][16 * F * u + row0]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s[t][j] = __builtin_fmaf(mkv[j], kLog2e, s[t][j]);
+        for (int j = 0; j < 4; ++j) s[u][j] = __builtin_fmaf(mk4[j], kLog2e, s[u][j]);
       }
     }
     if (rows < kWavePos) {                                 // only a sequence's last block has rows to mask
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int u = 0; u < Lanes::kGroups; ++u)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s[t][j] = (16 * t + 4 * g + j < rows) ? s[t][j] : -INFINITY;
+        for (int j = 0; j < 4; ++j) s[u][j] = (16 * F * u + row0 + j < rows) ? s[u][j] : -INFINITY;
     }
     // ---- value norms, their power-of-two scale
-    float vn[4][4];
+    f4 vn[Lanes::kGroups];
     float nmax = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float4 n4 = *reinterpret_cast<const float4*>(&vn_s[wave][16 * t + 4 * g]);
-      vn[t][0] = n4.x; vn[t][1] = n4.y; vn[t][2] = n4.z; vn[t][3] = n4.w;
-      nmax = fmaxf(nmax, fmaxf(fmaxf(n4.x, n4.y), fmaxf(n4.z, n4.w)));
+    for (int u = 0; u < Lanes::kGroups; ++u) {
+      vn[u] = *reinterpret_cast<const f4*>(&vn_s[wave][16 * F * u + row0]);
+      nmax = fmaxf(nmax, fmaxf(fmaxf(vn[u][0], vn[u][1]), fmaxf(vn[u][2], vn[u][3])));
     }
-    nmax = max_over_rows(nmax);
+    nmax = max_over_rows(Lanes::max_over_tiles(nmax));
     int ex = (int)((__float_as_uint(nmax) >> 23) & 0xFF);
     ex = ex < 27 ? (ex < 1 ? 127 : 27) : (ex > 227 ? 227 : ex);
     const float kexp = (float)(127 - ex);
@@ -925,10 +999,10 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     // ---- online softmax: rows >= 1, so the maximum of the step is finite unless a mask excludes them
     float mb = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int u = 0; u < Lanes::kGroups; ++u)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) mb = fmaxf(mb, s[t][j]);
-    mb = max_over_rows(mb);
+      for (int j = 0; j < 4; ++j) mb = fmaxf(mb, s[u][j]);
+    mb = max_over_rows(Lanes::max_over_tiles(mb));
     const float m_new = fmaxf(m_run, mb);
     const float R_new = (MASKED && m_new == -INFINITY ? 0.0f : m_new) - kexp;
     const float factor = __builtin_amdgcn_exp2f(R_run - R_new);      // 0 on the wave's first step
@@ -937,16 +1011,21 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     float lsum = 0.0f;
     uint32_t pa[2][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int u = 0; u < Lanes::kGroups; ++u) {
       float p[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        p[j] = __builtin_amdgcn_exp2f(s[t][j] - R_new);              // weight * 2^kexp
+        p[j] = __builtin_amdgcn_exp2f(s[u][j] - R_new);              // weight * 2^kexp
         lsum += p[j];
-        p[j] *= vn[t][j];
+        p[j] *= vn[u][j];
       }
-      pa[t >> 1][2 * (t & 1)] = pack_h2(p[0], p[1]);
-      pa[t >> 1][2 * (t & 1) + 1] = pack_h2(p[2], p[3]);
+      const uint32_t lo = pack_h2(p[0], p[1]), hi = pack_h2(p[2], p[3]);
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        const int t = F * u + f;
+        pa[t >> 1][2 * (t & 1)] = Lanes::take(lo, f);
+        pa[t >> 1][2 * (t & 1) + 1] = Lanes::take(hi, f);
+      }
     }
     l_run = l_run * factor + lsum;
     if (sidx > 0 && __any(factor != 1.0f)) {               // accumulator rows are heads 4g + j: factors through LDS
@@ -990,6 +1069,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   float l = l_run;
   l += shfl_xor_f(l, 16);
   l += shfl_xor_f(l, 32);
+  l = Lanes::sum_over_tiles(l);
   l *= inv_tscale;
   float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
   float* pml = a.ws_ml + part * (int64_t)(n_rep * 2);
@@ -1014,6 +1094,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     };
     int total = 0;
     for (int s0 = 0; s0 < a.n_seq; s0 += 64) total += wave_total(steps_of(s0 + lane));
+    total = __builtin_amdgcn_readfirstlane(total);
     const int per = max(2, (total + (int)gridDim.x - 1) / (int)gridDim.x);
     int at = wg * per, seq = 0, base = 0;
     const int end = min(total, at + per);
@@ -1034,7 +1115,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     }
     seq = __builtin_amdgcn_readfirstlane(seq);
     while (at < end) {
-      const int have = steps_of(seq), n = min(end, base + have) - at;
+      const int have = __builtin_amdgcn_readfirstlane(steps_of(seq)), n = min(end, base + have) - at;
       if (n > 0) {
         run(seq, (int64_t)(at - base) * kSStepPos, n, (int64_t)kvh * a.n_tiles_max + wg + seq);
         __syncthreads();                                                 // the merge has read what the next range overwrites
@@ -1516,25 +1597,23 @@ void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, co
 template <int BITS>
 void launch_packed_stream(dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb, int n_steps,
                           hipStream_t stream) {
-  if (a.parts) {
-    if constexpr (VField<BITS>::kQuad) {
-      if (std::memcmp(kcb.c, vcb.c, sizeof(kcb.c)) != 0) {
-        packed_stream_kernel<BITS, false, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);
-        return;
-      }
-    }
-    packed_stream_kernel<BITS, true, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);
-    return;
-  }
+#define TQ_STREAM(VQ_, F_)                                                                                             \
+  do {                                                                                                                 \
+    if (a.parts) packed_stream_kernel<BITS, VQ_, false, true, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);     \
+    else if (a.mask) packed_stream_kernel<BITS, VQ_, true, false, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps); \
+    else packed_stream_kernel<BITS, VQ_, false, false, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);      \
+  } while (0)
+  const int f = tiles_per_group(a.n_rep);
   if constexpr (VField<BITS>::kQuad) {
-    if (std::memcmp(kcb.c, vcb.c, sizeof(kcb.c)) != 0) {
-      if (a.mask) packed_stream_kernel<BITS, false, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);
-      else packed_stream_kernel<BITS, false><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);
+    if (std::memcmp(kcb.c, vcb.c, sizeof(kcb.c)) != 0) {                 // codebooks of their own are rare: one form for every n_rep
+      TQ_STREAM(false, 1);
       return;
     }
   }
-  if (a.mask) packed_stream_kernel<BITS, true, true><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);
-  else packed_stream_kernel<BITS><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);
+  if (f == 4) TQ_STREAM(true, 4);
+  else if (f == 2) TQ_STREAM(true, 2);
+  else TQ_STREAM(true, 1);
+#undef TQ_STREAM
 }
 
 template <int BITS>
