@@ -181,6 +181,10 @@ int tq_fill_rows(const tq_fill_segment* segments, int n_segments, tq_stream_t st
 #define TQ_SIGNS_MAX_SEEDS 4
 int tq_random_signs(const uint64_t* seeds /* HOST */, int n_seeds, int dim, float* signs, tq_stream_t stream);
 
+/* tq_fill_rows and tq_random_signs in one launch: all that a new cache needs before its first rows. */
+int tq_setup_rows(const tq_fill_segment* segments, int n_segments, const uint64_t* seeds /* HOST */, int n_seeds, int dim,
+                  float* signs, tq_stream_t stream);
+
 /*
  * Index rows to packed words and back (reference turboquant_mlx/packing.py:26-56 and 59-87): rows of dim indices,
  * integers of index_bytes = 1, 4 or 8 bytes, to rows of ceil(dim / vpw) words, and rows of words_per_row words to rows of

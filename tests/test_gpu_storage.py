@@ -43,6 +43,34 @@ def test_random_signs(tq, seeds, dim):
     assert got.tolist() == [sign_pattern(dim, s) for s in seeds]
 
 
+@pytest.mark.parametrize("seeds,dim,segments", [([42, 43], 128, 0), ([7], 64, 3), ([1, 2 ** 64 - 1, 3, 4], 257, 8), ([5, 6], 128, 11)])
+def test_signs_join_the_fill(tq, seeds, dim, segments):
+    """One launch for both; more segments than a launch takes; signs alone."""
+    from tqhip.rotation import sign_pattern
+    fill = tq.ops.StorageFill()
+    dst = [torch.full((2, 20 + i, 13), 5, dtype=torch.int32, device="cuda") for i in range(segments)]
+    for i, t in enumerate(dst):
+        fill.add(t, 13, i, 20 + i)
+    got = fill.signs(seeds, dim, torch.device("cuda"))
+    fill.run()
+    assert got.tolist() == [sign_pattern(dim, s) for s in seeds]
+    for i, t in enumerate(dst):
+        assert bool((t[:, :i] == 5).all()) and not t[:, i:].any()
+
+
+def test_an_insert_that_fails_leaves_no_sign_vectors_behind(tq, monkeypatch):
+    cache = tq.TurboQuantKVCache(bits=3)
+    k = torch.randn(1, 2, 30, 128, device="cuda")
+    monkeypatch.setattr(cache, "_fetch_buffers", lambda *a: (_ for _ in ()).throw(MemoryError()))
+    with pytest.raises(MemoryError):
+        cache.update_and_fetch(k, k)
+    assert cache._k_q is None and cache._v_q is None and cache.offset == 0 and cache.k_packed is None
+    monkeypatch.undo()
+    other = tq.TurboQuantKVCache(bits=3)
+    for got, want in zip(cache.update_and_fetch(k, k), other.update_and_fetch(k, k)):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dim,bits,rows,alloc,off", [(128, 3, 1, 256, 9), (128, 3, 48, 64, 16), (128, 4, 1001, 1024, 3),
                                                      (64, 2, 2001, 2048, 0), (256, 3, 700, 768, 1), (32, 1, 77, 80, 2)])
 def test_keys_and_values_in_one_launch(tq, dim, bits, rows, alloc, off):

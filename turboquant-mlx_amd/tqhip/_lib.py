@@ -79,6 +79,7 @@ PROTOTYPES = {
     "tq_encode_kv": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i, _fp, _l, _l, _l, _l, _i, _i, _i, _p]),
     "tq_dequant_kv": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _fp, _i, _l, _l, _l, _l, _l, _i, _i, _p]),
     "tq_fill_rows": (_i, [C.POINTER(FillSegment), _i, _p]),
+    "tq_setup_rows": (_i, [C.POINTER(FillSegment), _i, C.POINTER(C.c_uint64), _i, _i, _p, _p]),
     "tq_random_signs": (_i, [C.POINTER(C.c_uint64), _i, _i, _p, _p]),
     "tq_pack_indices": (_i, [_p, _i, _p, _l, _i, _i, _p]),
     "tq_unpack_indices": (_i, [_p, _p, _l, _i, _i, _i, _p]),

@@ -134,9 +134,10 @@ class TurboQuantKVCache:
                 return t.device
         return torch.device("cuda")
 
-    def _ensure_quantizer(self, k_dim, v_dim, device=None, in_order=True):
+    def _ensure_quantizer(self, k_dim, v_dim, device=None, in_order=True, fill=None):
         """in_order: what uses the sign vectors runs on the current stream (or waits for it), as the inserts do.  False
-        makes them with a blocking copy, for a restored cache that may be read from any stream at once."""
+        makes them with a blocking copy, for a restored cache that may be read from any stream at once.  fill: the sign
+        vectors join it, and the caller takes the quantizers back should it not run."""
         new_k, new_v = not self.v_only and self._k_q is None, self._v_q is None
         if not (new_k or new_v):
             return
@@ -148,7 +149,8 @@ class TurboQuantKVCache:
             ask.append((self.seed + 1, v_dim))
         made = {}
         if in_order and ask and self.sign_stream == "native" and device.type == "cuda" and len({d for _, d in ask}) == 1:
-            made = dict(zip((s for s, _ in ask), ops.random_signs([s for s, _ in ask], ask[0][1], device)))
+            seeds = [s for s, _ in ask]
+            made = dict(zip(seeds, (fill.signs if fill is not None else ops.random_signs)(seeds, ask[0][1], device).unbind(0)))
         tables = _tables(self.quant_bits)
         if new_k:
             self._k_q = _Quantizer(k_dim, self.quant_bits, self.seed, device, self._k_signs_given, self.sign_stream,
@@ -371,16 +373,21 @@ class TurboQuantKVCache:
         v_dim = values.shape[3]
         device = values.device
         self._dtype = keys.dtype
-        self._ensure_quantizer(k_dim, v_dim, device)
         prev = self.offset
         total = prev + S
         fill = ops.StorageFill()
-        new = self._grown_storage(B, H, _round_up(total, self.step), device, S, fill) if self._lacks_room(S) else {}
-        dtypes = [values.dtype] if self.v_only else [keys.dtype, values.dtype]
-        fresh = None if self.fused else self._fetch_buffers(B, H, prev, total, dtypes, device, fill)
-        made = {}
-        zeros = [self._zero_like(t, fill, made) for t in ((keys, values) if self.fused else (keys,) if self.v_only else ())]
-        fill.run()                                           # every allocation has succeeded: now the cache may change
+        held = self._k_q, self._v_q
+        try:
+            self._ensure_quantizer(k_dim, v_dim, device, fill=fill)
+            new = self._grown_storage(B, H, _round_up(total, self.step), device, S, fill) if self._lacks_room(S) else {}
+            dtypes = [values.dtype] if self.v_only else [keys.dtype, values.dtype]
+            fresh = None if self.fused else self._fetch_buffers(B, H, prev, total, dtypes, device, fill)
+            made = {}
+            zeros = [self._zero_like(t, fill, made) for t in ((keys, values) if self.fused else (keys,) if self.v_only else ())]
+            fill.run()                                       # every allocation has succeeded: now the cache may change
+        except BaseException:
+            self._k_q, self._v_q = held                      # their sign vectors may not have been made
+            raise
         self.__dict__.update(new)
         if made:
             self._zero_scalars.update(made)

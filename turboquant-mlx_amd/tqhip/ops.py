@@ -249,10 +249,16 @@ def dequant_kv_into(k_packed, k_norms, k_signs, k_out: torch.Tensor, v_packed, v
 
 class StorageFill:
     """Collects what fresh cache storage needs besides its new rows -- the prefix of the storage it replaces, zeros behind
-    the new rows -- and does it in one launch (tq_fill_rows).  Keeps the tensors alive until then."""
+    the new rows, the sign vectors of a new cache -- and does it in one launch (tq_setup_rows).  Keeps the tensors alive until then."""
 
     def __init__(self):
-        self._segments, self._keep = [], []
+        self._segments, self._keep, self._signs = [], [], None
+
+    def signs(self, seeds, dim: int, device) -> torch.Tensor:
+        """random_signs, made by run(): once, at most TQ_SIGNS_MAX_SEEDS seeds."""
+        out = torch.empty((len(seeds), dim), dtype=torch.float32, device=device)
+        self._signs = (_seed_array(seeds), len(seeds), dim, out)
+        return out
 
     def add(self, dst: torch.Tensor, inner: int, zero_from: int, zero_to: int, src: torch.Tensor | None = None, src_stride: int = 0,
             copy: int = 0, axis: int | None = None) -> None:
@@ -291,19 +297,28 @@ class StorageFill:
 
     def run(self) -> None:
         segs, self._segments = self._segments, []
-        for at in range(0, len(segs), _lib.FILL_MAX_SEGMENTS):
+        signs, self._signs = self._signs, None
+        for at in range(0, max(len(segs), 1 if signs else 0), _lib.FILL_MAX_SEGMENTS):
             part = segs[at:at + _lib.FILL_MAX_SEGMENTS]
             arr = (_lib.FillSegment * len(part))(*part)
-            _lib.check(_lib.load().tq_fill_rows(arr, len(part), _stream(self._keep[0][0])))
+            if signs:
+                seeds, n, dim, out = signs
+                _lib.check(_lib.load().tq_setup_rows(arr, len(part), seeds, n, dim, out.data_ptr(), _stream(out)))
+                signs = None
+            else:
+                _lib.check(_lib.load().tq_fill_rows(arr, len(part), _stream(self._keep[0][0])))
         self._keep = []
+
+
+def _seed_array(seeds):
+    return (C.c_uint64 * len(seeds))(*[s & 0xFFFFFFFFFFFFFFFF for s in seeds])
 
 
 def random_signs(seeds, dim: int, device) -> torch.Tensor:
     """(len(seeds), dim) float32 rows of +-1, row i = sign_pattern(dim, seeds[i]) of the rotation module, made on the GPU on
     the current stream (tq_random_signs)."""
     out = torch.empty((len(seeds), dim), dtype=torch.float32, device=device)
-    arr = (C.c_uint64 * len(seeds))(*[s & 0xFFFFFFFFFFFFFFFF for s in seeds])
-    _lib.check(_lib.load().tq_random_signs(arr, len(seeds), dim, out.data_ptr(), _stream(out)))
+    _lib.check(_lib.load().tq_random_signs(_seed_array(seeds), len(seeds), dim, out.data_ptr(), _stream(out)))
     return out
 
 
