@@ -31,6 +31,11 @@ def _mask_rows(mask, b: int, n_q: int, total: int):
     return m
 
 
+def _rows(queries):
+    """The one token of (B, n_heads, 1, dim) queries."""
+    return queries.squeeze(2)
+
+
 def _stored(cache, B):
     """Packed keys and values and their norms of the first B sequences of the cache (which may hold more)."""
     ts = (cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms)
@@ -66,7 +71,7 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
         od = queries.dtype if queries.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
         if (ops.vonly_sparse_supported(dim, bits, n_rep) or dim == 64) and total > 0 and dim == cache._v_dim:
             # one call: the kernels rotate the query themselves
-            out = ops.flash_from_query(queries[:, :, 0, :], kq.signs, cache.k_packed, cache.k_norms, cache.v_packed,
+            out = ops.flash_from_query(_rows(queries), kq.signs, cache.k_packed, cache.k_norms, cache.v_packed,
                                        cache.v_norms, kq.centroids, vq.centroids, vq.signs, dim, bits, attn_scale,
                                        n_rep=n_rep, seq_len=total, mask=m, out_dtype=od, sparse_v_threshold=thr)
         else:
@@ -74,7 +79,7 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
             out = ops.flash_decode(q_rot, cache.k_packed, cache.k_norms, cache.v_packed, cache.v_norms,
                                    kq.centroids, vq.centroids, vq.signs, dim, bits, attn_scale, n_rep=n_rep,
                                    seq_len=total, mask=m, out_dtype=od, sparse_v_threshold=thr)
-        out = out[:, :, None, :]
+        out = out.unsqueeze(2)
         return out if out.dtype == queries.dtype else out.to(queries.dtype)
 
     if v_buffer is None and B > 0 and total > 0 and dim == cache._v_dim and ops.vonly_sparse_supported(dim, bits, n_rep):
@@ -84,8 +89,8 @@ def turboquant_attention(queries: torch.Tensor, cache, attn_scale: float, mask=N
             m = ops.decode_mask_rows(mask, B, n_q, total, queries.device)
             if m is None:
                 m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
-        out = ops.composed_decode(queries[:, :, 0, :], kq.signs, *_stored(cache, B), kq.centroids, vq.centroids, vq.signs, dim,
-                                  bits, attn_scale, n_rep=n_rep, seq_len=total, mask=m, threshold=thr)[:, :, None, :]
+        out = ops.composed_decode(_rows(queries), kq.signs, *_stored(cache, B), kq.centroids, vq.centroids, vq.signs, dim,
+                                  bits, attn_scale, n_rep=n_rep, seq_len=total, mask=m, threshold=thr).unsqueeze(2)
         return out if out.dtype == queries.dtype else out.to(queries.dtype)
     outputs = []
     for b in range(B):
@@ -138,10 +143,9 @@ def vonly_decode_attention(queries: torch.Tensor, cache, attn_scale: float, mask
             if m is None:
                 m = torch.stack([_mask_rows(mask, b, n_q, total).expand(n_q, total) for b in range(B)])
         od = queries.dtype if queries.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
-        out = ops.vonly_decode(queries[:, :, 0, :], kc.keys, tq.v_packed, tq.v_norms, vq.centroids, vq.signs,
+        out = ops.vonly_decode(_rows(queries), kc.keys, tq.v_packed, tq.v_norms, vq.centroids, vq.signs,
                                dim, bits, attn_scale, n_rep=n_rep, seq_len=total, mask=m, out_dtype=od,
-                               sparse_v_threshold=thr)
-        out = out[:, :, None, :]                           # written in the query dtype by the merge pass
+                               sparse_v_threshold=thr).unsqueeze(2)   # written in the query dtype by the merge pass
         return out if out.dtype == queries.dtype else out.to(queries.dtype)
     outputs = []
     for b in range(B):

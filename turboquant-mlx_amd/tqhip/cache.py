@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import torch
 
-from . import ops
+from . import attention, ops
 from .kvcache import make_mask_for
 from .quantizer import gaussian_boundaries, gaussian_codebook
 from .rotation import random_diagonal_sign
@@ -45,8 +45,15 @@ class _Quantizer:
         self.centroids, self.boundaries = tables if tables is not None else _tables(bits)
 
 
+# The widths' tables, never handed out: a cache's are copies of its own (2 us, against 6 for making them)
+with torch.device("cpu"):
+    _TABLE_MASTERS = {bits: (c := gaussian_codebook(bits), gaussian_boundaries(c)) for bits in (1, 2, 3, 4)}
+
+
 def _tables(bits):
-    centroids = gaussian_codebook(bits)
+    if bits in _TABLE_MASTERS and torch._C._len_torch_function_stack() == 0 and torch._C._len_torch_dispatch_stack() == 0:
+        return tuple(t.clone() for t in _TABLE_MASTERS[bits])
+    centroids = gaussian_codebook(bits)                      # under a mode: whatever it makes of them (a default device, say)
     return centroids, gaussian_boundaries(centroids)
 
 
@@ -66,6 +73,10 @@ def _group_stride(t: torch.Tensor, inner: int) -> int:
     """Rows between consecutive (b, h) groups of a [B, H, T, inner] (or [B, H, T] with inner=1)
     tensor whose rows are dense and whose batch stride is H head strides -- true for the cache's
     own allocations and for time-slices of them."""
+    if t.is_contiguous():
+        shape = t.shape
+        if (len(shape) == 4 and shape[3] == inner) or (inner == 1 and len(shape) == 3):
+            return shape[2]
     if not _is_grouped(t, inner):
         raise ValueError("cache storage must be row-contiguous [B, H, T, *]; call .contiguous() first")
     return t.stride(1) // inner
@@ -323,7 +334,6 @@ class TurboQuantKVCache:
         insert position and the attended length from it when they run, so the step can be recorded in a HIP
         graph once and replayed while the caller advances the tensor; set `offset` afterwards.  `out`
         (B, n_heads, dim) receives the result when given."""
-        from . import attention
         B, n_q, S_q, dim = queries.shape
         H = values.shape[1]
         ok = (not self.v_only and S_q == 1 and values.shape[2] == 1 and keys.shape == values.shape

@@ -43,12 +43,16 @@ def _need_gpu(*tensors):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream(t: torch.Tensor):
-    """Raw hipStream_t of torch's current stream on the tensor's device."""
+def _stream_id(t: torch.Tensor) -> int:
+    """Raw hipStream_t of torch's current stream on the tensor's device, as the library and the workspaces take it."""
     if _raw_stream is not None:                       # avoids building a torch.cuda.Stream object per call
         idx = t.device.index
-        return C.c_void_p(_raw_stream(torch.cuda.current_device() if idx is None else idx))
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+        return _raw_stream(torch.cuda.current_device() if idx is None else idx)
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _stream(t: torch.Tensor):
+    return C.c_void_p(_stream_id(t))
 
 
 def _ptr(t):
@@ -270,7 +274,7 @@ class StorageFill:
             return
         if axis is None:
             axis = dst.dim() - (2 if inner > 1 else 1)
-        rows = dst.size(axis)
+        rows = dst.shape[axis]
         if dst.stride(axis) != inner or copy > rows or zero_to > rows:
             raise ValueError(f"rows of {inner} elements up to {max(copy, zero_to)} along axis {axis} of {tuple(dst.shape)}")
         if not dst.is_cuda:                                  # storage of a cache that has not met the GPU yet
@@ -345,8 +349,11 @@ def vonly_append_into(keys: torch.Tensor, values: torch.Tensor, signs: torch.Ten
         raise ValueError(f"keys {tuple(keys.shape)} and values {tuple(values.shape)} must have one shape")
     if k_f16.dtype != torch.float16 or not k_f16.is_contiguous():
         raise ValueError("k_f16 must be a contiguous float16 tensor")
-    for name, t in (("k_f16", k_f16), ("v_packed", v_packed), ("v_norms", v_norms)) + ((("v_raw", v_raw),) if v_raw is not None else ()):
-        if tuple(t.shape[:2]) != (B, H) or t.shape[2] < position + S:
+    for name, t in (("k_f16", k_f16), ("v_packed", v_packed), ("v_norms", v_norms), ("v_raw", v_raw)):
+        if t is None:
+            continue
+        b, h, rows = t.shape[:3]
+        if b != B or h != H or rows < position + S:
             raise ValueError(f"{name} {tuple(t.shape)} cannot hold positions {position}..{position + S} of {B} x {H} groups")
     if v_raw is not None and (v_raw.dtype != values.dtype or not v_raw.is_contiguous()):
         raise ValueError("v_raw must be contiguous and of the dtype of values")
@@ -365,12 +372,11 @@ def vonly_append_into(keys: torch.Tensor, values: torch.Tensor, signs: torch.Ten
             _ptr(pos_dev), _stream(values)))
         return
     _lib.check(lib.tq_vonly_append(
-        _ptr(keys), _dt(keys), _ptr(values), _dt(values), _ptr(signs), _host_table(boundaries),
-        C.c_void_p(k_f16.data_ptr() + position * D * 2),
-        None if v_raw is None else C.c_void_p(v_raw.data_ptr() + position * D * v_raw.element_size()),
-        C.c_void_p(v_packed.data_ptr() + position * pd * 4), C.c_void_p(v_norms.data_ptr() + position * 4),
+        keys.data_ptr(), _dt(keys), values.data_ptr(), _dt(values), signs.data_ptr(), _host_table(boundaries),
+        k_f16.data_ptr() + position * D * 2, None if v_raw is None else v_raw.data_ptr() + position * D * v_raw.element_size(),
+        v_packed.data_ptr() + position * pd * 4, v_norms.data_ptr() + position * 4,
         B * H, S, k_f16.shape[2], 0 if v_raw is None else v_raw.shape[2], v_packed.shape[2], v_norms.shape[2],
-        D, bits, var, _stream(values)))
+        D, bits, var, _stream_id(values)))
 
 
 def fused_quantize(vectors: torch.Tensor, signs: torch.Tensor, boundaries, dim: int, bits: int,
@@ -439,12 +445,10 @@ def dequant_into(packed: torch.Tensor, norms: torch.Tensor, centroids, signs: to
     pd = packed_dim(dim, bits)
     lib = _lib.load()
     _lib.check(lib.tq_dequant(
-        C.c_void_p(packed.data_ptr() + packed_row_offset * pd * 4),
-        C.c_void_p(norms.data_ptr() + norms_row_offset * 4),
-        _host_table(centroids), _ptr(signs),
-        C.c_void_p(out.data_ptr() + out_row_offset * dim * out.element_size()), _dt(out),
+        packed.data_ptr() + packed_row_offset * pd * 4, norms.data_ptr() + norms_row_offset * 4, _host_table(centroids),
+        signs.data_ptr(), out.data_ptr() + out_row_offset * dim * out.element_size(), _dt(out),
         n_groups, rows_per_group, packed_group_stride, norms_group_stride, out_group_stride,
-        dim, bits, _stream(out)))
+        dim, bits, _stream_id(out)))
 
 
 def _dequant(packed, norms, centroids, signs, dim, bits, dtype):
@@ -641,31 +645,22 @@ def count_active_positions(weights: torch.Tensor, threshold: float = 1e-5) -> in
 def _decode_shape(*, n_seq, n_kv, n_rep, dim, bits, block_size, seq_len, seq_offsets, k_strides, kn_strides,
                   v_strides, vn_strides, mask, mask_strides, attn_scale, out_dtype,
                   allow_mma: bool = True) -> DecodeShape:
-    sh = DecodeShape()
-    sh.n_seq, sh.n_kv_heads, sh.n_rep, sh.dim, sh.bits, sh.block_size = n_seq, n_kv, n_rep, dim, bits, block_size
-    sh.seq_len = seq_len
-    sh.seq_offsets = seq_offsets.data_ptr() if seq_offsets is not None else None
-    sh.k_seq_stride, sh.k_head_stride = k_strides
-    sh.kn_seq_stride, sh.kn_head_stride = kn_strides
-    sh.v_seq_stride, sh.v_head_stride = v_strides
-    sh.vn_seq_stride, sh.vn_head_stride = vn_strides
-    sh.mask = mask.data_ptr() if mask is not None else None
-    sh.mask_seq_stride, sh.mask_head_stride = mask_strides
-    sh.attn_scale = float(attn_scale)
-    sh.out_dtype = _DTYPES[out_dtype]
-    sh.allow_mma = 1 if allow_mma else 0
-    return sh
+    return DecodeShape(n_seq, n_kv, n_rep, dim, bits, block_size, seq_len,                 # the fields in their order
+                       seq_offsets.data_ptr() if seq_offsets is not None else None, *k_strides, *kn_strides, *v_strides, *vn_strides,
+                       mask.data_ptr() if mask is not None else None, *mask_strides, float(attn_scale), _DTYPES[out_dtype],
+                       1 if allow_mma else 0)
 
 
 def _check_rows(T: int, ragged: bool, n_seq: int, **tensors):
     """The kernels trust the attended length: refuse one that exceeds what the tensors hold (cache layout: rows
     per (sequence, head); ragged batch: the rows of all sequences together) before anything is launched."""
     for name, t in tensors.items():
-        rows = t.shape[-2] if name in ("k", "k_packed", "v_packed") else t.shape[-1]
+        shape, matrix = t.shape, name in ("k", "k_packed", "v_packed")
+        rows = shape[-2] if matrix else shape[-1]
         if T > rows:
             raise ValueError(f"attended length {T} exceeds the {rows} rows of {name}")
-        if not ragged and t.dim() >= 3 + (name in ("k", "k_packed", "v_packed")) and t.shape[0] != n_seq:
-            raise ValueError(f"{name} holds {t.shape[0]} sequences, the query {n_seq}")
+        if not ragged and len(shape) >= 3 + matrix and shape[0] != n_seq:
+            raise ValueError(f"{name} holds {shape[0]} sequences, the query {n_seq}")
 
 
 def _check_offsets(seq_offsets: torch.Tensor, n_seq: int, validate: bool, **tensors) -> None:
@@ -691,32 +686,36 @@ def _check_offsets(seq_offsets: torch.Tensor, n_seq: int, validate: bool, **tens
 def _kv_layout(t: torch.Tensor, inner: int, ragged: bool):
     """Strides in rows for KV addressing.  Accepts [H, T, inner] (one sequence or ragged batch) or
     [B, H, T, inner] (cache layout); the last two axes must be row-contiguous."""
-    if t.dim() == 3:
+    st = t.stride()
+    if len(st) == 3:
         t, hs = _head_layout_3d(t, inner)
         return t, (0, hs)
-    if t.dim() != 4:
+    if len(st) != 4:
         raise ValueError(f"expected a 3-D or 4-D KV tensor, got shape {tuple(t.shape)}")
-    if t.stride(3) != 1 or t.stride(2) != inner or t.stride(1) % inner or t.stride(0) % inner:
+    if st[3] != 1 or st[2] != inner or st[1] % inner or st[0] % inner:
         t = t.contiguous()
-    return t, (t.stride(0) // inner, t.stride(1) // inner)
+        st = t.stride()
+    return t, (st[0] // inner, st[1] // inner)
 
 
 def _norm_layout(t: torch.Tensor):
-    if t.dim() == 2:
+    st = t.stride()
+    if len(st) == 2:
         t, hs = _head_layout_2d(t)
         return t, (0, hs)
-    if t.dim() != 3:
+    if len(st) != 3:
         raise ValueError(f"expected a 2-D or 3-D norm tensor, got shape {tuple(t.shape)}")
-    if t.stride(2) != 1:
+    if st[2] != 1:
         t = t.contiguous()
-    return t, (t.stride(0), t.stride(1))
+        st = t.stride()
+    return t, st[:2]
 
 
 def _mask_layout(mask, n_seq: int, n_q: int, seq_len: int, device):
     """Additive float mask broadcastable to (n_seq, n_q, seq_len) -> (tensor, (seq_stride, head_stride))."""
     if mask is None:
         return None, (0, 0)
-    m = mask.to(device=device, dtype=torch.float32)
+    m = mask if mask.dtype == torch.float32 and mask.device == device else mask.to(device=device, dtype=torch.float32)
     while m.dim() < 3:
         m = m.unsqueeze(0)
     if m.shape[-1] != seq_len or m.shape[0] not in (1, n_seq) or m.shape[1] not in (1, n_q):
@@ -737,27 +736,32 @@ def decode_mask_rows(mask: torch.Tensor, n_seq: int, n_q: int, seq_len: int, dev
     (tq_mask_rows).  None for forms that need more than that (the caller builds the rows with tensor operations)."""
     if mask.device != device or mask.dtype not in _MASK_DTYPES or type(mask) is not torch.Tensor:
         return None
-    d = mask.dim()
+    shape, strides, d = mask.shape, mask.stride(), mask.dim()          # as (sequences, heads, positions), from the mask's first element
     if d == 4:
-        m = mask[:, :, 0, :]
+        (b, h, rows, t), (sb, sh, _, st) = shape, strides
+        if rows == 0:                                 # as indexing it
+            mask[:, :, 0, :]
     elif d == 3:
-        m = mask[:, 0:1, :]
-    elif d in (1, 2):
-        m = mask[None] if d == 2 else mask[None, None]
+        (b, h, t), (sb, sh, st) = shape, strides
+        h = min(h, 1)
+    elif d == 2:
+        (h, t), (sh, st) = shape, strides
+        b, sb = 1, h * sh
+    elif d == 1:
+        (t,), (st,) = shape, strides
+        b, h, sb, sh = 1, 1, t * st, t * st
     else:
         return None
-    b, h, t = m.shape
     if t != seq_len or t == 0 or h not in (1, n_q) or b == 0 or 1 < b < n_seq:
         return None
-    m = m[:n_seq]
-    b = m.shape[0]
-    if m.dtype == torch.float32 and m.stride(2) == 1:
-        return m
+    b = min(b, n_seq)
+    if mask.dtype == torch.float32 and st == 1:
+        return mask.as_strided((b, h, t), (sb, sh, st), mask.storage_offset())
     row_len = (t + 3) // 4 * 4                        # 16-byte rows: the kernels read four positions at a time
-    out = torch.empty((b, h, row_len), dtype=torch.float32, device=m.device)
-    sb, sh, st = m.stride()
-    _lib.check(_lib.load().tq_mask_rows(m.data_ptr(), _MASK_DTYPES[m.dtype], sb, sh, st, out.data_ptr(), b, h, t, row_len, _stream(m)))
-    return out[:, :, :t]
+    out = torch.empty((b, h, row_len), dtype=torch.float32, device=mask.device)
+    _lib.check(_lib.load().tq_mask_rows(mask.data_ptr(), _MASK_DTYPES[mask.dtype], sb, sh, st, out.data_ptr(), b, h, t, row_len,
+                                        _stream_id(mask)))
+    return out if row_len == t else out[:, :, :t]
 
 
 def flash_decode(q_rot: torch.Tensor, k_packed, k_norms, v_packed, v_norms, k_centroids, v_centroids,
@@ -894,20 +898,15 @@ def flash_from_query(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_no
                        vn_strides=vns, mask=mask, mask_strides=ms, attn_scale=attn_scale, out_dtype=out_dtype,
                        allow_mma=True)
     lib = _lib.load()
-    stream = _stream(q)
+    stream = _stream_id(q)
     thr = float(sparse_v_threshold) if sparse_v_threshold and sparse_v_threshold > 0.0 else 0.0
     need = (lib.tq_vonly_sparse_workspace_bytes(n_seq, n_q, T) if thr > 0.0
             else lib.tq_workspace_bytes(_lib.TQ_OP_FLASH_DECODE, n_seq, n_q, T, dim))
-    ws = _workspace(q.device, stream.value or 0, need)
-    if dim == 64:
-        _lib.check(lib.tq_flash_decode_from_q64(
-            _ptr(q), _dt(q), _ptr(k_signs), _ptr(k_packed), _ptr(k_norms), _ptr(v_packed), _ptr(v_norms),
-            _host_table(k_centroids), _host_table(v_centroids), _ptr(v_signs), _ptr(out), _ptr(ws), ws.numel(), C.byref(sh), stream))
-        return out
-    _lib.check(lib.tq_flash_decode_from_q(
-        _ptr(q), _dt(q), _ptr(k_signs), _ptr(k_packed), _ptr(k_norms), _ptr(v_packed), _ptr(v_norms),
-        _host_table(k_centroids), _host_table(v_centroids), _ptr(v_signs), thr, _ptr(out),
-        _ptr(ws), ws.numel(), C.byref(sh), stream))
+    ws = _workspace(q.device, stream, need)
+    head = (q.data_ptr(), _DTYPES[q.dtype], k_signs.data_ptr(), k_packed.data_ptr(), k_norms.data_ptr(), v_packed.data_ptr(),
+            v_norms.data_ptr(), _host_table(k_centroids), _host_table(v_centroids), v_signs.data_ptr())
+    tail = (out.data_ptr(), ws.data_ptr(), ws.numel(), C.byref(sh), stream)
+    _lib.check(lib.tq_flash_decode_from_q64(*head, *tail) if dim == 64 else lib.tq_flash_decode_from_q(*head, thr, *tail))
     return out
 
 
@@ -932,27 +931,27 @@ def composed_decode(q: torch.Tensor, k_signs, k_packed, k_norms, v_packed, v_nor
     q = q.contiguous()
     k_packed, ks = _kv_layout(_u32(k_packed), pd, False)
     v_packed, vs = _kv_layout(_u32(v_packed), pd, False)
-    k_norms, kns = _norm_layout(k_norms.to(torch.float32))
-    v_norms, vns = _norm_layout(v_norms.to(torch.float32))
+    k_norms, kns = _norm_layout(k_norms if k_norms.dtype == torch.float32 else k_norms.to(torch.float32))
+    v_norms, vns = _norm_layout(v_norms if v_norms.dtype == torch.float32 else v_norms.to(torch.float32))
     _check_rows(seq_len, False, n_seq, k_packed=k_packed, k_norms=k_norms, v_packed=v_packed, v_norms=v_norms)
     k_signs, v_signs = _as_f32_dev(k_signs, q), _as_f32_dev(v_signs, q)
     mask, ms = _mask_layout(mask, n_seq, n_q, seq_len, q.device)
     out = torch.empty((n_seq, n_q, dim), dtype=q.dtype, device=q.device)
     lib = _lib.load()
-    stream = _stream(q)
+    stream = _stream_id(q)
     per_call = max(1, min(n_seq, _COMPOSED_WORKSPACE // max(1, lib.tq_vonly_sparse_workspace_bytes(1, n_q, seq_len))))
     need = lib.tq_vonly_sparse_workspace_bytes(per_call, n_q, seq_len)
-    ws = _workspace(q.device, stream.value or 0, need) if need <= _COMPOSED_KEPT else torch.empty(need, dtype=torch.uint8, device=q.device)
+    ws = _workspace(q.device, stream, need) if need <= _COMPOSED_KEPT else torch.empty(need, dtype=torch.uint8, device=q.device)
     for first in range(0, n_seq, per_call):
         n = min(per_call, n_seq - first)
         sh = _decode_shape(n_seq=n, n_kv=n_q // n_rep, n_rep=n_rep, dim=dim, bits=bits, block_size=16, seq_len=seq_len,
                            seq_offsets=None, k_strides=ks, kn_strides=kns, v_strides=vs, vn_strides=vns,
                            mask=mask if mask is None or ms[0] == 0 else mask[first:], mask_strides=ms, attn_scale=attn_scale,
                            out_dtype=q.dtype)
+        qp, kp, kn, vp, vn, op = (t.data_ptr() + first * t.stride(0) * t.element_size() for t in (q, k_packed, k_norms, v_packed, v_norms, out))
         _lib.check(lib.tq_composed_decode(
-            q[first:].data_ptr(), _dt(q), k_signs.data_ptr(), k_packed[first:].data_ptr(), k_norms[first:].data_ptr(),
-            v_packed[first:].data_ptr(), v_norms[first:].data_ptr(), _host_table(k_centroids), _host_table(v_centroids),
-            v_signs.data_ptr(), threshold, out[first:].data_ptr(), ws.data_ptr(), ws.numel(), C.byref(sh), stream))
+            qp, _DTYPES[q.dtype], k_signs.data_ptr(), kp, kn, vp, vn, _host_table(k_centroids), _host_table(v_centroids),
+            v_signs.data_ptr(), threshold, op, ws.data_ptr(), ws.numel(), C.byref(sh), stream))
     return out
 
 
@@ -1036,29 +1035,26 @@ def vonly_decode(q: torch.Tensor, k: torch.Tensor, v_packed, v_norms, v_centroid
                        mask=mask, mask_strides=ms, attn_scale=attn_scale, out_dtype=out_dtype,
                        allow_mma=bool(_mma_flag(precision)))
     lib = _lib.load()
-    stream = _stream(q)
+    stream = _stream_id(q)
+    head = (q.data_ptr(), _DTYPES[q.dtype], k.data_ptr(), v_packed.data_ptr(), v_norms.data_ptr(), _host_table(v_centroids),
+            v_signs.data_ptr())
     if static_scratch:
         if sparse_v_threshold and sparse_v_threshold > 0.0:
             raise ValueError("static_scratch serves the dense step only (sparse_v_threshold = 0)")
-        _lib.check(lib.tq_vonly_decode_attn_static(
-            _ptr(q), _dt(q), _ptr(k), _ptr(v_packed), _ptr(v_norms), _host_table(v_centroids), _ptr(v_signs),
-            _ptr(out), C.byref(sh), stream))
+        _lib.check(lib.tq_vonly_decode_attn_static(*head, out.data_ptr(), C.byref(sh), stream))
         return out
     if sparse_v_threshold and sparse_v_threshold > 0.0:
         if not (vonly_threshold_supported(dim, bits, n_rep) and T > 0):
             raise ValueError("thresholded V-only decode needs dim 128, n_rep <= 16 and a non-empty cache; "
                              "compose dense_qk_scores, softmax_rows and sparse_v_matvec for other shapes")
         need = lib.tq_vonly_sparse_workspace_bytes(n_seq, n_q, T)
-        ws = _workspace(q.device, stream.value or 0, need)
-        _lib.check(lib.tq_vonly_sparse_decode_attn(
-            _ptr(q), _dt(q), _ptr(k), _ptr(v_packed), _ptr(v_norms), _host_table(v_centroids), _ptr(v_signs),
-            float(sparse_v_threshold), _ptr(out), _ptr(ws), ws.numel(), C.byref(sh), stream))
+        ws = _workspace(q.device, stream, need)
+        _lib.check(lib.tq_vonly_sparse_decode_attn(*head, float(sparse_v_threshold), out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                                   C.byref(sh), stream))
         return out
     need = lib.tq_workspace_bytes(_lib.TQ_OP_VONLY_DECODE, n_seq, n_q, T, dim)
-    ws = _workspace(q.device, stream.value or 0, need)
-    _lib.check(lib.tq_vonly_decode_attn(
-        _ptr(q), _dt(q), _ptr(k), _ptr(v_packed), _ptr(v_norms), _host_table(v_centroids), _ptr(v_signs),
-        _ptr(out), _ptr(ws), ws.numel(), C.byref(sh), stream))
+    ws = _workspace(q.device, stream, need)
+    _lib.check(lib.tq_vonly_decode_attn(*head, out.data_ptr(), ws.data_ptr(), ws.numel(), C.byref(sh), stream))
     return out
 
 
@@ -1169,12 +1165,12 @@ def step_call_unchecked(step, keys: torch.Tensor, values: torch.Tensor, q: torch
     """The library call of vonly_decode_step / packed_decode_step without their argument checks, for the cache
     objects, which have established shapes, dtypes and devices themselves: keys / values / q / out are contiguous
     and hold (B, heads, dim) elements in any view of that memory (a (B, heads, 1, dim) tensor qualifies)."""
-    stream = _stream(q)
-    _step_workspace(step, q.device, stream.value or 0)
+    stream = _stream_id(q)
+    _step_workspace(step, q.device, stream)
     lib = _lib.load()
     if isinstance(position, torch.Tensor):
         fn = lib.tq_packed_decode_step_at if packed else lib.tq_vonly_decode_step_at
-        pos = C.c_void_p(position.data_ptr())
+        pos = position.data_ptr()
     else:
         fn = lib.tq_packed_decode_step if packed else lib.tq_vonly_decode_step
         pos = position

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import torch
 
+from . import attention, ops
 from .cache import TurboQuantKVCache, _round_up
 from .kvcache import KVCache
 
@@ -66,7 +67,6 @@ class VOnlyTurboQuantCache:
     _FUSED_APPEND_MAX_TOKENS = 16
 
     def _append_fused(self, keys, values) -> bool:
-        from . import ops
         kc, tq = self._k_cache, self._v_tq
         B, H, S, v_dim = values.shape
         if (not 0 < S <= self._FUSED_APPEND_MAX_TOKENS or keys.shape != values.shape or not values.is_cuda
@@ -118,7 +118,6 @@ class VOnlyTurboQuantCache:
         once and replayed, the caller advancing the tensor by one after every step and calling `set_offset`
         when it is done replaying; `reserve` keeps the storage from moving meanwhile.  `out` (B, n_heads, dim)
         receives the result when given."""
-        from . import attention, ops
         kc, tq = self._k_cache, self._v_tq
         B, n_q, S_q, dim = queries.shape
         H = values.shape[1]
