@@ -217,6 +217,121 @@ __device__ __forceinline__ void value_products(const u4& A, const uint32_t (&VI)
   }
 }
 
+// What a lane needs of a packed key row as the A operand of four score products: the words of 32 elements, read from global memory
+// as they lie and cut up in registers.  Which elements meet in a product is free as long as the query's are chosen alike, so a
+// lane's are those of whole words: elements 32 g .. 32 g + 31, and at three bits, where a row is thirteen words of ten (the last
+// of eight), the three words 3 g .. 3 g + 2 and two elements of the last.
+template <int BITS>
+struct KeyQuarter {
+  static constexpr int kPd = VField<BITS>::kPd;
+  uint32_t w[BITS == 3 ? 4 : BITS];
+  __device__ __forceinline__ void load(const char* base, uint32_t row_bytes, int g) {
+    if constexpr (BITS == 3) {
+      typedef uint32_t u3 __attribute__((ext_vector_type(3), aligned(4)));
+      const u3 x = (*reinterpret_cast<const u3*>(base + (row_bytes + 12 * g)));
+      w[0] = x[0]; w[1] = x[1]; w[2] = x[2];
+      w[3] = *reinterpret_cast<const uint32_t*>(base + (row_bytes + 48));
+    } else if constexpr (BITS == 4) {
+      const u4 x = load_stream(base + (row_bytes + 16 * g));
+      w[0] = x[0]; w[1] = x[1]; w[2] = x[2]; w[3] = x[3];
+    } else if constexpr (BITS == 2) {
+      typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+      const u2 x = __builtin_nontemporal_load(reinterpret_cast<const u2*>(base + (row_bytes + 8 * g)));
+      w[0] = x[0]; w[1] = x[1];
+    } else {
+      w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + (row_bytes + 4 * g)));
+    }
+  }
+  // the same for rows at any 4-byte address
+  __device__ __forceinline__ void load_any(const char* base, uint32_t row_bytes, int g) {
+    if constexpr (BITS == 3) {
+      load(base, row_bytes, g);
+    } else {
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(base + (row_bytes + 4 * BITS * g));
+#pragma unroll
+      for (int i = 0; i < BITS; ++i) w[i] = src[i];
+    }
+  }
+  // the fields of the eight elements of product kb from bit 0 on; bits above them are garbage
+  __device__ __forceinline__ uint32_t field(int kb, int g) const {
+    if constexpr (BITS == 3) {
+      if (kb < 3) return w[kb];                                          // elements 0 .. 7 of a word; 8 and 9 of all make the fourth
+      return (w[0] >> 24) | ((w[1] >> 18) & 0xFC0u) | ((w[2] >> 12) & 0x3F000u) | ((w[3] >> (6 * g)) << 18);
+    } else if constexpr (BITS == 4) {
+      return w[kb];
+    } else if constexpr (BITS == 2) {
+      return w[kb >> 1] >> (16 * (kb & 1));
+    } else {
+      return w[0] >> (8 * kb);
+    }
+  }
+  // the pair of query elements (in units of two) that meets fields 2 jp and 2 jp + 1 of product kb
+  __device__ static __forceinline__ int pair(int kb, int jp, int g) {
+    if constexpr (BITS == 3) return kb < 3 ? 15 * g + 5 * kb + jp : jp < 3 ? 15 * g + 5 * jp + 4 : 60 + g;
+    else return 16 * g + 4 * kb + jp;
+  }
+};
+
+// Scores of four 16-position tiles in the lanes of 16 / F query heads.  A score product leaves head n16 in lanes n16 + 16 g, position
+// 4 g + j of the tile in register j, and with few heads most lanes hold nothing: the arithmetic on the scores would run F times
+// for one use.  So the tiles F u .. F u + F - 1 share a register group, tile F u + f in lanes n16 = 16 f / F + head (one lane shift
+// within the rows of 16 per register in, half of one per register of weights out).  What lanes past the heads hold afterwards is
+// other tiles' numbers: rows of the value products that nothing reads.
+// Four heads: 75 -> 69 us for sixteen ragged sequences (64 instead of 180 vector operations on the scores of a step); with uniform block bounds and
+// offsets that never change in the requests of whole blocks 67 - 68.
+template <int F>
+struct HeadLanes {
+  static constexpr int kGroups = 4 / F, kStep = 16 / F;
+  typedef f4 Group;
+  // first position of group u in a lane
+  __device__ static __forceinline__ int row(int u, int n16, int g) { return 16 * (F * u + n16 / kStep) + 4 * g; }
+  template <int BY>
+  __device__ static __forceinline__ float into(float old, float x) {      // lanes BY .. BY + kStep - 1 of a row of 16: x of the lanes 0 .. kStep - 1
+    constexpr int kBanks = (kStep == 4 ? 0x1 : kStep == 8 ? 0x3 : 0xF) << (BY / 4);
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), 0x110 + BY, 0xF, kBanks, false));
+  }
+  __device__ static __forceinline__ void put(Group (&s)[kGroups], int t, const f4& acc) {
+    const int u = t / F, f = t % F;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (f == 0) s[u][j] = acc[j];
+      else if constexpr (F == 2) s[u][j] = into<8>(s[u][j], acc[j]);
+      else if constexpr (F == 4) s[u][j] = f == 1 ? into<4>(s[u][j], acc[j]) : f == 2 ? into<8>(s[u][j], acc[j]) : into<12>(s[u][j], acc[j]);
+    }
+  }
+  template <int BY>
+  __device__ static __forceinline__ uint32_t from(uint32_t x) {           // lanes 0 .. kStep - 1: x of the lanes BY further
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x100 + BY, 0xF, 0xF, true);
+  }
+  __device__ static __forceinline__ uint32_t take(uint32_t x, int f) {
+    if (f == 0) return x;
+    if constexpr (F == 2) return from<8>(x);
+    else if constexpr (F == 4) return f == 1 ? from<4>(x) : f == 2 ? from<8>(x) : from<12>(x);
+    return x;
+  }
+  template <int BY>
+  __device__ static __forceinline__ float ror(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x120 + BY, 0xF, 0xF, true));
+  }
+  __device__ static __forceinline__ float max_over_tiles(float x) {
+    if constexpr (F >= 2) x = fmaxf(x, ror<8>(x));
+    if constexpr (F >= 4) x = fmaxf(x, ror<4>(x));
+    return x;
+  }
+  __device__ static __forceinline__ float sum_over_tiles(float x) {
+    if constexpr (F >= 2) x += ror<8>(x);
+    if constexpr (F >= 4) x += ror<4>(x);
+    return x;
+  }
+};
+// Tiles that share registers at n_rep query heads per kv head.
+inline int tiles_per_group(int n_rep) { return n_rep <= 4 ? 4 : n_rep <= 8 ? 2 : 1; }
+
+// a value that every lane holds alike, as one
+__device__ __forceinline__ int64_t uniform64(int64_t x) {
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
+}
+
 // grid = (n_tiles_max, n_kv, n_seq), NW * 64 threads, a tile of NW * 64 positions.  BITS: width of the packed keys and
 // values (a cache has one width for both).  WPE = waves per SIMD the registers are budgeted for: 4 lets two eight-wave
 // workgroups share a CU (the flash mode then spills some registers, which large grids repay); 3 is the flash mode
@@ -225,12 +340,18 @@ __device__ __forceinline__ void value_products(const u4& A, const uint32_t (&VI)
 // its SIMD to itself.
 // Centroids come from the pair tables here: a workgroup decodes 512 positions once, which does not repay building the
 // 32 KB quad table (measured: scores over 65 536 positions 10.65 us with pairs, 10.95 us with quads).
-template <int MODE, int BITS = 3, int WPE = 4, int NW = kWaves>
+// Keys go straight into registers (KeyQuarter) and F tiles of scores share a register group (flash mode, HeadLanes): one token step
+// of 32 / 8 heads at 1 500 positions, tile pass 8.3 -> 7.6 us.
+template <int MODE, int BITS = 3, int WPE = 4, int NW = kWaves, int F = 1>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   static_assert(NW == kWaves || (NW == 4 && MODE == kFlash), "the four-wave shape exists for the flash mode");
   constexpr int kThr = NW * 64, kPos = NW * kWavePos;               // threads and positions of a workgroup
+  static_assert(F == 1 || MODE == kFlash, "tiles share register groups in the flash mode");
   using VF = VField<BITS>;
+  using KQ = KeyQuarter<BITS>;
+  using Lanes = HeadLanes<F>;
+  constexpr int kGroups = Lanes::kGroups;
   constexpr int kVPd = VF::kPd;                                      // words per packed row
   constexpr bool GIVEN = MODE == kWeights || MODE == kSoftWeights;   // weights come from memory, no keys
   constexpr bool HAS_K = !GIVEN;
@@ -247,8 +368,9 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   __shared__ __align__(16) MergeLds<NW> mg_s;
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, g = lane >> 4;
+  const int head = n16 % Lanes::kStep, pos0 = Lanes::row(0, n16, g);     // of this lane's scores: head, first position of group 0
   const int tile = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
   const int n_rep = a.n_rep;
   const int n_q = a.n_kv * n_rep;
@@ -282,7 +404,8 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
     }
   }
   float my_kn = 0.0f, my_vn = 0.0f;
-  PackedBlockT<kVPd> kb_, vb_;
+  PackedBlockT<kVPd> vb_;
+  KQ kq[4];                                                           // the lane's quarters of key rows 16 t + n16, clamped into the tile
   if (HAS_V) {
     my_vn = load_stream(a.v_norms + (int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first + tile_p0 + crow);
     load_block<true>(vb_, a.v_packed + ((int64_t)seq * a.v_seq_stride + (int64_t)kvh * a.v_head_stride + first +
@@ -290,8 +413,10 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   }
   if (HAS_K) {
     my_kn = load_stream(a.k_norms + (int64_t)seq * a.kn_seq_stride + (int64_t)kvh * a.kn_head_stride + first + tile_p0 + crow);
-    load_block<HAS_V>(kb_, a.k_packed + ((int64_t)seq * a.k_seq_stride + (int64_t)kvh * a.k_head_stride + first +
-                                  tile_p0 + wrow0) * kVPd, lane, wrow0, rows_here);
+    const char* ktile = reinterpret_cast<const char*>(
+        a.k_packed + ((int64_t)seq * a.k_seq_stride + (int64_t)kvh * a.k_head_stride + first + tile_p0) * kVPd);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) kq[t].load_any(ktile, (uint32_t)min(wrow0 + 16 * t + n16, last_row) * (kVPd * 4), g);
   }
   // given weights: lane (head n16, group g) takes positions 16t + 4g + j
   float wgt[4][4];
@@ -362,19 +487,17 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   uint32_t* stage = reinterpret_cast<uint32_t*>(big_s) + wave * 1024;
 
   // ---- V: norms, table indices --------------------------------------------------------------------------
-  float vn[4][4];
+  f4 vn[kGroups];
   float inv_tscale = 1.0f, kexp = 0.0f;
   uint32_t VI[2][8];
   if (HAS_V) {
     float nmax = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float4 n4 = *reinterpret_cast<const float4*>(&vn_s[wave][16 * t + 4 * g]);
-      vn[t][0] = n4.x; vn[t][1] = n4.y; vn[t][2] = n4.z; vn[t][3] = n4.w;
-      nmax = fmaxf(nmax, fmaxf(fmaxf(n4.x, n4.y), fmaxf(n4.z, n4.w)));
+    for (int u = 0; u < kGroups; ++u) {
+      vn[u] = *reinterpret_cast<const f4*>(&vn_s[wave][16 * F * u + pos0]);
+      nmax = fmaxf(nmax, fmaxf(fmaxf(vn[u][0], vn[u][1]), fmaxf(vn[u][2], vn[u][3])));
     }
-    nmax = fmaxf(nmax, shfl_xor_f(nmax, 16));
-    nmax = fmaxf(nmax, shfl_xor_f(nmax, 32));
+    nmax = max_over_rows(Lanes::max_over_tiles(nmax));
     int ex = (int)((__float_as_uint(nmax) >> 23) & 0xFF);
     ex = ex < 27 ? (ex < 1 ? 127 : 27) : (ex > 227 ? 227 : ex);
     kexp = (float)(127 - ex);                            // weights carry 2^kexp: through the exponent (kFlash) ...
@@ -382,9 +505,7 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
     if (GIVEN) {                                         // ... or, for given weights, on the norms
       const float tscale = __uint_as_float((uint32_t)(254 - ex) << 23);
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vn[t][j] *= tscale;
+      for (int u = 0; u < kGroups; ++u) vn[u] *= tscale;
     }
 
     stage_block(vb_, stage, lane);
@@ -395,44 +516,44 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   }
 
   // ---- K: scores ----------------------------------------------------------------------------------------
-  float s[4][4];
+  typename Lanes::Group s[kGroups];
   const bool mask_vec = a.mask && ((reinterpret_cast<uintptr_t>(a.mask) & 15) == 0) && ((a.mask_seq_stride & 3) == 0) &&
                         ((a.mask_head_stride & 3) == 0);      // uniform
   if (HAS_K) {
     u4 qreg[4], qlow[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      qreg[kb] = *reinterpret_cast<const u4*>(&q_s[n16][(4 * kb + g) * 4]);
-      qlow[kb] = *reinterpret_cast<const u4*>(&ql_s[n16][(4 * kb + g) * 4]);
-    }
-    stage_block(kb_, stage, lane);                       // the V image has been consumed
-    int kw0[4], ksl[4], ksh[4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) VF::pos(4 * kb + g, kw0[kb], ksl[kb], ksh[kb]);
+      for (int jp = 0; jp < 4; ++jp) {
+        qreg[kb][jp] = q_s[n16][KQ::pair(kb, jp, g)];
+        qlow[kb][jp] = ql_s[n16][KQ::pair(kb, jp, g)];
+      }
+    }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
-      const uint32_t* krow = stage + (16 * t + n16) * kVPd;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
-        const uint32_t f = VF::field_raw(krow + kw0[kb], ksl[kb], ksh[kb]);
-        const u4 ka = key_operand<BITS, KQUAD>(f, quad_s, lutk_s);
+        const u4 ka = key_operand<BITS, KQUAD>(kq[t].field(kb, g), quad_s, lutk_s);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, qreg[kb]),
                                                      acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, qlow[kb]),
                                                      acc, 0, 0, 0);
       }
-      const float4 kn4 = *reinterpret_cast<const float4*>(&kn_s[wave][16 * t + 4 * g]);
-      const float knv[4] = {kn4.x, kn4.y, kn4.z, kn4.w};
+      Lanes::put(s, t, acc);
+    }
+#pragma unroll
+    for (int u = 0; u < kGroups; ++u) {
+      const int row0 = wrow0 + 16 * F * u + pos0;
+      const f4 kn4 = *reinterpret_cast<const f4*>(&kn_s[wave][16 * F * u + pos0]);
       float mk[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (SOFT && a.mask && n16 < n_rep)
-        load_mask4(a.mask + (int64_t)seq * a.mask_seq_stride + ((int64_t)kvh * n_rep + n16) * a.mask_head_stride + tile_p0 +
-                       wrow0 + 16 * t + 4 * g, wrow0 + 16 * t + 4 * g, rows_here, mask_vec, mk);
+      if (SOFT && a.mask && head < n_rep)
+        load_mask4(a.mask + (int64_t)seq * a.mask_seq_stride + ((int64_t)kvh * n_rep + head) * a.mask_head_stride + tile_p0 + row0, row0,
+                   rows_here, mask_vec, mk);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int row = wrow0 + 16 * t + 4 * g + j;
-        const float v = SOFT ? __builtin_fmaf(mk[j], kLog2e, acc[j] * knv[j]) : acc[j] * knv[j];
-        s[t][j] = (row < rows_here) ? v : -INFINITY;
+        const float v = SOFT ? __builtin_fmaf(mk[j], kLog2e, s[u][j] * kn4[j]) : s[u][j] * kn4[j];
+        s[u][j] = (row0 + j < rows_here) ? v : -INFINITY;
       }
     }
     if (MODE == kScores || MODE == kSoftScores) {
@@ -440,19 +561,17 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
       if (MODE == kSoftScores) {
         float m = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < kGroups; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
-        m = fmaxf(m, shfl_xor_f(m, 16));
-        m = fmaxf(m, shfl_xor_f(m, 32));
+        m = max_over_rows(m);
         const float msafe = (m == -INFINITY) ? 0.0f : m;
         float l = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < kGroups; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) l += __builtin_amdgcn_exp2f(s[t][j] - msafe);
-        l += shfl_xor_f(l, 16);
-        l += shfl_xor_f(l, 32);
+        l = sum_over_rows(l);
         if (g == 0) {
           m_s[wave][n16] = m;
           l_s[wave][n16] = l;
@@ -464,7 +583,7 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
       // 16-byte accesses both ways).
       f4* sc = reinterpret_cast<f4*>(stage);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) sc[n16 * 16 + ((4 * t + g) ^ n16)] = f4{s[t][0], s[t][1], s[t][2], s[t][3]};
+      for (int t = 0; t < kGroups; ++t) sc[n16 * 16 + ((4 * t + g) ^ n16)] = s[t];
       const int64_t row_len = (MODE == kSoftScores) ? a.w_stride : len;
       const bool vec_ok = ((row_len & 3) == 0) && ((reinterpret_cast<uintptr_t>(a.scores) & 15) == 0);   // uniform
 #pragma unroll
@@ -569,27 +688,30 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   if (MODE == kFlash) {
     m = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int u = 0; u < kGroups; ++u)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
-    m = fmaxf(m, shfl_xor_f(m, 16));
-    m = fmaxf(m, shfl_xor_f(m, 32));
+      for (int j = 0; j < 4; ++j) m = fmaxf(m, s[u][j]);
+    m = max_over_rows(Lanes::max_over_tiles(m));
   }
   const float bias = kexp - ((m == -INFINITY) ? 0.0f : m);
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
+  for (int u = 0; u < kGroups; ++u) {
     float p[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      p[j] = (MODE == kFlash) ? __builtin_amdgcn_exp2f(s[t][j] + bias) : wgt[t][j];   // kFlash: weight * 2^kexp
+      p[j] = (MODE == kFlash) ? __builtin_amdgcn_exp2f(s[u][j] + bias) : wgt[u][j];   // kFlash: weight * 2^kexp
       l += p[j];
-      p[j] *= vn[t][j];
+      p[j] *= vn[u][j];
     }
-    pa[t >> 1][2 * (t & 1)] = pack_h2(p[0], p[1]);
-    pa[t >> 1][2 * (t & 1) + 1] = pack_h2(p[2], p[3]);
+    const uint32_t lo = pack_h2(p[0], p[1]), hi = pack_h2(p[2], p[3]);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const int t = F * u + f;
+      pa[t >> 1][2 * (t & 1)] = Lanes::take(lo, f);
+      pa[t >> 1][2 * (t & 1) + 1] = Lanes::take(hi, f);
+    }
   }
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(Lanes::sum_over_tiles(l));
   if (MODE == kFlash) l *= inv_tscale;
 
   // ---- values ------------------------------------------------------------------------------------------
@@ -643,111 +765,6 @@ constexpr int kSWaves = 4;
 constexpr int kSThreads = kSWaves * 64;
 constexpr int kSStepPos = kSWaves * kWavePos;     // 256 positions per workgroup step
 constexpr int kSImageBytes = 4096;                // 209 pieces of 16 bytes, rounded up; 256 pieces at four bits
-
-// What a lane needs of a packed key row as the A operand of four score products: the words of 32 elements, read from global memory
-// as they lie and cut up in registers.  Which elements meet in a product is free as long as the query's are chosen alike, so a
-// lane's are those of whole words: elements 32 g .. 32 g + 31, and at three bits, where a row is thirteen words of ten (the last
-// of eight), the three words 3 g .. 3 g + 2 and two elements of the last.
-template <int BITS>
-struct KeyQuarter {
-  static constexpr int kPd = VField<BITS>::kPd;
-  uint32_t w[BITS == 3 ? 4 : BITS];
-  __device__ __forceinline__ void load(const char* base, uint32_t row_bytes, int g) {
-    if constexpr (BITS == 3) {
-      typedef uint32_t u3 __attribute__((ext_vector_type(3), aligned(4)));
-      const u3 x = (*reinterpret_cast<const u3*>(base + (row_bytes + 12 * g)));
-      w[0] = x[0]; w[1] = x[1]; w[2] = x[2];
-      w[3] = *reinterpret_cast<const uint32_t*>(base + (row_bytes + 48));
-    } else if constexpr (BITS == 4) {
-      const u4 x = load_stream(base + (row_bytes + 16 * g));
-      w[0] = x[0]; w[1] = x[1]; w[2] = x[2]; w[3] = x[3];
-    } else if constexpr (BITS == 2) {
-      typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-      const u2 x = __builtin_nontemporal_load(reinterpret_cast<const u2*>(base + (row_bytes + 8 * g)));
-      w[0] = x[0]; w[1] = x[1];
-    } else {
-      w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + (row_bytes + 4 * g)));
-    }
-  }
-  // the fields of the eight elements of product kb from bit 0 on; bits above them are garbage
-  __device__ __forceinline__ uint32_t field(int kb, int g) const {
-    if constexpr (BITS == 3) {
-      if (kb < 3) return w[kb];                                          // elements 0 .. 7 of a word; 8 and 9 of all make the fourth
-      return (w[0] >> 24) | ((w[1] >> 18) & 0xFC0u) | ((w[2] >> 12) & 0x3F000u) | ((w[3] >> (6 * g)) << 18);
-    } else if constexpr (BITS == 4) {
-      return w[kb];
-    } else if constexpr (BITS == 2) {
-      return w[kb >> 1] >> (16 * (kb & 1));
-    } else {
-      return w[0] >> (8 * kb);
-    }
-  }
-  // the pair of query elements (in units of two) that meets fields 2 jp and 2 jp + 1 of product kb
-  __device__ static __forceinline__ int pair(int kb, int jp, int g) {
-    if constexpr (BITS == 3) return kb < 3 ? 15 * g + 5 * kb + jp : jp < 3 ? 15 * g + 5 * jp + 4 : 60 + g;
-    else return 16 * g + 4 * kb + jp;
-  }
-};
-
-// Scores of four 16-position tiles in the lanes of 16 / F query heads.  A score product leaves head n16 in lanes n16 + 16 g, position
-// 4 g + j of the tile in register j, and with few heads most lanes hold nothing: the arithmetic on the scores would run F times
-// for one use.  So the tiles F u .. F u + F - 1 share a register group, tile F u + f in lanes n16 = 16 f / F + head (one lane shift
-// within the rows of 16 per register in, half of one per register of weights out).  What lanes past the heads hold afterwards is
-// other tiles' numbers: rows of the value products that nothing reads.
-// Four heads: 75 -> 69 us for sixteen ragged sequences (64 instead of 180 vector operations on the scores of a step); with uniform block bounds and
-// offsets that never change in the requests of whole blocks 67 - 68.
-template <int F>
-struct HeadLanes {
-  static constexpr int kGroups = 4 / F, kStep = 16 / F;
-  typedef f4 Group;
-  // first position of group u in a lane
-  __device__ static __forceinline__ int row(int u, int n16, int g) { return 16 * (F * u + n16 / kStep) + 4 * g; }
-  template <int BY>
-  __device__ static __forceinline__ float into(float old, float x) {      // lanes BY .. BY + kStep - 1 of a row of 16: x of the lanes 0 .. kStep - 1
-    constexpr int kBanks = (kStep == 4 ? 0x1 : kStep == 8 ? 0x3 : 0xF) << (BY / 4);
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), 0x110 + BY, 0xF, kBanks, false));
-  }
-  __device__ static __forceinline__ void put(Group (&s)[kGroups], int t, const f4& acc) {
-    const int u = t / F, f = t % F;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (f == 0) s[u][j] = acc[j];
-      else if constexpr (F == 2) s[u][j] = into<8>(s[u][j], acc[j]);
-      else if constexpr (F == 4) s[u][j] = f == 1 ? into<4>(s[u][j], acc[j]) : f == 2 ? into<8>(s[u][j], acc[j]) : into<12>(s[u][j], acc[j]);
-    }
-  }
-  template <int BY>
-  __device__ static __forceinline__ uint32_t from(uint32_t x) {           // lanes 0 .. kStep - 1: x of the lanes BY further
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x100 + BY, 0xF, 0xF, true);
-  }
-  __device__ static __forceinline__ uint32_t take(uint32_t x, int f) {
-    if (f == 0) return x;
-    if constexpr (F == 2) return from<8>(x);
-    else if constexpr (F == 4) return f == 1 ? from<4>(x) : f == 2 ? from<8>(x) : from<12>(x);
-    return x;
-  }
-  template <int BY>
-  __device__ static __forceinline__ float ror(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x120 + BY, 0xF, 0xF, true));
-  }
-  __device__ static __forceinline__ float max_over_tiles(float x) {
-    if constexpr (F >= 2) x = fmaxf(x, ror<8>(x));
-    if constexpr (F >= 4) x = fmaxf(x, ror<4>(x));
-    return x;
-  }
-  __device__ static __forceinline__ float sum_over_tiles(float x) {
-    if constexpr (F >= 2) x += ror<8>(x);
-    if constexpr (F >= 4) x += ror<4>(x);
-    return x;
-  }
-};
-// Tiles that share registers at n_rep query heads per kv head.
-inline int tiles_per_group(int n_rep) { return n_rep <= 4 ? 4 : n_rep <= 8 ? 2 : 1; }
-
-// a value that every lane holds alike, as one
-__device__ __forceinline__ int64_t uniform64(int64_t x) {
-  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
-}
 
 // The arguments in the kernel's argument segment, and which of the two a form reads.
 typedef const __attribute__((address_space(4))) PackedArgs ConstArgs;
@@ -1602,11 +1619,20 @@ template <int BITS>
 void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb,
                          hipStream_t stream) {
   switch (mode) {
-    case kFlash:
-      if (shape == kTilesFourWaves) packed_tile_mfma_kernel<kFlash, BITS, 2, 4><<<grid, 256, 0, stream>>>(a, kcb, vcb);
-      else if (shape == kTilesOnePerCu) packed_tile_mfma_kernel<kFlash, BITS, 3><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb);
-      else packed_tile_mfma_kernel<kFlash, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb);
+    case kFlash: {
+#define TQ_FLASH_TILES(F_)                                                                                                         \
+  do {                                                                                                                             \
+    if (shape == kTilesFourWaves) packed_tile_mfma_kernel<kFlash, BITS, 2, 4, F_><<<grid, 256, 0, stream>>>(a, kcb, vcb);          \
+    else if (shape == kTilesOnePerCu) packed_tile_mfma_kernel<kFlash, BITS, 3, kWaves, F_><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb); \
+    else packed_tile_mfma_kernel<kFlash, BITS, 4, kWaves, F_><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb);                     \
+  } while (0)
+      const int f = tiles_per_group(a.n_rep);
+      if (f == 4) TQ_FLASH_TILES(4);
+      else if (f == 2) TQ_FLASH_TILES(2);
+      else TQ_FLASH_TILES(1);
+#undef TQ_FLASH_TILES
       break;
+    }
     case kScores: packed_tile_mfma_kernel<kScores, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb); break;
     case kSoftScores: packed_tile_mfma_kernel<kSoftScores, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb); break;
     case kWeights: packed_tile_mfma_kernel<kWeights, BITS><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb); break;
