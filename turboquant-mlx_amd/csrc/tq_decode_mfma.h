@@ -333,8 +333,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
     vn[t][0] = n4.x; vn[t][1] = n4.y; vn[t][2] = n4.z; vn[t][3] = n4.w;
     nmax = fmaxf(nmax, fmaxf(fmaxf(n4.x, n4.y), fmaxf(n4.z, n4.w)));
   }
-  nmax = fmaxf(nmax, shfl_xor_f(nmax, 16));
-  nmax = fmaxf(nmax, shfl_xor_f(nmax, 32));
+  nmax = max_over_rows(nmax);
   // power-of-two scale 2^kexp, kexp = -floor(log2 nmax) (clamped to +-100): keeps P * norm inside half
   // range whatever the norms are.  It enters through the exponent of the weights (exact), not as
   // a multiplication of the norms.
@@ -437,8 +436,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
-  m = fmaxf(m, shfl_xor_f(m, 16));
-  m = fmaxf(m, shfl_xor_f(m, 32));
+  m = max_over_rows(m);
   // PLAIN: s is the raw product and attn_scale > 0 (host check), so the maximum commutes with the
   // scaling; weights = 2^(s * cs - m * cs + kexp) in one fma + v_exp_f32.
   const float arg_scale = PLAIN ? cs : 1.0f;
@@ -458,8 +456,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
     pa[t >> 1][2 * (t & 1)] = pack_h2(p[0], p[1]);
     pa[t >> 1][2 * (t & 1) + 1] = pack_h2(p[2], p[3]);
   }
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(l);
   l *= inv_tscale;
 
   // ---- values ------------------------------------------------------------------------------------------
@@ -629,16 +626,14 @@ __global__ __launch_bounds__(WAVES * 64) void vonly_scores_kernel(MfmaArgs a) {
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
-  m = fmaxf(m, shfl_xor_f(m, 16));
-  m = fmaxf(m, shfl_xor_f(m, 32));
+  m = max_over_rows(m);
   const float msafe = (m == -INFINITY) ? 0.0f : m;
   float l = 0.0f;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) l += __builtin_amdgcn_exp2f(s[t][j] - msafe);
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(l);
   if (g == 0) {
     m_s[wave][n16] = m;
     l_s[wave][n16] = l;
@@ -863,8 +858,7 @@ __device__ __forceinline__ void vonly_stream_body(const MfmaArgs& a, const Codeb
       vn[t][0] = n4.x; vn[t][1] = n4.y; vn[t][2] = n4.z; vn[t][3] = n4.w;
       nmax = fmaxf(nmax, fmaxf(fmaxf(n4.x, n4.y), fmaxf(n4.z, n4.w)));
     }
-    nmax = fmaxf(nmax, shfl_xor_f(nmax, 16));
-    nmax = fmaxf(nmax, shfl_xor_f(nmax, 32));
+    nmax = max_over_rows(nmax);
     int ex = (int)((__float_as_uint(nmax) >> 23) & 0xFF);
     ex = ex < 27 ? (ex < 1 ? 127 : 27) : (ex > 227 ? 227 : ex);
     const float kexp = (float)(127 - ex);
@@ -925,8 +919,7 @@ __device__ __forceinline__ void vonly_stream_body(const MfmaArgs& a, const Codeb
     // ---- online softmax
     float mb = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
                      fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-    mb = fmaxf(mb, shfl_xor_f(mb, 16));
-    mb = fmaxf(mb, shfl_xor_f(mb, 32));
+    mb = max_over_rows(mb);
     const float m_new = fmaxf(m_run, mb * cs);            // log2 units; attn_scale > 0 (host check)
     // RAGGED: a wave whose rows so far all lie past the end has seen nothing yet (m_new = -inf): it keeps its
     // empty state (weights 2^-inf = 0, no rescale) instead of forming -inf - -inf
@@ -979,8 +972,7 @@ __device__ __forceinline__ void vonly_stream_body(const MfmaArgs& a, const Codeb
   // ---- merge the eight waves (merge_waves): m is the running maximum, the weight sum and the accumulators carry
   // 2^kexp of the last step
   float l = l_run;
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(l);
   l *= inv_tscale;
   const int64_t grp = (int64_t)seq * a.n_kv + kvh;
   float* pS = a.ws_S + (grp * a.n_tiles_max + tile) * (int64_t)(n_rep * kD);
@@ -1179,13 +1171,11 @@ __device__ __forceinline__ void merge_rows_body(
         kidx[i] = (int)n;
         d += c * qr[i];
       }
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) d += shfl_xor_f(d, m);
+      d = wave_sum(d);
       d = (d * knrm) * inv_dim;
     } else {
       d = qx[0] * kx[0] + qx[1] * kx[1];
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) d += shfl_xor_f(d, m);
+      d = wave_sum(d);
     }
     if (lane == 0) {
       ml_s[8][0] = ok ? d * f.cs : -INFINITY;

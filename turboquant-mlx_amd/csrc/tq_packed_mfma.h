@@ -1084,8 +1084,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   // ---- merge the four waves (merge_waves): a wave deposits into its own image area.  A wave that saw no valid
   // row has m = -inf, l = 0 and zero accumulators.
   float l = l_run;
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(l);
   l = Lanes::sum_over_tiles(l);
   l *= inv_tscale;
   float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
@@ -1335,8 +1334,7 @@ void packed_stream_scores_kernel(PackedArgs a, Codebook kcb, int n_steps) {
 
   // ---- one (maximum, sum) pair per head for the workgroup's range; a wave without rows has (-inf, 0)
   float l = l_run;
-  l += shfl_xor_f(l, 16);
-  l += shfl_xor_f(l, 32);
+  l = sum_over_rows(l);
   if (g == 0) {
     m_s[wave][n16] = m_run;
     l_s[wave][n16] = l;
