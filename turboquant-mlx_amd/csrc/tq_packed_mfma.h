@@ -334,8 +334,8 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
 
 // grid = (n_tiles_max, n_kv, n_seq), NW * 64 threads, a tile of NW * 64 positions.  BITS: width of the packed keys and
 // values (a cache has one width for both).  WPE = waves per SIMD the registers are budgeted for: 4 lets two eight-wave
-// workgroups share a CU (the flash mode then spills some registers, which large grids repay); 3 is the flash mode
-// without spills, for grids that give a CU one workgroup at most.  NW = 4 (flash mode, budget of two waves per SIMD)
+// workgroups share a CU; 3 leaves the flash mode's scheduler more registers, for grids that give a CU one workgroup at most (14 000
+// positions of 32 / 8 heads 9.5 us, with the budget of 4 10.5).  NW = 4 (flash mode, budget of two waves per SIMD)
 // is for short caches whose eight-wave tiles would fill at most half of the CUs: twice the workgroups, each wave with
 // its SIMD to itself.
 // Centroids come from the pair tables here: a workgroup decodes 512 positions once, which does not repay building the
