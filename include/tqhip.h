@@ -336,15 +336,19 @@ int tq_mask_rows(const void* mask, int mask_dtype, int64_t seq_stride, int64_t h
 
 /*
  * Which tile pass tq_flash_decode takes on the matrix-core path for a batch of this shape:
- * 0 = one workgroup per 512-position tile; n >= 2 = the streaming pass, one workgroup per
- * n * 256 consecutive positions (large batches; masked != 0: a mask with a row per query head -- one that the
- * heads share counts as none).  Informational: lets a caller or a test
+ * 0 = one workgroup per 512-position tile; n >= 2 = the streaming pass, which leaves one partial per
+ * n * 256 consecutive positions of a sequence (large batches; masked != 0: a mask with a row per query head -- one that the
+ * heads share counts as none).  So the result of a sequence depends, besides its own rows and query, on what this
+ * function takes and on no other sequence's length or contents.  Informational: lets a caller or a test
  * know which kernel a shape exercises.  No counterpart in the reference (one kernel per call,
  * flash_attention.py:168-274).  The plan sees no pointers: it describes three-bit tensors (rows at any
  * 4-byte offset) and tensors of widths 1, 2 and 4 that are 16-byte aligned; tq_flash_decode sends a
  * tensor of width 1, 2 or 4 at another offset to the tile pass whatever the plan says.
  */
 int tq_flash_decode_plan(int n_seq, int n_kv_heads, int64_t max_seq_len, int ragged, int masked);
+/* The workgroups per kv head that take the partials of a streamed ragged batch without a mask in equal shares; 0: one each.
+ * Informational like the plan; the results are the same bits. */
+int tq_flash_decode_groups(int n_seq, int n_kv_heads, int64_t max_seq_len);
 
 /*
  * Decode attention for a V-only cache: fp16 keys, packed values, dense softmax (threshold 0):

@@ -1,5 +1,5 @@
-"""Ragged decode batches whose steps are cut into equal ranges over the workgroups, against the float32 kernels, which take
-one sequence after the other."""
+"""Ragged decode batches on the streaming pass, with a workgroup per partial and with the partials shared out in equal ranges of
+steps, against the float32 kernels, which take one sequence after the other."""
 import math
 
 import pytest
@@ -19,23 +19,29 @@ def tq():
 
 # lengths at the edges of a step (256 positions) and of a workgroup's share, empty sequences first, last and in a row, more
 # sequences than a wavefront has lanes, kv heads that do not divide the launch, one long sequence, a bound on the lengths far
-# above them, a launch cut down to what the workspace holds (three sequences of one kv head)
+# above them, fewer steps than workgroups; partials of two, three and four steps; last: the partials are shared out
 CASES = [
-    ([0, 0, 5000, 256, 0, 1, 4097, 20000, 255, 0], 8, 4, 0),
-    ([(i * 97) % 700 for i in range(70)] + [0, 6000], 4, 2, 0),
-    ([70001], 8, 1, 0),
-    ([16384, 8192, 512, 8191, 8193], 6, 7, 0),
-    ([43777, 3, 30000], 1, 16, 0),
-    ([300, 40, 1, 3100, 2900, 3000], 8, 4, 9341),
+    ([0, 0, 5000, 256, 0, 1, 4097, 20000, 255, 0], 8, 4, 0, True),
+    ([(i * 97) % 700 for i in range(70)] + [0, 6000], 4, 2, 0, True),
+    ([70001], 8, 1, 0, False),
+    ([16384, 8192, 512, 8191, 8193], 6, 7, 0, False),
+    ([43777, 3, 30000], 1, 16, 0, False),
+    ([300, 40, 1, 3100, 2900, 3000], 8, 4, 9341, False),
+    ([100001], 16, 1, 0, True),
+    ([max(0, 1024 * (i % 7) + i % 3 - 1) for i in range(39)] + [6259], 6, 7, 0, True),
+    ([66000, 3, 30000] + [0] * 20 + [257], 1, 16, 0, True),
+    ([4138, 768, 0, 1537, 3000, 4138, 2304, 1, 767, 769], 32, 4, 0, True),
+    ([2320] + [33 * i for i in range(69)], 8, 5, 0, True),
 ]
 
 
 @pytest.mark.parametrize("bits", [3, 1, 2, 4])
-@pytest.mark.parametrize("lens,n_kv,n_rep,bound", CASES)
-def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound):
+@pytest.mark.parametrize("lens,n_kv,n_rep,bound,shared", CASES)
+def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound, shared):
     D, n_seq, rows = 128, len(lens), sum(lens)
     longest = bound or max(lens)
     assert tq._lib.load().tq_flash_decode_plan(n_seq, n_kv, longest, 1, 0) >= 2          # a streaming launch
+    assert (tq._lib.load().tq_flash_decode_groups(n_seq, n_kv, longest) > 0) == shared
     g = torch.Generator(device="cuda")
     g.manual_seed(rows + bits)
     cb = tq.quantizer.gaussian_codebook(bits)
@@ -67,3 +73,38 @@ def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound):
             # weights enter the products as fp16, 2^-11 of the sum of |weight x value|, and the peaked head's sum is a few values, as
             # large as the row's largest result: the bar of 1e-3 + 2e-3 of the row's magnitude is four times that
             assert ((got[i] - want[0]).abs() <= 1e-3 + 2e-3 * want[0].abs().amax(-1, keepdim=True)).all(), (i, n)
+
+
+# partials of two, three and four steps, in shared-out ranges and a workgroup each; the bound on the lengths and the number of
+# sequences stay, the lengths beside one sequence change: its partials then fall to other workgroups, alone or behind others
+@pytest.mark.parametrize("n_seq,n_kv,n_rep,bound,steps,shared", [(3, 8, 4, 9000, 2, False), (70, 8, 4, 2320, 2, True),
+                                                                 (10, 32, 8, 4138, 3, True), (4, 16, 1, 40000, 4, True)])
+def test_neighbours_change_no_bit(tq, n_seq, n_kv, n_rep, bound, steps, shared):
+    D, bits = 128, 3
+    lib = tq._lib.load()
+    assert lib.tq_flash_decode_plan(n_seq, n_kv, bound, 1, 0) == steps
+    assert (lib.tq_flash_decode_groups(n_seq, n_kv, bound) > 0) == shared
+    cb = tq.quantizer.gaussian_codebook(bits)
+    bd = tq.quantizer.gaussian_boundaries(cb)
+    ks, vs = (tq.random_diagonal_sign(D, seed=s, device="cuda") for s in (42, 43))
+    own = bound - 500                                                                     # a last step of part of its rows
+    g = torch.Generator(device="cuda").manual_seed(bound)
+    x = [torch.randn((n_kv, own, D), generator=g, device="cuda") for _ in range(2)]
+    q = torch.randn((n_seq, n_kv * n_rep, D), generator=g, device="cuda")
+    first = None
+    for at, others in ((0, [bound] * (n_seq - 1)), (0, [700] * (n_seq - 1)), (n_seq - 1, [bound // 2 + 77 * i for i in range(n_seq - 1)]),
+                       (1, [0] * (n_seq - 2) + [700]), (0, [500])):
+        lens = others[:at] + [own] + others[at:]
+        if lib.tq_flash_decode_plan(len(lens), n_kv, bound, 1, 0) != steps:
+            continue                                                                      # the last one: fewer sequences, the same partials
+        sides, a = [], sum(lens[:at])
+        for s, mine in zip((ks, vs), x):
+            rows = torch.randn((n_kv, sum(lens), D), generator=g, device="cuda")
+            rows[:, a:a + own] = mine
+            p, n = tq.fused_quantize(rows.view(-1, D), s, bd, D, bits)
+            sides += [p.view(n_kv, sum(lens), -1), n.view(n_kv, sum(lens))]
+        offs = torch.tensor([0] + lens, device="cuda").cumsum(0).to(torch.int32)
+        queries = q.roll(at, 0)[:len(lens)]
+        out = tq.flash_decode_from_q(queries, ks, *sides, cb, cb, vs, D, bits, D ** -0.5, n_rep=n_rep, seq_offsets=offs, max_seq_len=bound)
+        first = out[at] if first is None else first
+        assert torch.equal(out[at], first), lens

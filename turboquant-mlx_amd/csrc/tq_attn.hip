@@ -978,8 +978,7 @@ void launch_packed_stream_bits(int bits, dim3 grid, const tqm::PackedArgs& a, co
 // per CU) about 4.2 us, and with more workgroups than that the launch runs in rounds whose set-up overlaps.
 // So: the smallest step count that brings the launch down to 256 workgroups, or the smallest that brings it
 // down to 512, whichever costs less; at most 8 steps, and at most 4 for ragged batches (true lengths
-// unknown on the host, max_seq_len is an upper bound), which keeps the tail of the launch short (ragged batches without a mask
-// only learn from this that they stream: their steps are spread evenly, see launch_packed_mfma).  Measured,
+// unknown on the host, max_seq_len is an upper bound), which keeps the tail of the launch short.  Measured,
 // one sequence of 32 / 8 heads: 24 576 positions 16.7 us with 3 steps (256 workgroups) against 17.9 with 2
 // (384) and 22.4 as single tiles; 18 432 positions 17.0 with 3 steps, 18.2 with 2, 22.0 as single tiles; 36 864
 // positions 21.7 with 3 (384 workgroups), 26.5 with 2 (576), 22.3 with 5 (232).
@@ -1012,6 +1011,16 @@ int flash_stream_steps(int n_seq, int n_kv, int64_t max_seq_len, bool ragged) {
     return best_n;
   }
   return (alone && alone * 27 <= shared * 42) ? alone : shared;
+}
+
+// Workgroups per kv head that share the pieces of a streamed ragged batch out (tq_packed_mfma.h, SPREAD), two per CU; 0: a workgroup
+// of its own per piece.  The pieces are counted from the bound on the lengths; the partials are the same bits either way.  Up to
+// three rounds of 512 workgroups a piece each is level or faster, since nothing has to be derived from the offsets and shares are
+// whole pieces too.  32 / 8 heads, three bits, call in us, shared out against a piece each: 576 pieces (8 sequences up to 9 000 positions) 38.1 / 31.5,
+// 960 (8 x 4 heads, 30 000) 38.2 / 37.8, 1 344 (12 sequences, 14 000) 44.6 / 38.8, 1 536 (64 sequences, 2 500) 44.9 / 39.2 and (24, 8 000)
+// 50.2 / 55.9, 2 048 (32 sequences, 8 000) 60.8 / 72.3, 4 096 (16 sequences, 32 768) 76.2 / 96.0.
+int flash_spread_groups(int n_seq, int n_kv, int64_t max_pieces) {
+  return (int64_t)n_seq * n_kv * max_pieces > 1536 ? std::max(1, 512 / n_kv) : 0;
 }
 
 // Matrix-core path over packed keys/values: MODE = tqm::kFlash (tq_flash_decode) or tqm::kWeights
@@ -1060,19 +1069,16 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
                          (sh.bits == 3 || (tq::aligned(k_packed, 16) && tq::aligned(v_packed, 16)));
   const int n_steps = stream_ok ? flash_stream_steps(sh.n_seq, sh.n_kv_heads, sh.seq_len,
                                                      sh.seq_offsets != nullptr || len_dev != nullptr) : 0;
-  // A ragged batch without a mask: equal ranges of the steps of all sequences (tq_packed_mfma.h, SPREAD), two workgroups per CU --
-  // as many as fit beside each other -- and as many partials as the workspace holds beside their list.
-  const int64_t spread = sh.seq_offsets && !sh.mask ? std::min<int64_t>(std::max(1, 512 / sh.n_kv_heads), (int64_t)sh.n_seq * (n_tiles - 2)) : 0;
-  if (n_steps >= 2 && spread >= 1) {
-    a.n_seq = sh.n_seq;
-    a.n_tiles_max = (int)spread + sh.n_seq;
-    a.ws_ml = a.ws_S + (size_t)a.n_tiles_max * n_q * tqm::kD;
-    a.parts = (int2*)(a.ws_ml + (size_t)a.n_tiles_max * n_q * 2);
-    launch_packed_stream_bits(sh.bits, dim3((unsigned)spread, sh.n_kv_heads), a, kcb, vcb, 0, stream);
-  } else if (n_steps >= 2) {
+  if (n_steps >= 2) {
     tile_pos = tqm::kSStepPos * n_steps;
     a.n_tiles_max = (int)((sh.seq_len + tile_pos - 1) / tile_pos);
     dim3 grid(a.n_tiles_max, sh.n_kv_heads, sh.n_seq);
+    const int groups = sh.seq_offsets && !sh.mask ? flash_spread_groups(sh.n_seq, sh.n_kv_heads, a.n_tiles_max) : 0;
+    if (groups) {
+      a.n_seq = sh.n_seq;
+      a.piece_steps = n_steps;
+      grid = dim3(groups, sh.n_kv_heads);
+    }
     launch_packed_stream_bits(sh.bits, grid, a, kcb, vcb, n_steps, stream);
   } else if (n_tiles_real > 0) {
     const int64_t wgs8 = (int64_t)n_tiles * sh.n_kv_heads * sh.n_seq;
@@ -1118,7 +1124,7 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
 #define LAUNCH_MERGE_P(TO)                                                                                    \
   tqm::decode_merge_rows_kernel<TO, MODE == tqm::kFlash><<<mgrid, tqm::kMergeThreads, 0, stream>>>(            \
       a.ws_S, a.ws_ml, sh.seq_offsets, sh.seq_len, n_parts, sh.n_kv_heads, sh.n_rep, v_signs, inv_dim, (TO*)out, tile_pos, \
-      len_dev, len_bias, a.parts)
+      len_dev, len_bias)
   if (sh.out_dtype == TQ_F16) { LAUNCH_MERGE_P(__half); }
   else if (sh.out_dtype == TQ_BF16) { LAUNCH_MERGE_P(__hip_bfloat16); }
   else { LAUNCH_MERGE_P(float); }
@@ -1521,6 +1527,11 @@ extern "C" int tq_mask_rows(const void* mask, int mask_dtype, int64_t seq_stride
 extern "C" int tq_flash_decode_plan(int n_seq, int n_kv_heads, int64_t max_seq_len, int ragged, int masked) {
   if (n_seq < 1 || n_kv_heads < 1 || max_seq_len < 0) return 0;
   return masked ? 0 : flash_stream_steps(n_seq, n_kv_heads, max_seq_len, ragged != 0);
+}
+
+extern "C" int tq_flash_decode_groups(int n_seq, int n_kv_heads, int64_t max_seq_len) {
+  const int64_t n = tq_flash_decode_plan(n_seq, n_kv_heads, max_seq_len, 1, 0);
+  return n ? flash_spread_groups(n_seq, n_kv_heads, (max_seq_len + tqm::kSStepPos * n - 1) / (tqm::kSStepPos * n)) : 0;
 }
 
 extern "C" int tq_flash_decode(const float* q_rot, const uint32_t* k_packed, const float* k_norms,

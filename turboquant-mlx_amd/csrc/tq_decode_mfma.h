@@ -1082,8 +1082,7 @@ template <typename TO, bool NORM, int U, bool FRESH>
 __device__ __forceinline__ void merge_rows_body(
     const float* __restrict__ ws_S, const float* __restrict__ ws_ml, const int32_t* __restrict__ seq_offsets,
     int64_t seq_len, int n_tiles_max, int n_kv, int n_rep, const float* __restrict__ signs, float inv_dim,
-    TO* __restrict__ out, int tile_pos, const int64_t* __restrict__ len_dev, int64_t len_bias, const FreshToken* ft,
-    const int2* __restrict__ parts) {
+    TO* __restrict__ out, int tile_pos, const int64_t* __restrict__ len_dev, int64_t len_bias, const FreshToken* ft) {
   __shared__ __align__(16) float acc_s[FRESH ? 9 : 8][kD];
   __shared__ float ml_s[FRESH ? 9 : 8][2];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1097,15 +1096,10 @@ __device__ __forceinline__ void merge_rows_body(
     const int64_t want = *len_dev + len_bias;
     len = want < 0 ? 0 : (want < len ? want : len);
   }
+  const int n_tiles = (int)((len + tile_pos - 1) / tile_pos);
   const int64_t grp = (int64_t)seq * n_kv + kvh;
-  int n_tiles = (int)((len + tile_pos - 1) / tile_pos);
-  int64_t part0 = grp * n_tiles_max;
-  if (parts) {                                           // spread streaming pass: n_tiles_max partials per kv head, the sequence's in a row
-    n_tiles = parts[seq].y;
-    part0 = (int64_t)kvh * n_tiles_max + parts[seq].x;
-  }
-  const float* gS = ws_S + part0 * (int64_t)(n_rep * kD) + r * kD + 4 * eq;
-  const float* gml = ws_ml + part0 * (int64_t)(n_rep * 2) + r * 2;
+  const float* gS = ws_S + grp * n_tiles_max * (int64_t)(n_rep * kD) + r * kD + 4 * eq;
+  const float* gml = ws_ml + grp * n_tiles_max * (int64_t)(n_rep * 2) + r * 2;
   // issued first: the signs are only needed at the very end, their latency hides behind everything else
   const float sign0 = signs[lane], sign1 = signs[lane + 64];
   bool fresh_wave = false;
@@ -1277,10 +1271,9 @@ template <typename TO, bool NORM, int U = 8>
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_rows_kernel(
     const float* __restrict__ ws_S, const float* __restrict__ ws_ml, const int32_t* __restrict__ seq_offsets,
     int64_t seq_len, int n_tiles_max, int n_kv, int n_rep, const float* __restrict__ signs, float inv_dim,
-    TO* __restrict__ out, int tile_pos, const int64_t* __restrict__ len_dev = nullptr, int64_t len_bias = 0,
-    const int2* __restrict__ parts = nullptr) {
+    TO* __restrict__ out, int tile_pos, const int64_t* __restrict__ len_dev = nullptr, int64_t len_bias = 0) {
   merge_rows_body<TO, NORM, U, false>(ws_S, ws_ml, seq_offsets, seq_len, n_tiles_max, n_kv, n_rep, signs, inv_dim, out,
-                                      tile_pos, len_dev, len_bias, nullptr, parts);
+                                      tile_pos, len_dev, len_bias, nullptr);
 }
 
 // The merge pass of a decode step that inserts its token here (see FreshToken): 320 threads.
@@ -1290,7 +1283,7 @@ __global__ __launch_bounds__(kMergeThreads + 64) void decode_merge_fresh_kernel(
     int n_rep, const float* __restrict__ signs, float inv_dim, TO* __restrict__ out, int tile_pos,
     const int64_t* __restrict__ len_dev, FreshToken ft) {
   merge_rows_body<TO, true, U, true>(ws_S, ws_ml, nullptr, seq_len, n_tiles_max, n_kv, n_rep, signs, inv_dim, out,
-                                     tile_pos, len_dev, 0, &ft, nullptr);
+                                     tile_pos, len_dev, 0, &ft);
 }
 
 // Which tile kernel a launch uses (chosen by the host from the length, the mask / offsets and the alignment).

@@ -56,7 +56,7 @@ struct PackedArgs {
   float v_unscale;            // 1 / the scale the value table was multiplied by on the host
   float threshold;            // kWeights
   int32_t n_seq;              // spread streaming pass: sequences
-  int2* parts;                //   out, per sequence: its first partial of a kv head and their number (n_tiles_max = partials per kv head)
+  int32_t piece_steps;        //   steps per partial; 0 in the other passes
 };
 
 // copy one wave's 64 packed rows of PD words each (3328 bytes at three bits) from global memory into its LDS area:
@@ -751,12 +751,17 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
 // -inf scores.  Rows of the other widths are 16, 32 or 64 bytes: every row of a 16-byte aligned
 // tensor is aligned (the host sends other tensors to the tile pass), and a block is 64, 128 or 256 pieces.
 //
-// SPREAD (ragged batches): the grid is (gridDim.x, n_kv), about two workgroups per CU, and the steps of all sequences, one after
-// the other, are cut into gridDim.x equal ranges (at least two steps each), which the workgroups derive from the offsets.  A range
-// may end one sequence and begin the next: each piece leaves a partial of its own, number (workgroup + sequence) of its kv head --
-// along the list one or the other grows by one at every cut -- and the merge pass reads from a.parts which are a sequence's.
-// Against one workgroup per four steps of a sequence, whose set-up of about 5 us then stands beside 4 x 4.2 us of steps and
-// whose number is no multiple of what the chip holds: sixteen sequences of 4K to 32K positions, 32 / 8 heads, 125.7 -> 90.1 us (the pass 113.6 -> 80.6).
+// SPREAD (ragged batches): the grid is (gridDim.x, n_kv), about two workgroups per CU.  A sequence is summed in pieces of
+// a.piece_steps steps from its own beginning, a partial each, which is what the form without SPREAD gives a workgroup: the result
+// of a sequence is the same bits whatever the lengths beside it are.  The steps of all sequences, one after the other, are cut
+// into gridDim.x equal ranges, which the workgroups derive from the offsets, and a workgroup takes the pieces that begin in its
+// range; between two pieces of a sequence it leaves the partial and goes on with the next step's rows already on their way.
+// Against one workgroup per piece, whose set-up of about 5 us then stands beside 4 x 4.2 us of steps and whose number is no
+// multiple of what the chip holds: sixteen sequences of 4K to 32K positions, 32 / 8 heads, the call 96 - 98 us with a workgroup per
+// piece, 75 - 87 this way.  (Ranges that may end inside a piece took 67 - 76, but then the lengths beside a sequence decide where
+// its partial sums end, and with that 3e-4 of its result.)
+// Workgroups 256 apart share a CU, so the second half of them takes its ranges one further: a range that ends late makes the next
+// one short, and the same range of another kv head would be as long (3 - 5 %).
 //
 // Mask: one value per position, like the norms, two steps ahead of its use, so that a step that the mask excludes for a
 // wave (left padding) neither fetches its packed rows nor computes: 8 sequences x 32 / 8 heads of 6003 positions, a quarter of
@@ -797,10 +802,11 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   __shared__ __align__(16) float alpha_s[kSWaves][kHeadsMax];
   __shared__ __align__(16) MergeLds<kSWaves> mg_s;
 
-  const int wg = blockIdx.x, kvh = blockIdx.y;
+  const int kvh = blockIdx.y;
+  const int wg = SPREAD ? (int)((blockIdx.x + blockIdx.y * gridDim.x / 256) % gridDim.x) : (int)blockIdx.x;
 
-  // n_steps steps of sequence seq from position wg_p0 on, into partial `part`
-  auto run = [&](const int seq, const int64_t wg_p0, const int n_steps, const int64_t part) __attribute__((always_inline)) {
+  // n_steps steps of sequence seq from position wg_p0 on, into partial `part` (SPREAD: and those behind it, one per piece)
+  auto run = [&](const int seq, const int64_t wg_p0, const int n_steps, int64_t part) __attribute__((always_inline)) {
   int tid = threadIdx.x;
   ConstArgs* again = (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   // Several ranges in a row: what a range derives from the lane and from the arguments is derived again for the next one. Kept in
@@ -948,6 +954,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
 #pragma unroll
   for (int et = 0; et < 8; ++et) accS[et] = f4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, R_run = -INFINITY, l_run = 0.0f, inv_tscale = 1.0f;
+  int done = 0;                                          // steps summed up since the last partial
 
   // one step on the buffers (kq, vq, kn, vn); `next()` issues the loads of the following step
   auto step = [&](int sidx, KQ (&kq)[4], u4 (&vq)[kLoads], float kn, float vn_, float mk, auto&& next) {
@@ -1045,7 +1052,7 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
       }
     }
     l_run = l_run * factor + lsum;
-    if (sidx > 0 && __any(factor != 1.0f)) {               // accumulator rows are heads 4g + j: factors through LDS
+    if (done > 0 && __any(factor != 1.0f)) {               // accumulator rows are heads 4g + j: factors through LDS
       if (g == 0) alpha_s[wave][n16] = factor;
       const float4 a4 = *reinterpret_cast<const float4*>(&alpha_s[wave][4 * g]);
       const float av[4] = {a4.x, a4.y, a4.z, a4.w};
@@ -1064,6 +1071,34 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     }
   };
 
+  // ---- merge the four waves (merge_waves): a wave deposits into its own image area.  A wave that saw no valid
+  // row has m = -inf, l = 0 and zero accumulators.
+  auto leave_partial = [&]() {
+    float l = l_run;
+    l = sum_over_rows(l);
+    l = Lanes::sum_over_tiles(l);
+    l *= inv_tscale;
+    float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
+    float* pml = a.ws_ml + part * (int64_t)(n_rep * 2);
+    static_assert(kSImageBytes >= 8 * kD * 4 && kSImageBytes % 16 == 0, "a wave's image area holds its eight deposit rows");
+    merge_waves<kSWaves>(mg_s, big_s, kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml, tid);
+  };
+  // Behind step s: a piece that another one follows.  All of its steps are whole (the sequence goes on), so no wave has stopped
+  // and all of them meet at the barriers.
+  auto end_step = [&](int s) {
+    ++done;
+    if (SPREAD && done == a.piece_steps && s + 1 < n_steps) {
+      leave_partial();
+      __syncthreads();                                     // the partial has been read from the images
+      ++part;
+      done = 0;
+      m_run = R_run = -INFINITY;
+      l_run = 0.0f;
+#pragma unroll
+      for (int et = 0; et < 8; ++et) accS[et] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+
   // Steps come in pairs so that the two register buffers keep their names; the rows of step s + 1 are requested as
   // the first thing step s does.  A wave stops at its first step without rows (steps only run out at the end of the
   // sequence).
@@ -1073,24 +1108,15 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
       issue(sidx + 1, excluded(mkB), kqB, vqB, knB, vnB);
       if (MASKED) mkA = mask_of(sidx + 2);
     });
+    end_step(sidx);
     if (sidx + 1 >= n_steps || rows_left_of(sidx + 1) <= 0) break;
     step(sidx + 1, kqB, vqB, knB, vnB, mkB, [&]() {
       issue(sidx + 2, excluded(mkA), kqA, vqA, knA, vnA);
       if (MASKED) mkB = mask_of(sidx + 3);
     });
+    end_step(sidx + 1);
   }
-
-
-  // ---- merge the four waves (merge_waves): a wave deposits into its own image area.  A wave that saw no valid
-  // row has m = -inf, l = 0 and zero accumulators.
-  float l = l_run;
-  l = sum_over_rows(l);
-  l = Lanes::sum_over_tiles(l);
-  l *= inv_tscale;
-  float* pS = a.ws_S + part * (int64_t)(n_rep * kD);
-  float* pml = a.ws_ml + part * (int64_t)(n_rep * 2);
-  static_assert(kSImageBytes >= 8 * kD * 4 && kSImageBytes % 16 == 0, "a wave's image area holds its eight deposit rows");
-  merge_waves<kSWaves>(mg_s, big_s, kSImageBytes, accS, m_run, l, inv_tscale, a.v_unscale, n_rep, pS, pml, tid);
+  leave_partial();
   };
 
   const PackedArgs& a = args;
@@ -1099,44 +1125,41 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
     const int seq = blockIdx.z;
     run(seq, (int64_t)wg * kSStepPos * max_steps, max_steps, ((int64_t)seq * a.n_kv + kvh) * a.n_tiles_max + wg);
   } else {
-    // steps of all sequences in a row: this workgroup's are at .. end - 1, `base` those of the sequences before `seq`
+    // steps of all sequences in a row: this workgroup's pieces begin at at .. end - 1, `base` is where `seq` does
     if (tid < 64) VF::fill(lutk_s, kcb, tid);
     else if (tid < 128) VF::fill(lutv_s, vcb, tid - 64);
     __syncthreads();
     if (KQUAD) VF::fill_quad(quad_s, lutk_s, tid, kSThreads);            // the first range's barrier makes it visible
-    auto steps_of = [&](int s) {
+    const int piece = a.piece_steps;
+    auto steps_of = [&](int s) {                                         // no more than there are partials for
       const int64_t len = s < a.n_seq ? (int64_t)a.seq_offsets[s + 1] - a.seq_offsets[s] : 0;
-      return len > 0 ? (int)((len + kSStepPos - 1) / kSStepPos) : 0;
+      return len > 0 ? (int)min((len + kSStepPos - 1) / kSStepPos, (int64_t)a.n_tiles_max * piece) : 0;
     };
     int total = 0;
     for (int s0 = 0; s0 < a.n_seq; s0 += 64) total += wave_total(steps_of(s0 + lane));
     total = __builtin_amdgcn_readfirstlane(total);
-    const int per = max(2, (total + (int)gridDim.x - 1) / (int)gridDim.x);
-    int at = wg * per, seq = 0, base = 0;
-    const int end = min(total, at + per);
-    const bool listing = wg == 0 && kvh == 0 && wave == 0;               // the merge pass's list of partials
-    bool found = false;
+    const int per = total / (int)gridDim.x, more = total % (int)gridDim.x;
+    const int at = wg * per + min(wg, more), end = at + per + (wg < more ? 1 : 0);
+    int seq = 0, base = 0;
     for (int s0 = 0, before = 0; s0 < a.n_seq; s0 += 64) {
       const int mine = steps_of(s0 + lane), upto = before + wave_scan(mine, lane);
-      if (listing && s0 + lane < a.n_seq)
-        a.parts[s0 + lane] = make_int2((upto - mine) / per + s0 + lane, mine > 0 ? (upto - 1) / per - (upto - mine) / per + 1 : 0);
       const uint64_t past = __ballot(upto > at);
-      if (!found && past) {
-        found = true;
+      if (past) {
         const int l = __builtin_ctzll(past);
         seq = s0 + l;
         base = __builtin_amdgcn_readlane(upto - mine, l);
+        break;
       }
       before = __builtin_amdgcn_readlane(upto, 63);
     }
     seq = __builtin_amdgcn_readfirstlane(seq);
-    while (at < end) {
-      const int have = __builtin_amdgcn_readfirstlane(steps_of(seq)), n = min(end, base + have) - at;
-      if (n > 0) {
-        run(seq, (int64_t)(at - base) * kSStepPos, n, (int64_t)kvh * a.n_tiles_max + wg + seq);
+    while (at < end && base < end) {                                      // end <= total: sequences are left
+      const int have = __builtin_amdgcn_readfirstlane(steps_of(seq));
+      const int p0 = (max(at - base, 0) + piece - 1) / piece, p1 = (min(end - base, have) + piece - 1) / piece;
+      if (p0 < p1) {
+        run(seq, (int64_t)p0 * piece * kSStepPos, min(have, p1 * piece) - p0 * piece, ((int64_t)seq * a.n_kv + kvh) * a.n_tiles_max + p0);
         __syncthreads();                                                 // the merge has read what the next range overwrites
       }
-      at += n;
       base += have;
       ++seq;
     }
@@ -1612,7 +1635,7 @@ void packed_stream_weights_kernel(PackedArgs a, Codebook vcb, int n_steps) {
 // points, 1, 2 and 4 in translation units of their own (the widths compile in parallel).
 //   launch_packed_tiles: the tile pass in `mode`; shape (flash mode): kTilesOnePerCu when the grid gives a CU one
 //     workgroup at most, kTilesFourWaves for workgroups of four waves (tiles of 256 positions)
-//   launch_packed_stream: the streaming flash pass (no mask, or one that the query heads share; a.parts set: the spread form, no mask); rows of widths other than 3 must be 16-byte aligned
+//   launch_packed_stream: the streaming flash pass (no mask, or one that the query heads share; a.piece_steps set: the spread form, no mask); rows of widths other than 3 must be 16-byte aligned
 template <int BITS>
 void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb,
                          hipStream_t stream) {
@@ -1643,7 +1666,7 @@ void launch_packed_stream(dim3 grid, const PackedArgs& a, const Codebook& kcb, c
                           hipStream_t stream) {
 #define TQ_STREAM(VQ_, F_)                                                                                             \
   do {                                                                                                                 \
-    if (a.parts) packed_stream_kernel<BITS, VQ_, false, true, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);     \
+    if (a.piece_steps) packed_stream_kernel<BITS, VQ_, false, true, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, 0);     \
     else if (a.mask) packed_stream_kernel<BITS, VQ_, true, false, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps); \
     else packed_stream_kernel<BITS, VQ_, false, false, F_><<<grid, kSThreads, 0, stream>>>(a, kcb, vcb, n_steps);      \
   } while (0)
