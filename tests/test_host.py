@@ -4,6 +4,8 @@ masks) matches the oracle.  No kernel is launched here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -401,3 +403,29 @@ def test_decode_from_the_query_refuses_what_no_entry_serves(dim, n_rep, threshol
     t = torch.zeros(1)
     with pytest.raises(ValueError, match="dim 64 without a threshold"):
         ops.flash_from_query(t, t, t, t, t, t, t, t, t, dim, 3, 0.1, n_rep=n_rep, sparse_v_threshold=threshold)
+
+
+def test_codebook_tables_outlive_no_mode():
+    """A cache's tables are real tensors of its own whatever the mode under which the package is imported, or a cache is made first."""
+    code = f"""
+import sys
+sys.path.insert(0, {os.path.dirname(os.path.dirname(os.path.abspath(_lib.__file__)))!r})
+import torch
+from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
+with FakeTensorMode():
+    import tqhip
+    from tqhip import cache
+    from tqhip.quantizer import gaussian_boundaries, gaussian_codebook
+    assert all(type(t) is FakeTensor for t in cache._tables(3))
+torch.func.functionalize(lambda x: x + cache._tables(2)[0].sum())(torch.ones(1))
+with torch.device("meta"):
+    assert cache._tables(4)[0].device.type == "meta"
+for bits in (1, 2, 3, 4):
+    c = gaussian_codebook(bits)
+    for _ in range(2):
+        got = cache._tables(bits)
+        assert all(type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in got)
+        assert torch.equal(got[0], c) and torch.equal(got[1], gaussian_boundaries(c))
+        got[0].zero_(), got[1].zero_()
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)

@@ -45,16 +45,21 @@ class _Quantizer:
         self.centroids, self.boundaries = tables if tables is not None else _tables(bits)
 
 
-# The widths' tables, never handed out: a cache's are copies of its own (2 us, against 6 for making them)
-with torch.device("cpu"):
-    _TABLE_MASTERS = {bits: (c := gaussian_codebook(bits), gaussian_boundaries(c)) for bits in (1, 2, 3, 4)}
+_TABLE_MASTERS = {}     # the widths' tables as first made outside any mode, never handed out: a cache's are copies (2 us, against 6)
 
 
 def _tables(bits):
-    if bits in _TABLE_MASTERS and torch._C._len_torch_function_stack() == 0 and torch._C._len_torch_dispatch_stack() == 0:
-        return tuple(t.clone() for t in _TABLE_MASTERS[bits])
-    centroids = gaussian_codebook(bits)                      # under a mode: whatever it makes of them (a default device, say)
-    return centroids, gaussian_boundaries(centroids)
+    """(centroids, boundaries) of a width, host tensors of the caller's own; under a mode whatever it makes of them."""
+    if torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack():
+        centroids = gaussian_codebook(bits)
+        return centroids, gaussian_boundaries(centroids)
+    if bits not in _TABLE_MASTERS:
+        centroids = gaussian_codebook(bits)
+        made = centroids, gaussian_boundaries(centroids)
+        if any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in made):
+            return made
+        _TABLE_MASTERS[bits] = made
+    return tuple(t.clone() for t in _TABLE_MASTERS[bits])
 
 
 def _round_up(n, step):
