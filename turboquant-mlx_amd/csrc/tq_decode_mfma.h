@@ -181,7 +181,22 @@ __device__ __forceinline__ void merge_waves(MergeLds<NW>& mg, unsigned char* are
 // narrow V path drop out, and K / V addresses are a uniform base plus a lane-constant offset.
 // QF32: the queries are float32 and enter as an fp16 value plus the fp16 remainder of that rounding (two
 // matrix instructions per key operand), which keeps float32-query fidelity; otherwise fp16 (or bf16) queries.
-template <bool PLAIN, bool QF32, int NW, int BITS>
+// PERMUTE: the reductions over the four lane rows go through the LDS permute instead of the vector unit's row swaps.  Shorter by a few
+// registers where the allocation needs them: see vonly_tile_mfma_kernel.
+template <bool PERMUTE>
+__device__ __forceinline__ float rows_max(float v) {
+  if constexpr (!PERMUTE) return max_over_rows(v);
+  v = fmaxf(v, shfl_xor_f(v, 16));
+  return fmaxf(v, shfl_xor_f(v, 32));
+}
+template <bool PERMUTE>
+__device__ __forceinline__ float rows_sum(float v) {
+  if constexpr (!PERMUTE) return sum_over_rows(v);
+  v += shfl_xor_f(v, 16);
+  return v + shfl_xor_f(v, 32);
+}
+
+template <bool PLAIN, bool QF32, int NW, int BITS, bool PERMUTE = false>
 __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codebook& vcb, const int64_t first,
                                                 const int64_t len) {
   using VF = VField<BITS>;
@@ -333,7 +348,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
     vn[t][0] = n4.x; vn[t][1] = n4.y; vn[t][2] = n4.z; vn[t][3] = n4.w;
     nmax = fmaxf(nmax, fmaxf(fmaxf(n4.x, n4.y), fmaxf(n4.z, n4.w)));
   }
-  nmax = max_over_rows(nmax);
+  nmax = rows_max<PERMUTE>(nmax);
   // power-of-two scale 2^kexp, kexp = -floor(log2 nmax) (clamped to +-100): keeps P * norm inside half
   // range whatever the norms are.  It enters through the exponent of the weights (exact), not as
   // a multiplication of the norms.
@@ -436,7 +451,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) m = fmaxf(m, s[t][j]);
-  m = max_over_rows(m);
+  m = rows_max<PERMUTE>(m);
   // PLAIN: s is the raw product and attn_scale > 0 (host check), so the maximum commutes with the
   // scaling; weights = 2^(s * cs - m * cs + kexp) in one fma + v_exp_f32.
   const float arg_scale = PLAIN ? cs : 1.0f;
@@ -456,7 +471,7 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
     pa[t >> 1][2 * (t & 1)] = pack_h2(p[0], p[1]);
     pa[t >> 1][2 * (t & 1) + 1] = pack_h2(p[2], p[3]);
   }
-  l = sum_over_rows(l);
+  l = rows_sum<PERMUTE>(l);
   l *= inv_tscale;
 
   // ---- values ------------------------------------------------------------------------------------------
@@ -479,6 +494,9 @@ __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codeboo
   merge_waves<NW>(mg_s, big_s, 4096, accS, m, l, inv_tscale, a.v_unscale, n_rep, pS, pml);
 }
 
+// Four-wave tiles have 168 registers.  Two forms need more and spill fewer with the LDS permute (masked three-bit tiles of fp16 queries 9 ->
+// 4, whole tiles of float32 queries 15 -> 12): a masked cache of 16 384 positions, 28 / 4 heads, 13.3 -> 12.0 us a call, float32 queries
+// over 16 384 positions 13.05 -> 12.4.  Every other form is as fast or faster with the row swaps (8 191 positions 10.4 -> 10.0).
 template <bool PLAIN, bool QF32, int NW, int BITS = 3>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 3, NW == 8 ? 2 : 3)))
 void vonly_tile_mfma_kernel(MfmaArgs a, Codebook vcb) {
@@ -490,7 +508,8 @@ void vonly_tile_mfma_kernel(MfmaArgs a, Codebook vcb) {
     const int64_t want = *a.len_dev + a.len_bias;
     len = want < 0 ? 0 : (want < len ? want : len);
   }
-  vonly_tile_body<PLAIN, QF32, NW, BITS>(a, vcb, first, len);
+  constexpr bool kPermute = NW == 4 && (PLAIN ? QF32 && BITS > 1 : !QF32 && BITS == 3);
+  vonly_tile_body<PLAIN, QF32, NW, BITS, kPermute>(a, vcb, first, len);
 }
 
 // The same pass for unmasked caches of ANY length (host-checked: no mask, no ragged offsets, positive scale,
