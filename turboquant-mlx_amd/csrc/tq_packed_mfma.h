@@ -70,20 +70,17 @@ struct PackedBlockT {
   uint32_t d[PD];
   bool wide;
 };
-using PackedBlock = PackedBlockT<kPdim>;
 
-// STREAM: streaming loads (load_stream).  They pay in the passes that decode values (given weights: 11.9 -> 11.7 us at
-// 32 768 positions) and cost where a pass only scores keys and writes as many bytes as it reads (65 536 positions:
-// 10.7 -> 11.0 us), so the score-only passes keep the default policy.
-template <bool STREAM, int PD>
+// Streaming loads (load_stream): given weights 11.9 -> 11.7 us at 32 768 positions.
+template <int PD>
 __device__ __forceinline__ void load_block(PackedBlockT<PD>& b, const uint32_t* block, int lane, int wrow0, int rows_here) {
   constexpr int kFull = PackedBlockT<PD>::kFull, kTail = PackedBlockT<PD>::kTail;
   b.wide = (wrow0 + kWavePos <= rows_here) && ((reinterpret_cast<uintptr_t>(block) & 15) == 0);
   if (b.wide) {
     const u4* b4 = reinterpret_cast<const u4*>(block);
 #pragma unroll
-    for (int i = 0; i < kFull; ++i) b.q[i] = STREAM ? load_stream(b4 + i * 64 + lane) : b4[i * 64 + lane];
-    if (kTail) b.q[kFull] = STREAM ? load_stream(b4 + kFull * 64 + (lane & (kTail - 1))) : b4[kFull * 64 + (lane & (kTail - 1))];
+    for (int i = 0; i < kFull; ++i) b.q[i] = load_stream(b4 + i * 64 + lane);
+    if (kTail) b.q[kFull] = load_stream(b4 + kFull * 64 + (lane & (kTail - 1)));
   } else {
     const int valid_words = max(0, rows_here - wrow0) * PD;
     const uint32_t* tile_base = block - (int64_t)wrow0 * PD;          // row 0 of the tile: always valid
@@ -408,7 +405,7 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   KQ kq[4];                                                           // the lane's quarters of key rows 16 t + n16, clamped into the tile
   if (HAS_V) {
     my_vn = load_stream(a.v_norms + (int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first + tile_p0 + crow);
-    load_block<true>(vb_, a.v_packed + ((int64_t)seq * a.v_seq_stride + (int64_t)kvh * a.v_head_stride + first +
+    load_block(vb_, a.v_packed + ((int64_t)seq * a.v_seq_stride + (int64_t)kvh * a.v_head_stride + first +
                                   tile_p0 + wrow0) * kVPd, lane, wrow0, rows_here);
   }
   if (HAS_K) {
@@ -577,7 +574,7 @@ void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
           l_s[wave][n16] = l;
         }
       }
-      // The wave's 64 x n_rep scores leave through its LDS area (the key image has been consumed), so that a
+      // The wave's 64 x n_rep scores leave through its LDS area (idle here: keys wait in registers), so that a
       // store instruction writes whole 256-byte runs of a head's row instead of 64 separate floats: the
       // area is [16 heads][16 units of 4 positions], the unit index xor-ed with the head (conflict-free
       // 16-byte accesses both ways).
@@ -846,9 +843,9 @@ void packed_stream_kernel(PackedArgs args, Codebook kcb, Codebook vcb, int max_s
   auto rows_left_of = [&](int s) { return min(max(wave_rows - s * kSStepPos, 0), kWavePos); };
   // Requests the rows of step s.  Every call issues the same loads whatever s is: a piece past the end of the sequence
   // is fetched from the last piece of the block that holds a valid byte, a norm past the end (and everything of a step
-  // past the workgroup's last) from the first piece / row of the workgroup's range, which exists, so that no branch
-  // surrounds a load -- the compiler can then count the requests in flight and wait for one buffer's rows while the
-  // other buffer's are still on their way.  What comes back for a row that does not exist is real data of another row:
+  // past the workgroup's last) from the first piece / row of the workgroup's range, which exists.  The one branch, on whether
+  // the block is whole, has as many loads in the same order on both sides -- the compiler can then count the requests in
+  // flight and wait for one buffer's rows while the other buffer's are still on their way.  What comes back for a row that does not exist is real data of another row:
   // finite, and its score is set to -inf.
   // Addresses are a base that is the same for the wavefront plus a 32-bit offset per lane, which for a whole block (all but a
   // sequence's last) never changes: its loads take no vector instruction at all.
@@ -1184,7 +1181,8 @@ void packed_stream_scores_kernel(PackedArgs a, Codebook kcb, int n_steps) {
   __shared__ __align__(16) unsigned char big_s[kSWaves * kSImageBytes];   // per wave: K image, then its 64 x 16 scores
   __shared__ uint32_t lutk_s[VF::kLut < 64 ? 64 : VF::kLut];
   __shared__ __align__(16) uint2 quad_s[KQUAD ? VF::kQuadEntries : 1];
-  // the rotated query (fp16 value and remainder, 8 KB) is staged in the image area: it is in registers before any image is written
+  // the rotated query (fp16 value and remainder, 8.5 KB) is staged in the image area: it is in registers before any image is written
+  static_assert(2 * kHeadsMax * kQPitch * 4 <= sizeof(big_s), "the staged query fits the images");
   uint32_t (*q_s)[kQPitch] = reinterpret_cast<uint32_t (*)[kQPitch]>(big_s);
   uint32_t (*ql_s)[kQPitch] = reinterpret_cast<uint32_t (*)[kQPitch]>(big_s + kHeadsMax * kQPitch * 4);
   __shared__ __align__(16) float kn_s[kSWaves][kWavePos];
@@ -1215,7 +1213,7 @@ void packed_stream_scores_kernel(PackedArgs a, Codebook kcb, int n_steps) {
     const int64_t left = s < n_steps ? len - p0w : 0;
     return (int)(left < 0 ? 0 : (left > kWavePos ? kWavePos : left));
   };
-  // requests as in packed_stream_kernel: the same loads whatever s is, no branch around a load
+  // requests as in packed_stream_kernel, here without the branch on whole blocks: the same loads whatever s is
   const char* k_base = krow0 + wg_p0 * (kPd * 4) - kmis;
   const float* kn_base = knrow0 + wg_p0;
   auto issue = [&](int s, u4 (&kq)[kLoads], float& kn) {
@@ -1432,7 +1430,7 @@ void packed_stream_weights_kernel(PackedArgs a, Codebook vcb, int n_steps) {
   const float* vnrow0 = a.v_norms + (int64_t)seq * a.vn_seq_stride + (int64_t)kvh * a.vn_head_stride + first;
   const int wave_rows = (int)min(len - wg_p0, (int64_t)n_steps * kSStepPos) - wave * kWavePos;
   auto rows_left_of = [&](int s) { return min(max(wave_rows - s * kSStepPos, 0), kWavePos); };
-  // Requests of a step: the same loads whatever s is, no branch around a load (see packed_stream_kernel).  The scores
+  // Requests of a step: as many loads in the same order whatever s is where the rows are aligned (see packed_stream_kernel).  The scores
   // of the lane's head (heads past n_rep: head 0) at four positions of the wave's rows come as one 16-byte
   // piece per register group (rows of `weights` are w_stride floats, a multiple of four, from a 16-byte aligned base; a row's
   // padding and the pieces of blocks past the end are read and then masked).

@@ -136,7 +136,7 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
     for (int t = 0; t < 4; ++t)
       kq[t].load_any(reinterpret_cast<const char*>(block - (int64_t)wrow0 * kPd), (uint32_t)min(wrow0 + 16 * t + n16, last_row) * (kPd * 4), g);
   } else {
-    load_block<true>(blk, block, lane, wrow0, rows_here);
+    load_block(blk, block, lane, wrow0, rows_here);
   }
   // given weights: four positions of the lane's head per group
   float wgt[kGroups][4];
@@ -278,7 +278,7 @@ void split_tile_kernel(SplitArgs a, Codebook cb) {
         l_s[wave][n16] = l;
       }
     }
-    // The wave's 64 x n_rep scores leave through its LDS area (the key image has been consumed): a store
+    // The wave's 64 x n_rep scores leave through its LDS area (idle here: keys wait in registers): a store
     // instruction then writes whole 256-byte runs of a head's row.  Area = [16 heads][16 units of 4 positions],
     // the unit index xor-ed with the head (conflict-free 16-byte accesses both ways).
     f4* sc = reinterpret_cast<f4*>(stage);
