@@ -1217,8 +1217,8 @@ def test_flash_streaming_pass_group_sizes_and_leading_offset(tq, n_kv, n_rep):
     (2, 8, 2, 9001, True),       # 288, masked: two eight-wave workgroups per CU
     (1, 2, 16, 257, False), (3, 1, 7, 256, True)])
 def test_flash_tile_pass_workgroup_shapes(tq, n_seq, n_kv, n_rep, T, masked):
-    """The three shapes of the packed tile pass in its flash mode (chosen by how many tiles the call has), each
-    against the oracle, lengths that end inside a wave's rows and one row into a tile, with and without a mask."""
+    """The packed tile pass in its flash mode with workgroups of four waves and of eight (chosen by how many tiles the call has), the
+    latter one and two to a CU, against the oracle, lengths that end inside a wave's rows and one row into a tile, with and without a mask."""
     rng = np.random.default_rng(5 * T + n_rep)
     D, bits, sc = 128, 3, 1 / math.sqrt(128)
     n_q = n_kv * n_rep

@@ -1095,8 +1095,7 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
       launch_packed_tiles_bits(sh.bits, MODE, tqm::kTilesFourWaves, grid, a, kcb, vcb, stream);
     } else {
       dim3 grid(n_tiles, sh.n_kv_heads, sh.n_seq);
-      // at most one workgroup per CU: the flash variant with registers to spare
-      launch_packed_tiles_bits(sh.bits, MODE, wgs8 <= 256 ? tqm::kTilesOnePerCu : tqm::kTilesDefault, grid, a, kcb, vcb, stream);
+      launch_packed_tiles_bits(sh.bits, MODE, tqm::kTilesDefault, grid, a, kcb, vcb, stream);
     }
   }
   TQ_CHECK_LAUNCH(who);

@@ -23,7 +23,7 @@
 namespace tqm {
 
 enum PackedMode { kFlash = 0, kScores = 1, kWeights = 2, kSoftWeights = 3, kSoftScores = 4 };
-enum PackedTileShape { kTilesDefault = 0, kTilesOnePerCu = 1, kTilesFourWaves = 2 };
+enum PackedTileShape { kTilesDefault = 0, kTilesFourWaves = 1 };
 
 struct PackedArgs {
   const float* q_rot;         // kFlash / kScores: [n_seq, n_q, 128] f32, pre-rotated; or NULL with q_raw set
@@ -330,17 +330,17 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
 }
 
 // grid = (n_tiles_max, n_kv, n_seq), NW * 64 threads, a tile of NW * 64 positions.  BITS: width of the packed keys and
-// values (a cache has one width for both).  WPE = waves per SIMD the registers are budgeted for: 4 lets two eight-wave
-// workgroups share a CU; 3 leaves the flash mode's scheduler more registers, for grids that give a CU one workgroup at most (14 000
-// positions of 32 / 8 heads 9.5 us, with the budget of 4 10.5).  NW = 4 (flash mode, budget of two waves per SIMD)
+// values (a cache has one width for both).  Two eight-wave workgroups share a CU (100 - 116 registers of the 128 that four waves per
+// SIMD have; a budget of three waves, for grids of one workgroup per CU, was level or up to 1.5 % slower at four widths and eight
+// grids).  NW = 4 (flash mode, budget of two waves per SIMD)
 // is for short caches whose eight-wave tiles would fill at most half of the CUs: twice the workgroups, each wave with
 // its SIMD to itself.
 // Centroids come from the pair tables here: a workgroup decodes 512 positions once, which does not repay building the
 // 32 KB quad table (measured: scores over 65 536 positions 10.65 us with pairs, 10.95 us with quads).
 // Keys go straight into registers (KeyQuarter) and F tiles of scores share a register group (flash mode, HeadLanes): one token step
 // of 32 / 8 heads at 1 500 positions, tile pass 8.3 -> 7.6 us.
-template <int MODE, int BITS = 3, int WPE = 4, int NW = kWaves, int F = 1>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <int MODE, int BITS = 3, int NW = kWaves, int F = 1>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == kWaves ? 4 : 2, NW == kWaves ? 4 : 2)))
 void packed_tile_mfma_kernel(PackedArgs a, Codebook kcb, Codebook vcb) {
   static_assert(NW == kWaves || (NW == 4 && MODE == kFlash), "the four-wave shape exists for the flash mode");
   constexpr int kThr = NW * 64, kPos = NW * kWavePos;               // threads and positions of a workgroup
@@ -1631,8 +1631,8 @@ void packed_stream_weights_kernel(PackedArgs a, Codebook vcb, int n_steps) {
 
 // Launchers of the kernels above for one width.  Instantiated once per width: 3 beside the host code of the entry
 // points, 1, 2 and 4 in translation units of their own (the widths compile in parallel).
-//   launch_packed_tiles: the tile pass in `mode`; shape (flash mode): kTilesOnePerCu when the grid gives a CU one
-//     workgroup at most, kTilesFourWaves for workgroups of four waves (tiles of 256 positions)
+//   launch_packed_tiles: the tile pass in `mode`; shape (flash mode): kTilesFourWaves for workgroups of four waves (tiles of 256
+//     positions)
 //   launch_packed_stream: the streaming flash pass (no mask, or one that the query heads share; a.piece_steps set: the spread form, no mask); rows of widths other than 3 must be 16-byte aligned
 template <int BITS>
 void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, const Codebook& kcb, const Codebook& vcb,
@@ -1641,9 +1641,8 @@ void launch_packed_tiles(int mode, int shape, dim3 grid, const PackedArgs& a, co
     case kFlash: {
 #define TQ_FLASH_TILES(F_)                                                                                                         \
   do {                                                                                                                             \
-    if (shape == kTilesFourWaves) packed_tile_mfma_kernel<kFlash, BITS, 2, 4, F_><<<grid, 256, 0, stream>>>(a, kcb, vcb);          \
-    else if (shape == kTilesOnePerCu) packed_tile_mfma_kernel<kFlash, BITS, 3, kWaves, F_><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb); \
-    else packed_tile_mfma_kernel<kFlash, BITS, 4, kWaves, F_><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb);                     \
+    if (shape == kTilesFourWaves) packed_tile_mfma_kernel<kFlash, BITS, 4, F_><<<grid, 256, 0, stream>>>(a, kcb, vcb);             \
+    else packed_tile_mfma_kernel<kFlash, BITS, kWaves, F_><<<grid, kMfmaThreads, 0, stream>>>(a, kcb, vcb);                        \
   } while (0)
       const int f = tiles_per_group(a.n_rep);
       if (f == 4) TQ_FLASH_TILES(4);
