@@ -974,18 +974,21 @@ void launch_packed_stream_bits(int bits, dim3 grid, const tqm::PackedArgs& a, co
 
 // Steps of 256 positions that one workgroup of the streaming flash pass runs through, or 0 for the
 // single-tile pass (at most 512 steps in all).  A step of a wave that has its SIMD to itself (at most
-// one four-wave workgroup per CU, 256 on this part) takes about 2.7 us, a step that shares it (up to two
-// per CU) about 4.2 us, and with more workgroups than that the launch runs in rounds whose set-up overlaps.
+// one four-wave workgroup per CU, 256 on this part) takes about 2.0 us, a step that shares it (up to two
+// per CU) about 2.9 us, and with more workgroups than that the launch runs in rounds whose set-up overlaps.
 // So: the smallest step count that brings the launch down to 256 workgroups, or the smallest that brings it
 // down to 512, whichever costs less; at most 8 steps, and at most 4 for ragged batches (true lengths
 // unknown on the host, max_seq_len is an upper bound), which keeps the tail of the launch short.  Measured,
-// one sequence of 32 / 8 heads: 24 576 positions 16.7 us with 3 steps (256 workgroups) against 17.9 with 2
-// (384) and 22.4 as single tiles; 18 432 positions 17.0 with 3 steps, 18.2 with 2, 22.0 as single tiles; 36 864
-// positions 21.7 with 3 (384 workgroups), 26.5 with 2 (576), 22.3 with 5 (232).
+// one sequence of 32 / 8 heads, three bits, the replayed call: 24 576 positions 17.3 us with 3 steps (256 workgroups)
+// against 17.6 with 2 (384) and 17.5 as single tiles; 36 864 positions 20.4 with 3 (384 workgroups), 25.6 with 2 (576),
+// 21.5 with 5 (232), 23.1 as tiles; 131 072 positions 35.8 with 8, 42.3 with 4, 53.4 with 2, 47.5 as tiles.  Over 34 shapes (1 - 16
+// sequences, 2 - 8 kv heads, 1 100 - 131 072 positions) the choice is within 2 % of the best of 2 - 8 steps and tiles, but for one
+// sequence of two kv heads with 131 072 positions, where four steps leave the merge pass half as many partials (21.6 against 22.9).
+// The prices in the code are from kernels whose steps took 2.7 and 4.2 us: the same ratio.
 int flash_stream_steps(int n_seq, int n_kv, int64_t max_seq_len, bool ragged) {
   const int64_t steps = (max_seq_len + tqm::kSStepPos - 1) / tqm::kSStepPos;
   const int64_t groups = (int64_t)n_seq * n_kv;
-  if (groups * steps <= 512) return 0;            // up to 256 eight-wave tiles: the tile pass is as fast (14.7 against 14.9 us)
+  if (groups * steps <= 512) return 0;            // up to 256 eight-wave tiles: the tile pass is faster (16 384 positions 13.8 us, 15.2 with 2 steps)
   const int cap = ragged ? 4 : 8;
   int alone = 0, shared = 0;                      // step counts that leave at most 256 / 512 workgroups
   for (int n = 2; n <= cap; ++n) {
@@ -995,11 +998,10 @@ int flash_stream_steps(int n_seq, int n_kv, int64_t max_seq_len, bool ragged) {
   }
   if (!shared) {
     // More than two workgroups per CU even at the cap: the launch runs in rounds of 512 workgroups.  A full round costs
-    // the steps of a workgroup at the shared rate (4.2 us each) plus a set-up of about 5 us (the stamps of the kernel; a
-    // sweep of the count over a ragged batch of 16 sequences: 116 / 117 / 108 / 108 us at 2 / 3 / 4 / 6 steps); a last round of at most 256
+    // the steps of a workgroup at the shared rate plus a set-up of about 5 us (the stamps of the kernel); a last round of at most 256
     // workgroups runs its steps at the rate of a wave that has its SIMD to itself.  The cheapest count, ties to the
-    // larger.  16 sequences x 8 kv heads x 40 steps: five steps (1024 workgroups, two full rounds) instead of eight
-    // (640: a second round that is a quarter full), 61 -> 54 us on one box.
+    // larger.  16 sequences x 8 kv heads x 40 steps: five steps (1024 workgroups, two full rounds) 47.7 us, eight
+    // (640: a second round that is a quarter full) 54.6, four 52.4, tiles 56.7.
     int best_n = cap;
     int64_t best = INT64_MAX;
     for (int n = 2; n <= cap; ++n) {
@@ -1084,7 +1086,9 @@ int launch_packed_mfma(const float* q_rot_or_weights, const uint32_t* k_packed, 
     const int64_t wgs8 = (int64_t)n_tiles * sh.n_kv_heads * sh.n_seq;
     // Short caches (the eight-wave tiles fill at most half of the CUs): workgroups of FOUR waves over tiles of 256
     // positions, so that a wave has its SIMD to itself -- a tile's time is one wave's chain of key decode, softmax and
-    // value decode, which a second wave on the SIMD stretches.  The partials of the finer tiles must fit the workspace.
+    // value decode, which a second wave on the SIMD stretches.  The partials of the finer tiles must fit the workspace.  32 / 8 heads,
+    // the replayed call, four waves against eight: 1 500 positions 10.1 / 11.4 us, 8 192 (128 tiles of eight) 11.7 / 12.5, 9 000 (144)
+    // 13.6 / 12.7.
     const int n_tiles4 = (int)((sh.seq_len + 4 * tqm::kWavePos - 1) / (4 * tqm::kWavePos));
     const size_t need4 = (size_t)sh.n_seq * n_q * n_tiles4 * (tqm::kD + 2) * sizeof(float);
     if (MODE == tqm::kFlash && wgs8 <= 128 && workspace_bytes >= need4) {
