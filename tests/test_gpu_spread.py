@@ -6,6 +6,8 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+import edge_rows  # noqa: E402
+
 pytestmark = pytest.mark.gpu
 
 
@@ -47,13 +49,21 @@ def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound, shared):
     cb = tq.quantizer.gaussian_codebook(bits)
     bd = tq.quantizer.gaussian_boundaries(cb)
     ks, vs = (tq.random_diagonal_sign(D, seed=s, device="cuda") for s in (42, 43))
+    steps = tq._lib.load().tq_flash_decode_plan(n_seq, n_kv, longest, 1, 0)
+    x = [torch.randn((n_kv, rows, D), generator=g, device="cuda") for _ in range(2)]
+    q = torch.randn((n_seq, n_kv * n_rep, D), generator=g, device="cuda")
+    first = [sum(lens[:i]) for i in range(n_seq)]
+    edges = [edge_rows.edge_positions(n, (64, 256, 256 * steps)) if n else [] for n in lens]
+    for i, n in enumerate(lens):                                                          # weight on the rows at the edges of blocks and partials
+        if n:
+            edge_rows.plant(*(t[:, first[i]:first[i] + n] for t in x), q[i], edges[i], kappa={1: 0.8, 2: 0.94}.get(bits, 1.0))
+    q[:, 0] *= 8                                                                          # a head whose maximum moves late
     sides = []
-    for s in (ks, vs):
-        p, n = tq.fused_quantize(torch.randn((n_kv * rows, D), generator=g, device="cuda"), s, bd, D, bits)
+    for s, t in zip((ks, vs), x):
+        p, n = tq.fused_quantize(t.view(-1, D), s, bd, D, bits)
         sides += [p.view(n_kv, rows, -1), n.view(n_kv, rows)]
     kp, kn, vp, vn = sides
-    q = torch.randn((n_seq, n_kv * n_rep, D), generator=g, device="cuda")
-    q[:, 0] *= 8                                                                          # a head whose maximum moves late
+    del x
     offs = torch.tensor([0] + lens, device="cuda").cumsum(0).to(torch.int32)
     sc = 1 / math.sqrt(D)
     q_rot = tq.prerotate_query(q.view(-1, D), ks).view(n_seq, -1, D)
@@ -66,13 +76,12 @@ def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound, shared):
             if n == 0:
                 assert not got[i].any()
                 continue
-            a = sum(lens[:i])
-            want = tq.flash_decode(q_rot[i:i + 1], kp[:, a:a + n], kn[:, a:a + n], vp[:, a:a + n], vn[:, a:a + n], cb, cb * other, vs,
-                                   D, bits, sc, n_rep=n_rep, seq_offsets=torch.tensor([0, n], device="cuda", dtype=torch.int32),
-                                   max_seq_len=n, precision="fp32")
-            # weights enter the products as fp16, 2^-11 of the sum of |weight x value|, and the peaked head's sum is a few values, as
-            # large as the row's largest result: the bar of 1e-3 + 2e-3 of the row's magnitude is four times that
-            assert ((got[i] - want[0]).abs() <= 1e-3 + 2e-3 * want[0].abs().amax(-1, keepdim=True)).all(), (i, n)
+            mine = [t[:, first[i]:first[i] + n] for t in (kp, kn, vp, vn)]
+            want = tq.flash_decode(q_rot[i:i + 1], *mine, cb, cb * other, vs, D, bits, sc, n_rep=n_rep,
+                                   seq_offsets=torch.tensor([0, n], device="cuda", dtype=torch.int32), max_seq_len=n, precision="fp32")
+            k, v = (tq.packed_dequantize(p.reshape(n_kv * n, -1), m.reshape(-1), c, sign, D, bits).view(n_kv, n, D)
+                    for p, m, c, sign in ((mine[0], mine[1], cb, ks), (mine[2], mine[3], cb * other, vs)))
+            edge_rows.check(got[i], want[0], q[i], k, v, sc, edges[i], edge_rows.fp16_weights_bound(v))
 
 
 # partials of two, three and four steps, in shared-out ranges and a workgroup each; the bound on the lengths and the number of
