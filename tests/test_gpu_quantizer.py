@@ -82,3 +82,24 @@ def test_boundaries_without_a_level_line_and_empty_calls(tq):
     assert idx.shape == (0, 128) and norms.shape == (0,)
     with pytest.raises(RuntimeError):
         pq.quantize(x.cpu())
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,dim", [(1, 64), (100, 64), (7, 128), (100, 128), (8200, 128), (31, 256)])
+def test_levels_of_the_other_variant(tq, bits, n, dim):
+    """Thresholds of the variant without a half-step at the boundaries: another level line, also below the row count from which
+    words come from the streaming encoder."""
+    pq = tq.PolarQuantizer(dim, bits=bits)
+    for dtype in (torch.float16, torch.float32):
+        x = _rows(n, dim, dtype, 7 * dim + n)
+        packed, norms = tq.fused_quantize(x, pq.signs, pq.boundaries, dim, bits, variant="metal")
+        idx, got_norms = tq.ops.quantize_indices(x, pq.signs, pq.boundaries, dim, bits, variant="metal")
+        assert torch.equal(idx, tq.unpack_indices(packed, bits, dim))
+        assert torch.equal(_bits_of(got_norms), _bits_of(norms))
+
+
+def test_rows_of_another_width_are_refused(tq):
+    pq = tq.PolarQuantizer(128, bits=3)
+    for shape in ((100, 64), (100, 2, 128)):
+        with pytest.raises((RuntimeError, ValueError)):
+            tq.ops.quantize_indices(torch.zeros(shape, device="cuda"), pq.signs, pq.boundaries, 128, 3)

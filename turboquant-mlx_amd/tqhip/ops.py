@@ -403,7 +403,7 @@ def fused_quantize(vectors: torch.Tensor, signs: torch.Tensor, boundaries, dim: 
 def quantize_indices(x: torch.Tensor, signs: torch.Tensor, boundaries, dim: int, bits: int, variant: str = "mlx"):
     """fused_quantize and unpack_indices of (n, dim) rows: (n, dim) uint8 levels and (n,) float32 norms, in one launch
     (tq_quantize) where it takes the call."""
-    if dim in (64, 128, 256) and x.dtype in _DTYPES and _native_pack(x):
+    if dim in (64, 128, 256) and x.dtype in _DTYPES and x.shape[1:] == (dim,) and _native_pack(x):
         rows = x.contiguous()
         signs = _as_f32_dev(signs, rows)
         n = rows.shape[0]
@@ -422,8 +422,8 @@ def quantize_indices(x: torch.Tensor, signs: torch.Tensor, boundaries, dim: int,
 def dequantize_indices(indices: torch.Tensor, norms: torch.Tensor, centroids, signs: torch.Tensor, dim: int, bits: int) -> torch.Tensor:
     """pack_indices and packed_dequantize of (n, dim) levels: (n, dim) float32, in one launch (tq_dequantize) for bytes."""
     n = indices.shape[0]
-    if (dim in (64, 128, 256) and indices.dtype == torch.uint8 and _native_pack(indices) and norms.is_cuda
-            and norms.shape[0] == n and type(norms) is torch.Tensor):
+    if (dim in (64, 128, 256) and indices.dtype == torch.uint8 and indices.shape[1:] == (dim,) and _native_pack(indices)
+            and norms.is_cuda and norms.shape == (n,) and type(norms) is torch.Tensor):
         rows = indices.contiguous()
         norms = norms.to(torch.float32).contiguous()
         signs = _as_f32_dev(signs, rows)
