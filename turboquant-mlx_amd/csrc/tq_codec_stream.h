@@ -129,10 +129,10 @@ constexpr int kEncPasses = 4;     // passes per wavefront once there are rows en
 // destination rows are consecutive.  RAGGED = true takes any row count (a prompt's length is no multiple of
 // anything): a pass takes the next kVecs rows whatever their groups, every lane derives its own vector's group once
 // per pass and the destination rows of the pass are shared through LDS; rows past the end repeat the last one and
-// and are not stored.  What it costs over the other form is a dozen instructions per 2048 elements.
+// are not stored.  What it costs over the other form is a dozen instructions per 2048 elements.
 //
 // INDICES: the levels leave as one byte each instead of packed words, `packed` standing for n_rows x D bytes without groups
-// (RAGGED).  Bound by memory like the packing form (256 bytes in, 132 out per fp16 row of 128): 100 003 rows in one launch 13.4 us
+// (RAGGED).  Bound as the packing form is (256 bytes in, 132 out per fp16 row of 128): 100 003 rows in one launch 12.4 - 13.6 us by the box,
 // against 12.7 us of encoding and 5.4 us of unpacking the words again.
 template <int D, typename T, int BITS, bool RAGGED, bool INDICES = false>
 __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, Thresholds thr, EncodeGuess gs, RowMap rm,
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(kBlock) void encode_rows_kernel(EncodeSides sides, 
 // chunks as they lie (8 bytes each, 16 kLanes bytes of a row per instruction) and looks pairs up from them.  Bytes past the width
 // mean what packing them first would give: words of the summed, shifted bytes, cut to `word_bits` (three bits: whether the two
 // bits above a word's ten fields reach the next chunk depends on the kernel that reads the words); a wavefront that meets one
-// builds the words of its pass.  100 003 rows of 128 to float32 13.6 us against 8.1 us of packing and 11.6 us of this kernel
+// builds the words of its pass.  100 003 rows of 128 to float32 13.2 - 13.6 us against 8.1 us of packing and 11.6 us of this kernel
 // on the words.
 template <int D, typename TO, int BITS, bool RAGGED, bool INDICES = false>
 __global__ __launch_bounds__(kBlock) void dequant_rows_kernel(DequantSides sides, Codebook cbk, float s, RowMap rm,
