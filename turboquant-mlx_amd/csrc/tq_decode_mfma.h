@@ -172,17 +172,6 @@ __device__ __forceinline__ void merge_waves(MergeLds<NW>& mg, unsigned char* are
   }
 }
 
-// grid = (n_tiles_max, n_kv, n_seq), NW * 64 threads: a workgroup of NW waves owns NW * 64 consecutive positions.
-// NW = 8 (one workgroup per CU) is the faster shape when the tiles of a launch fill the CUs exactly once; NW = 4
-// lets two or three workgroups share a CU, so a launch whose tile count is not a multiple of the CU count does
-// not pay a second, nearly empty round of workgroups.
-// PLAIN = no mask, no ragged offsets, seq_len a multiple of the tile, 16-byte aligned V rows (checked
-// by the host): every tile is full, so the row clamps, the validity selects, the mask reads and the
-// narrow V path drop out, and K / V addresses are a uniform base plus a lane-constant offset.
-// QF32: the queries are float32 and enter as an fp16 value plus the fp16 remainder of that rounding (two
-// matrix instructions per key operand), which keeps float32-query fidelity; otherwise fp16 (or bf16) queries.
-// PERMUTE: the reductions over the four lane rows go through the LDS permute instead of the vector unit's row swaps.  Shorter by a few
-// registers where the allocation needs them: see vonly_tile_mfma_kernel.
 template <bool PERMUTE>
 __device__ __forceinline__ float rows_max(float v) {
   if constexpr (!PERMUTE) return max_over_rows(v);
@@ -196,6 +185,17 @@ __device__ __forceinline__ float rows_sum(float v) {
   return v + shfl_xor_f(v, 32);
 }
 
+// grid = (n_tiles_max, n_kv, n_seq), NW * 64 threads: a workgroup of NW waves owns NW * 64 consecutive positions.
+// NW = 8 (one workgroup per CU) is the faster shape when the tiles of a launch fill the CUs exactly once; NW = 4
+// lets two or three workgroups share a CU, so a launch whose tile count is not a multiple of the CU count does
+// not pay a second, nearly empty round of workgroups.
+// PLAIN = no mask, no ragged offsets, seq_len a multiple of the tile, 16-byte aligned V rows (checked
+// by the host): every tile is full, so the row clamps, the validity selects, the mask reads and the
+// narrow V path drop out, and K / V addresses are a uniform base plus a lane-constant offset.
+// QF32: the queries are float32 and enter as an fp16 value plus the fp16 remainder of that rounding (two
+// matrix instructions per key operand), which keeps float32-query fidelity; otherwise fp16 (or bf16) queries.
+// PERMUTE: the reductions over the four lane rows go through the LDS permute instead of the vector unit's row swaps.  Shorter by a few
+// registers where the allocation needs them: see vonly_tile_mfma_kernel.
 template <bool PLAIN, bool QF32, int NW, int BITS, bool PERMUTE = false>
 __device__ __forceinline__ void vonly_tile_body(const MfmaArgs& a, const Codebook& vcb, const int64_t first,
                                                 const int64_t len) {
