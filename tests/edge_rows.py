@@ -24,18 +24,18 @@ def plant(k, v, q, at, kappa=1.0):
     v[:, at] *= 3
 
 
-def check(got, want, q, k, v, scale, at, bound, majority=True):
-    """|got - want| <= bound(w, smax) elementwise, and the loss of any planted row would be more than twice that in half of the heads.
+def check(got, want, q, k, v, scale, at, bound):
+    """|got - want| <= bound(w, terms) elementwise, and the loss of any planted row would be more than twice that in half of the heads.
 
-    q (n_q, d), k and v (n_kv, n, d) as the kernels see them; bound takes the weights (n_kv, n_rep, n) and the largest
-    score magnitude (n_kv, n_rep, 1) and gives (n_kv, n_rep, d)."""
+    q (n_q, d), k and v (n_kv, n, d) as the kernels see them; bound takes the weights (n_kv, n_rep, n) and the largest sum of the
+    magnitudes of a score's terms (n_kv, n_rep, 1) and gives (n_kv, n_rep, d)."""
     n_kv, n, d = k.shape
-    s = torch.matmul(q.float().view(n_kv, -1, d), k.float().transpose(1, 2).contiguous()) * scale
-    w = torch.softmax(s, -1)
-    b = bound(w, s.abs().amax(-1, keepdim=True))
+    q, kt = q.float().view(n_kv, -1, d), k.float().transpose(1, 2).contiguous()
+    w = torch.softmax(torch.matmul(q, kt) * scale, -1)
+    b = bound(w, torch.matmul(q.abs(), kt.abs()).amax(-1, keepdim=True) * scale)
     got, want = got.float().view(b.shape), want.float().view(b.shape)
     assert ((got - want).abs() <= b).all(), float(((got - want).abs() / b).max())
-    if n == 1 or not majority:
+    if n == 1:
         return
     for p in at:
         wp = w[:, :, p, None]
@@ -44,19 +44,20 @@ def check(got, want, q, k, v, scale, at, bound, majority=True):
         assert seen.float().mean() >= 0.5, (p, float(seen.float().mean()))
 
 
-def fp16_weights_bound(v, centroid_eps=2.0 ** -14):
+def fp16_weights_bound(v, bits):
     """What a pass over packed keys and values may lose whose weights enter the products as fp16.
 
     A weight times its row's norm is rounded once (2^-11), below fp16's normal range to 2^-25 of the row's largest; the
-    centroids are fp16 numbers within centroid_eps (every element of a value by that share of the row's norm at most, and every
-    score by that share of its terms: sum |q_i k_i|, bounded for Gaussian vectors by 2 / pi of d against sqrt(d) for a score of 1, hence
-    the larger of eight and the score, twice for numerator and sum)."""
+    centroids are fp16 numbers under a scale that leaves the worst of them within 2^-13.2 at four bits and 2^-15.6 below: every element
+    of a value is off by that share of the row's norm at most, and every score by that share of its terms, which moves a weight twice, in the
+    numerator and in the sum."""
+    eps = 2.0 ** (-13 if bits == 4 else -15)
     v = v.float()
     norm = v.norm(dim=-1, keepdim=True)
 
-    def bound(w, smax):
+    def bound(w, terms):
         share = torch.matmul(w, v.abs())
-        return (share * (2.0 ** -11 + 2 * centroid_eps * smax.clamp_min(8.0))
-                + torch.matmul(w, norm) * centroid_eps
+        return (share * (2.0 ** -11 + 2 * eps * terms)
+                + torch.matmul(w, norm) * eps
                 + w.amax(-1, keepdim=True) * v.shape[1] * 2.0 ** -25 * v.abs().amax())
     return bound

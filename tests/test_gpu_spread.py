@@ -81,7 +81,7 @@ def test_spread_ranges(tq, bits, lens, n_kv, n_rep, bound, shared):
                                    seq_offsets=torch.tensor([0, n], device="cuda", dtype=torch.int32), max_seq_len=n, precision="fp32")
             k, v = (tq.packed_dequantize(p.reshape(n_kv * n, -1), m.reshape(-1), c, sign, D, bits).view(n_kv, n, D)
                     for p, m, c, sign in ((mine[0], mine[1], cb, ks), (mine[2], mine[3], cb * other, vs)))
-            edge_rows.check(got[i], want[0], q[i], k, v, sc, edges[i], edge_rows.fp16_weights_bound(v))
+            edge_rows.check(got[i], want[0], q[i], k, v, sc, edges[i], edge_rows.fp16_weights_bound(v, bits))
 
 
 # partials of two, three and four steps, in shared-out ranges and a workgroup each; the bound on the lengths and the number of

@@ -45,6 +45,6 @@ def test_threshold_streams_at_every_head_count(tq, bits, n_rep, T):
         vp, vn = kv.v_packed[b, :, :T], kv.v_norms[b, :, :T]
         want = tq.sparse_v_matvec(w, vp, vn, vq.centroids, vq.signs, D, bits, threshold=thr, n_rep=n_rep, precision="fp32")
         values = tq.packed_dequantize(vp.reshape(n_kv * T, -1), vn.reshape(-1), vq.centroids, vq.signs, D, bits).view(n_kv, T, D)
-        close = edge_rows.fp16_weights_bound(values)
+        close = edge_rows.fp16_weights_bound(values, bits)
         # and two weights at the threshold may round to its other side (rows between the edges have values of one to five)
-        edge_rows.check(got[b, :, 0], want, q[b, :, 0], k[b], values, sc, edges, lambda w, smax: close(w, smax) + 2 * thr * 5)
+        edge_rows.check(got[b, :, 0], want, q[b, :, 0], k[b], values, sc, edges, lambda w, terms: close(w, terms) + 2 * thr * 5)
